@@ -1,20 +1,41 @@
-// fp32 MFMA GEMM for gfx950: C[M,N] = op(A)[M,K] * B[K,N] (+ C).
+// fp32 GEMM for gfx950: C[M,N] = op(A)[M,K] * B[K,N] (+ C).
 //
 // Replaces the cuBLAS sgemm calls of the reference (lib/blas.h:48-61): the
 // time-fused input projection x*W (lib/lstm_forward_gpu.cu.cc:340-348) and the
 // three batched backward products dW, dR, dx (lib/lstm_backward_gpu.cu.cc:374-402).
 //
-// Design: 128x128 output tile per 256-thread workgroup (4 wavefronts, each a 64x64
-// quadrant = 2x2 v_mfma_f32_32x32x2_f32 tiles), K consumed 16 at a time through a
-// double-buffered LDS stage.  Both operand tiles sit in LDS k-major, so a wavefront
-// reads the 32 consecutive floats of one k for each half of its lanes, which is the
-// operand layout of the 32x32x2 instruction and is bank-conflict free.
+// The product runs on the bf16 matrix cores, which multiply 16 times as fast as the fp32 ones,
+// without giving up precision: every float is the exact sum of three bfloat16 (8 + 8 + 8 bits
+// of significand), the products of those are exact in fp32, and of the nine the six that can
+// reach a float's 24 bits are accumulated in fp32 (Henry, Tang and Heinecke, "Leveraging the
+// bfloat16 artificial intelligence datatype for higher-precision computations", 2019).  The
+// three left out are below 2^-24 of the largest.  The five small products have an accumulator
+// of their own, so that the large one is rounded once per 16 k where the fp32 instruction
+// (32x32x2) rounds eight times.  Measured against float64, normal operands: 0.3 - 0.4 of the
+// fp32 instruction's error (2-norm, K = 75 .. 160000).  A tile in which that does not work --
+// infinities, NaNs, values within 0.4 % of the largest float, results so small that the third
+// parts fall below the smallest bfloat16 -- is computed again with the fp32 instruction.
 //
-// Work distribution: output tiles are handed out in rounds of one tile per CU for as
-// long as whole rounds remain; the tiles of the last, partial round (all tiles, when
-// there are fewer tiles than CUs: dW, dR with K = T*N) are cut along K into pieces so
-// that the pieces again fill the chip evenly.  Pieces park partial tiles; a second,
-// bandwidth-bound kernel adds the pieces of a tile in index order, so results do not
+// Design: 128x128 output tile per 256-thread workgroup (4 wavefronts, each a 64x64 quadrant =
+// 2x2 v_mfma_f32_32x32x16_bf16 tiles), K consumed 32 at a time.  A stage is read as float,
+// split in registers and put into LDS as three planes of [k / 8][row][k % 8]: an operand of
+// the instruction is then one 16-byte LDS read per lane at consecutive addresses.  Operands
+// whose rows run along the output (B, and A stored transposed) are read 8 k deep per thread,
+// so that putting 8 k side by side is a choice of registers.  Two workgroups share a CU and one
+// splits while the other multiplies; the multiplying one has the higher wave priority (3-8 %).
+// What bounds it: the bf16 matrix cores, at the clock the chip's power allows (a bare loop of
+// these MFMAs on random data reaches 1700 TFLOP/s = 283 of fp32 product, 1430 with the splitting's
+// share of vector instructions beside them).  Measured, fp32 instruction before -> now:
+// 8192^3 140 -> 199 TFLOP/s; 6400 x 2048 x 512 110 -> 148; 6400 x 512 x 2048 113 -> 153;
+// 512 x 2048 x 6400 119 -> 170 (with the kernel that adds the K pieces).
+// One accumulator instead of two leaves registers for three workgroups per CU: 213 TFLOP/s at
+// 8192^3 and 0-5 % on the other shapes, with 2.5 times the error.  256x128 tiles (8 wavefronts, two LDS
+// stages) 195; 16x16x32 instructions 197 with one accumulator.
+//
+// Work distribution: whole tiles for as long as they fill rounds of two per CU; the tiles of
+// the last, partial round (all tiles, when there are few: dW, dR with K = T*N) are cut along K
+// into pieces so that the pieces again fill the chip evenly.  Pieces park partial tiles; a
+// second, bandwidth-bound kernel adds the pieces of a tile in index order, so results do not
 // depend on scheduling.  Whole tiles are numbered so that each XCD (one L2) works on a
 // contiguous run of them; the pieces follow, dealt round-robin over the XCDs.
 #include "common.h"
@@ -33,17 +54,16 @@ constexpr int kXcds = 8;
 
 // Operand panels are read through buffer resources: a 16-byte load at any 4-byte aligned
 // offset, elements beyond the resource's range read as zero and never fault.  That keeps the
-// K loop free of branches (the compiler can then overlap the loads of the next step with the
-// MFMAs of this one); `valid` (how many of the four elements belong to the problem) is applied
-// with selects.
+// K loops free of branches (the compiler can then overlap the loads of the next step with the
+// MFMAs of this one).
 typedef unsigned int uint4_t __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_panel(const float* base, long long floats) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, (int)(floats * 4), 0x00020000);
 }
 
-// The load is issued here; `valid` is applied by masked4() when the data is used, so that
-// nothing waits for the load in between.
+// The load is issued here; `valid` (how many of the four elements belong to the problem) is
+// applied by masked4() when the data is used, so that nothing waits for the load in between.
 __device__ __forceinline__ uint4_t load4_raw(__amdgpu_buffer_rsrc_t panel, long long float_offset,
                                              int valid) {
   const unsigned int off = valid > 0 ? (unsigned int)(float_offset * 4) : 0x7ffffff0u;
@@ -59,12 +79,11 @@ __device__ __forceinline__ float4_t masked4(uint4_t u, int valid) {
   return v;
 }
 
-// One BM x 128 output tile over the K range [k_begin, k_end): BM = 128 (each wavefront a
-// 64x64 quadrant) or 64 (each a 32x64 quadrant) for outputs too small to fill the chip with
-// 128-row tiles.  part == null: the tile goes to C (+= when accumulate); otherwise the whole
-// [BM][BN] partial tile is parked at `part`.  `smem`: 2 * (BK * (BM + 4) + B_STAGE) floats.
-template <bool TRANS_A, int BM, bool INTERIOR = false>
-__device__ __forceinline__ void gemm_tile(int M, int N, int K,
+// One BM x 128 output tile over the K range [k_begin, k_end) with the fp32 instruction: what
+// split_tile() falls back on when its operands do not split.  Arguments as there; `smem`:
+// 2 * (BK * (BM + 4) + B_STAGE) floats.
+template <bool TRANS_A, int BM>
+__device__ __forceinline__ void float_tile(int M, int N, int K,
                                           const float* __restrict__ A, int lda,
                                           const float* __restrict__ B, int ldb,
                                           float* __restrict__ C, int ldc, int accumulate,
@@ -109,47 +128,20 @@ __device__ __forceinline__ void gemm_tile(int M, int N, int K,
               : make_panel(A + (size_t)m0 * lda, (long long)(rows_here - 1) * lda + K);
   const __amdgpu_buffer_rsrc_t b_panel = make_panel(B + n0, (long long)(K - 1) * ldb + cols_here);
 
-  // INTERIOR (every tile whole, K and the K pieces multiples of BK): a thread's offsets into
-  // the panels are fixed and the step enters as the instruction's scalar offset, so that a
-  // step's loads cost no vector instruction besides themselves (everything the vector units
-  // do in this loop is time the matrix units stand still).
-  unsigned int a_voff[A_PASSES], b_voff[2];
-#pragma unroll
-  for (int i = 0; i < A_PASSES; ++i)
-    a_voff[i] = TRANS_A ? (unsigned int)((((tid / TA_COLS) + TA_ROWS * i) * lda + (tid % TA_COLS) * 4) * 4)
-                        : (unsigned int)((((tid >> 2) + 64 * i) * lda + (tid & 3) * 4) * 4);
-#pragma unroll
-  for (int i = 0; i < 2; ++i) b_voff[i] = (unsigned int)((((tid >> 5) + 8 * i) * ldb + (tid & 31) * 4) * 4);
-
   auto load_global = [&](int kk) {
-    if constexpr (INTERIOR) {
-      const int a_soff = TRANS_A ? kk * lda * 4 : kk * 4;
-      const int b_soff = kk * ldb * 4;
-#pragma unroll
-      for (int i = 0; i < A_PASSES; ++i) {
-        a_valid[i] = 4;
-        a_raw[i] = __builtin_amdgcn_raw_buffer_load_b128(a_panel, a_voff[i], a_soff, 0);
-      }
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        b_valid[i] = 4;
-        b_raw[i] = __builtin_amdgcn_raw_buffer_load_b128(b_panel, b_voff[i], b_soff, 0);
-      }
-      return;
-    }
 #pragma unroll
     for (int i = 0; i < A_PASSES; ++i) {
       if (TRANS_A) {
         const int ak = (tid / TA_COLS) + TA_ROWS * i;
         const int am = (tid % TA_COLS) * 4;
         const int k = kk + ak;
-        a_valid[i] = INTERIOR ? 4 : ((k < k_end) ? (rows_here - am) : 0);
+        a_valid[i] = (k < k_end) ? (rows_here - am) : 0;
         a_raw[i] = load4_raw(a_panel, (long long)k * lda + am, a_valid[i]);
       } else {
         const int arow = (tid >> 2) + 64 * i;
         const int ak = (tid & 3) * 4;
         const int k = kk + ak;
-        a_valid[i] = INTERIOR ? 4 : ((arow < rows_here) ? (k_end - k) : 0);
+        a_valid[i] = (arow < rows_here) ? (k_end - k) : 0;
         a_raw[i] = load4_raw(a_panel, (long long)arow * lda + k, a_valid[i]);
       }
     }
@@ -158,7 +150,7 @@ __device__ __forceinline__ void gemm_tile(int M, int N, int K,
       const int bk = (tid >> 5) + 8 * i;
       const int bn = (tid & 31) * 4;
       const int k = kk + bk;
-      b_valid[i] = INTERIOR ? 4 : ((k < k_end) ? (cols_here - bn) : 0);
+      b_valid[i] = (k < k_end) ? (cols_here - bn) : 0;
       b_raw[i] = load4_raw(b_panel, (long long)k * ldb + bn, b_valid[i]);
     }
   };
@@ -274,20 +266,239 @@ __device__ __forceinline__ void gemm_tile(int M, int N, int K,
     }
 }
 
-// Runs one tile (or K piece of a tile) with the loop that fits it: whole tiles whose K range
-// is a multiple of BK need no masks (gemm_tile's INTERIOR), the tiles on the edges of a ragged
-// problem do.
-template <bool TRANS_A, int BM>
-__device__ __forceinline__ void gemm_any_tile(int M, int N, int K, const float* __restrict__ A, int lda,
-                                              const float* __restrict__ B, int ldb,
-                                              float* __restrict__ C, int ldc, int accumulate,
-                                              int tm, int tn, int k_begin, int k_end,
-                                              float* __restrict__ part, float* smem) {
-  const bool whole = M - tm * BM >= BM && N - tn * BN >= BN && (k_end - k_begin) % BK == 0;
-  if (whole)
-    gemm_tile<TRANS_A, BM, true>(M, N, K, A, lda, B, ldb, C, ldc, accumulate, tm, tn, k_begin, k_end, part, smem);
-  else
-    gemm_tile<TRANS_A, BM, false>(M, N, K, A, lda, B, ldb, C, ldc, accumulate, tm, tn, k_begin, k_end, part, smem);
+
+// ---- the product on the bf16 matrix cores ------------------------------------------------
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef float float2_t __attribute__((ext_vector_type(2)));
+
+constexpr int SK = 32;  // k of one LDS stage
+// Bytes of one group of 8 k of `rows` rows in one plane (the padding puts the groups that a
+// wavefront writes side by side on different banks), and of an operand's three planes.
+constexpr int split_group_bytes(int rows) { return rows * 16 + 64; }
+constexpr int split_operand_bytes(int rows) { return 3 * (SK / 8) * split_group_bytes(rows); }
+
+__device__ __forceinline__ unsigned int pack_bf16(float a, float b) {
+  const float2_t v = {a, b};
+  return __builtin_bit_cast(unsigned int, __builtin_convertvector(v, bf16x2_t));
+}
+
+__device__ __forceinline__ float bf16_low(unsigned int u) { return __uint_as_float(u << 16); }
+__device__ __forceinline__ float bf16_high(unsigned int u) { return __uint_as_float(u & 0xffff0000u); }
+
+// Eight consecutive k of one row, split into three bf16 each and stored into the three planes.
+__device__ __forceinline__ void split_store(const float (&f)[8], char* at, int plane_bytes) {
+  uint4_t p[3];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    float a = f[2 * j], b = f[2 * j + 1];
+    const unsigned int hi = pack_bf16(a, b);
+    a -= bf16_low(hi);
+    b -= bf16_high(hi);
+    const unsigned int mid = pack_bf16(a, b);
+    a -= bf16_low(mid);
+    b -= bf16_high(mid);
+    p[0][j] = hi;
+    p[1][j] = mid;
+    p[2][j] = pack_bf16(a, b);
+  }
+#pragma unroll
+  for (int q = 0; q < 3; ++q) *reinterpret_cast<uint4_t*>(at + q * plane_bytes) = p[q];
+}
+
+// A bfloat16 cannot hold what lies below 2^-133.  When everything a wavefront computed is smaller
+// than this, that may be visible (the loss is at most 2^-134 per operand element): 2^-90 leaves
+// it below a float's rounding for partners up to 2^7 and K up to 2^13.
+constexpr float kTinyTile = 0x1p-90f;
+
+// One BM x 128 output tile, BM = 64 * MI, over the K range [k_begin, k_end): MI = 2 (each
+// wavefront a 64x64 quadrant) or 1 (each a 32x64 quadrant) for outputs of at most 64 rows.
+// k_begin is a multiple of SK, k_end too unless it is K.  part == null: the tile goes to C
+// (+= when accumulate); otherwise the whole [BM][BN] partial tile is parked at `part` (columns
+// and rows beyond the problem hold nothing of use).
+// `smem`: split_operand_bytes(BM) + split_operand_bytes(BN) bytes.
+template <bool TRANS_A, int MI>
+__device__ __forceinline__ void split_tile(int M, int N, int K, const float* __restrict__ A, int lda,
+                                           const float* __restrict__ B, int ldb, float* __restrict__ C,
+                                           int ldc, int accumulate, int tm, int tn, int k_begin, int k_end,
+                                           float* __restrict__ part, char* smem) {
+  constexpr int BM = 64 * MI;
+  constexpr int WM = 32 * MI;
+  constexpr int A_GROUP = split_group_bytes(BM), B_GROUP = split_group_bytes(BN);
+  constexpr int A_PLANE = (SK / 8) * A_GROUP, B_PLANE = (SK / 8) * B_GROUP;
+  char* As = smem;
+  char* Bs = smem + split_operand_bytes(BM);
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wr = wave >> 1, wc = wave & 1;
+
+  const int rows_here = (M - m0) < BM ? (M - m0) : BM;
+  const int cols_here = (N - n0) < BN ? (N - n0) : BN;
+  const __amdgpu_buffer_rsrc_t a_panel =
+      TRANS_A ? make_panel(A + m0, (long long)(K - 1) * lda + rows_here)
+              : make_panel(A + (size_t)m0 * lda, (long long)(rows_here - 1) * lda + K);
+  const __amdgpu_buffer_rsrc_t b_panel = make_panel(B + n0, (long long)(K - 1) * ldb + cols_here);
+
+  float16_t acc[MI][2], low[MI][2];  // the products of the first parts; the five smaller ones
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = low[i][j][e] = 0.f;
+
+  // A thread's share of a stage: 8 consecutive k of MI rows of A and 2 columns of B.  Rows, columns
+  // and k beyond the problem read as zero or as what lies there, which reaches only outputs
+  // that nobody keeps -- except k beyond the end of a row of A, masked in store_lds().
+  // Where the rows run along the output, a wavefront takes 8 k of all of them, a lane MI (2)
+  // neighbours, and neighbour i goes to MFMA tile i: writes to LDS stay consecutive, and a lane
+  // ends up with two neighbouring columns of C.
+  float a_raw[MI][8], b_raw[2][8];
+  auto load_global = [&](int kk) {
+    if constexpr (TRANS_A) {
+      const unsigned int base = ((unsigned)(kk + 8 * wave) * (unsigned)lda + (unsigned)(lane * MI)) * 4u;
+#pragma unroll
+      for (int r = 0; r < 8; ++r) {
+        const unsigned int off = base + (unsigned)(r * lda) * 4u;
+        if constexpr (MI == 2) {
+          const auto u = __builtin_amdgcn_raw_buffer_load_b64(a_panel, off, 0, 0);
+          a_raw[0][r] = __uint_as_float(u[0]);
+          a_raw[1][r] = __uint_as_float(u[1]);
+        } else {
+          a_raw[0][r] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(a_panel, off, 0, 0));
+        }
+      }
+    } else {
+      const unsigned int base = ((unsigned)(tid >> 2) * (unsigned)lda + (unsigned)(kk + 8 * (tid & 3))) * 4u;
+#pragma unroll
+      for (int i = 0; i < MI; ++i) {
+        const unsigned int off = base + (unsigned)(64 * i * lda) * 4u;
+        const uint4_t u = __builtin_amdgcn_raw_buffer_load_b128(a_panel, off, 0, 0);
+        const uint4_t w = __builtin_amdgcn_raw_buffer_load_b128(a_panel, off + 16u, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          a_raw[i][e] = __uint_as_float(u[e]);
+          a_raw[i][4 + e] = __uint_as_float(w[e]);
+        }
+      }
+    }
+    const unsigned int base = ((unsigned)(kk + 8 * wave) * (unsigned)ldb + (unsigned)(lane * 2)) * 4u;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      const auto u = __builtin_amdgcn_raw_buffer_load_b64(b_panel, base + (unsigned)(r * ldb) * 4u, 0, 0);
+      b_raw[0][r] = __uint_as_float(u[0]);
+      b_raw[1][r] = __uint_as_float(u[1]);
+    }
+  };
+
+  auto store_lds = [&](int kk) {
+    if constexpr (TRANS_A) {
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+        split_store(a_raw[i], As + wave * A_GROUP + ((lane >> 5) * WM + 32 * i + (lane & 31)) * 16, A_PLANE);
+    } else {
+      if (kk + SK > k_end) {  // the last stage of a ragged K: what follows a row is another row
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) a_raw[i][e] = kk + 8 * (tid & 3) + e < k_end ? a_raw[i][e] : 0.f;
+      }
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+        split_store(a_raw[i], As + (tid & 3) * A_GROUP + ((tid >> 2) + 64 * i) * 16, A_PLANE);
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      split_store(b_raw[j], Bs + wave * B_GROUP + ((lane >> 5) * 64 + 32 * j + (lane & 31)) * 16, B_PLANE);
+  };
+
+  auto fragment = [&](const char* at) { return *reinterpret_cast<const bf16x8_t*>(at); };
+  auto compute = [&]() {
+    const char* as = As + (lane >> 5) * A_GROUP + (wr * WM + (lane & 31)) * 16;
+    const char* bs = Bs + (lane >> 5) * B_GROUP + (wc * 64 + (lane & 31)) * 16;
+#pragma unroll
+    for (int s = 0; s < SK / 16; ++s) {
+      bf16x8_t b[2][3];
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int q = 0; q < 3; ++q) b[j][q] = fragment(bs + q * B_PLANE + 2 * s * B_GROUP + 32 * 16 * j);
+#pragma unroll
+      for (int i = 0; i < MI; ++i) {
+        bf16x8_t a[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) a[q] = fragment(as + q * A_PLANE + 2 * s * A_GROUP + 32 * 16 * i);
+          // the smallest partial products first
+        constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+        for (int p = 0; p < 6; ++p)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            float16_t& to = p < 5 ? low[i][j] : acc[i][j];
+            to = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[pa[p]], b[j][pb[p]], to, 0, 0, 0);
+          }
+      }
+    }
+  };
+
+  load_global(k_begin);
+  for (int kk = k_begin; kk < k_end; kk += SK) {
+    store_lds(kk);
+    __syncthreads();
+    if (kk + SK < k_end) load_global(kk + SK);
+    __builtin_amdgcn_s_setprio(1);
+    compute();
+    __builtin_amdgcn_s_setprio(0);
+    __syncthreads();
+  }
+
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] += low[i][j];
+  // An operand that is not finite, or rounds to infinity as a bfloat16, gives NaNs here, and parts
+  // below the smallest bfloat16 are lost: such tiles are computed again on the float matrix cores.
+  float finite = 0.f, largest = 0.f;
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        finite = fmaf(acc[i][j][e], 0.f, finite);
+        largest = fmaxf(largest, fabsf(acc[i][j][e]));
+      }
+  const bool tiny = __all(largest < kTinyTile) && __any(largest > 0.f);
+  if (__syncthreads_or(!(finite == 0.f) || tiny)) {
+    float_tile<TRANS_A, BM>(M, N, K, A, lda, B, ldb, C, ldc, accumulate, tm, tn, k_begin, k_end, part,
+                           reinterpret_cast<float*>(smem));
+    return;
+  }
+
+  const int col = wc * 64 + 2 * (lane & 31);
+  // Whole tiles with 8-byte aligned rows: a lane's two columns in one store.
+  const bool wide = cols_here == BN && (ldc & 1) == 0 && (reinterpret_cast<uintptr_t>(C) & 7) == 0;
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int q = 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
+      const int row = TRANS_A ? wr * WM + MI * q + i : wr * WM + 32 * i + q;
+      if (part != nullptr) {
+        const float2_t v = {acc[i][0][e], acc[i][1][e]};
+        *reinterpret_cast<float2_t*>(part + row * BN + col) = v;
+      } else if (row < rows_here) {
+        float* p = C + (size_t)(m0 + row) * ldc + n0 + col;
+        if (wide) {
+          float2_t v = {acc[i][0][e], acc[i][1][e]};
+          if (accumulate) v += *reinterpret_cast<const float2_t*>(p);
+          *reinterpret_cast<float2_t*>(p) = v;
+          continue;
+        }
+        if (col < cols_here) p[0] = accumulate ? p[0] + acc[i][0][e] : acc[i][0][e];
+        if (col + 1 < cols_here) p[1] = accumulate ? p[1] + acc[i][1][e] : acc[i][1][e];
+      }
+    }
 }
 
 template <bool TRANS_A, int BM>
@@ -298,7 +509,7 @@ void gemm_f32_kernel(int M, int N, int K,
                      float* __restrict__ C, int ldc, int accumulate,
                      int tiles_n, int whole_tiles, int splits, int k_per_split,
                      float* __restrict__ partial) {
-  __shared__ __attribute__((aligned(16))) float smem[2 * BK * (BM + 4) + 2 * B_STAGE];
+  __shared__ __attribute__((aligned(16))) float smem[(split_operand_bytes(BM) + split_operand_bytes(BN)) / 4];
   // Workgroups [0, whole_tiles) compute one whole tile each.  Ids are handed to the XCDs
   // round-robin; XCD x gets the x-th contiguous chunk of the tile list so that neighbours
   // in the list share an L2.  Workgroups from whole_tiles on compute one K piece of one of
@@ -344,8 +555,8 @@ void gemm_f32_kernel(int M, int N, int K,
     k_end = (k_begin + k_per_split < K) ? (k_begin + k_per_split) : K;
     part = partial + ((size_t)t * splits + split) * BM * BN;
   }
-  gemm_any_tile<TRANS_A, BM>(M, N, K, A, lda, B, ldb, C, ldc, accumulate, tile / tiles_n, tile % tiles_n,
-                             k_begin, k_end, part, smem);
+  split_tile<TRANS_A, BM / 64>(M, N, K, A, lda, B, ldb, C, ldc, accumulate, tile / tiles_n, tile % tiles_n,
+                             k_begin, k_end, part, reinterpret_cast<char*>(smem));
 }
 
 // Two products with the same N and K in one launch (dW = x^T dv and dR = h^T dv of a backward
@@ -364,7 +575,7 @@ struct GemmPair {
 template <int BM>
 __global__ __launch_bounds__(256, 2)
 void gemm_f32_pair_kernel(GemmPair p) {
-  __shared__ __attribute__((aligned(16))) float smem[2 * BK * (BM + 4) + 2 * B_STAGE];
+  __shared__ __attribute__((aligned(16))) float smem[(split_operand_bytes(BM) + split_operand_bytes(BN)) / 4];
   const int j = blockIdx.x;
   const int tile = j / p.splits;
   const int k_begin = (j % p.splits) * p.k_per_split;
@@ -372,11 +583,11 @@ void gemm_f32_pair_kernel(GemmPair p) {
   float* part = p.splits > 1 ? p.partial + (size_t)j * BM * BN : nullptr;
   const int tm = tile / p.tiles_n, tn = tile % p.tiles_n;
   if (tm < p.tiles_m1)
-    gemm_any_tile<false, BM>(p.M1, p.N, p.K, p.A1, p.lda1, p.B1, p.ldb1, p.C1, p.ldc1, p.accumulate,
-                             tm, tn, k_begin, k_end, part, smem);
+    split_tile<false, BM / 64>(p.M1, p.N, p.K, p.A1, p.lda1, p.B1, p.ldb1, p.C1, p.ldc1, p.accumulate,
+                             tm, tn, k_begin, k_end, part, reinterpret_cast<char*>(smem));
   else
-    gemm_any_tile<true, BM>(p.M2, p.N, p.K, p.A2, p.lda2, p.B2, p.ldb2, p.C2, p.ldc2, p.accumulate,
-                            tm - p.tiles_m1, tn, k_begin, k_end, part, smem);
+    split_tile<true, BM / 64>(p.M2, p.N, p.K, p.A2, p.lda2, p.B2, p.ldb2, p.C2, p.ldc2, p.accumulate,
+                            tm - p.tiles_m1, tn, k_begin, k_end, part, reinterpret_cast<char*>(smem));
 }
 
 // For the split tiles (tile index whole_tiles + blockIdx.x): C tile (+)= sum over its
@@ -448,6 +659,19 @@ struct GemmPlan {
   size_t scratch_bytes;
 };
 
+// What `tiles` tiles cut into s pieces each cost, in units of what one CU needs for a whole tile
+// while two workgroups share it (41 ns * K).  A piece costs as much as 48 k more (its first
+// loads, its write-out); workgroups run in rounds of two per CU, and a round of at most one
+// per CU takes three quarters of a full one; the partial tiles cost 128 KiB of traffic a piece
+// at 4.5 TB/s, the kernel that adds them up 3 us.
+double list_cost(long long tiles, int s, int K, int cus) {
+  const long long pieces = tiles * s, slots = 2LL * cus, left = pieces % slots;
+  const double rounds = (double)(pieces / slots) + (left == 0 ? 0.0 : left <= cus ? 0.75 : 1.0);
+  double c = 2.0 * rounds * (1.0 / s + 48.0 / K);
+  if (s > 1) c += (0.71 * (double)pieces + 73.0) / K;
+  return c;
+}
+
 GemmPlan plan_gemm(int M, int N, int K) {
   GemmPlan g;
   g.tiles_n = (N + BN - 1) / BN;
@@ -458,37 +682,28 @@ GemmPlan plan_gemm(int M, int N, int K) {
   const int tiles_m = (M + g.bm - 1) / g.bm;
   const long long tiles = (long long)tiles_m * g.tiles_n;
 
-  // Whole rounds of one tile per CU run unsplit; the `rest` tiles of the last round are each
-  // cut into `splits` K pieces.  In units of the time one CU needs for one whole tile, s
-  // pieces per tile cost ceil(rest*s/CUs)/s for the arithmetic plus 0.25*rest*s/K for
-  // writing and re-reading the partial tiles (128 KiB per piece at the chip's memory rate
-  // against 2*128*128*K flops at one CU's MFMA rate); a launch that consists of fewer than
-  // two pieces per CU pays 20 % more (a lone workgroup cannot hide its own load latency;
-  // measured 5-9 % between 1 and 2 pieces per CU at 128 x 8192 x 2048 with the traffic term).
-  // The cheapest s is taken, a piece keeping at least 64 of K.  The choice depends on the
-  // shape only, so results are reproducible.
-  const long long whole = tiles >= cus ? tiles / cus * cus : 0;
-  g.rest = (int)(tiles - whole);
+  // Either all tiles whole, or whole tiles for full rounds of two per CU and the `rest` cut
+  // into the cheapest number of K pieces; the choice depends on the shape only, so results are
+  // reproducible.  (Measured, us: 6400 x 512 x 2048, 200 tiles, in 1 / 2 / 4 / 5 pieces 122 / 84 /
+  // 91 / 87; 512 x 8192 x 3200, 256 tiles, in 1 / 2 / 4: 190 / 143 / 154; 12800 x 2048 x 512, 1600
+  // tiles, whole 162, the last 64 in 4 pieces 150; 6400 x 2048 x 512, 800 tiles, whole 82, the
+  // last 32 in 4 pieces 85.)
+  const long long whole = tiles / (2 * cus) * (2 * cus);
   int splits = 1;
+  g.rest = (int)(tiles - whole);
   if (g.rest > 0) {
-    const int k_iters = (K + BK - 1) / BK;
-    int s_max = k_iters / 4;
+    int s_max = K / 64;
     if (s_max > 64) s_max = 64;
-    auto cost = [&](int s) {
-      const long long pieces = (long long)g.rest * s;
-      double c = (double)((pieces + cus - 1) / cus) / s;
-      if (whole == 0 && pieces < 2LL * cus) c *= 1.2;
-      if (s > 1) c += 0.25 * (double)g.rest * s / K;
-      return c;
-    };
+    double best = list_cost(tiles, 1, K, cus) - list_cost(whole, 1, K, cus);
     // At most four pieces per CU: that bounds the partial tiles of any product (64 KiB a
     // piece) by a size callers who lend the library its scratch memory can plan for.
-    double best = cost(1);
-    for (int s = 2; s <= s_max && (long long)g.rest * s <= 4LL * cus; ++s)
-      if (cost(s) < best - 1e-9) { best = cost(s); splits = s; }
+    for (int s = 2; s <= s_max && (long long)g.rest * s <= 4LL * cus; ++s) {
+      const double c = list_cost(g.rest, s, K, cus);
+      if (c < best - 1e-9) { best = c; splits = s; }
+    }
   }
   g.k_per_split = (K + splits - 1) / splits;
-  g.k_per_split = (g.k_per_split + BK - 1) / BK * BK;
+  g.k_per_split = (g.k_per_split + SK - 1) / SK * SK;
   g.splits = (K + g.k_per_split - 1) / g.k_per_split;
   const bool split = g.splits > 1;
   // Unsplit "rest" tiles are ordinary whole tiles.
@@ -620,23 +835,14 @@ int gemm_f32_pair(hipStream_t stream, int M1, int M2, int N, int K, const float*
     HASTE_HIP_PROPAGATE(gemm_f32(stream, false, M1, N, K, A1, lda1, B1, ldb1, C1, ldc1, accumulate));
     return gemm_f32(stream, true, M2, N, K, A2, lda2, B2, ldb2, C2, ldc2, accumulate);
   }
-  // The cost model of plan_gemm for a list in which every tile is cut.
-  const int k_iters = (K + BK - 1) / BK;
-  int s_max = k_iters / 4;
+  int s_max = K / 64;
   if (s_max > 64) s_max = 64;
-  auto cost = [&](int s) {
-    const long long pieces = tiles * s;
-    double c = (double)((pieces + cus - 1) / cus) / s;
-    if (pieces < 2LL * cus) c *= 1.2;
-    if (s > 1) c += 0.25 * (double)tiles * s / K;
-    return c;
-  };
   int splits = 1;
-  double best = cost(1);
+  double best = list_cost(tiles, 1, K, cus);
   for (int s = 2; s <= s_max && tiles * s <= 4LL * cus; ++s)
-    if (cost(s) < best - 1e-9) { best = cost(s); splits = s; }
+    if (list_cost(tiles, s, K, cus) < best - 1e-9) { best = list_cost(tiles, s, K, cus); splits = s; }
   int k_per_split = (K + splits - 1) / splits;
-  k_per_split = (k_per_split + BK - 1) / BK * BK;
+  k_per_split = (k_per_split + SK - 1) / SK * SK;
   splits = (K + k_per_split - 1) / k_per_split;
 
   GemmPair p;

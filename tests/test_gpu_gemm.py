@@ -124,3 +124,73 @@ def test_gemm_operand_of_more_than_2_gib(trans_a):
         ref += a_slab @ b[k0:k0 + step].double()
     err = float((out.double() - ref).abs().max() / ref.abs().max())
     assert err < 1e-5, err
+
+
+def _bound(a64, b64, K):
+    """What fp32 accumulation of exact products can be off by, element by element: one rounding
+    (at most 2^-23: the matrix unit may truncate) per 16 k of the sum of the large partial
+    products, 5 of the small ones, which are 2^-8 of them, and one each for adding the two sums
+    and up to 64 K pieces; the partial products left out are 2^-24."""
+    return (K / 16 * (1 + 5 / 256) + 66) * 2.0 ** -23 * (np.abs(a64) @ np.abs(b64))
+
+
+@pytest.mark.parametrize("trans_a", [False, True])
+@pytest.mark.parametrize("M,N,K", [
+    (1, 1, 1), (63, 127, 31), (64, 128, 32), (65, 129, 33), (127, 2, 63), (128, 130, 64), (129, 255, 65),
+    (66, 3, 7), (192, 257, 1029), (70, 70, 4099)])
+@pytest.mark.parametrize("scale_a,scale_b", [(1.0, 1.0), (1e-37, 1.0), (1e-20, 1e-18), (1e30, 1e-30), (1e18, 1e18)])
+def test_gemm_edges_and_range(trans_a, M, N, K, scale_a, scale_b):
+    """Every edge of the 64 / 128 x 128 tiles and of the 32 k of a stage, operands from the smallest
+    to the largest floats (what a float cannot represent of the result excepted)."""
+    import torch
+    from haste_amd import ops
+    r = np.random.default_rng(M + 31 * N + 17 * K)
+    a = (r.standard_normal((K, M) if trans_a else (M, K)) * scale_a).astype(np.float32)
+    b = (r.standard_normal((K, N)) * scale_b).astype(np.float32)
+    print("gemm edges", trans_a, M, N, K, scale_a, scale_b, flush=True)
+    out = host(ops.gemm(dev(a), dev(b), trans_a=trans_a)).astype(np.float64)
+    torch.cuda.synchronize()
+    a64, b64 = (a.T if trans_a else a).astype(np.float64), b.astype(np.float64)
+    assert np.all(np.abs(out - a64 @ b64) <= _bound(a64, b64, K) + K * 2.0 ** -149)
+
+
+@pytest.mark.parametrize("trans_a", [False, True])
+def test_gemm_operands_that_are_not_finite(trans_a):
+    """Infinities, NaNs and values beyond the largest bfloat16 give what float arithmetic gives, and
+    leave the rest of their tile alone."""
+    import torch
+    from haste_amd import ops
+    r = np.random.default_rng(3)
+    M, N, K = 200, 150, 96
+    a, b = r.standard_normal((M, K)).astype(np.float32), r.standard_normal((K, N)).astype(np.float32)
+    a[3, 5], a[100, 7], b[9, 20], a[150, 11] = np.inf, -np.inf, np.nan, 3.4e38
+    b[11] = np.where(np.abs(b[11]) > 1, b[11] / 4, b[11])
+    b[5, 30] = 0.0
+    out = host(ops.gemm(dev(a.T if trans_a else a), dev(b), trans_a=trans_a))
+    torch.cuda.synchronize()
+    with np.errstate(invalid="ignore"):
+        ref = a.astype(np.float64) @ b.astype(np.float64)
+    assert np.array_equal(np.isnan(out), np.isnan(ref))
+    inf = np.isinf(ref)
+    assert np.array_equal(out[inf], ref[inf].astype(np.float32))
+    rows = [i for i in range(M) if i not in (3, 100, 150)]
+    cols = [j for j in range(N) if j != 20]
+    a64, b64 = a[rows].astype(np.float64), b[:, cols].astype(np.float64)
+    assert np.all(np.abs(out[np.ix_(rows, cols)] - a64 @ b64) <= _bound(a64, b64, K))
+
+
+@pytest.mark.parametrize("M,N,K", [(512, 512, 512), (256, 512, 6400), (128, 128, 40000)])
+def test_gemm_is_at_least_as_accurate_as_float_products(M, N, K):
+    """Against the float64 product: no further from it than a float32 product whose partial sums
+    are rounded every two k, as the fp32 matrix instruction rounds them (on the CPU)."""
+    import torch
+    from haste_amd import ops
+    g = torch.Generator().manual_seed(M + K)
+    a, b = torch.randn(M, K, generator=g), torch.randn(K, N, generator=g)
+    out = ops.gemm(a.cuda(), b.cuda()).cpu().double()
+    rows = slice(0, 16)
+    ref = a[rows].double() @ b.double()
+    acc = torch.zeros(16, N)
+    for k in range(0, K, 2):
+        acc = (acc.double() + a[rows, k:k + 2].double() @ b[k:k + 2].double()).float()
+    assert (out[rows] - ref).norm() <= (acc.double() - ref).norm()
