@@ -391,7 +391,8 @@ struct LnLstmBwdParams {
   const float* R_t;        // [4H,H]
   const float* c;          // [T+1,N,H]
   const float* dh_new;     // [T+1,N,H]
-  const float* dc_new;     // [T+1,N,H]
+  const float* dc_new;     // [T+1,N,H]; without dc_given some tensor of that shape, not used
+  int dc_given;
   float* db;               // [4H]
   float* dh;               // [N,H]
   float* dc;               // [N,H]
@@ -660,7 +661,7 @@ void ln_lstm_backward_kernel(LnLstmBwdParams p) {
         accs[pp][9] += dln3;
 
         const float gi = s[pp].vt[0], gg = s[pp].vt[1], gf = s[pp].vt[2];
-        const float base = s[pp].dcn + dc[pp] + s[pp].is3 * gd3[pp];
+        const float base = (p.dc_given ? s[pp].dcn : 0.f) + dc[pp] + s[pp].is3 * gd3[pp];
         const float X = 2.0f * xc3[pp] * invH;
         const float k[3] = {d_sigmoid_f(gi) * gg, d_tanh_f(gg) * gi, d_sigmoid_f(gf) * s[pp].c0};
         float F = 0.f, G = 0.f, x2 = 0.f;
@@ -712,7 +713,7 @@ void ln_lstm_backward_kernel(LnLstmBwdParams p) {
         const float dmu = (-2.0f * rs[1] * dsigma * invH) - (rs[2] * is3);
         const float dc_ln = (2.0f * xc3[pp] * dsigma * invH) + (is3 * gd3[pp]) + (dmu * invH);
         const float gi = s[pp].vt[0], gg = s[pp].vt[1], gf = s[pp].vt[2];
-        const float dc_total = s[pp].dcn + dc[pp] + dc_ln;
+        const float dc_total = (p.dc_given ? s[pp].dcn : 0.f) + dc[pp] + dc_ln;
         const float df = s[pp].c0 * dc_total;
         dc[pp] = gf * dc_total;
         const float di = gg * dc_total;
@@ -935,7 +936,7 @@ int haste_hip_layer_norm_lstm_backward_f32(int steps, int batch_size, int input_
   (void)beta_h;
   const int T = steps, N = batch_size, C = input_size, H = hidden_size;
   HASTE_HIP_REQUIRE(T > 0 && N > 0 && C > 0 && H > 0);
-  HASTE_HIP_REQUIRE(W_t && R_t && x_t && h && c && dh_new && dc_new);
+  HASTE_HIP_REQUIRE(W_t && R_t && x_t && h && c && dh_new);
   HASTE_HIP_REQUIRE(dx && dW && dR && db && dh && dc && act_Wx && gamma1 && dgamma1);
   HASTE_HIP_REQUIRE(act_Wx_norm && act_Rh && gamma2 && dgamma2 && cache2 && gamma_h);
   HASTE_HIP_REQUIRE(dgamma_h && dbeta_h && cache3 && act_c_norm);
@@ -961,7 +962,9 @@ int haste_hip_layer_norm_lstm_backward_f32(int steps, int batch_size, int input_
 
   LnLstmBwdParams p;
   p.T = T; p.N = N; p.H = H;
-  p.R_t = R_t; p.c = c; p.dh_new = dh_new; p.dc_new = dc_new;
+  p.R_t = R_t; p.c = c; p.dh_new = dh_new;
+  p.dc_new = dc_new != nullptr ? dc_new : dh_new;
+  p.dc_given = dc_new != nullptr;
   p.db = db; p.dh = dh; p.dc = dc; p.v = act_Wx_norm; p.act_Rh = act_Rh;
   p.gamma2 = gamma2; p.dgamma2 = dgamma2; p.cache2 = cache2;
   p.gamma_h = gamma_h; p.dgamma_h = dgamma_h; p.dbeta_h = dbeta_h; p.cache3 = cache3;

@@ -420,7 +420,8 @@ struct LstmBwdParams {
   const float* c;       // [T,N,H] cell state before each step
   const float* c_next;  // [T,N,H] cell state after each step (may be c + N*H)
   const float* dh_next; // [T,N,H] upstream gradient of the h each step produced
-  const float* dc_next; // [T,N,H] same for c
+  const float* dc_next; // [T,N,H] same for c; without dc_given some tensor of that shape, not used
+  int dc_given;
   float* db;            // [4H] accumulated
   float* dh;            // [N,H] in/out
   float* dc;            // [N,H] in/out
@@ -589,7 +590,7 @@ void lstm_backward_kernel(LstmBwdParams p) {
       if (act[pp]) {
         const StepIn s = nxt[pp];
         const float gi = s.vt[0], gg = s.vt[1], gf = s.vt[2], go = s.vt[3];
-        float dc_total = s.dcn + dc[pp];
+        float dc_total = (p.dc_given ? s.dcn : 0.f) + dc[pp];
         float dh_total = s.dhn + dh[pp];
         const float c_tanh = tanh_f(s.c1);
         if (zoneout) {
@@ -713,6 +714,7 @@ struct LstmScatterCell {
   static constexpr int kInputs = 9;  // v (4 gates), c before and after, dh_next, dc_next, mask
   static constexpr int kSums = 4;
   float dh, dc, dh_keep;
+  bool dc_given;
   float gi, gg, gf, go, c0, dhn, m, c_tanh, k_c, k_i, k_g, k_f, k_o, dc_total;
 
   __device__ __forceinline__ static float* pieces(const Params& p) { return p.xdv; }
@@ -730,6 +732,7 @@ struct LstmScatterCell {
   __device__ __forceinline__ void load_state(const Params& p, size_t e, bool mine) {
     dh = mine ? p.dh[e] : 0.f;
     dc = mine ? p.dc[e] : 0.f;
+    dc_given = p.dc_given != 0;
     dh_keep = 0.f;
   }
   __device__ __forceinline__ void store_state(const Params& p, size_t e) const {
@@ -745,7 +748,7 @@ struct LstmScatterCell {
     k_g = d_tanh_f(gg);
     k_f = d_sigmoid_f(gf);
     k_o = d_sigmoid_f(go);
-    dc_total = sv[7] + dc;
+    dc_total = (dc_given ? sv[7] : 0.f) + dc;
   }
   __device__ __forceinline__ void add_gathered(float sum) { dh = dh_keep + sum; }
   __device__ __forceinline__ float4_t step(bool act, bool zoneout, float (&sums)[kSums]) {
@@ -912,7 +915,7 @@ int lstm_backward_impl(hipStream_t stream, int T, int N, int C, int H,
                        float* dx, float* dW, float* dR, float* db, float* dh, float* dc, float* v,
                        const float* zoneout_mask) {
   HASTE_HIP_REQUIRE(T > 0 && N > 0 && C > 0 && H > 0);
-  HASTE_HIP_REQUIRE(W_t && R_t && x_t && h && c && c_next && dh_next && dc_next);
+  HASTE_HIP_REQUIRE(W_t && R_t && x_t && h && c && c_next && dh_next);
   HASTE_HIP_REQUIRE(dx && dW && dR && db && dh && dc && v);
   const BackwardTile tile = pick_backward_tile(4 * H, N, H, 4 * 16, 0, true);
   if (!tile.ok)
@@ -942,7 +945,9 @@ int lstm_backward_impl(hipStream_t stream, int T, int N, int C, int H,
 
   LstmBwdParams p;
   p.T = T; p.N = N; p.H = H;
-  p.R_t = R_t; p.c = c; p.c_next = c_next; p.dh_next = dh_next; p.dc_next = dc_next;
+  p.R_t = R_t; p.c = c; p.c_next = c_next; p.dh_next = dh_next;
+  p.dc_next = dc_next != nullptr ? dc_next : dh_next;
+  p.dc_given = dc_next != nullptr;
   p.db = db; p.dh = dh; p.dc = dc; p.v = v; p.zoneout_mask = zoneout_mask;
   p.db_partial = ws.scratch;
   p.xdv = ws.scratch + (db_floats + 3) / 4 * 4;
@@ -1024,11 +1029,11 @@ int haste_hip_lstm_backward_f32(int steps, int batch_size, int input_size, int h
                                 float* dh, float* dc, float* v,
                                 const float* zoneout_mask, void* stream) {
   (void)b;  // unused by the reference as well (lib/lstm_backward_gpu.cu.cc:319-405)
-  HASTE_HIP_REQUIRE(c && dh_new && dc_new && batch_size > 0 && hidden_size > 0);
+  HASTE_HIP_REQUIRE(c && dh_new && batch_size > 0 && hidden_size > 0);
   const size_t NH = (size_t)batch_size * hidden_size;
   return haste_hip::lstm_backward_impl(haste_hip::as_stream(stream), steps, batch_size, input_size,
                                        hidden_size, W_t, R_t, x_t, h, c, c + NH, dh_new + NH,
-                                       dc_new + NH, dx, dW, dR, db, dh, dc, v, zoneout_mask);
+                                       dc_new != nullptr ? dc_new + NH : nullptr, dx, dW, dR, db, dh, dc, v, zoneout_mask);
 }
 
 int haste_hip_lstm_forward_iterate_f32(int training, int batch_size, int input_size,

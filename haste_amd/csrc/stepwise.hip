@@ -512,7 +512,7 @@ void lstm_backward_pointwise(int N, int H, const T* __restrict__ c, const T* __r
   const int n = (int)(idx / H), j = (int)(idx % H);
   const size_t g0 = (size_t)n * 4 * H + j;
   const T gi = v_t[g0], gg = v_t[g0 + H], gf = v_t[g0 + 2 * (size_t)H], go = v_t[g0 + 3 * (size_t)H];
-  T dc_total = dc_next[idx] + dc[idx];
+  T dc_total = (dc_next != nullptr ? dc_next[idx] : T(0)) + dc[idx];
   T dh_total = dh_next[idx] + (dh[idx] + pend.at(idx));
   const T c_tanh = Fn<T>::tanh_(c_next[idx]);
   T dh_keep = T(0);
@@ -689,7 +689,7 @@ void ln_lstm_gate_grad(int N, int H, const T* __restrict__ c, const T* __restric
   const int n = (int)(idx / H), j = (int)(idx % H);
   const size_t g0 = (size_t)n * 4 * H + j;
   const T gi = v_t[g0], gg = v_t[g0 + H], gf = v_t[g0 + 2 * (size_t)H];
-  const T dc_total = dc_next[idx] + dc[idx] + dc_ln[idx];
+  const T dc_total = (dc_next != nullptr ? dc_next[idx] : T(0)) + dc[idx] + dc_ln[idx];
   const T df = c[idx] * dc_total;
   const T di = gg * dc_total;
   const T dg = gi * dc_total;
@@ -811,7 +811,7 @@ int lstm_backward_steps(hipStream_t stream, int steps, int N, int C, int H, cons
     for (int t = steps - 1; t >= 0; --t) {
       lstm_backward_pointwise<T><<<blocks_for(NH), dim3(kThreads), 0, stream>>>(
           N, H, c + (size_t)t * NH, c_next + (size_t)t * NH, dh_next + (size_t)t * NH,
-          dc_next + (size_t)t * NH, dh, pend, dc, v + (size_t)t * N4H,
+          dc_next != nullptr ? dc_next + (size_t)t * NH : nullptr, dh, pend, dc, v + (size_t)t * N4H,
           zoneout_mask ? zoneout_mask + (size_t)t * NH : nullptr);
       HASTE_LAUNCHED();
       // dh += dv_t * R^T
@@ -953,7 +953,7 @@ int ln_lstm_backward_steps(hipStream_t stream, int steps, int N, int C, int H, c
       HASTE_HIP_PROPAGATE(ln_backward_rows<T>(stream, (size_t)N, H, gamma_h, c + (size_t)(t + 1) * NH, cn_t, cn_t,
                                               dgamma_h, dbeta_h, cache3 + (size_t)t * N * 2, partial));
       ln_lstm_gate_grad<T><<<blocks_for(NH), dim3(kThreads), 0, stream>>>(
-          N, H, c + (size_t)t * NH, dc_new + (size_t)(t + 1) * NH, dc, cn_t, v_t);
+          N, H, c + (size_t)t * NH, dc_new != nullptr ? dc_new + (size_t)(t + 1) * NH : nullptr, dc, cn_t, v_t);
       HASTE_LAUNCHED();
       // through the norm of h*R, in place over act_Rh[t]
       HASTE_HIP_PROPAGATE(ln_backward_rows<T>(stream, (size_t)N, 4 * H, gamma2, rh_t, v_t, rh_t, dgamma2,
@@ -1240,11 +1240,12 @@ int haste_hip_lstm_backward_f64(int steps, int batch_size, int input_size, int h
                                 const double* zoneout_mask, void* stream) {
   (void)b;
   HASTE_HIP_REQUIRE(steps > 0 && batch_size > 0 && input_size > 0 && hidden_size > 0);
-  HASTE_HIP_REQUIRE(W_t && R_t && x_t && h && c && dh_new && dc_new);
+  HASTE_HIP_REQUIRE(W_t && R_t && x_t && h && c && dh_new);
   HASTE_HIP_REQUIRE(dx && dW && dR && db && dh && dc && v);
   const size_t NH = (size_t)batch_size * hidden_size;
   return lstm_backward_steps<double>(as_stream(stream), steps, batch_size, input_size, hidden_size,
-                                     W_t, R_t, x_t, h, c, c + NH, dh_new + NH, dc_new + NH, dx, dW, dR,
+                                     W_t, R_t, x_t, h, c, c + NH, dh_new + NH,
+                                     dc_new != nullptr ? dc_new + NH : nullptr, dx, dW, dR,
                                      db, dh, dc, v, zoneout_mask);
 }
 
@@ -1271,7 +1272,7 @@ int haste_hip_lstm_backward_iterate_f64(int batch_size, int input_size, int hidd
                                         const double* zoneout_mask, void* stream) {
   (void)b;
   HASTE_HIP_REQUIRE(batch_size > 0 && input_size > 0 && hidden_size > 0);
-  HASTE_HIP_REQUIRE(W_t && R_t && x_t && h && c && c_new && dh_new && dc_new);
+  HASTE_HIP_REQUIRE(W_t && R_t && x_t && h && c && c_new && dh_new);
   HASTE_HIP_REQUIRE(dx && dW && dR && db && dh && dc && v);
   return lstm_backward_steps<double>(as_stream(stream), 1, batch_size, input_size, hidden_size, W_t,
                                      R_t, x_t, h, c, c_new, dh_new, dc_new, dx, dW, dR, db, dh, dc, v,
@@ -1409,7 +1410,7 @@ int haste_hip_layer_norm_lstm_backward_f64(int steps, int batch_size, int input_
   (void)b;
   (void)beta_h;
   HASTE_HIP_REQUIRE(steps > 0 && batch_size > 0 && input_size > 0 && hidden_size > 0);
-  HASTE_HIP_REQUIRE(W_t && R_t && x_t && h && c && dh_new && dc_new);
+  HASTE_HIP_REQUIRE(W_t && R_t && x_t && h && c && dh_new);
   HASTE_HIP_REQUIRE(dx && dW && dR && db && dh && dc && act_Wx && gamma1 && dgamma1);
   HASTE_HIP_REQUIRE(act_Wx_norm && act_Rh && gamma2 && dgamma2 && cache2 && gamma_h);
   HASTE_HIP_REQUIRE(dgamma_h && dbeta_h && cache3 && act_c_norm);

@@ -25,11 +25,6 @@ from . import ops
 __all__ = ["LSTM", "GRU", "IndRNN", "LayerNormLSTM", "LayerNormGRU", "LayerNormIndRNN"]
 
 
-def _time_major_t(x):
-    """[T,N,C] -> [C,T,N], the layout the backward passes take x in."""
-    return ops.transpose(x) if x.is_cuda else x.permute(2, 0, 1).contiguous()
-
-
 def _t(w):
     return ops.transpose(w) if w.is_cuda and w.is_contiguous() else w.t().contiguous()
 
@@ -48,151 +43,230 @@ def _no_training_backward(name):
 
 
 # ---- autograd glue (reference frameworks/pytorch/lstm.py:69-88 and siblings) -------------
-class _LSTMFunction(torch.autograd.Function):
+# The functions return what the layers return -- the states after each step and what `wanted` asks for
+# of every state -- and not the [T+1,N,H] sequences the ops work on: differentiating slices of those
+# would fill and copy a sequence per slice, where the backward ops take the gradients of the outputs
+# as they come (a training step of the IndRNN at T=2500 N=64 H=4096, 2.6 GB per sequence: 10.0 -> 8.7 ms;
+# of the LSTM at N=128 T=100 C=H=512 1399 -> 1367 us).
+def _alias(seq, first):
+    """seq[first:] (or seq[-1]) as a tensor on the same memory that is no view to autograd."""
+    a = seq[first:] if first >= 0 else seq[-1]
+    return seq.new_empty(0).set_(a)
+
+
+def _wanted_states(seqs, wanted):
+    """What a layer returns of its state sequences [T+1,N,H]: "last" [N,H], "all" [T,N,H], or the states
+    at the steps in an index tensor [N]."""
+    if torch.is_tensor(wanted):
+        cols = torch.arange(seqs[0].size(1), device=wanted.device)
+        return tuple(seq[wanted, cols] for seq in seqs)
+    return tuple(_alias(seq, 1 if wanted == "all" else -1) for seq in seqs)
+
+
+def _upstream(like, grad_steps, grad_wanted, wanted):
+    """The gradients of a state sequence `like` [T+1,N,H] from those of the states after each step and of
+    the wanted states (either may be None): (gradients [T,N,H] or [T+1,N,H], or None; more of the last
+    states, [N,H] or None)."""
+    if grad_wanted is None:
+        return grad_steps if grad_steps is None else grad_steps.contiguous(), None
+    if not torch.is_tensor(wanted):
+        if wanted == "last":
+            return grad_steps if grad_steps is None else grad_steps.contiguous(), grad_wanted
+        return (grad_wanted if grad_steps is None else grad_steps + grad_wanted).contiguous(), None
+    full = torch.zeros_like(like) if grad_steps is None else torch.empty_like(like)
+    if grad_steps is not None:
+        full[1:] = grad_steps
+        full[0].zero_()
+    # one entry per batch row: nothing is indexed twice
+    cols = torch.arange(like.size(1), device=like.device)
+    full[wanted, cols] = full[wanted, cols] + grad_wanted
+    return full, None
+
+
+def _upstream_h(h, grad_y, grad_h, wanted):
+    grad, last = _upstream(h, grad_y, grad_h, wanted)
+    return h.new_zeros((h.size(0) - 1,) + h.shape[1:]) if grad is None else grad, last
+
+
+def _initial(ctx, *grads):
+    """The gradients of the initial states, inputs 4, 5 of every function, where they are tensors."""
+    return tuple(g if ctx.needs_input_grad[4 + i] else None for i, g in enumerate(grads))
+
+
+class _RecurrenceFunction(torch.autograd.Function):
+    """forward(ctx, training, zoneout_prob, wanted, ...) -> the outputs named above; the subclasses call
+    the ops."""
+
     @staticmethod
-    def forward(ctx, training, zoneout_prob, x, h0, c0, kernel, recurrent_kernel, bias, zoneout_mask,
+    def finish(ctx, training, wanted, saved, *seqs):
+        """Saves what the backward pass needs; (y, wanted states of each sequence)."""
+        h = seqs[0]
+        y = _alias(h, 1)
+        states = _wanted_states(seqs, wanted)
+        # the outputs that share memory with h and c too: if a caller changes them, autograd notices
+        ctx.save_for_backward(y, *states, *saved)
+        ctx.training, ctx.wanted, ctx.count = training, wanted, len(seqs)
+        ctx.set_materialize_grads(False)
+        return (y,) + states
+
+    @staticmethod
+    def restore(ctx):
+        return ctx.saved_tensors[1 + ctx.count:]
+
+
+class _NoGradients:
+    """Stands in for a context where there is nothing to differentiate."""
+
+    def save_for_backward(self, *tensors):
+        pass
+
+    def set_materialize_grads(self, value):
+        pass
+
+
+class _LSTMFunction(_RecurrenceFunction):
+    @staticmethod
+    def forward(ctx, training, zoneout_prob, wanted, x, h0, c0, kernel, recurrent_kernel, bias, zoneout_mask,
                 dropconnect_mask, dropconnect_scale):
         h, c, cache = ops.lstm_forward(training, zoneout_prob, x, h0, c0, kernel, recurrent_kernel,
                                        bias, zoneout_mask, dropconnect_mask, dropconnect_scale)
-        ctx.save_for_backward(x, kernel, recurrent_kernel, bias, zoneout_mask, h, c, cache,
-                              dropconnect_mask if dropconnect_mask is not None else x.new_empty(0))
-        ctx.training = training
         ctx.dropconnect_scale = dropconnect_scale
-        ctx.mark_non_differentiable(zoneout_mask)
-        return h, c
+        return _RecurrenceFunction.finish(
+            ctx, training, wanted,
+            (x, kernel, recurrent_kernel, bias, zoneout_mask, h, c, cache, dropconnect_mask), h, c)
 
     @staticmethod
-    def backward(ctx, grad_h, grad_c):
+    def backward(ctx, grad_y, grad_h, grad_c):
         if not ctx.training:
             raise _no_training_backward("LSTM")
-        x, kernel, recurrent_kernel, bias, zoneout_mask, h, c, cache, dmask = ctx.saved_tensors
-        if dmask.numel():
+        x, kernel, recurrent_kernel, bias, zoneout_mask, h, c, cache, dmask = _RecurrenceFunction.restore(ctx)
+        if dmask is not None:
             recurrent_kernel = recurrent_kernel * dmask * ctx.dropconnect_scale
         _single_shot(ctx, "LSTM")  # the backward pass overwrites the activation cache
+        dh_new, dh_last = _upstream_h(h, grad_y, grad_h, ctx.wanted)
+        dc_new, dc_last = _upstream(c, None, grad_c, ctx.wanted)
         dx, dh, dc, dW, dR, db = ops.lstm_backward(
-            _time_major_t(x), _t(kernel), _t(recurrent_kernel), bias, zoneout_mask, h, c,
-            cache, grad_h.contiguous(), grad_c.contiguous())
-        if dmask.numel():
+            *ops.transpose3(x, kernel, recurrent_kernel), bias, zoneout_mask, h, c, cache, dh_new, dc_new,
+            dh_last, dc_last)
+        if dmask is not None:
             dR = dR * dmask * ctx.dropconnect_scale
-        return None, None, dx, dh, dc, dW, dR, db, None, None, None
+        return (None, None, None, dx) + _initial(ctx, dh, dc) + (dW, dR, db, None, None, None)
 
 
-class _GRUFunction(torch.autograd.Function):
+class _GRUFunction(_RecurrenceFunction):
     @staticmethod
-    def forward(ctx, training, zoneout_prob, x, h0, kernel, recurrent_kernel, bias, recurrent_bias,
+    def forward(ctx, training, zoneout_prob, wanted, x, h0, kernel, recurrent_kernel, bias, recurrent_bias,
                 zoneout_mask, dropconnect_mask, dropconnect_scale):
         h, cache = ops.gru_forward(training, zoneout_prob, x, h0, kernel, recurrent_kernel, bias,
                                    recurrent_bias, zoneout_mask, dropconnect_mask, dropconnect_scale)
-        ctx.save_for_backward(x, kernel, recurrent_kernel, bias, recurrent_bias, zoneout_mask, h, cache,
-                              dropconnect_mask if dropconnect_mask is not None else x.new_empty(0))
-        ctx.training = training
         ctx.dropconnect_scale = dropconnect_scale
-        ctx.mark_non_differentiable(zoneout_mask)
-        return h
+        return _RecurrenceFunction.finish(
+            ctx, training, wanted,
+            (x, kernel, recurrent_kernel, bias, recurrent_bias, zoneout_mask, h, cache, dropconnect_mask), h)
 
     @staticmethod
-    def backward(ctx, grad_h):
+    def backward(ctx, grad_y, grad_h):
         if not ctx.training:
             raise _no_training_backward("GRU")
-        x, kernel, recurrent_kernel, bias, recurrent_bias, zoneout_mask, h, cache, dmask = ctx.saved_tensors
-        if dmask.numel():
+        (x, kernel, recurrent_kernel, bias, recurrent_bias, zoneout_mask, h, cache,
+         dmask) = _RecurrenceFunction.restore(ctx)
+        if dmask is not None:
             recurrent_kernel = recurrent_kernel * dmask * ctx.dropconnect_scale
+        dh_new, dh_last = _upstream_h(h, grad_y, grad_h, ctx.wanted)
         dx, dh, dW, dR, dbx, dbr = ops.gru_backward(
-            _time_major_t(x), _t(kernel), _t(recurrent_kernel), bias, recurrent_bias, zoneout_mask, h,
-            cache, grad_h.contiguous())
-        if dmask.numel():
+            *ops.transpose3(x, kernel, recurrent_kernel), bias, recurrent_bias, zoneout_mask, h, cache, dh_new,
+            dh_last)
+        if dmask is not None:
             dR = dR * dmask * ctx.dropconnect_scale
-        return None, None, dx, dh, dW, dR, dbx, dbr, None, None, None
+        return (None, None, None, dx) + _initial(ctx, dh) + (dW, dR, dbx, dbr, None, None, None)
 
 
-class _IndRNNFunction(torch.autograd.Function):
+class _IndRNNFunction(_RecurrenceFunction):
     @staticmethod
-    def forward(ctx, training, zoneout_prob, x, h0, kernel, recurrent_scale, bias, zoneout_mask):
+    def forward(ctx, training, zoneout_prob, wanted, x, h0, kernel, recurrent_scale, bias, zoneout_mask):
         h = ops.indrnn_forward(training, zoneout_prob, x, h0, kernel, recurrent_scale, bias, zoneout_mask)
-        ctx.save_for_backward(x, kernel, recurrent_scale, bias, zoneout_mask, h)
-        ctx.training = training
-        ctx.mark_non_differentiable(zoneout_mask)
-        return h
+        return _RecurrenceFunction.finish(ctx, training, wanted,
+                                          (x, kernel, recurrent_scale, bias, zoneout_mask, h), h)
 
     @staticmethod
-    def backward(ctx, grad_h):
+    def backward(ctx, grad_y, grad_h):
         if not ctx.training:
             raise _no_training_backward("IndRNN")
-        x, kernel, recurrent_scale, bias, zoneout_mask, h = ctx.saved_tensors
-        dx, dh, dW, du, db = ops.indrnn_backward(_time_major_t(x), _t(kernel), recurrent_scale, bias,
-                                                 zoneout_mask, h, grad_h.contiguous())
-        return None, None, dx, dh, dW, du, db, None
+        x, kernel, recurrent_scale, bias, zoneout_mask, h = _RecurrenceFunction.restore(ctx)
+        dh_new, dh_last = _upstream_h(h, grad_y, grad_h, ctx.wanted)
+        dx, dh, dW, du, db = ops.indrnn_backward(ops.transpose(x), ops.transpose(kernel), recurrent_scale, bias,
+                                                 zoneout_mask, h, dh_new, dh_last)
+        return (None, None, None, dx) + _initial(ctx, dh) + (dW, du, db, None)
 
 
-class _LayerNormIndRNNFunction(torch.autograd.Function):
+class _LayerNormIndRNNFunction(_RecurrenceFunction):
     @staticmethod
-    def forward(ctx, training, zoneout_prob, x, h0, kernel, recurrent_scale, bias, gamma, zoneout_mask):
+    def forward(ctx, training, zoneout_prob, wanted, x, h0, kernel, recurrent_scale, bias, gamma, zoneout_mask):
         h, act_Wx, cache = ops.layer_norm_indrnn_forward(training, zoneout_prob, x, h0, kernel,
                                                          recurrent_scale, bias, gamma, zoneout_mask)
-        ctx.save_for_backward(x, kernel, recurrent_scale, bias, gamma, zoneout_mask, h, act_Wx, cache)
-        ctx.training = training
-        ctx.mark_non_differentiable(zoneout_mask)
-        return h
+        return _RecurrenceFunction.finish(
+            ctx, training, wanted, (x, kernel, recurrent_scale, bias, gamma, zoneout_mask, h, act_Wx, cache), h)
 
     @staticmethod
-    def backward(ctx, grad_h):
+    def backward(ctx, grad_y, grad_h):
         if not ctx.training:
             raise _no_training_backward("LayerNormIndRNN")
-        x, kernel, recurrent_scale, bias, gamma, zoneout_mask, h, act_Wx, cache = ctx.saved_tensors
+        (x, kernel, recurrent_scale, bias, gamma, zoneout_mask, h, act_Wx,
+         cache) = _RecurrenceFunction.restore(ctx)
+        dh_new, dh_last = _upstream_h(h, grad_y, grad_h, ctx.wanted)
         dx, dh, dW, du, db, dgamma = ops.layer_norm_indrnn_backward(
-            _time_major_t(x), _t(kernel), recurrent_scale, bias, gamma, zoneout_mask, h, act_Wx, cache,
-            grad_h.contiguous())
-        return None, None, dx, dh, dW, du, db, dgamma, None
+            ops.transpose(x), ops.transpose(kernel), recurrent_scale, bias, gamma, zoneout_mask, h, act_Wx, cache,
+            dh_new, dh_last)
+        return (None, None, None, dx) + _initial(ctx, dh) + (dW, du, db, dgamma, None)
 
 
-class _LayerNormLSTMFunction(torch.autograd.Function):
+class _LayerNormLSTMFunction(_RecurrenceFunction):
     @staticmethod
-    def forward(ctx, training, zoneout_prob, x, h0, c0, kernel, recurrent_kernel, bias, gamma, gamma_h,
+    def forward(ctx, training, zoneout_prob, wanted, x, h0, c0, kernel, recurrent_kernel, bias, gamma, gamma_h,
                 beta_h, zoneout_mask):
         outs = ops.layer_norm_lstm_forward(training, zoneout_prob, x, h0, c0, kernel, recurrent_kernel,
                                            bias, gamma, gamma_h, beta_h, zoneout_mask)
-        ctx.save_for_backward(x, kernel, recurrent_kernel, bias, gamma, gamma_h, beta_h, zoneout_mask,
-                              *outs)
-        ctx.training = training
-        ctx.mark_non_differentiable(zoneout_mask)
-        return outs[0], outs[1]
+        return _RecurrenceFunction.finish(
+            ctx, training, wanted,
+            (x, kernel, recurrent_kernel, bias, gamma, gamma_h, beta_h, zoneout_mask) + tuple(outs), *outs[:2])
 
     @staticmethod
-    def backward(ctx, grad_h, grad_c):
+    def backward(ctx, grad_y, grad_h, grad_c):
         if not ctx.training:
             raise _no_training_backward("LayerNormLSTM")
         (x, kernel, recurrent_kernel, bias, gamma, gamma_h, beta_h, zoneout_mask, h, c, act_Wx,
-         act_Wx_norm, cache1, act_Rh, cache2, act_c_norm, cache3) = ctx.saved_tensors
+         act_Wx_norm, cache1, act_Rh, cache2, act_c_norm, cache3) = _RecurrenceFunction.restore(ctx)
         _single_shot(ctx, "LayerNormLSTM")  # the saved activations are overwritten below
-        grads = ops.layer_norm_lstm_backward(
-            _time_major_t(x), _t(kernel), _t(recurrent_kernel), bias, gamma, gamma_h, beta_h,
+        dh_new, dh_last = _upstream_h(h, grad_y, grad_h, ctx.wanted)
+        dc_new, dc_last = _upstream(c, None, grad_c, ctx.wanted)
+        dx, dh, dc, *grads = ops.layer_norm_lstm_backward(
+            *ops.transpose3(x, kernel, recurrent_kernel), bias, gamma, gamma_h, beta_h,
             zoneout_mask, h, c, act_Wx, act_Wx_norm, cache1, act_Rh, cache2, act_c_norm, cache3,
-            grad_h.contiguous(), grad_c.contiguous())
-        return (None, None) + tuple(grads) + (None,)
+            dh_new, dc_new, dh_last, dc_last)
+        return (None, None, None, dx) + _initial(ctx, dh, dc) + tuple(grads) + (None,)
 
 
-class _LayerNormGRUFunction(torch.autograd.Function):
+class _LayerNormGRUFunction(_RecurrenceFunction):
     @staticmethod
-    def forward(ctx, training, zoneout_prob, x, h0, kernel, recurrent_kernel, bias, recurrent_bias,
+    def forward(ctx, training, zoneout_prob, wanted, x, h0, kernel, recurrent_kernel, bias, recurrent_bias,
                 gamma, zoneout_mask):
         outs = ops.layer_norm_gru_forward(training, zoneout_prob, x, h0, kernel, recurrent_kernel, bias,
                                           recurrent_bias, gamma, zoneout_mask)
-        ctx.save_for_backward(x, kernel, recurrent_kernel, bias, recurrent_bias, gamma, zoneout_mask,
-                              *outs)
-        ctx.training = training
-        ctx.mark_non_differentiable(zoneout_mask)
-        return outs[0]
+        return _RecurrenceFunction.finish(
+            ctx, training, wanted,
+            (x, kernel, recurrent_kernel, bias, recurrent_bias, gamma, zoneout_mask) + tuple(outs), outs[0])
 
     @staticmethod
-    def backward(ctx, grad_h):
+    def backward(ctx, grad_y, grad_h):
         if not ctx.training:
             raise _no_training_backward("LayerNormGRU")
         (x, kernel, recurrent_kernel, bias, recurrent_bias, gamma, zoneout_mask, h, cache, act_Wx,
-         cache1, act_Rh, cache2) = ctx.saved_tensors
-        grads = ops.layer_norm_gru_backward(
-            _time_major_t(x), _t(kernel), _t(recurrent_kernel), bias, recurrent_bias, gamma,
-            zoneout_mask, h, cache, act_Wx, cache1, act_Rh, cache2, grad_h.contiguous())
-        return (None, None) + tuple(grads) + (None,)
+         cache1, act_Rh, cache2) = _RecurrenceFunction.restore(ctx)
+        dh_new, dh_last = _upstream_h(h, grad_y, grad_h, ctx.wanted)
+        dx, dh, *grads = ops.layer_norm_gru_backward(
+            *ops.transpose3(x, kernel, recurrent_kernel), bias, recurrent_bias, gamma,
+            zoneout_mask, h, cache, act_Wx, cache1, act_Rh, cache2, dh_new, dh_last)
+        return (None, None, None, dx) + _initial(ctx, dh) + tuple(grads) + (None,)
 
 
 # ---- the time loop in plain torch (reference *Script functions, e.g. frameworks/pytorch/
@@ -291,11 +365,12 @@ class _RNNBase(nn.Module):
     def _time_major(self, x):
         return x.permute(1, 0, 2) if self.batch_first else x
 
-    def _initial_state(self, x, state, count):
-        """`count` tensors of shape [N,H]: zeros, or the caller's [1,N,H] states checked."""
+    def _initial_state(self, x, state, count, fused=False):
+        """`count` tensors of shape [N,H]: zeros (None where the fused ops run: they preset them), or
+        the caller's [1,N,H] states checked."""
         shape = [1, x.shape[1], self.hidden_size]
         if state is None:
-            return tuple(x.new_zeros(shape[1:]) for _ in range(count))
+            return (None,) * count if fused else tuple(x.new_zeros(shape[1:]) for _ in range(count))
         states = (state,) if count == 1 else state
         if count > 1 and (not isinstance(states, (tuple, list)) or len(states) != count):
             raise ValueError("RNN state must be a tuple of %d tensors" % count)
@@ -304,6 +379,20 @@ class _RNNBase(nn.Module):
                 raise ValueError("RNN state has invalid shape; expected %s, got %s"
                                  % (shape, list(s.shape) if torch.is_tensor(s) else type(s)))
         return tuple(s[0].contiguous() for s in states)
+
+    def _wanted(self, lengths, device):
+        """Which states the fused functions are to return (see _wanted_states)."""
+        if self.return_state_sequence:
+            return "all"
+        return "last" if lengths is None else torch.as_tensor(lengths, device=device, dtype=torch.long)
+
+    def _fused(self, function, *args):
+        """The fused pass; without gradients autograd is not told of it."""
+        return function.apply(*args) if torch.is_grad_enabled() else function.forward(_NoGradients(), *args)
+
+    def _fused_state(self, states):
+        """A state as the layer returns it, from what the fused functions return of it."""
+        return (self._time_major(states) if self.return_state_sequence else states).unsqueeze(0)
 
     def _final_state(self, seq, lengths):
         """seq: [T+1,N,H] state after every step (slot 0 = initial state)."""
@@ -319,7 +408,7 @@ class _RNNBase(nn.Module):
         # 1 = take the new value (reference frameworks/pytorch/base_rnn.py:64-70)
         if self.zoneout:
             return x.new_empty(x.shape[0], x.shape[1], self.hidden_size).bernoulli_(1.0 - self.zoneout)
-        return x.new_empty(0, 0, 0)
+        return None
 
     def _dropconnect_mask(self, weight):
         """(mask, scale) for inverted dropout on the recurrent matrix, or (None, 1.0)."""
@@ -402,17 +491,19 @@ class LSTM(_RNNBase):
         """input [T,N,C] ([N,T,C] if batch_first) -> (output, (h_n, c_n)); h_n, c_n are [1,N,H],
         taken at `lengths` when given (the output itself is not masked)."""
         x = self._time_major(input)
-        h0, c0 = self._initial_state(x, state, 2)
+        fused = self._is_cuda()
+        h0, c0 = self._initial_state(x, state, 2, fused)
         dmask, dscale = self._dropconnect_mask(self.recurrent_kernel)
         zmask = self._zoneout_mask(x)
-        if self._is_cuda():
+        if fused:
             self._check_fused(x)
-            h, c = _LSTMFunction.apply(self.training, self.zoneout, x.contiguous(), h0, c0,
-                                       self.kernel.contiguous(), self.recurrent_kernel.contiguous(),
-                                       self.bias.contiguous(), zmask, dmask, dscale)
-        else:
-            h, c = _eager_lstm(self.training, self.zoneout, x, h0, c0, self.kernel,
-                               _dropped(self.recurrent_kernel, dmask, dscale), self.bias, zmask)
+            wanted = self._wanted(lengths, x.device)
+            y, h, c = self._fused(_LSTMFunction, self.training, self.zoneout, wanted, x.contiguous(), h0, c0,
+                                  self.kernel.contiguous(), self.recurrent_kernel.contiguous(),
+                                  self.bias.contiguous(), zmask, dmask, dscale)
+            return self._time_major(y), (self._fused_state(h), self._fused_state(c))
+        h, c = _eager_lstm(self.training, self.zoneout, x, h0, c0, self.kernel,
+                           _dropped(self.recurrent_kernel, dmask, dscale), self.bias, zmask)
         return self._time_major(h[1:]), (self._final_state(h, lengths), self._final_state(c, lengths))
 
 
@@ -452,19 +543,21 @@ class GRU(_RNNBase):
 
     def forward(self, input, state=None, lengths=None):
         x = self._time_major(input)
-        (h0,) = self._initial_state(x, state, 1)
+        fused = self._is_cuda()
+        (h0,) = self._initial_state(x, state, 1, fused)
         dmask, dscale = self._dropconnect_mask(self.recurrent_kernel)
         zmask = self._zoneout_mask(x)
-        if self._is_cuda():
+        if fused:
             self._check_fused(x)
-            h = _GRUFunction.apply(self.training, self.zoneout, x.contiguous(), h0,
-                                   self.kernel.contiguous(), self.recurrent_kernel.contiguous(),
-                                   self.bias.contiguous(), self.recurrent_bias.contiguous(),
-                                   zmask, dmask, dscale)
-        else:
-            h = _eager_gru(self.training, self.zoneout, x, h0, self.kernel,
-                           _dropped(self.recurrent_kernel, dmask, dscale), self.bias,
-                           self.recurrent_bias, zmask)
+            wanted = self._wanted(lengths, x.device)
+            y, h = self._fused(_GRUFunction, self.training, self.zoneout, wanted, x.contiguous(), h0,
+                               self.kernel.contiguous(), self.recurrent_kernel.contiguous(),
+                               self.bias.contiguous(), self.recurrent_bias.contiguous(),
+                               zmask, dmask, dscale)
+            return self._time_major(y), self._fused_state(h)
+        h = _eager_gru(self.training, self.zoneout, x, h0, self.kernel,
+                       _dropped(self.recurrent_kernel, dmask, dscale), self.bias,
+                       self.recurrent_bias, zmask)
         return self._time_major(h[1:]), self._final_state(h, lengths)
 
 
@@ -490,16 +583,18 @@ class IndRNN(_RNNBase):
 
     def forward(self, input, state=None, lengths=None):
         x = self._time_major(input)
-        (h0,) = self._initial_state(x, state, 1)
+        fused = self._is_cuda()
+        (h0,) = self._initial_state(x, state, 1, fused)
         zmask = self._zoneout_mask(x)
-        if self._is_cuda():
+        if fused:
             self._check_fused(x)
-            h = _IndRNNFunction.apply(self.training, self.zoneout, x.contiguous(), h0,
-                                      self.kernel.contiguous(), self.recurrent_scale.contiguous(),
-                                      self.bias.contiguous(), zmask)
-        else:
-            h = _eager_indrnn(self.training, self.zoneout, x, h0, self.kernel, self.recurrent_scale,
-                              self.bias, zmask)
+            wanted = self._wanted(lengths, x.device)
+            y, h = self._fused(_IndRNNFunction, self.training, self.zoneout, wanted, x.contiguous(), h0,
+                               self.kernel.contiguous(), self.recurrent_scale.contiguous(),
+                               self.bias.contiguous(), zmask)
+            return self._time_major(y), self._fused_state(h)
+        h = _eager_indrnn(self.training, self.zoneout, x, h0, self.kernel, self.recurrent_scale,
+                          self.bias, zmask)
         return self._time_major(h[1:]), self._final_state(h, lengths)
 
 
@@ -526,16 +621,18 @@ class LayerNormIndRNN(_RNNBase):
 
     def forward(self, input, state=None, lengths=None):
         x = self._time_major(input)
-        (h0,) = self._initial_state(x, state, 1)
+        fused = self._is_cuda()
+        (h0,) = self._initial_state(x, state, 1, fused)
         zmask = self._zoneout_mask(x)
-        if self._is_cuda():
+        if fused:
             self._check_fused(x)
-            h = _LayerNormIndRNNFunction.apply(self.training, self.zoneout, x.contiguous(), h0,
-                                               self.kernel.contiguous(), self.recurrent_scale.contiguous(),
-                                               self.bias.contiguous(), self.gamma.contiguous(), zmask)
-        else:
-            h = _eager_indrnn(self.training, self.zoneout, x, h0, self.kernel, self.recurrent_scale,
-                              self.bias, zmask, gamma=self.gamma)
+            wanted = self._wanted(lengths, x.device)
+            y, h = self._fused(_LayerNormIndRNNFunction, self.training, self.zoneout, wanted, x.contiguous(), h0,
+                               self.kernel.contiguous(), self.recurrent_scale.contiguous(),
+                               self.bias.contiguous(), self.gamma.contiguous(), zmask)
+            return self._time_major(y), self._fused_state(h)
+        h = _eager_indrnn(self.training, self.zoneout, x, h0, self.kernel, self.recurrent_scale,
+                          self.bias, zmask, gamma=self.gamma)
         return self._time_major(h[1:]), self._final_state(h, lengths)
 
 
@@ -569,19 +666,21 @@ class LayerNormLSTM(_RNNBase):
 
     def forward(self, input, state=None, lengths=None):
         x = self._time_major(input)
-        h0, c0 = self._initial_state(x, state, 2)
+        fused = self._is_cuda()
+        h0, c0 = self._initial_state(x, state, 2, fused)
         dmask, dscale = self._dropconnect_mask(self.recurrent_kernel)
         R = _dropped(self.recurrent_kernel, dmask, dscale)
         zmask = self._zoneout_mask(x)
-        if self._is_cuda():
+        if fused:
             self._check_fused(x)
-            h, c = _LayerNormLSTMFunction.apply(self.training, self.zoneout, x.contiguous(), h0, c0,
-                                                self.kernel.contiguous(), R.contiguous(),
-                                                self.bias.contiguous(), self.gamma.contiguous(),
-                                                self.gamma_h.contiguous(), self.beta_h.contiguous(), zmask)
-        else:
-            h, c = _eager_lstm(self.training, self.zoneout, x, h0, c0, self.kernel, R, self.bias, zmask,
-                               gamma=self.gamma, gamma_h=self.gamma_h, beta_h=self.beta_h)
+            wanted = self._wanted(lengths, x.device)
+            y, h, c = self._fused(_LayerNormLSTMFunction, self.training, self.zoneout, wanted, x.contiguous(), h0, c0,
+                                  self.kernel.contiguous(), R.contiguous(),
+                                  self.bias.contiguous(), self.gamma.contiguous(),
+                                  self.gamma_h.contiguous(), self.beta_h.contiguous(), zmask)
+            return self._time_major(y), (self._fused_state(h), self._fused_state(c))
+        h, c = _eager_lstm(self.training, self.zoneout, x, h0, c0, self.kernel, R, self.bias, zmask,
+                           gamma=self.gamma, gamma_h=self.gamma_h, beta_h=self.beta_h)
         return self._time_major(h[1:]), (self._final_state(h, lengths), self._final_state(c, lengths))
 
 
@@ -609,17 +708,19 @@ class LayerNormGRU(_RNNBase):
 
     def forward(self, input, state=None, lengths=None):
         x = self._time_major(input)
-        (h0,) = self._initial_state(x, state, 1)
+        fused = self._is_cuda()
+        (h0,) = self._initial_state(x, state, 1, fused)
         dmask, dscale = self._dropconnect_mask(self.recurrent_kernel)
         R = _dropped(self.recurrent_kernel, dmask, dscale)
         zmask = self._zoneout_mask(x)
-        if self._is_cuda():
+        if fused:
             self._check_fused(x)
-            h = _LayerNormGRUFunction.apply(self.training, self.zoneout, x.contiguous(), h0,
-                                            self.kernel.contiguous(), R.contiguous(),
-                                            self.bias.contiguous(), self.recurrent_bias.contiguous(),
-                                            self.gamma.contiguous(), zmask)
-        else:
-            h = _eager_gru(self.training, self.zoneout, x, h0, self.kernel, R, self.bias,
-                           self.recurrent_bias, zmask, gamma=self.gamma)
+            wanted = self._wanted(lengths, x.device)
+            y, h = self._fused(_LayerNormGRUFunction, self.training, self.zoneout, wanted, x.contiguous(), h0,
+                               self.kernel.contiguous(), R.contiguous(),
+                               self.bias.contiguous(), self.recurrent_bias.contiguous(),
+                               self.gamma.contiguous(), zmask)
+            return self._time_major(y), self._fused_state(h)
+        h = _eager_gru(self.training, self.zoneout, x, h0, self.kernel, R, self.bias,
+                       self.recurrent_bias, zmask, gamma=self.gamma)
         return self._time_major(h[1:]), self._final_state(h, lengths)

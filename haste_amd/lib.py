@@ -4,8 +4,11 @@ The library must have been built (python -m haste_amd.build); there is no fallba
 loading fails loudly when it is missing.
 """
 import ctypes
+import functools
 import os
 import re
+
+import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libhaste_hip.so")
@@ -49,30 +52,41 @@ def load():
     return lib
 
 
-def _arg(a):
-    import torch
-    if a is None:
-        return ctypes.c_void_p(0)
-    if isinstance(a, torch.Tensor):
-        return ctypes.c_void_p(a.data_ptr())
-    if isinstance(a, bool):
-        return ctypes.c_int(int(a))
-    if isinstance(a, int):
-        return ctypes.c_int(a)
-    if isinstance(a, float):
-        return ctypes.c_float(a)
-    raise TypeError("unsupported argument type %r" % type(a))
+_TYPES = {"int": ctypes.c_int, "float": ctypes.c_float, "size_t": ctypes.c_size_t}
+_entries = {}
+
+
+def entry(name):
+    """Entry point `name` with the argument types its declaration in include/haste_hip.h has: the
+    arguments of a call are then converted by ctypes itself (a wrapper object per argument, made in
+    Python, costs more than the rest of a short call).  None when the library has no such entry."""
+    fn = _entries.get(name)
+    if fn is None:
+        try:
+            fn = load()[name]  # a function object of this module's own: its argument types are nobody else's
+        except AttributeError:
+            return None
+        fn.restype = ctypes.c_int
+        fn.argtypes = [ctypes.c_void_p if "*" in p else _TYPES[p.split()[-2]] for p in _parameters()[name]]
+        _entries[name] = fn
+    return fn
+
+
+@functools.lru_cache(maxsize=None)
+def _parameters():
+    with open(HEADER_PATH) as f:
+        text = re.sub(r"/\*.*?\*/", "", f.read(), flags=re.S)
+    found = re.findall(r"\b(haste_hip_[a-z0-9_]+)\s*\(([^()]*)\)", text)
+    return {name: [p.strip() for p in params.split(",")] for name, params in found}
 
 
 def call(name, *args, stream=None):
-    """Calls entry point `name` with ints/floats/tensors(None = NULL) plus the stream."""
-    import torch
-    lib = load()
-    fn = getattr(lib, name)
-    fn.restype = ctypes.c_int
+    """Calls entry point `name` with ints/floats/tensors/addresses (None = NULL) plus the stream."""
+    fn = entry(name)
+    if fn is None:
+        raise AttributeError("libhaste_hip.so has no entry point " + name)
     if stream is None:
         stream = torch.cuda.current_stream().cuda_stream
-    cargs = [_arg(a) for a in args] + [ctypes.c_void_p(stream)]
-    rc = fn(*cargs)
+    rc = fn(*[a.data_ptr() if isinstance(a, torch.Tensor) else a for a in args], stream)
     if rc != 0:
         raise HasteHipError(rc, name)

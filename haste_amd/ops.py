@@ -14,11 +14,13 @@ from . import lib
 def _check(*tensors):
     # reference frameworks/pytorch/support.h:20-22 (CHECK_INPUT)
     for t in tensors:
+        if t is None:
+            continue
         if not t.is_cuda:
             raise ValueError("tensor must be a GPU tensor")
         if not t.is_contiguous():
             raise ValueError("tensor must be contiguous")
-        if t.numel() and t.dtype not in _SUFFIX:
+        if t.dtype not in _SUFFIX and t.numel():
             raise ValueError("only float32, float64 and (GRU) float16 are implemented")
 
 
@@ -29,11 +31,17 @@ def _call(entry, *args):
     """Calls `entry` + "_f32" / "_f64" according to the tensors among `args`, which must all
     have one dtype (the reference's bindings dispatch the same way, AT_DISPATCH_FLOATING_TYPES,
     frameworks/pytorch/lstm.cc:65)."""
-    dtypes = {a.dtype for a in args if isinstance(a, torch.Tensor) and a.numel()}
-    if len(dtypes) != 1:
-        raise ValueError("all tensors of a call must have the same dtype, got %s" % sorted(map(str, dtypes)))
-    name = entry + _SUFFIX[dtypes.pop()]
-    if not hasattr(lib.load(), name):
+    dtype = None
+    for a in args:
+        if isinstance(a, torch.Tensor) and a.dtype is not dtype and a.numel():
+            if dtype is not None:
+                dtypes = {t.dtype for t in args if isinstance(t, torch.Tensor) and t.numel()}
+                raise ValueError("all tensors of a call must have the same dtype, got %s" % sorted(map(str, dtypes)))
+            dtype = a.dtype
+    if dtype is None:
+        raise ValueError("all tensors of a call must have the same dtype, got []")
+    name = entry + _SUFFIX[dtype]
+    if lib.entry(name) is None:
         # as in the reference, half exists for the GRU only (lib/gru_forward_gpu.cu.cc:373)
         raise ValueError("%s is not implemented" % name)
     lib.call(name, *args)
@@ -114,8 +122,40 @@ def _zeros(opts, *shapes):
     return [flat[a:a + n].view(shp) for a, n, shp in zip(starts, sizes, shapes)]
 
 
+def _given(mask):
+    return mask is not None and mask.numel() > 0
+
+
 def _mask_or_none(has_zoneout, zoneout_mask):
     return zoneout_mask if has_zoneout else None
+
+
+def _first_states(T, N, H, first, opts):
+    """State sequences [T+1,N,H], one per tensor in `first`, with slot 0 preset to it (None: zeros) by
+    one kernel for all of them."""
+    seqs = [torch.empty(T + 1, N, H, **opts) for _ in first]
+    given = [(q[0], f) for q, f in zip(seqs, first) if f is not None]
+    empty = [q[0] for q, f in zip(seqs, first) if f is None]
+    if given:
+        torch._foreach_copy_([q for q, _ in given], [f for _, f in given])
+    if empty:
+        torch._foreach_zero_(empty)
+    return seqs
+
+
+def _upstream(grad, T):
+    """The address a backward entry point takes for the gradients of the states: it expects
+    [T+1,N,H] and reads slots 1 .. T, so gradients [T,N,H] of the states after each step are handed
+    over as they are, with the address of the slot before them."""
+    if grad is None or grad.shape[0] == T + 1:
+        return grad
+    return grad.data_ptr() - grad[0].numel() * grad.element_size()
+
+
+def _carried(opts, *pairs):
+    """_zeros() of the shapes in `pairs` of (shape, initial value or None)."""
+    out = _zeros(opts, *[shape for shape, start in pairs if start is None])
+    return [out.pop(0) if start is None else start.clone() for _, start in pairs]
 
 
 def gemm(a, b, out=None, trans_a=False, accumulate=False):
@@ -145,20 +185,17 @@ def transpose(a, out=None):
 
 
 def transpose3(a, b, c):
-    """transpose() of three float32 tensors in one launch: the x_t, W_t, R_t a backward pass asks
-    its caller for (reference frameworks/pytorch/lstm.py:84-86)."""
+    """transpose() of three tensors in one launch: the x_t, W_t, R_t a backward pass asks its caller
+    for (reference frameworks/pytorch/lstm.py:84-86)."""
+    _check(a, b, c)
     outs = []
     args = []
     for m in (a, b, c):
-        _check(m)
-        if m.dtype != torch.float32:
-            return transpose(a), transpose(b), transpose(c)
         cols = m.shape[-1]
-        rows = m.numel() // cols
         out = torch.empty((cols,) + tuple(m.shape[:-1]), device=m.device, dtype=m.dtype)
         outs.append(out)
-        args += [rows, cols, m, out]
-    lib.call("haste_hip_transpose3_f32", *args)
+        args += [m.numel() // cols, cols, m, out]
+    _call("haste_hip_transpose3", *args)
     return tuple(outs)
 
 
@@ -167,13 +204,11 @@ def lstm_forward(training, zoneout_prob, x, h0, c0, kernel, recurrent_kernel, bi
                  dropconnect_mask=None, dropconnect_scale=1.0):
     T, N, C = x.shape
     H = recurrent_kernel.shape[0]
-    has_zoneout = bool(zoneout_prob) and zoneout_mask.numel() > 0
+    has_zoneout = bool(zoneout_prob) and _given(zoneout_mask)
     _check(x, h0, c0, kernel, recurrent_kernel, bias, zoneout_mask)
     opts = dict(device=x.device, dtype=x.dtype)
-    output = torch.empty(T + 1, N, H, **opts)
-    output_state = torch.empty(T + 1, N, H, **opts)
+    output, output_state = _first_states(T, N, H, (h0, c0), opts)
     cache = torch.empty(T, N, 4 * H, **opts)
-    torch._foreach_copy_([output[0], output_state[0]], [h0, c0])  # one kernel for both
     zp = float(zoneout_prob) if has_zoneout else 0.0
     mask = _mask_or_none(has_zoneout, zoneout_mask)
     if dropconnect_mask is None:
@@ -187,16 +222,20 @@ def lstm_forward(training, zoneout_prob, x, h0, c0, kernel, recurrent_kernel, bi
     return output, output_state, cache
 
 
-def lstm_backward(x_t, kernel_t, recurrent_kernel_t, bias, zoneout_mask, h, c, cache, dh_new, dc_new):
+def lstm_backward(x_t, kernel_t, recurrent_kernel_t, bias, zoneout_mask, h, c, cache, dh_new, dc_new,
+                  dh_last=None, dc_last=None):
+    """dh_new, dc_new: gradients of the states, [T+1,N,H] (slot 0 is not read) or [T,N,H]; dc_new may
+    be None (zeros).  dh_last, dc_last: more gradient of the last states, [N,H]."""
     C, T, N = x_t.shape
     H = recurrent_kernel_t.shape[1]
-    has_zoneout = zoneout_mask.numel() > 0
+    has_zoneout = _given(zoneout_mask)
     _check(x_t, kernel_t, recurrent_kernel_t, bias, zoneout_mask, h, c, cache, dh_new, dc_new)
     opts = dict(device=x_t.device, dtype=x_t.dtype)
     dx = torch.empty(T, N, C, **opts)
-    dW, dR, db, dh, dc = _zeros(opts, (C, 4 * H), (H, 4 * H), (4 * H,), (N, H), (N, H))
+    dW, dR, db, dh, dc = _carried(opts, ((C, 4 * H), None), ((H, 4 * H), None), ((4 * H,), None),
+                                  ((N, H), dh_last), ((N, H), dc_last))
     _call("haste_hip_lstm_backward", T, N, C, H, kernel_t, recurrent_kernel_t, bias, x_t,
-             h, c, dh_new, dc_new, dx, dW, dR, db, dh, dc, cache,
+             h, c, _upstream(dh_new, T), _upstream(dc_new, T), dx, dW, dR, db, dh, dc, cache,
              _mask_or_none(has_zoneout, zoneout_mask))
     return dx, dh, dc, dW, dR, db
 
@@ -271,13 +310,12 @@ def gru_forward(training, zoneout_prob, x, h0, kernel, recurrent_kernel, bias, r
                 zoneout_mask, dropconnect_mask=None, dropconnect_scale=1.0):
     T, N, C = x.shape
     H = recurrent_kernel.shape[0]
-    has_zoneout = bool(zoneout_prob) and zoneout_mask.numel() > 0
+    has_zoneout = bool(zoneout_prob) and _given(zoneout_mask)
     _check(x, h0, kernel, recurrent_kernel, bias, recurrent_bias, zoneout_mask)
     opts = dict(device=x.device, dtype=x.dtype)
-    output = torch.empty(T + 1, N, H, **opts)
+    (output,) = _first_states(T, N, H, (h0,), opts)
     cache = torch.empty(T, N, 4 * H, **opts)
     tmp_Wx = torch.empty(T, N, 3 * H, **opts)
-    output[0] = h0
     zp = float(zoneout_prob) if has_zoneout else 0.0
     mask = _mask_or_none(has_zoneout, zoneout_mask)
     if dropconnect_mask is None:
@@ -292,18 +330,19 @@ def gru_forward(training, zoneout_prob, x, h0, kernel, recurrent_kernel, bias, r
 
 
 def gru_backward(x_t, kernel_t, recurrent_kernel_t, bias, recurrent_bias, zoneout_mask, h, cache,
-                 dh_new):
+                 dh_new, dh_last=None):
     C, T, N = x_t.shape
     H = recurrent_kernel_t.shape[1]
-    has_zoneout = zoneout_mask.numel() > 0
+    has_zoneout = _given(zoneout_mask)
     _check(x_t, kernel_t, recurrent_kernel_t, bias, recurrent_bias, zoneout_mask, h, cache, dh_new)
     opts = dict(device=x_t.device, dtype=x_t.dtype)
     dx = torch.empty(T, N, C, **opts)
-    dW, dR, dbx, dbr, dh = _zeros(opts, (C, 3 * H), (H, 3 * H), (3 * H,), (3 * H,), (N, H))
+    dW, dR, dbx, dbr, dh = _carried(opts, ((C, 3 * H), None), ((H, 3 * H), None), ((3 * H,), None),
+                                    ((3 * H,), None), ((N, H), dh_last))
     dp = torch.empty(T, N, 3 * H, **opts)
     dq = torch.empty(T, N, 3 * H, **opts)
     _call("haste_hip_gru_backward", T, N, C, H, kernel_t, recurrent_kernel_t, bias,
-             recurrent_bias, x_t, h, cache, dh_new, dx, dW, dR, dbx, dbr, dh, dp, dq,
+             recurrent_bias, x_t, h, cache, _upstream(dh_new, T), dx, dW, dR, dbx, dbr, dh, dp, dq,
              _mask_or_none(has_zoneout, zoneout_mask))
     return dx, dh, dW, dR, dbx, dbr
 
@@ -332,29 +371,28 @@ def layer_norm_backward(x, gamma, dy, cache=None, with_beta=True, in_place=False
 def indrnn_forward(training, zoneout_prob, x, h0, kernel, recurrent_scale, bias, zoneout_mask):
     T, N, C = x.shape
     H = recurrent_scale.shape[0]
-    has_zoneout = bool(zoneout_prob) and zoneout_mask.numel() > 0
+    has_zoneout = bool(zoneout_prob) and _given(zoneout_mask)
     _check(x, h0, kernel, recurrent_scale, bias, zoneout_mask)
     opts = dict(device=x.device, dtype=x.dtype)
-    output = torch.empty(T + 1, N, H, **opts)
+    (output,) = _first_states(T, N, H, (h0,), opts)
     workspace = torch.empty(T, N, H, **opts)
-    output[0] = h0
     _call("haste_hip_indrnn_forward", bool(training), T, N, C, H, kernel, recurrent_scale,
              bias, x, output, workspace, float(zoneout_prob) if has_zoneout else 0.0,
              _mask_or_none(has_zoneout, zoneout_mask))
     return output
 
 
-def indrnn_backward(x_t, kernel_t, recurrent_scale, bias, zoneout_mask, h, dh_new):
+def indrnn_backward(x_t, kernel_t, recurrent_scale, bias, zoneout_mask, h, dh_new, dh_last=None):
     C, T, N = x_t.shape
     H = recurrent_scale.shape[0]
-    has_zoneout = zoneout_mask.numel() > 0
+    has_zoneout = _given(zoneout_mask)
     _check(x_t, kernel_t, recurrent_scale, bias, zoneout_mask, h, dh_new)
     opts = dict(device=x_t.device, dtype=x_t.dtype)
     dx = torch.empty(T, N, C, **opts)
-    dW, du, db, dh = _zeros(opts, (C, H), (H,), (H,), (N, H))
+    dW, du, db, dh = _carried(opts, ((C, H), None), ((H,), None), ((H,), None), ((N, H), dh_last))
     workspace = torch.empty(T, N, H, **opts)
     _call("haste_hip_indrnn_backward", T, N, C, H, kernel_t, recurrent_scale, bias, x_t, h,
-             dh_new, dx, dW, du, db, dh, workspace, _mask_or_none(has_zoneout, zoneout_mask))
+             _upstream(dh_new, T), dx, dW, du, db, dh, workspace, _mask_or_none(has_zoneout, zoneout_mask))
     return dx, dh, dW, du, db
 
 
@@ -363,14 +401,13 @@ def layer_norm_indrnn_forward(training, zoneout_prob, x, h0, kernel, recurrent_s
                               zoneout_mask):
     T, N, C = x.shape
     H = recurrent_scale.shape[0]
-    has_zoneout = bool(zoneout_prob) and zoneout_mask.numel() > 0
+    has_zoneout = bool(zoneout_prob) and _given(zoneout_mask)
     _check(x, h0, kernel, recurrent_scale, bias, gamma, zoneout_mask)
     opts = dict(device=x.device, dtype=x.dtype)
-    output = torch.empty(T + 1, N, H, **opts)
+    (output,) = _first_states(T, N, H, (h0,), opts)
     workspace = torch.empty(T, N, H, **opts)
     act_Wx = torch.empty(T, N, H, **opts)
     act_Wx_norm_cache = torch.empty(T, N, 2, **opts)
-    output[0] = h0
     _call("haste_hip_layer_norm_indrnn_forward", bool(training), T, N, C, H, kernel,
              recurrent_scale, bias, x, output, workspace, act_Wx, gamma[0], act_Wx_norm_cache,
              float(zoneout_prob) if has_zoneout else 0.0, _mask_or_none(has_zoneout, zoneout_mask))
@@ -378,18 +415,18 @@ def layer_norm_indrnn_forward(training, zoneout_prob, x, h0, kernel, recurrent_s
 
 
 def layer_norm_indrnn_backward(x_t, kernel_t, recurrent_scale, bias, gamma, zoneout_mask, h, act_Wx,
-                               act_Wx_norm_cache, dh_new):
+                               act_Wx_norm_cache, dh_new, dh_last=None):
     C, T, N = x_t.shape
     H = recurrent_scale.shape[0]
-    has_zoneout = zoneout_mask.numel() > 0
+    has_zoneout = _given(zoneout_mask)
     _check(x_t, kernel_t, recurrent_scale, bias, gamma, zoneout_mask, h, act_Wx, dh_new)
     opts = dict(device=x_t.device, dtype=x_t.dtype)
     dx = torch.empty(T, N, C, **opts)
-    dW, du, db, dh = _zeros(opts, (C, H), (H,), (H,), (N, H))
+    dW, du, db, dh = _carried(opts, ((C, H), None), ((H,), None), ((H,), None), ((N, H), dh_last))
     workspace = torch.empty(T, N, H, **opts)
     dgamma = torch.zeros_like(gamma)
     _call("haste_hip_layer_norm_indrnn_backward", T, N, C, H, kernel_t, recurrent_scale, bias,
-             x_t, h, dh_new, dx, dW, du, db, dh, workspace, act_Wx, gamma[0], dgamma[0],
+             x_t, h, _upstream(dh_new, T), dx, dW, du, db, dh, workspace, act_Wx, gamma[0], dgamma[0],
              _mask_or_none(has_zoneout, zoneout_mask))
     return dx, dh, dW, du, db, dgamma
 
@@ -399,11 +436,10 @@ def layer_norm_lstm_forward(training, zoneout_prob, x, h0, c0, kernel, recurrent
                             gamma, gamma_h, beta_h, zoneout_mask):
     T, N, C = x.shape
     H = recurrent_kernel.shape[0]
-    has_zoneout = bool(zoneout_prob) and zoneout_mask.numel() > 0
+    has_zoneout = bool(zoneout_prob) and _given(zoneout_mask)
     _check(x, h0, c0, kernel, recurrent_kernel, bias, gamma, gamma_h, beta_h, zoneout_mask)
     opts = dict(device=x.device, dtype=x.dtype)
-    output = torch.empty(T + 1, N, H, **opts)
-    output_state = torch.empty(T + 1, N, H, **opts)
+    output, output_state = _first_states(T, N, H, (h0, c0), opts)
     act_Wx = torch.empty(T, N, 4 * H, **opts)
     act_Wx_norm = torch.empty(T, N, 4 * H, **opts)
     act_Wx_norm_cache = torch.empty(T, N, 2, **opts)
@@ -411,8 +447,6 @@ def layer_norm_lstm_forward(training, zoneout_prob, x, h0, c0, kernel, recurrent
     act_Rh_norm_cache = torch.empty(T, N, 2, **opts)
     act_c_norm = torch.empty(T, N, H, **opts)
     act_c_norm_cache = torch.empty(T, N, 2, **opts)
-    output[0] = h0
-    output_state[0] = c0
     _call("haste_hip_layer_norm_lstm_forward", bool(training), T, N, C, H, kernel,
              recurrent_kernel, bias, x, output, output_state, act_Wx, None,
              gamma[0], act_Wx_norm_cache, act_Wx_norm, act_Rh, gamma[1], act_Rh_norm_cache,
@@ -424,19 +458,21 @@ def layer_norm_lstm_forward(training, zoneout_prob, x, h0, c0, kernel, recurrent
 
 def layer_norm_lstm_backward(x_t, kernel_t, recurrent_kernel_t, bias, gamma, gamma_h, beta_h,
                              zoneout_mask, h, c, act_Wx, act_Wx_norm, act_Wx_norm_cache, act_Rh,
-                             act_Rh_norm_cache, act_c_norm, act_c_norm_cache, dh_new, dc_new):
+                             act_Rh_norm_cache, act_c_norm, act_c_norm_cache, dh_new, dc_new,
+                             dh_last=None, dc_last=None):
     C, T, N = x_t.shape
     H = recurrent_kernel_t.shape[1]
-    has_zoneout = zoneout_mask.numel() > 0
+    has_zoneout = _given(zoneout_mask)
     _check(x_t, kernel_t, recurrent_kernel_t, bias, gamma, gamma_h, beta_h, zoneout_mask, h, c,
            act_Wx, act_Wx_norm, act_Wx_norm_cache, act_Rh, act_Rh_norm_cache, act_c_norm,
            act_c_norm_cache, dh_new, dc_new)
     opts = dict(device=x_t.device, dtype=x_t.dtype)
     dx = torch.empty(T, N, C, **opts)
-    dW, dR, db, dgamma, dgamma_h, dbeta_h, dh, dc = _zeros(
-        opts, (C, 4 * H), (H, 4 * H), (4 * H,), tuple(gamma.shape), (H,), (H,), (N, H), (N, H))
+    dW, dR, db, dgamma, dgamma_h, dbeta_h, dh, dc = _carried(
+        opts, ((C, 4 * H), None), ((H, 4 * H), None), ((4 * H,), None), (tuple(gamma.shape), None),
+        ((H,), None), ((H,), None), ((N, H), dh_last), ((N, H), dc_last))
     _call("haste_hip_layer_norm_lstm_backward", T, N, C, H, kernel_t, recurrent_kernel_t,
-             bias, x_t, h, c, dh_new, dc_new, dx, dW, dR, db, dh, dc,
+             bias, x_t, h, c, _upstream(dh_new, T), _upstream(dc_new, T), dx, dW, dR, db, dh, dc,
              act_Wx, gamma[0], dgamma[0], act_Wx_norm, act_Rh, gamma[1], dgamma[1],
              act_Rh_norm_cache, gamma_h, beta_h, dgamma_h, dbeta_h, act_c_norm_cache, act_c_norm,
              _mask_or_none(has_zoneout, zoneout_mask))
@@ -448,17 +484,16 @@ def layer_norm_gru_forward(training, zoneout_prob, x, h0, kernel, recurrent_kern
                            recurrent_bias, gamma, zoneout_mask):
     T, N, C = x.shape
     H = recurrent_kernel.shape[0]
-    has_zoneout = bool(zoneout_prob) and zoneout_mask.numel() > 0
+    has_zoneout = bool(zoneout_prob) and _given(zoneout_mask)
     _check(x, h0, kernel, recurrent_kernel, bias, recurrent_bias, gamma, zoneout_mask)
     opts = dict(device=x.device, dtype=x.dtype)
-    output = torch.empty(T + 1, N, H, **opts)
+    (output,) = _first_states(T, N, H, (h0,), opts)
     cache = torch.empty(T, N, 4 * H, **opts)
     act_Wx = torch.empty(T, N, 3 * H, **opts)
     tmp_Wx_norm = torch.empty(T, N, 3 * H, **opts)
     act_Wx_norm_cache = torch.empty(T, N, 2, **opts)
     act_Rh = torch.empty(T, N, 3 * H, **opts)
     act_Rh_norm_cache = torch.empty(T, N, 2, **opts)
-    output[0] = h0
     _call("haste_hip_layer_norm_gru_forward", bool(training), T, N, C, H, kernel,
              recurrent_kernel, bias, recurrent_bias, x, output, cache if training else None,
              act_Wx, gamma[0], act_Wx_norm_cache, tmp_Wx_norm, act_Rh, gamma[1], act_Rh_norm_cache,
@@ -469,20 +504,20 @@ def layer_norm_gru_forward(training, zoneout_prob, x, h0, kernel, recurrent_kern
 
 def layer_norm_gru_backward(x_t, kernel_t, recurrent_kernel_t, bias, recurrent_bias, gamma,
                             zoneout_mask, h, cache, act_Wx, act_Wx_norm_cache, act_Rh,
-                            act_Rh_norm_cache, dh_new):
+                            act_Rh_norm_cache, dh_new, dh_last=None):
     C, T, N = x_t.shape
     H = recurrent_kernel_t.shape[1]
-    has_zoneout = zoneout_mask.numel() > 0
+    has_zoneout = _given(zoneout_mask)
     _check(x_t, kernel_t, recurrent_kernel_t, bias, recurrent_bias, gamma, zoneout_mask, h, cache,
            act_Wx, act_Wx_norm_cache, act_Rh, act_Rh_norm_cache, dh_new)
     opts = dict(device=x_t.device, dtype=x_t.dtype)
     dx = torch.empty(T, N, C, **opts)
-    dW, dR, dbx, dbr, dh, dgamma = _zeros(opts, (C, 3 * H), (H, 3 * H), (3 * H,), (3 * H,), (N, H),
-                                          tuple(gamma.shape))
+    dW, dR, dbx, dbr, dh, dgamma = _carried(opts, ((C, 3 * H), None), ((H, 3 * H), None), ((3 * H,), None),
+                                            ((3 * H,), None), ((N, H), dh_last), (tuple(gamma.shape), None))
     dp = torch.empty(T, N, 3 * H, **opts)
     dq = torch.empty(T, N, 3 * H, **opts)
     _call("haste_hip_layer_norm_gru_backward", T, N, C, H, kernel_t, recurrent_kernel_t, bias,
-             recurrent_bias, x_t, h, cache, dh_new, dx, dW, dR, dbx, dbr, dh, dp, dq,
+             recurrent_bias, x_t, h, cache, _upstream(dh_new, T), dx, dW, dR, dbx, dbr, dh, dp, dq,
              act_Wx, gamma[0], dgamma[0], act_Rh, gamma[1], dgamma[1], act_Rh_norm_cache,
              _mask_or_none(has_zoneout, zoneout_mask))
     return dx, dh, dW, dR, dbx, dbr, dgamma

@@ -168,7 +168,9 @@ int haste_hip_lstm_forward_dropconnect_f32(int training, int steps, int batch_si
  * W_t[4H,C] R_t[4H,H] b[4H] (unused) x_t[C,T,N] h,c[T+1,N,H] dh_new,dc_new[T+1,N,H]
  * dx[T,N,C] (assigned) dW[C,4H] dR[H,4H] db[4H] (accumulated into) dh,dc[N,H] (in/out,
  * zero on entry, d h0 / d c0 on return) v[T,N,4H] (in: activations, out: gate gradients)
- * zoneout_mask[T,N,H] or NULL. */
+ * zoneout_mask[T,N,H] or NULL.  In this and every other backward entry point slot 0 of dh_new and
+ * dc_new is never read; dc_new may be NULL (no gradient enters through the cell states); what
+ * dh, dc hold on entry counts as further gradient of the last states. */
 int haste_hip_lstm_backward_f32(int steps, int batch_size, int input_size, int hidden_size,
                                 const float* W_t, const float* R_t, const float* b,
                                 const float* x_t, const float* h, const float* c,
@@ -399,6 +401,9 @@ int haste_hip_gemm_f64(int trans_a, int M, int N, int K,
                        const double* A, int lda, const double* B, int ldb,
                        double* C, int ldc, int accumulate, void* stream);
 int haste_hip_transpose_f64(int rows, int cols, const double* in, double* out, void* stream);
+int haste_hip_transpose3_f64(int rows0, int cols0, const double* in0, double* out0,
+                             int rows1, int cols1, const double* in1, double* out1,
+                             int rows2, int cols2, const double* in2, double* out2, void* stream);
 int haste_hip_lstm_forward_f64(int training, int steps, int batch_size, int input_size,
                                int hidden_size,
                                const double* W, const double* R, const double* b, const double* x,
@@ -555,6 +560,9 @@ int haste_hip_layer_norm_indrnn_backward_f64(int steps, int batch_size, int inpu
 int haste_hip_gemm_f16(int trans_a, int M, int N, int K, const void* A, int lda, const void* B,
                        int ldb, void* C, int ldc, int accumulate, void* stream);
 int haste_hip_transpose_f16(int rows, int cols, const void* in, void* out, void* stream);
+int haste_hip_transpose3_f16(int rows0, int cols0, const void* in0, void* out0,
+                             int rows1, int cols1, const void* in1, void* out1,
+                             int rows2, int cols2, const void* in2, void* out2, void* stream);
 /* C[M,N] (+)= A[M,K] * Bt[N,K]^T with fp32 accumulation and an fp32 result: the product kernel
  * of the half GRU's passes over more than one step.  Bt holds IEEE binary16 values, A binary16
  * or (a_is_float != 0) fp32 values that are rounded to half as they are read; both have the

@@ -97,6 +97,10 @@ def test_three_transposes_in_one_launch(shapes):
     outs = ops.transpose3(*ms)
     for m, out in zip(ms, outs):
         assert torch.equal(out, ops.transpose(m))
+    for dtype in (torch.float64, torch.float16):
+        cast = [m.to(dtype) for m in ms]
+        for m, out in zip(cast, ops.transpose3(*cast)):
+            assert torch.equal(out, ops.transpose(m))
 
 
 @pytest.mark.parametrize("trans_a", [True, False])

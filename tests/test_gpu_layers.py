@@ -256,3 +256,51 @@ def test_self_consistency_fused_vs_plain_loop(name, regularised):
         for k, p in rnn.named_parameters():
             ref = p.grad
             assert float((grads1[k] - ref).abs().max()) < 2e-3 * max(float(ref.abs().max()), 1e-6), k
+
+
+@pytest.mark.parametrize("name,dtype,H", [
+    (n, d, h) for n in ("LSTM", "GRU", "IndRNN", "LayerNormLSTM", "LayerNormGRU", "LayerNormIndRNN")
+    for d, h in ((torch.float32, 24), (torch.float64, 24), (torch.float32, 300))] + [
+    ("LSTM", torch.float32, 1200), ("LayerNormLSTM", torch.float32, 1200), ("GRU", torch.float16, 64)])
+@pytest.mark.parametrize("wanted", ["last", "lengths", "all"])
+@pytest.mark.parametrize("through", ["y", "state", "both"])
+def test_gradients_enter_through_every_output(name, dtype, H, wanted, through):
+    """Gradients of the outputs, of the final states (at the sequences' ends, or at lengths), of the state
+    sequences and of their combinations, against the plain loop on the CPU in double: the fused
+    backward passes take them without a [T+1,N,H] sequence being made of them."""
+    T, N, C = 5, 3, 8
+    torch.manual_seed(11)
+    layer = getattr(haste_amd, name)(C, H, return_state_sequence=wanted == "all", batch_first=wanted == "all")
+    layer = layer.to(dtype)
+    ref = getattr(haste_amd, name)(C, H, return_state_sequence=wanted == "all", batch_first=wanted == "all").double()
+    ref.load_state_dict(layer.state_dict())
+    layer = layer.cuda()
+    x = torch.randn(*((N, T, C) if wanted == "all" else (T, N, C))).to(dtype)
+    lengths = [5, 1, 3] if wanted == "lengths" else None
+    results = []
+    for net, at in ((layer, x.cuda()), (ref, x.double())):
+        at.requires_grad_(True)
+        y, state = net(at, lengths=lengths)
+        states = state if isinstance(state, tuple) else (state,)
+        outs = ([y] if through != "state" else []) + (list(states) if through != "y" else [])
+        g = torch.Generator().manual_seed(4)
+        torch.autograd.backward(outs, [torch.randn(o.shape, generator=g).to(o) for o in outs])
+        results.append([y, *states, at.grad] + [p.grad for p in net.parameters()])
+    print(name, dtype, H, wanted, through, flush=True)
+    for got, want in zip(*results):
+        if want is None or got is None:
+            assert want is None or not want.abs().max()
+            continue
+        assert relerr(npy(got), npy(want)) < {torch.float32: TOL, torch.float64: 1e-10, torch.float16: 2e-2}[dtype]
+
+
+def test_outputs_that_are_changed_are_noticed():
+    """The outputs share memory with what the backward pass reads."""
+    layer = haste_amd.LSTM(4, 8).cuda()
+    for which in ("y", "h", "c"):
+        y, (h, c) = layer(torch.randn(3, 2, 4, device="cuda", requires_grad=True))
+        loss = (y * y).sum()
+        with torch.no_grad():
+            {"y": y, "h": h, "c": c}[which].add_(1.0)
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            loss.backward()
