@@ -29,6 +29,20 @@ int gemm_f64(hipStream_t stream, bool trans_a, int M, int N, int K, const double
 size_t gemm_f64_scratch_bytes(int M, int N, int K);
 int gemm_f64_chunks(hipStream_t stream, int M, int N, int K, const double* A, int lda, const double* B,
                     int ldb, size_t scratch_offset, const double** partial, int* chunks);
+// recurrent_f64.hip: all steps of the double LSTM and GRU in one launch.
+size_t recurrence64_scratch_bytes(int in_gates, int out_gates, int steps, int N, int H);
+int lstm_forward_recurrence64(hipStream_t stream, int training, int T, int N, int H, const double* R, const double* b,
+                              const double* h, const double* c, double* h_out, double* c_out, double* v,
+                              float zoneout_prob, const double* mask, void* exchange);
+int gru_forward_recurrence64(hipStream_t stream, int training, int T, int N, int H, const double* R, const double* bx,
+                             const double* br, const double* h, const double* wx, double* h_out, double* v,
+                             float zoneout_prob, const double* mask, void* exchange);
+int lstm_backward_recurrence64(hipStream_t stream, int T, int N, int H, const double* R_t, const double* c,
+                               const double* c_next, const double* dh_next, const double* dc_next, double* dh,
+                               double* dc, double* v, const double* mask, void* exchange);
+int gru_backward_recurrence64(hipStream_t stream, int T, int N, int H, const double* R_t, const double* h,
+                              const double* v, const double* dh_next, double* dh, double* dp, double* dq,
+                              const double* mask, void* exchange);
 int gemm_f16(hipStream_t stream, bool trans_a, int M, int N, int K, const void* A, int lda,
              const void* B, int ldb, void* C, int ldc, bool accumulate);
 // gru_half.hip: the half GRU over more than one step, on the fp32 kernels.
@@ -273,6 +287,25 @@ int open_scratch(hipStream_t stream, size_t own_bytes, size_t gemm_bytes, Scratc
   sc->used = 0;
   sc->own = own_bytes;
   return HASTE_HIP_OK;
+}
+
+// Scratch for the exchange tiles of a recurrence in one launch (recurrent_f64.hip), 0 when the
+// call runs step by step: always for float (its persistent kernels are the callers of this file),
+// and for double when the shape does not fit the chip, while the stream is being captured (a
+// persistent launch needs a control block that replays wipe, and these calls never had one in
+// their graphs), and in memory lent by the caller that is too small for the tiles.
+template <typename T>
+size_t one_launch_bytes(hipStream_t, int, int, int, int, int, size_t) { return 0; }
+template <>
+size_t one_launch_bytes<double>(hipStream_t stream, int in_gates, int out_gates, int steps, int N, int H, size_t others) {
+  const size_t bytes = padded(recurrence64_scratch_bytes(in_gates, out_gates, steps, N, H));
+  if (bytes == 0) return 0;
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &capture) != hipSuccess) (void)hipGetLastError();
+  if (capture != hipStreamCaptureStatusNone) return 0;
+  Workspace ws;
+  if (get_workspace(stream, 0, &ws) != HASTE_HIP_OK) return 0;
+  return ws.caller_owned && ws.scratch_bytes < others + bytes + 256 ? 0 : bytes;
 }
 
 // ---- small kernels ------------------------------------------------------------------
@@ -771,13 +804,20 @@ int lstm_forward_steps(hipStream_t stream, int training, int steps, int N, int C
                        T* h_out, T* c_out, T* v, float zoneout_prob, const T* zoneout_mask,
                        const T* dc_mask, float dc_scale) {
   const size_t NH = (size_t)N * H, N4H = NH * 4, r_count = (size_t)H * 4 * H;
-  const size_t own = padded(N4H * sizeof(T)) + (dc_mask ? padded(r_count * sizeof(T)) : 0);
+  size_t own = padded(N4H * sizeof(T)) + (dc_mask ? padded(r_count * sizeof(T)) : 0);
+  const size_t room = max2(gemm_room<T>(steps * N, 4 * H, C), gemm_room<T>(N, 4 * H, H));
+  const size_t tiles = one_launch_bytes<T>(stream, 1, 4, steps, N, H, own + room);
+  own += tiles;
   Scratch sc;
-  HASTE_HIP_PROPAGATE(open_scratch(stream, own, max2(gemm_room<T>(steps * N, 4 * H, C), gemm_room<T>(N, 4 * H, H)), &sc));
+  HASTE_HIP_PROPAGATE(open_scratch(stream, own, room, &sc));
   T* rh = sc.take<T>(N4H);
   const T* Ruse;
   HASTE_HIP_PROPAGATE(effective_r(stream, r_count, R, dc_mask, dc_scale, dc_mask ? sc.take<T>(r_count) : nullptr, &Ruse));
   HASTE_HIP_PROPAGATE(gemm(stream, false, steps * N, 4 * H, C, x, C, W, 4 * H, v, 4 * H, false, sc.gemm_offset()));
+  if constexpr (std::is_same<T, double>::value)
+    if (tiles > 0)
+      return lstm_forward_recurrence64(stream, training, steps, N, H, Ruse, b, h, c, h_out, c_out, v, zoneout_prob,
+                                       zoneout_mask, sc.take<char>(tiles));
   ScopedKernelTimer timer("lstm_forward_steps", stream);
   for (int t = 0; t < steps; ++t) {
     const T* h_t = t == 0 ? h : h_out + (size_t)(t - 1) * NH;
@@ -799,13 +839,18 @@ int lstm_backward_steps(hipStream_t stream, int steps, int N, int C, int H, cons
                         T* dc, T* v, const T* zoneout_mask) {
   const size_t NH = (size_t)N * H, N4H = NH * 4;
   const int TN = steps * N;
-  const size_t own = column_sum_bytes<T>((size_t)TN, 4 * H);
+  const size_t sums = column_sum_bytes<T>((size_t)TN, 4 * H);
   size_t room = max2(gemm_room<T>(N, H, 4 * H), gemm_room<T>(C, 4 * H, TN));
   room = max2(room, max2(gemm_room<T>(H, 4 * H, TN), gemm_room<T>(TN, C, 4 * H)));
+  const size_t tiles = one_launch_bytes<T>(stream, 4, 1, steps, N, H, sums + room);
   Scratch sc;
-  HASTE_HIP_PROPAGATE(open_scratch(stream, own, room, &sc));
-  void* partial = sc.take<char>(own);
-  {
+  HASTE_HIP_PROPAGATE(open_scratch(stream, sums + tiles, room, &sc));
+  void* partial = sc.take<char>(sums);
+  if (tiles > 0) {
+    if constexpr (std::is_same<T, double>::value)
+      HASTE_HIP_PROPAGATE(lstm_backward_recurrence64(stream, steps, N, H, R_t, c, c_next, dh_next, dc_next, dh, dc, v,
+                                                     zoneout_mask, sc.take<char>(tiles)));
+  } else {
     ScopedKernelTimer timer("lstm_backward_steps", stream);
     StepProduct<T> pend;
     for (int t = steps - 1; t >= 0; --t) {
@@ -832,13 +877,20 @@ int gru_forward_steps(hipStream_t stream, int training, int steps, int N, int C,
                       T* tmp_Wx, float zoneout_prob, const T* zoneout_mask, const T* dc_mask,
                       float dc_scale) {
   const size_t NH = (size_t)N * H, N3H = NH * 3, N4H = NH * 4, r_count = (size_t)H * 3 * H;
-  const size_t own = padded(N3H * sizeof(T)) + (dc_mask ? padded(r_count * sizeof(T)) : 0);
+  size_t own = padded(N3H * sizeof(T)) + (dc_mask ? padded(r_count * sizeof(T)) : 0);
+  const size_t room = max2(gemm_room<T>(steps * N, 3 * H, C), gemm_room<T>(N, 3 * H, H));
+  const size_t tiles = one_launch_bytes<T>(stream, 1, 3, steps, N, H, own + room);
+  own += tiles;
   Scratch sc;
-  HASTE_HIP_PROPAGATE(open_scratch(stream, own, max2(gemm_room<T>(steps * N, 3 * H, C), gemm_room<T>(N, 3 * H, H)), &sc));
+  HASTE_HIP_PROPAGATE(open_scratch(stream, own, room, &sc));
   T* rh = sc.take<T>(N3H);
   const T* Ruse;
   HASTE_HIP_PROPAGATE(effective_r(stream, r_count, R, dc_mask, dc_scale, dc_mask ? sc.take<T>(r_count) : nullptr, &Ruse));
   HASTE_HIP_PROPAGATE(gemm(stream, false, steps * N, 3 * H, C, x, C, W, 3 * H, tmp_Wx, 3 * H, false, sc.gemm_offset()));
+  if constexpr (std::is_same<T, double>::value)
+    if (tiles > 0)
+      return gru_forward_recurrence64(stream, training, steps, N, H, Ruse, bx, br, h, tmp_Wx, h_out, v, zoneout_prob,
+                                      zoneout_mask, sc.take<char>(tiles));
   ScopedKernelTimer timer("gru_forward_steps", stream);
   for (int t = 0; t < steps; ++t) {
     const T* h_t = t == 0 ? h : h_out + (size_t)(t - 1) * NH;
@@ -859,13 +911,18 @@ int gru_backward_steps(hipStream_t stream, int steps, int N, int C, int H, const
                        T* dW, T* dR, T* dbx, T* dbr, T* dh, T* dp, T* dq, const T* zoneout_mask) {
   const size_t NH = (size_t)N * H, N3H = NH * 3, N4H = NH * 4;
   const int TN = steps * N;
-  const size_t own = column_sum_bytes<T>((size_t)TN, 3 * H);
+  const size_t sums = column_sum_bytes<T>((size_t)TN, 3 * H);
   size_t room = max2(gemm_room<T>(N, H, 3 * H), gemm_room<T>(C, 3 * H, TN));
   room = max2(room, max2(gemm_room<T>(H, 3 * H, TN), gemm_room<T>(TN, C, 3 * H)));
+  const size_t tiles = one_launch_bytes<T>(stream, 3, 1, steps, N, H, sums + room);
   Scratch sc;
-  HASTE_HIP_PROPAGATE(open_scratch(stream, own, room, &sc));
-  void* partial = sc.take<char>(own);
-  {
+  HASTE_HIP_PROPAGATE(open_scratch(stream, sums + tiles, room, &sc));
+  void* partial = sc.take<char>(sums);
+  if (tiles > 0) {
+    if constexpr (std::is_same<T, double>::value)
+      HASTE_HIP_PROPAGATE(gru_backward_recurrence64(stream, steps, N, H, R_t, h, v, dh_next, dh, dp, dq, zoneout_mask,
+                                                    sc.take<char>(tiles)));
+  } else {
     ScopedKernelTimer timer("gru_backward_steps", stream);
     StepProduct<T> pend;
     for (int t = steps - 1; t >= 0; --t) {

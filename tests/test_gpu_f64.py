@@ -146,3 +146,46 @@ def test_f64_cpp_classes(monkeypatch, cell):
         test_gpu_cpp_api.test_cpp_gru(T, N, C, H, zoneout, ln)
     else:
         test_gpu_cpp_api.test_cpp_indrnn(T, N, C, H, zoneout, ln)
+
+
+# The recurrences in one launch: weights in registers alone and shared with LDS, 8 and 16 units per
+# workgroup, groups within and across XCDs, ragged last units, rows and quarters of the contraction;
+# (4, 70, 8, 768): forward too large for it, backward not.
+ONE_LAUNCH_SHAPES = [(4, 1, 4, 1), (5, 64, 8, 512), (4, 128, 8, 512), (4, 16, 8, 513), (6, 33, 12, 300), (4, 20, 8, 700),
+                     (4, 70, 8, 768), (4, 113, 4, 72), (4, 129, 4, 250)]
+
+
+@pytest.mark.parametrize("zoneout", [0.0, 0.3])
+@pytest.mark.parametrize("T,N,C,H", ONE_LAUNCH_SHAPES)
+def test_f64_recurrence_in_one_launch(double_precision, T, N, C, H, zoneout):
+    test_gpu_lstm.test_lstm_training_forward_backward(T, N, C, H, zoneout)
+    test_gpu_gru.test_gru_training_forward_backward(T, N, C, H, zoneout)
+
+
+@pytest.mark.parametrize("T,N,C,H", ONE_LAUNCH_SHAPES[1:5])
+def test_f64_inference_in_one_launch(double_precision, T, N, C, H):
+    test_gpu_lstm.test_lstm_inference_forward(0.25, T, N, C, H)
+    test_gpu_gru.test_gru_inference_forward(0.25, T, N, C, H)
+
+
+def test_f64_recurrence_under_capture():
+    """A captured call runs step by step; every replay gives what the eager call gives to rounding."""
+    import torch
+    from haste_amd import ops
+    T, N, C, H = 6, 20, 16, 64
+    r = np.random.default_rng(5)
+    arrays = [dev64(r.uniform(-0.3, 0.3, s)) for s in ((T, N, C), (N, H), (N, H), (C, 4 * H), (H, 4 * H), (4 * H,))]
+    x, h0, c0, W, R, b = arrays
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        ops.lstm_forward(False, 0.0, x, h0, c0, W, R, b, dev64(None))
+        stream.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            h, c, _ = ops.lstm_forward(False, 0.0, x, h0, c0, W, R, b, dev64(None))
+    for k in range(3):
+        x.copy_(dev64(r.uniform(-1, 1, (T, N, C))))
+        graph.replay()
+        eager, _, _ = ops.lstm_forward(False, 0.0, x, h0, c0, W, R, b, dev64(None))
+        torch.cuda.synchronize()
+        assert relerr(host(h), host(eager)) < 1e-13, k
