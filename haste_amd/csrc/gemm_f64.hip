@@ -5,8 +5,12 @@
 // Bound: MFMA (fp64 peak 78.6 TFLOP/s), algorithmic flops 2*M*N*K.  A workgroup of four
 // wavefronts owns a 64 x 64 tile of C; a wavefront owns 32 x 32 of it as 2 x 2 MFMA tiles.
 // Operand panels of 32 k go through LDS k-major ([k][m], [k][n]): the lanes of one MFMA
-// operand read 16 consecutive doubles of one k row.  A product with few tiles and a long
-// contraction (the recurrent product of one step: 64 x 512 x 2048 is 8 tiles) is cut along K
+// operand read 16 consecutive doubles of one k row.  Measured, panels loaded in runs of 256 - 512
+// bytes and requested three ahead (one ahead and in runs of 16 bytes before): 512 x 2048 x 6400
+// 359 -> 312 us, with A transposed 405 -> 295 (45 TFLOP/s, one workgroup per CU); products of many
+// tiles were and are bound by the matrix cores, 64 - 75 % busy: 6400 x 2048 x 512 300, 4096^3 56
+// TFLOP/s.  A product with few tiles and a long
+// contraction (the product of one step over 70 rows: 128 x 512 x 2048 is 16 tiles) is cut along K
 // into pieces, each a workgroup of its own, which park partial results in the stream's scratch
 // buffer; a second kernel adds a tile's pieces in index order.  How a product is cut depends
 // on its shape only, so results are reproducible.  Lane layout of the instruction (checked on
@@ -24,15 +28,21 @@ typedef unsigned int uint4_t __attribute__((ext_vector_type(4)));
 constexpr unsigned int kNowhere = 0x7ffffff0u;  // an offset beyond any buffer resource's range: the load returns zeros
 
 constexpr int DM = 64, DN = 64, DK = 32;
-constexpr int DPITCH = 64 + 1;  // doubles per k row in LDS (odd: the transposing stores of A spread over the banks)
+
+// Where element i (row of A, column of B) of panel row k lies in LDS.  The operand reads of an
+// instruction take 16 elements of four consecutive k, the transposing stores of A one k of every
+// second of 32 and four rows: the exclusive or with bits of k spreads both evenly over the banks
+// (two words each) and keeps neighbouring elements side by side.
+__device__ __forceinline__ int panel_at(int k, int i) {
+  return k * 64 + (i ^ (((k >> 1) & 3) << 2) ^ (((k >> 3) ^ k) & 1) << 4);
+}
 
 template <bool TRANS_A>
 __global__ __launch_bounds__(256)
 void gemm_f64_kernel(int M, int N, int K, const double* __restrict__ A, int lda,
                      const double* __restrict__ B, int ldb, double* __restrict__ C, int ldc,
                      int accumulate, int k_per_piece, double* __restrict__ part, int panels_ok) {
-  __shared__ double As[DK][DPITCH];
-  __shared__ double Bs[DK][DPITCH];
+  __shared__ double2_t panels[2][2][DK * 64 / 2];  // [buffer][A, B]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int m0 = blockIdx.y * DM, n0 = blockIdx.x * DN;
   const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
@@ -49,68 +59,64 @@ void gemm_f64_kernel(int M, int N, int K, const double* __restrict__ A, int lda,
       fast ? (int)((TRANS_A ? (long long)(K - 1) * lda + M : (long long)(M - 1) * lda + K) * 8) : 0, 0x00020000);
   const __amdgpu_buffer_rsrc_t pb = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<double*>(B), 0, fast ? (int)(((long long)(K - 1) * ldb + N) * 8) : 0, 0x00020000);
-  const unsigned int a_voff = TRANS_A ? (unsigned int)(((tid >> 3) * lda + m0 + (tid & 7) * 8) * 8)
-                                      : (unsigned int)(((m0 + (tid >> 2)) * lda + (tid & 3) * 8) * 8);
-  const unsigned int b_voff = (unsigned int)(((tid >> 3) * ldb + n0 + (tid & 7) * 8) * 8);
+  // Load i of a panel: where rows run along k (A not transposed) 16 lanes take the 32 k of a row and
+  // i counts 16 rows, otherwise 32 lanes take the 64 elements of one k and i counts 8 k -- a
+  // wavefront's load is runs of 256 or 512 bytes.
+  const int rrow = tid >> 4, rk = (tid & 15) * 2;
+  const int ck = tid >> 5, ci = (tid & 31) * 2;
+  const unsigned int a_voff = TRANS_A ? (unsigned int)((ck * lda + m0 + ci) * 8)
+                                      : (unsigned int)(((m0 + rrow) * lda + rk) * 8);
+  const unsigned int a_step = (unsigned int)((TRANS_A ? 8 : 16) * lda) * 8u, b_step = (unsigned int)ldb * 64u;
+  const unsigned int b_voff = (unsigned int)((ck * ldb + n0 + ci) * 8);
   double4_t acc[2][2];
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
     for (int b = 0; b < 2; ++b) acc[a][b] = double4_t{0.0, 0.0, 0.0, 0.0};
 
-  // A thread's 8 elements of each operand panel.  The panel of step k0 + DK is requested before
-  // the MFMAs of step k0, so that the loads' latency (what a step of this short loop costs
-  // otherwise) passes beside them.
-  double ra[8], rb[8];
-  auto request = [&](int k0) {
+  // A thread's 8 elements of each operand panel.  Panels are requested three ahead of the MFMAs
+  // (two in registers, one in LDS): a product with one workgroup per CU has nothing else to do
+  // while it waits for memory.
+  double2_t ra[2][4], rb[2][4];
+  auto request = [&](int set, int k0) {
     if (fast) {
       const int sa = TRANS_A ? k0 * lda * 8 : k0 * 8, sb = k0 * ldb * 8;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const double2_t va = __builtin_bit_cast(double2_t, __builtin_amdgcn_raw_buffer_load_b128(pa, a_voff + 16 * i, sa, 0));
-        const double2_t vb = __builtin_bit_cast(double2_t, __builtin_amdgcn_raw_buffer_load_b128(pb, b_voff + 16 * i, sb, 0));
-        ra[2 * i] = va[0];
-        ra[2 * i + 1] = va[1];
-        rb[2 * i] = vb[0];
-        rb[2 * i + 1] = vb[1];
+        ra[set][i] = __builtin_bit_cast(double2_t, __builtin_amdgcn_raw_buffer_load_b128(pa, a_voff + i * a_step, sa, 0));
+        rb[set][i] = __builtin_bit_cast(double2_t, __builtin_amdgcn_raw_buffer_load_b128(pb, b_voff + i * b_step, sb, 0));
       }
       return;
     }
-    if (TRANS_A) {
-      const int gk = k0 + (tid >> 3), m8 = (tid & 7) * 8;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int gm = m0 + m8 + i;
-        ra[i] = (gm < M && gk < K) ? A[(size_t)gk * lda + gm] : 0.0;
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        if (TRANS_A) {
+          const int gk = k0 + ck + 8 * i, gm = m0 + ci + e;
+          ra[set][i][e] = (gm < M && gk < K) ? A[(size_t)gk * lda + gm] : 0.0;
+        } else {
+          const int gk = k0 + rk + e, gm = m0 + rrow + 16 * i;
+          ra[set][i][e] = (gm < M && gk < K) ? A[(size_t)gm * lda + gk] : 0.0;
+        }
+        const int gk = k0 + ck + 8 * i, gn = n0 + ci + e;
+        rb[set][i][e] = (gn < N && gk < K) ? B[(size_t)gk * ldb + gn] : 0.0;
       }
-    } else {
-      const int gm = m0 + (tid >> 2), k8 = (tid & 3) * 8;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int gk = k0 + k8 + i;
-        ra[i] = (gm < M && gk < K) ? A[(size_t)gm * lda + gk] : 0.0;
-      }
-    }
-    const int gk = k0 + (tid >> 3), n8 = (tid & 7) * 8;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int gn = n0 + n8 + i;
-      rb[i] = (gn < N && gk < K) ? B[(size_t)gk * ldb + gn] : 0.0;
-    }
   };
-  auto park = [&]() {
-    if (TRANS_A) {
-      const int k = tid >> 3, m8 = (tid & 7) * 8;
+  auto park = [&](int set, int buffer) {
+    double2_t* as = panels[buffer][0];
+    double2_t* bs = panels[buffer][1];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) As[k][m8 + i] = ra[i];
-    } else {
-      const int m = tid >> 2, k8 = (tid & 3) * 8;
+    for (int i = 0; i < 4; ++i) {
+      if (TRANS_A) {
+        as[panel_at(ck + 8 * i, ci) / 2] = ra[set][i];
+      } else {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) As[k8 + i][m] = ra[i];
+        for (int e = 0; e < 2; ++e)
+          reinterpret_cast<double*>(as)[panel_at(rk + e, rrow + 16 * i)] = ra[set][i][e];
+      }
+      bs[panel_at(ck + 8 * i, ci) / 2] = rb[set][i];
     }
-    const int k = tid >> 3, n8 = (tid & 7) * 8;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) Bs[k][n8 + i] = rb[i];
   };
 
   // this workgroup's piece of the contraction; request() and the loop below see its end as K
@@ -121,22 +127,34 @@ void gemm_f64_kernel(int M, int N, int K, const double* __restrict__ A, int lda,
     ldc = N;
     accumulate = 0;
   }
-  request(k_begin);
-  for (int k0 = k_begin; k0 < K; k0 += DK) {
-    park();
-    __syncthreads();
-    if (k0 + DK < K) request(k0 + DK);
+  // Panel p lies in buffer p % 2; at its turn the panel behind it is parked in the other buffer,
+  // which everybody has finished with, and the one three behind requested.
+  auto panel = [&](auto parity, int k0) {
+    constexpr int P = decltype(parity)::value;
+    if (k0 + DK < K) park(P ^ 1, P ^ 1);
+    if (k0 + 3 * DK < K) request(P ^ 1, k0 + 3 * DK);
+    const double* as = reinterpret_cast<const double*>(panels[P][0]);
+    const double* bs = reinterpret_cast<const double*>(panels[P][1]);
 #pragma unroll
     for (int kk = 0; kk < DK; kk += 4) {
       const int k = kk + (lane >> 4), o = lane & 15;
-      const double a0 = As[k][wm + o], a1 = As[k][wm + 16 + o];
-      const double b0 = Bs[k][wn + o], b1 = Bs[k][wn + 16 + o];
+      const double a0 = as[panel_at(k, wm + o)], a1 = as[panel_at(k, wm + 16 + o)];
+      const double b0 = bs[panel_at(k, wn + o)], b1 = bs[panel_at(k, wn + 16 + o)];
       acc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b0, acc[0][0], 0, 0, 0);
       acc[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b1, acc[0][1], 0, 0, 0);
       acc[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b0, acc[1][0], 0, 0, 0);
       acc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b1, acc[1][1], 0, 0, 0);
     }
     __syncthreads();
+  };
+  request(0, k_begin);
+  if (k_begin + DK < K) request(1, k_begin + DK);
+  park(0, 0);
+  if (k_begin + 2 * DK < K) request(0, k_begin + 2 * DK);
+  __syncthreads();
+  for (int k0 = k_begin; k0 < K; k0 += 2 * DK) {
+    panel(std::integral_constant<int, 0>{}, k0);
+    if (k0 + DK < K) panel(std::integral_constant<int, 1>{}, k0 + DK);
   }
 #pragma unroll
   for (int a = 0; a < 2; ++a)
