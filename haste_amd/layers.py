@@ -54,10 +54,18 @@ def _alias(seq, first):
     return seq.new_empty(0).set_(a)
 
 
+def _one_per_row(wanted, seq):
+    """Whether an index tensor is what the ops take: a step for every batch row (anything else that
+    indexing accepts is left to it)."""
+    return wanted.dim() == 1 and wanted.size(0) == seq.size(1) and wanted.is_contiguous() and seq.numel() > 0
+
+
 def _wanted_states(seqs, wanted):
     """What a layer returns of its state sequences [T+1,N,H]: "last" [N,H], "all" [T,N,H], or the states
     at the steps in an index tensor [N]."""
     if torch.is_tensor(wanted):
+        if _one_per_row(wanted, seqs[0]):
+            return ops.gather_states(seqs, wanted)
         cols = torch.arange(seqs[0].size(1), device=wanted.device)
         return tuple(seq[wanted, cols] for seq in seqs)
     return tuple(_alias(seq, 1 if wanted == "all" else -1) for seq in seqs)
@@ -73,6 +81,8 @@ def _upstream(like, grad_steps, grad_wanted, wanted):
         if wanted == "last":
             return grad_steps if grad_steps is None else grad_steps.contiguous(), grad_wanted
         return (grad_wanted if grad_steps is None else grad_steps + grad_wanted).contiguous(), None
+    if _one_per_row(wanted, like):
+        return ops.state_gradients(like, grad_steps, grad_wanted, wanted), None
     full = torch.zeros_like(like) if grad_steps is None else torch.empty_like(like)
     if grad_steps is not None:
         full[1:] = grad_steps

@@ -199,6 +199,31 @@ def transpose3(a, b, c):
     return tuple(outs)
 
 
+def gather_states(seqs, lengths):
+    """The states [N,H] of one or two sequences [T+1,N,H] at the steps lengths[N] (int64)."""
+    _check(*seqs)
+    T1, N, H = seqs[0].shape
+    outs = [torch.empty(N, H, device=s.device, dtype=s.dtype) for s in seqs]
+    second = seqs[1:] or (None,)
+    _call("haste_hip_gather_states", T1 - 1, N, H, seqs[0], second[0], lengths.data_ptr(), outs[0],
+          outs[1] if len(outs) > 1 else None)
+    return tuple(outs)
+
+
+def state_gradients(like, grad, last, lengths):
+    """Gradients [T,N,H] of the steps of a sequence `like` [T+1,N,H]: grad [T,N,H] (None: zeros) plus
+    last [N,H] at the steps lengths[N] (int64; step 0, the initial state, gets none)."""
+    T1, N, H = like.shape
+    if grad is not None and grad.stride(2) != 1:
+        grad = grad.contiguous()
+    last = last.contiguous()
+    _check(last)
+    out = torch.empty(T1 - 1, N, H, device=like.device, dtype=like.dtype)
+    step, row = (0, 0) if grad is None else grad.stride()[:2]
+    _call("haste_hip_state_gradients", T1 - 1, N, H, grad, step, row, last, lengths.data_ptr(), out)
+    return out
+
+
 # ---- LSTM (reference frameworks/pytorch/lstm.cc:31-157) ---------------------
 def lstm_forward(training, zoneout_prob, x, h0, c0, kernel, recurrent_kernel, bias, zoneout_mask,
                  dropconnect_mask=None, dropconnect_scale=1.0):

@@ -142,6 +142,19 @@ int haste_hip_transpose3_f32(int rows0, int cols0, const float* in0, float* out0
                              int rows1, int cols1, const float* in1, float* out1,
                              int rows2, int cols2, const float* in2, float* out2, void* stream);
 
+/* Batches whose sequences have lengths of their own (reference frameworks/pytorch/base_rnn.py:54-61).
+ * lengths: N 64-bit integers on the device, steps 0 (the initial state) .. T of a sequence
+ * [T+1,N,H], counted from the end when negative.
+ * gather_states: out0[n] = seq0[length of n][n], [N,H], and the same for seq1 unless it is NULL;
+ * a length that names no step gives NaNs.
+ * state_gradients: out[T,N,H] = grad (zeros when NULL; rows of H elements, the strides between
+ * steps and batch rows in elements) + last[N,H] at each row's last step (none for length 0). */
+int haste_hip_gather_states_f32(int T, int N, int H, const float* seq0, const float* seq1,
+                                const void* lengths, float* out0, float* out1, void* stream);
+int haste_hip_state_gradients_f32(int T, int N, int H, const float* grad, size_t step_stride,
+                                  size_t row_stride, const float* last, const void* lengths,
+                                  float* out, void* stream);
+
 /* ---- LSTM ----------------------------------------------------------------
  * reference lib/haste/lstm.h:118-129 (ForwardPass::Run), lib/lstm_forward_gpu.cu.cc:313-366.
  * W[C,4H] R[H,4H] b[4H] x[T,N,C] h,c[T+1,N,H] (slot 0 preset by the caller)
@@ -404,6 +417,11 @@ int haste_hip_transpose_f64(int rows, int cols, const double* in, double* out, v
 int haste_hip_transpose3_f64(int rows0, int cols0, const double* in0, double* out0,
                              int rows1, int cols1, const double* in1, double* out1,
                              int rows2, int cols2, const double* in2, double* out2, void* stream);
+int haste_hip_gather_states_f64(int T, int N, int H, const double* seq0, const double* seq1,
+                                const void* lengths, double* out0, double* out1, void* stream);
+int haste_hip_state_gradients_f64(int T, int N, int H, const double* grad, size_t step_stride,
+                                  size_t row_stride, const double* last, const void* lengths,
+                                  double* out, void* stream);
 int haste_hip_lstm_forward_f64(int training, int steps, int batch_size, int input_size,
                                int hidden_size,
                                const double* W, const double* R, const double* b, const double* x,
@@ -563,6 +581,11 @@ int haste_hip_transpose_f16(int rows, int cols, const void* in, void* out, void*
 int haste_hip_transpose3_f16(int rows0, int cols0, const void* in0, void* out0,
                              int rows1, int cols1, const void* in1, void* out1,
                              int rows2, int cols2, const void* in2, void* out2, void* stream);
+int haste_hip_gather_states_f16(int T, int N, int H, const void* seq0, const void* seq1,
+                                const void* lengths, void* out0, void* out1, void* stream);
+int haste_hip_state_gradients_f16(int T, int N, int H, const void* grad, size_t step_stride,
+                                  size_t row_stride, const void* last, const void* lengths,
+                                  void* out, void* stream);
 /* C[M,N] (+)= A[M,K] * Bt[N,K]^T with fp32 accumulation and an fp32 result: the product kernel
  * of the half GRU's passes over more than one step.  Bt holds IEEE binary16 values, A binary16
  * or (a_is_float != 0) fp32 values that are rounded to half as they are read; both have the

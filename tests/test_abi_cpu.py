@@ -69,6 +69,8 @@ def test_null_pointers_and_bad_dimensions_are_rejected_on_the_host(lib):
 
 def test_double_and_half_entry_points_reject_bad_arguments_too(lib):
     INVALID = 1
+    for sfx in ("_f32", "_f64", "_f16"):
+        assert _call(lib, "haste_hip_gather_states" + sfx, 3, 2, 2, *([None] * 5), None) == INVALID
     for sfx in ("_f64", "_f16"):
         assert _call(lib, "haste_hip_gemm" + sfx, 0, 4, 4, 4, None, 4, None, 4, None, 4, 0, None) == INVALID
         assert _call(lib, "haste_hip_transpose" + sfx, 4, 4, None, None, None) == INVALID

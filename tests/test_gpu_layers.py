@@ -304,3 +304,29 @@ def test_outputs_that_are_changed_are_noticed():
             {"y": y, "h": h, "c": c}[which].add_(1.0)
         with pytest.raises(RuntimeError, match="modified by an inplace operation"):
             loss.backward()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64, torch.float16])
+@pytest.mark.parametrize("T,N,H", [(1, 1, 1), (4, 3, 5), (7, 33, 256), (5, 2, 300)])
+def test_states_at_lengths_match_indexing(dtype, T, N, H):
+    """Gathered states and their gradients against tensor indexing, bit for bit: lengths 0 (the initial
+    state), T and counted from the end, gradients contiguous, batch first, broadcast and absent."""
+    from haste_amd import ops
+    gen = torch.Generator(device="cuda").manual_seed(T + N + H)
+    def rand(*s):
+        return torch.randn(*s, device="cuda", generator=gen).to(dtype)
+
+    seqs = [rand(T + 1, N, H), rand(T + 1, N, H)]
+    lengths = torch.randint(-T - 1, T + 1, (N,), device="cuda", generator=gen)
+    lengths[0] = T
+    rows = torch.arange(N, device="cuda")
+    for given in (seqs[:1], seqs):
+        for got, seq in zip(ops.gather_states(given, lengths), given):
+            assert torch.equal(got, seq[lengths, rows])
+    last = rand(N, H)
+    for grad in (rand(T, N, H), rand(N, T, H).permute(1, 0, 2), rand(1, 1, H).expand(T, N, H), rand(1, 1, 1).expand(T, N, H), None):
+        full = torch.zeros(T + 1, N, H, device="cuda", dtype=dtype)
+        if grad is not None:
+            full[1:] = grad
+        full[lengths, rows] = full[lengths, rows] + last
+        assert torch.equal(ops.state_gradients(seqs[0], grad, last, lengths), full[1:])
