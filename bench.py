@@ -479,8 +479,8 @@ def run_configs(args, torch, lib, ops, dev):
     forward (+ backward with the caller-side transposes) in ms per call, with the algorithmic
     flops of the matrix products (2*T*N*G*H*(C + H) forward, three times that forward +
     backward) and the fraction of the matrix cores' peak for the arithmetic type.  Also the
-    other instantiations of the reference at the metric shape: the double LSTM (step-wise regime:
-    one product and one pointwise launch per step) and the half GRU (fp32 recurrences on widened
+    other instantiations of the reference at the metric shape: the double LSTM (all steps of
+    a recurrence in one launch, products on the fp64 matrix cores) and the half GRU (fp32 recurrences on widened
     tensors, products on the half matrix cores)."""
     details = {}
 
