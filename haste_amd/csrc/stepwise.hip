@@ -355,8 +355,17 @@ void column_finish_kernel(int chunks, int cols, const typename Acc<T>::type* __r
   using A = typename Acc<T>::type;
   const int col = blockIdx.x * kThreads + threadIdx.x;
   if (col >= cols) return;
+  constexpr int kInFlight = 32;
   A s = A(0);
-  for (int k = 0; k < chunks; ++k) s += partial[(size_t)k * cols + col];
+  int k = 0;
+  for (; k + kInFlight <= chunks; k += kInFlight) {
+    A v[kInFlight];
+#pragma unroll
+    for (int u = 0; u < kInFlight; ++u) v[u] = partial[(size_t)(k + u) * cols + col];
+#pragma unroll
+    for (int u = 0; u < kInFlight; ++u) s += v[u];
+  }
+  for (; k < chunks; ++k) s += partial[(size_t)k * cols + col];
   out[col] = T(A(out[col]) + s);
 }
 
