@@ -164,6 +164,25 @@ int test_absent_workgroups();
 // their waits (for experiments).
 bool fused_input_enabled();
 
+// Whether a forward recurrence that can compute x * W (C inputs, `columns` outputs) beside its waits
+// does so.  The projection costs every step about 0.4 us at C = H = 512, however few the rows; the GEMM
+// costs its launches, the round trip of x * W and little per row, so that it wins when there are enough
+// steps of enough work each (C * H = 2^15: a step is no cheaper behind the GEMM, however many there are).
+// With 64 rows the two are level, training passes 1 % slower behind the GEMM.  Measured, inference, N = 8 / 16 / 32 / 64, beside the waits -> GEMM, us:
+//   LSTM T = 100 C = H = 512  233 / 234 / 239 / 335 -> 200 / 212 / 223 / 331
+//   LSTM T = 400 C = H = 512  831 / 832 / 837 / 1213 -> 663 / 700 / 760 / 1168
+//   LSTM T = 400 C = 128 H = 512  693 / 694 / 704 / 993 -> 637 / 650 / 669 / 968
+//   LSTM T = 100 C = 128 H = 512  196 / 197 / 201 / 283 -> 190 / 197 / 200 / 283
+//   LSTM T = 400 C = 128 H = 256  413 / 413 / 421 / 570 -> 436 / 448 / 455 / 575
+//   LSTM T = 25 C = H = 512  83 / 83 / 83 / 110 -> 77 / 84 / 87 / 119
+//   GRU T = 100 C = H = 512  222 / 223 / 226 / 293 -> 190 / 205 / 212 / 288
+//   GRU T = 25 C = H = 512  77 / 77 / 76 / 96 -> 73 / 78 / 81 / 109
+//   training, N = 5 / 16 / 32:  LSTM T = 400 C = H = 512  1621 / 1769 / 2096 -> 1435 / 1616 / 1937
+//   GRU T = 300 C = 128 H = 512  1015 / 1043 / 1177 -> 999 / 1030 / 1141
+// Where the GEMM's partial tiles would not fit memory the caller lent, or the workspace would have
+// to grow while the stream is captured, it stays in the recurrence.
+int input_projection_in_recurrence(hipStream_t stream, int T, int N, int C, int H, int columns, bool* fused);
+
 // C[M,N] = op(A)*B (+C): fp32 MFMA GEMM on `stream`.  The partial tiles of a split product
 // are kept `scratch_offset` bytes (a multiple of 16) into the stream's scratch buffer.
 int gemm_f32(hipStream_t stream, bool trans_a, int M, int N, int K,

@@ -843,9 +843,10 @@ int gru_forward_impl(hipStream_t stream, int training, int T, int N, int C, int 
   // wavefront's share of W (C/4 x 48 columns) fits its registers (the step's x*W GEMM, its split
   // reduce and the round trip of tmp_Wx through memory go away).  The partial tiles then have
   // rows of 64 columns: the slice's 48 and the candidate gate's x*W.
-  const bool fused = !wx_ready && !half_product && (paired || tile.nb == 4) && tile.hs == 16 &&
+  bool fused = !wx_ready && !half_product && (paired || tile.nb == 4) && tile.hs == 16 &&
                      tile.reg_groups == 0 && C <= 512 && C % 4 == 0 &&
-                     (reinterpret_cast<uintptr_t>(x) & 15u) == 0 && fused_input_enabled();
+                     (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
+  if (fused) HASTE_HIP_PROPAGATE(input_projection_in_recurrence(stream, T, N, C, H, 3 * H, &fused));
   const int xsg = C <= 256 ? 1 : 2;
   size_t lds_bytes = paired ? paired_lds : tile.lds_bytes;
   if (fused)

@@ -845,8 +845,9 @@ int lstm_forward_impl(hipStream_t stream, int training, int T, int N, int C, int
   // of its partial tiles; the projection's weights must fit the registers, C <= 512).
   // Otherwise: v = x * W for all steps at once.
   const int xsg = (C + 255) / 256;  // super-groups of 64 input features per wavefront
-  const bool fused = (paired || tile.nb == 4) && H > 192 && C <= 512 && C % 4 == 0 &&
-                     (reinterpret_cast<uintptr_t>(x) & 15u) == 0 && fused_input_enabled();
+  bool fused = (paired || tile.nb == 4) && H > 192 && C <= 512 && C % 4 == 0 &&
+                     (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
+  if (fused) HASTE_HIP_PROPAGATE(input_projection_in_recurrence(stream, T, N, C, H, 4 * H, &fused));
   if (!fused)
     HASTE_HIP_PROPAGATE(gemm_f32(stream, false, T * N, 4 * H, C, x, C, W, 4 * H, v, 4 * H, false));
 

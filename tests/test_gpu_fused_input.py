@@ -79,5 +79,40 @@ def test_input_projection_inside_the_recurrence_matches_the_separate_gemm():
                 assert relerr(v, ref) < 5e-6, (shape, k)
 
 
+@pytest.mark.parametrize("T,N,C,H", [(63, 9, 512, 512), (64, 9, 512, 512), (257, 29, 512, 256), (513, 3, 128, 256),
+                                     (70, 33, 512, 512)])
+@pytest.mark.parametrize("lent", [False, True])
+def test_either_side_of_the_rule_for_the_input_projection(T, N, C, H, lent):
+    """T * C * H, C * H and N just below and above what sends x*W to the GEMM, in the library's own workspace and in
+    memory that holds the recurrence's exchange tiles but not the GEMM's partial tiles, against
+    the oracle in fp64.  The bound is the forward parity tests'."""
+    import torch
+    from haste_amd import ops
+    from oracle import haste_oracle as O
+    print("projection rule", T, N, C, H, lent, flush=True)
+    p = problem(17 + T + N + C + H, T, N, C, H, 4, 0.0)
+    q = problem(18 + T + N + C + H, T, N, C, H, 3, 0.0)
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        memory = torch.empty(1 << 20, dtype=torch.uint8, device="cuda:0") if lent else None
+        if lent:
+            ops.set_workspace(memory)
+        try:
+            h, c, _ = ops.lstm_forward(True, 0.0, dev(p["x"]), dev(p["h0"]), dev(p["c0"]), dev(p["W"]), dev(p["R"]),
+                                       dev(p["b"]), torch.empty(0, device="cuda:0"))
+            with_gru = not lent or H >= 512  # below, the GRU takes the GEMM at any T
+            hg = None if not with_gru else ops.gru_forward(True, 0.0, dev(q["x"]), dev(q["h0"]), dev(q["W"]), dev(q["R"]), dev(q["b"]),
+                                    dev(q["b2"]), torch.empty(0, device="cuda:0"))[0]
+            s.synchronize()
+        finally:
+            s.synchronize()
+            if lent:
+                ops.set_workspace(None)
+    ho, co, _ = O.lstm_forward(p["W"], p["R"], p["b"], p["x"], p["h0"], p["c0"])
+    go, _ = O.gru_forward(q["W"], q["R"], q["b"], q["b2"], q["x"], q["h0"])
+    assert relerr(host(h), ho) < 1e-4 and relerr(host(c), co) < 1e-4
+    assert not with_gru or relerr(host(hg), go) < 1e-4
+
+
 if __name__ == "__main__":
     child(sys.argv[1])
