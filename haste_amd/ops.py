@@ -153,9 +153,17 @@ def _upstream(grad, T):
 
 
 def _carried(opts, *pairs):
-    """_zeros() of the shapes in `pairs` of (shape, initial value or None)."""
+    """_zeros() of the shapes in `pairs` of (shape, initial value or None).  An initial value may have
+    any strides (the gradient of a state that the caller transposed or summed comes that way); the
+    entry points take row-major tensors."""
+    for shape, start in pairs:
+        if start is not None and (tuple(start.shape) != tuple(shape) or start.dtype != opts["dtype"]
+                                  or start.device != opts["device"]):
+            raise ValueError("gradient of the last state must be %s, %s on %s, got %s, %s on %s"
+                             % (list(shape), opts["dtype"], opts["device"], list(start.shape), start.dtype, start.device))
     out = _zeros(opts, *[shape for shape, start in pairs if start is None])
-    return [out.pop(0) if start is None else start.clone() for _, start in pairs]
+    return [out.pop(0) if start is None else start.clone(memory_format=torch.contiguous_format)
+            for _, start in pairs]
 
 
 def gemm(a, b, out=None, trans_a=False, accumulate=False):

@@ -294,6 +294,39 @@ def test_gradients_enter_through_every_output(name, dtype, H, wanted, through):
         assert relerr(npy(got), npy(want)) < {torch.float32: TOL, torch.float64: 1e-10, torch.float16: 2e-2}[dtype]
 
 
+@pytest.mark.parametrize("name,dtype", [
+    (n, d) for n in ("LSTM", "GRU", "IndRNN", "LayerNormLSTM", "LayerNormGRU", "LayerNormIndRNN")
+    for d in (torch.float32, torch.float64)] + [("GRU", torch.float16)])
+@pytest.mark.parametrize("form", ["transposed", "broadcast"])
+def test_gradients_of_final_states_in_any_layout(name, dtype, form):
+    """Gradients of the final states that arrive with strides of their own: of a caller that works on
+    the transposed state, and of a sum (stride 0)."""
+    T, N, C, H = 5, 3, 8, 24
+    torch.manual_seed(12)
+    layer = getattr(haste_amd, name)(C, H).to(dtype)
+    ref = getattr(haste_amd, name)(C, H).double()
+    ref.load_state_dict(layer.state_dict())
+    layer = layer.cuda()
+    x = torch.randn(T, N, C).to(dtype)
+    start = torch.randn(2, N, H).to(dtype)
+    weight = torch.randn(2, H, N).to(dtype)
+    results = []
+    for net, at, first in ((layer, x.cuda(), start.cuda()), (ref, x.double(), start.double())):
+        at.requires_grad_(True)
+        first = [s.unsqueeze(0).requires_grad_(True) for s in first]
+        two = "LSTM" in name
+        _, state = net(at, tuple(first) if two else first[0])
+        states = state if two else (state,)
+        loss = 0.0
+        for s, w in zip(states, weight.to(at)):
+            loss = loss + ((s[0].t().contiguous() * w).sum() if form == "transposed" else s.sum())
+        loss.backward()
+        results.append([at.grad] + [s.grad for s in first[:len(states)]] + [p.grad for p in net.parameters()])
+    print(name, dtype, form, flush=True)
+    for got, want in zip(*results):
+        assert relerr(npy(got), npy(want)) < {torch.float32: TOL, torch.float64: 1e-10, torch.float16: 2e-2}[dtype]
+
+
 def test_outputs_that_are_changed_are_noticed():
     """The outputs share memory with what the backward pass reads."""
     layer = haste_amd.LSTM(4, 8).cuda()

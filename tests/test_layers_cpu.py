@@ -256,3 +256,20 @@ def test_mixed_cpu_and_gpu_parameters_are_refused():
     layer.parameters = lambda: [Fake(f) for f in (True, False, False, False)]
     with pytest.raises(ValueError, match="all be CUDA tensors or none"):
         layer._is_cuda()
+
+
+# ---- host side of the fused passes, on CPU tensors ----------------------------------------------
+def test_initial_gradients_are_row_major():
+    """A backward entry point gets the address of the gradients of the last states: whatever their
+    strides, it must be that of a row-major copy."""
+    from haste_amd import ops
+    opts = dict(device=torch.device("cpu"), dtype=torch.float32)
+    N, H = 3, 5
+    base = torch.randn(H, N)
+    for start in (base.t(), torch.randn(1, H).expand(N, H), torch.randn(()).expand(N, H), torch.randn(N, 2 * H)[:, ::2]):
+        zeros, got = ops._carried(opts, ((H, 4), None), ((N, H), start))
+        assert got.is_contiguous() and torch.equal(got, start) and got.data_ptr() != start.data_ptr()
+        assert tuple(zeros.shape) == (H, 4) and not zeros.any()
+    for wrong in (base, base.t().double(), torch.randn(1, N, H)):
+        with pytest.raises(ValueError, match="gradient of the last state"):
+            ops._carried(opts, ((N, H), wrong))
