@@ -115,12 +115,21 @@ class _RecurrenceFunction(torch.autograd.Function):
         states = _wanted_states(seqs, wanted)
         # the outputs that share memory with h and c too: if a caller changes them, autograd notices
         ctx.save_for_backward(y, *states, *saved)
+        if torch.is_tensor(wanted):  # often the caller's own tensor, filled again for the next batch
+            wanted = wanted.clone() if wanted.is_inference() else wanted
+            ctx.lengths_version = None if wanted.is_inference() else wanted._version  # None: in inference mode
         ctx.training, ctx.wanted, ctx.count = training, wanted, len(seqs)
         ctx.set_materialize_grads(False)
         return (y,) + states
 
     @staticmethod
-    def restore(ctx):
+    def restore(ctx, *state_grads):
+        """The saved tensors.  Gradients of states at lengths need the lengths of the forward pass (which
+        are not saved with the rest: a pass that only y's gradients enter may outlive them)."""
+        if (torch.is_tensor(ctx.wanted) and ctx.wanted._version != ctx.lengths_version
+                and any(g is not None for g in state_grads)):
+            raise RuntimeError("the lengths needed for gradient computation have been modified by an inplace "
+                               "operation since the forward pass")
         return ctx.saved_tensors[1 + ctx.count:]
 
 
@@ -149,7 +158,7 @@ class _LSTMFunction(_RecurrenceFunction):
     def backward(ctx, grad_y, grad_h, grad_c):
         if not ctx.training:
             raise _no_training_backward("LSTM")
-        x, kernel, recurrent_kernel, bias, zoneout_mask, h, c, cache, dmask = _RecurrenceFunction.restore(ctx)
+        x, kernel, recurrent_kernel, bias, zoneout_mask, h, c, cache, dmask = _RecurrenceFunction.restore(ctx, grad_h, grad_c)
         if dmask is not None:
             recurrent_kernel = recurrent_kernel * dmask * ctx.dropconnect_scale
         _single_shot(ctx, "LSTM")  # the backward pass overwrites the activation cache
@@ -179,7 +188,7 @@ class _GRUFunction(_RecurrenceFunction):
         if not ctx.training:
             raise _no_training_backward("GRU")
         (x, kernel, recurrent_kernel, bias, recurrent_bias, zoneout_mask, h, cache,
-         dmask) = _RecurrenceFunction.restore(ctx)
+         dmask) = _RecurrenceFunction.restore(ctx, grad_h)
         if dmask is not None:
             recurrent_kernel = recurrent_kernel * dmask * ctx.dropconnect_scale
         dh_new, dh_last = _upstream_h(h, grad_y, grad_h, ctx.wanted)
@@ -202,7 +211,7 @@ class _IndRNNFunction(_RecurrenceFunction):
     def backward(ctx, grad_y, grad_h):
         if not ctx.training:
             raise _no_training_backward("IndRNN")
-        x, kernel, recurrent_scale, bias, zoneout_mask, h = _RecurrenceFunction.restore(ctx)
+        x, kernel, recurrent_scale, bias, zoneout_mask, h = _RecurrenceFunction.restore(ctx, grad_h)
         dh_new, dh_last = _upstream_h(h, grad_y, grad_h, ctx.wanted)
         dx, dh, dW, du, db = ops.indrnn_backward(ops.transpose(x), ops.transpose(kernel), recurrent_scale, bias,
                                                  zoneout_mask, h, dh_new, dh_last)
@@ -222,7 +231,7 @@ class _LayerNormIndRNNFunction(_RecurrenceFunction):
         if not ctx.training:
             raise _no_training_backward("LayerNormIndRNN")
         (x, kernel, recurrent_scale, bias, gamma, zoneout_mask, h, act_Wx,
-         cache) = _RecurrenceFunction.restore(ctx)
+         cache) = _RecurrenceFunction.restore(ctx, grad_h)
         dh_new, dh_last = _upstream_h(h, grad_y, grad_h, ctx.wanted)
         dx, dh, dW, du, db, dgamma = ops.layer_norm_indrnn_backward(
             ops.transpose(x), ops.transpose(kernel), recurrent_scale, bias, gamma, zoneout_mask, h, act_Wx, cache,
@@ -245,7 +254,7 @@ class _LayerNormLSTMFunction(_RecurrenceFunction):
         if not ctx.training:
             raise _no_training_backward("LayerNormLSTM")
         (x, kernel, recurrent_kernel, bias, gamma, gamma_h, beta_h, zoneout_mask, h, c, act_Wx,
-         act_Wx_norm, cache1, act_Rh, cache2, act_c_norm, cache3) = _RecurrenceFunction.restore(ctx)
+         act_Wx_norm, cache1, act_Rh, cache2, act_c_norm, cache3) = _RecurrenceFunction.restore(ctx, grad_h, grad_c)
         _single_shot(ctx, "LayerNormLSTM")  # the saved activations are overwritten below
         dh_new, dh_last = _upstream_h(h, grad_y, grad_h, ctx.wanted)
         dc_new, dc_last = _upstream(c, None, grad_c, ctx.wanted)
@@ -271,7 +280,7 @@ class _LayerNormGRUFunction(_RecurrenceFunction):
         if not ctx.training:
             raise _no_training_backward("LayerNormGRU")
         (x, kernel, recurrent_kernel, bias, recurrent_bias, gamma, zoneout_mask, h, cache, act_Wx,
-         cache1, act_Rh, cache2) = _RecurrenceFunction.restore(ctx)
+         cache1, act_Rh, cache2) = _RecurrenceFunction.restore(ctx, grad_h)
         dh_new, dh_last = _upstream_h(h, grad_y, grad_h, ctx.wanted)
         dx, dh, *grads = ops.layer_norm_gru_backward(
             *ops.transpose3(x, kernel, recurrent_kernel), bias, recurrent_bias, gamma,

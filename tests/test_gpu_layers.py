@@ -339,6 +339,18 @@ def test_outputs_that_are_changed_are_noticed():
             loss.backward()
 
 
+@pytest.mark.parametrize("name", ["LSTM", "GRU", "IndRNN", "LayerNormLSTM", "LayerNormGRU", "LayerNormIndRNN"])
+def test_lengths_that_are_changed_are_noticed(name):
+    """A buffer of lengths that is filled again before the backward pass."""
+    layer = getattr(haste_amd, name)(4, 8).cuda()
+    lengths = torch.tensor([3, 1], device="cuda")
+    y, state = layer(torch.randn(3, 2, 4, device="cuda"), lengths=lengths)
+    last = state[0] if isinstance(state, tuple) else state
+    lengths.fill_(2)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        last.sum().backward()
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64, torch.float16])
 @pytest.mark.parametrize("T,N,H", [(1, 1, 1), (4, 3, 5), (7, 33, 256), (5, 2, 300)])
 def test_states_at_lengths_match_indexing(dtype, T, N, H):

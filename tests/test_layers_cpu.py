@@ -273,3 +273,82 @@ def test_initial_gradients_are_row_major():
     for wrong in (base, base.t().double(), torch.randn(1, N, H)):
         with pytest.raises(ValueError, match="gradient of the last state"):
             ops._carried(opts, ((N, H), wrong))
+
+
+@pytest.fixture
+def fused_lstm_on_cpu(monkeypatch):
+    """haste_amd.LSTM takes its fused path on CPU tensors, over stand-ins for the ops it calls: what the
+    layer does around them can be tested without a GPU."""
+    from haste_amd import layers
+
+    def forward(training, zoneout_prob, x, h0, c0, kernel, recurrent_kernel, bias, zoneout_mask, *dropconnect):
+        zeros = x.new_zeros(x.shape[1], recurrent_kernel.shape[0])
+        with torch.no_grad():
+            h, c = layers._eager_lstm(training, zoneout_prob, x.detach(), zeros if h0 is None else h0,
+                                      zeros if c0 is None else c0, kernel, recurrent_kernel, bias, zoneout_mask)
+        return h, c, x.new_zeros(1)
+
+    def backward(x_t, kernel_t, recurrent_kernel_t, bias, zoneout_mask, h, c, cache, dh_new, dc_new, dh_last, dc_last):
+        with torch.enable_grad():
+            leaves = [t.detach().clone().requires_grad_() for t in
+                      (x_t.permute(1, 2, 0), h[0], c[0], kernel_t.t(), recurrent_kernel_t.t(), bias)]
+            hh, cc = layers._eager_lstm(True, 0.0, *leaves, None)
+            loss = (hh[1:] * dh_new[-len(x_t[0]):]).sum() + (0.0 if dc_new is None else (cc[1:] * dc_new[-len(x_t[0]):]).sum())
+            loss = loss + (0.0 if dh_last is None else (hh[-1] * dh_last).sum())
+            loss = loss + (0.0 if dc_last is None else (cc[-1] * dc_last).sum())
+        return torch.autograd.grad(loss, leaves)
+
+    def state_gradients(like, grad, last, lengths):
+        full = torch.zeros_like(like)
+        if grad is not None:
+            full[1:] = grad
+        full[lengths, torch.arange(like.size(1))] += last
+        return full[1:]
+
+    for name, stand_in in (
+            ("lstm_forward", forward), ("lstm_backward", backward), ("state_gradients", state_gradients),
+            ("gather_states", lambda seqs, lengths: tuple(s[lengths, torch.arange(s.size(1))] for s in seqs)),
+            ("transpose3", lambda *t: tuple(m.permute(m.dim() - 1, *range(m.dim() - 1)).contiguous() for m in t))):
+        monkeypatch.setattr(layers.ops, name, stand_in)
+    monkeypatch.setattr(haste_amd.LSTM, "_is_cuda", lambda self: True)
+    monkeypatch.setattr(haste_amd.LSTM, "_check_fused", lambda self, x: None)
+    return haste_amd.LSTM
+
+
+def test_lengths_that_are_changed_are_noticed(fused_lstm_on_cpu):
+    """A buffer of lengths that is filled again between the passes: gradients of the states refuse, those of
+    the output do not need the lengths."""
+    T, N, C, H = 5, 3, 4, 6
+    torch.manual_seed(3)
+    layer = fused_lstm_on_cpu(C, H)
+    x = torch.randn(T, N, C)
+    grads = []
+    for change in (False, True):
+        for through in ("state", "y"):
+            layer.zero_grad(set_to_none=True)
+            lengths = torch.tensor([5, 1, 3])
+            y, (h, c) = layer(x, lengths=lengths)
+            if change:
+                lengths.copy_(torch.tensor([2, 2, 2]))
+            loss = y.square().sum() if through == "y" else h.square().sum() + c.sum()
+            if change and through == "state":
+                with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+                    loss.backward()
+                continue
+            loss.backward()
+            grads.append((through, layer.kernel.grad))
+    assert [g[0] for g in grads] == ["state", "y", "y"] and torch.equal(grads[1][1], grads[2][1])
+    ref = haste_amd.LSTM(C, H)
+    ref.load_state_dict(layer.state_dict())
+    ref._is_cuda = lambda: False
+    _, (h, c) = ref(x, lengths=[5, 1, 3])
+    (h.square().sum() + c.sum()).backward()
+    assert torch.allclose(grads[0][1], ref.kernel.grad, atol=1e-6)
+    with torch.inference_mode():
+        own = torch.tensor([5, 1, 3])
+        _, (h2, _) = layer(x, lengths=own)
+    assert torch.allclose(h2, h, atol=1e-6)
+    layer.zero_grad(set_to_none=True)
+    _, (h3, c3) = layer(x, lengths=own)  # a tensor made in inference mode has no version to look at
+    (h3.square().sum() + c3.sum()).backward()
+    assert torch.equal(layer.kernel.grad, grads[0][1])
