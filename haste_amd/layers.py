@@ -133,16 +133,6 @@ class _RecurrenceFunction(torch.autograd.Function):
         return ctx.saved_tensors[1 + ctx.count:]
 
 
-class _NoGradients:
-    """Stands in for a context where there is nothing to differentiate."""
-
-    def save_for_backward(self, *tensors):
-        pass
-
-    def set_materialize_grads(self, value):
-        pass
-
-
 class _LSTMFunction(_RecurrenceFunction):
     @staticmethod
     def forward(ctx, training, zoneout_prob, wanted, x, h0, c0, kernel, recurrent_kernel, bias, zoneout_mask,
@@ -405,10 +395,6 @@ class _RNNBase(nn.Module):
             return "all"
         return "last" if lengths is None else torch.as_tensor(lengths, device=device, dtype=torch.long)
 
-    def _fused(self, function, *args):
-        """The fused pass; without gradients autograd is not told of it."""
-        return function.apply(*args) if torch.is_grad_enabled() else function.forward(_NoGradients(), *args)
-
     def _fused_state(self, states):
         """A state as the layer returns it, from what the fused functions return of it."""
         return (self._time_major(states) if self.return_state_sequence else states).unsqueeze(0)
@@ -517,9 +503,9 @@ class LSTM(_RNNBase):
         if fused:
             self._check_fused(x)
             wanted = self._wanted(lengths, x.device)
-            y, h, c = self._fused(_LSTMFunction, self.training, self.zoneout, wanted, x.contiguous(), h0, c0,
-                                  self.kernel.contiguous(), self.recurrent_kernel.contiguous(),
-                                  self.bias.contiguous(), zmask, dmask, dscale)
+            y, h, c = _LSTMFunction.apply(self.training, self.zoneout, wanted, x.contiguous(), h0, c0,
+                                          self.kernel.contiguous(), self.recurrent_kernel.contiguous(),
+                                          self.bias.contiguous(), zmask, dmask, dscale)
             return self._time_major(y), (self._fused_state(h), self._fused_state(c))
         h, c = _eager_lstm(self.training, self.zoneout, x, h0, c0, self.kernel,
                            _dropped(self.recurrent_kernel, dmask, dscale), self.bias, zmask)
@@ -569,10 +555,10 @@ class GRU(_RNNBase):
         if fused:
             self._check_fused(x)
             wanted = self._wanted(lengths, x.device)
-            y, h = self._fused(_GRUFunction, self.training, self.zoneout, wanted, x.contiguous(), h0,
-                               self.kernel.contiguous(), self.recurrent_kernel.contiguous(),
-                               self.bias.contiguous(), self.recurrent_bias.contiguous(),
-                               zmask, dmask, dscale)
+            y, h = _GRUFunction.apply(self.training, self.zoneout, wanted, x.contiguous(), h0,
+                                      self.kernel.contiguous(), self.recurrent_kernel.contiguous(),
+                                      self.bias.contiguous(), self.recurrent_bias.contiguous(),
+                                      zmask, dmask, dscale)
             return self._time_major(y), self._fused_state(h)
         h = _eager_gru(self.training, self.zoneout, x, h0, self.kernel,
                        _dropped(self.recurrent_kernel, dmask, dscale), self.bias,
@@ -608,9 +594,9 @@ class IndRNN(_RNNBase):
         if fused:
             self._check_fused(x)
             wanted = self._wanted(lengths, x.device)
-            y, h = self._fused(_IndRNNFunction, self.training, self.zoneout, wanted, x.contiguous(), h0,
-                               self.kernel.contiguous(), self.recurrent_scale.contiguous(),
-                               self.bias.contiguous(), zmask)
+            y, h = _IndRNNFunction.apply(self.training, self.zoneout, wanted, x.contiguous(), h0,
+                                         self.kernel.contiguous(), self.recurrent_scale.contiguous(),
+                                         self.bias.contiguous(), zmask)
             return self._time_major(y), self._fused_state(h)
         h = _eager_indrnn(self.training, self.zoneout, x, h0, self.kernel, self.recurrent_scale,
                           self.bias, zmask)
@@ -646,9 +632,9 @@ class LayerNormIndRNN(_RNNBase):
         if fused:
             self._check_fused(x)
             wanted = self._wanted(lengths, x.device)
-            y, h = self._fused(_LayerNormIndRNNFunction, self.training, self.zoneout, wanted, x.contiguous(), h0,
-                               self.kernel.contiguous(), self.recurrent_scale.contiguous(),
-                               self.bias.contiguous(), self.gamma.contiguous(), zmask)
+            y, h = _LayerNormIndRNNFunction.apply(self.training, self.zoneout, wanted, x.contiguous(), h0,
+                                                  self.kernel.contiguous(), self.recurrent_scale.contiguous(),
+                                                  self.bias.contiguous(), self.gamma.contiguous(), zmask)
             return self._time_major(y), self._fused_state(h)
         h = _eager_indrnn(self.training, self.zoneout, x, h0, self.kernel, self.recurrent_scale,
                           self.bias, zmask, gamma=self.gamma)
@@ -693,10 +679,10 @@ class LayerNormLSTM(_RNNBase):
         if fused:
             self._check_fused(x)
             wanted = self._wanted(lengths, x.device)
-            y, h, c = self._fused(_LayerNormLSTMFunction, self.training, self.zoneout, wanted, x.contiguous(), h0, c0,
-                                  self.kernel.contiguous(), R.contiguous(),
-                                  self.bias.contiguous(), self.gamma.contiguous(),
-                                  self.gamma_h.contiguous(), self.beta_h.contiguous(), zmask)
+            y, h, c = _LayerNormLSTMFunction.apply(self.training, self.zoneout, wanted, x.contiguous(), h0, c0,
+                                                   self.kernel.contiguous(), R.contiguous(),
+                                                   self.bias.contiguous(), self.gamma.contiguous(),
+                                                   self.gamma_h.contiguous(), self.beta_h.contiguous(), zmask)
             return self._time_major(y), (self._fused_state(h), self._fused_state(c))
         h, c = _eager_lstm(self.training, self.zoneout, x, h0, c0, self.kernel, R, self.bias, zmask,
                            gamma=self.gamma, gamma_h=self.gamma_h, beta_h=self.beta_h)
@@ -735,10 +721,10 @@ class LayerNormGRU(_RNNBase):
         if fused:
             self._check_fused(x)
             wanted = self._wanted(lengths, x.device)
-            y, h = self._fused(_LayerNormGRUFunction, self.training, self.zoneout, wanted, x.contiguous(), h0,
-                               self.kernel.contiguous(), R.contiguous(),
-                               self.bias.contiguous(), self.recurrent_bias.contiguous(),
-                               self.gamma.contiguous(), zmask)
+            y, h = _LayerNormGRUFunction.apply(self.training, self.zoneout, wanted, x.contiguous(), h0,
+                                               self.kernel.contiguous(), R.contiguous(),
+                                               self.bias.contiguous(), self.recurrent_bias.contiguous(),
+                                               self.gamma.contiguous(), zmask)
             return self._time_major(y), self._fused_state(h)
         h = _eager_gru(self.training, self.zoneout, x, h0, self.kernel, R, self.bias,
                        self.recurrent_bias, zmask, gamma=self.gamma)

@@ -352,3 +352,23 @@ def test_lengths_that_are_changed_are_noticed(fused_lstm_on_cpu):
     _, (h3, c3) = layer(x, lengths=own)  # a tensor made in inference mode has no version to look at
     (h3.square().sum() + c3.sum()).backward()
     assert torch.equal(layer.kernel.grad, grads[0][1])
+
+
+@pytest.mark.filterwarnings("ignore")
+@pytest.mark.parametrize("grad", [True, False])
+def test_autograd_is_told_of_every_fused_pass(fused_lstm_on_cpu, grad):
+    """Also where there is nothing to differentiate: a trace holds the pass as one op (the kernels are not
+    seen by the tracer), and transforms that it has no rule for refuse instead of dropping what they carry."""
+    import torch.autograd.forward_ad as forward_ad
+    layer = fused_lstm_on_cpu(4, 6)
+    x = torch.randn(5, 3, 4)
+    with torch.set_grad_enabled(grad):
+        traced = torch.jit.trace(layer, (x,), check_trace=False)
+        assert "_LSTMFunction" in str(traced.inlined_graph)
+        other = torch.randn(5, 3, 4)
+        for got, want in zip((traced(other)[0], *traced(other)[1]), (layer(other)[0], *layer(other)[1])):
+            assert torch.equal(got, want)
+        with forward_ad.dual_level(), pytest.raises(RuntimeError, match="jvp"):
+            layer(forward_ad.make_dual(x, torch.ones_like(x)))
+        with pytest.raises(RuntimeError, match="vmap"):
+            torch.func.vmap(layer)(x.expand(2, 5, 3, 4))
