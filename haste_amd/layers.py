@@ -60,15 +60,21 @@ def _one_per_row(wanted, seq):
     return wanted.dim() == 1 and wanted.size(0) == seq.size(1) and wanted.is_contiguous() and seq.numel() > 0
 
 
+# Outputs that share memory must share a version counter, or autograd does not see that a change of one
+# (padding masked in place, say) changes another that was saved: the states of h that y holds are either
+# views of y, taken by the layer (None here), or a copy (3 us) where a view would bring back the gradients
+# of slices.
 def _wanted_states(seqs, wanted):
-    """What a layer returns of its state sequences [T+1,N,H]: "last" [N,H], "all" [T,N,H], or the states
-    at the steps in an index tensor [N]."""
+    """What a layer returns of its state sequences [T+1,N,H], h's first: "last" [N,H] ("last of y" where
+    nothing is differentiated), "all" [T,N,H], or the states at the steps in an index tensor [N].  None:
+    the layer takes it from y."""
     if torch.is_tensor(wanted):
         if _one_per_row(wanted, seqs[0]):
             return ops.gather_states(seqs, wanted)
         cols = torch.arange(seqs[0].size(1), device=wanted.device)
         return tuple(seq[wanted, cols] for seq in seqs)
-    return tuple(_alias(seq, 1 if wanted == "all" else -1) for seq in seqs)
+    h = seqs[0][-1].clone() if wanted == "last" else None
+    return (h,) + tuple(_alias(seq, 1 if wanted == "all" else -1) for seq in seqs[1:])
 
 
 def _upstream(like, grad_steps, grad_wanted, wanted):
@@ -80,7 +86,7 @@ def _upstream(like, grad_steps, grad_wanted, wanted):
     if not torch.is_tensor(wanted):
         if wanted == "last":
             return grad_steps if grad_steps is None else grad_steps.contiguous(), grad_wanted
-        return (grad_wanted if grad_steps is None else grad_steps + grad_wanted).contiguous(), None
+        return grad_wanted.contiguous(), None  # of c: those of h are y's
     if _one_per_row(wanted, like):
         return ops.state_gradients(like, grad_steps, grad_wanted, wanted), None
     full = torch.zeros_like(like) if grad_steps is None else torch.empty_like(like)
@@ -393,10 +399,14 @@ class _RNNBase(nn.Module):
         """Which states the fused functions are to return (see _wanted_states)."""
         if self.return_state_sequence:
             return "all"
-        return "last" if lengths is None else torch.as_tensor(lengths, device=device, dtype=torch.long)
+        if lengths is None:
+            return "last" if torch.is_grad_enabled() else "last of y"
+        return torch.as_tensor(lengths, device=device, dtype=torch.long)
 
-    def _fused_state(self, states):
-        """A state as the layer returns it, from what the fused functions return of it."""
+    def _fused_state(self, states, y=None):
+        """A state as the layer returns it, from what the fused functions return of it (None: y holds it)."""
+        if states is None:
+            states = y if self.return_state_sequence else y[-1]
         return (self._time_major(states) if self.return_state_sequence else states).unsqueeze(0)
 
     def _final_state(self, seq, lengths):
@@ -506,7 +516,7 @@ class LSTM(_RNNBase):
             y, h, c = _LSTMFunction.apply(self.training, self.zoneout, wanted, x.contiguous(), h0, c0,
                                           self.kernel.contiguous(), self.recurrent_kernel.contiguous(),
                                           self.bias.contiguous(), zmask, dmask, dscale)
-            return self._time_major(y), (self._fused_state(h), self._fused_state(c))
+            return self._time_major(y), (self._fused_state(h, y), self._fused_state(c))
         h, c = _eager_lstm(self.training, self.zoneout, x, h0, c0, self.kernel,
                            _dropped(self.recurrent_kernel, dmask, dscale), self.bias, zmask)
         return self._time_major(h[1:]), (self._final_state(h, lengths), self._final_state(c, lengths))
@@ -559,7 +569,7 @@ class GRU(_RNNBase):
                                       self.kernel.contiguous(), self.recurrent_kernel.contiguous(),
                                       self.bias.contiguous(), self.recurrent_bias.contiguous(),
                                       zmask, dmask, dscale)
-            return self._time_major(y), self._fused_state(h)
+            return self._time_major(y), self._fused_state(h, y)
         h = _eager_gru(self.training, self.zoneout, x, h0, self.kernel,
                        _dropped(self.recurrent_kernel, dmask, dscale), self.bias,
                        self.recurrent_bias, zmask)
@@ -597,7 +607,7 @@ class IndRNN(_RNNBase):
             y, h = _IndRNNFunction.apply(self.training, self.zoneout, wanted, x.contiguous(), h0,
                                          self.kernel.contiguous(), self.recurrent_scale.contiguous(),
                                          self.bias.contiguous(), zmask)
-            return self._time_major(y), self._fused_state(h)
+            return self._time_major(y), self._fused_state(h, y)
         h = _eager_indrnn(self.training, self.zoneout, x, h0, self.kernel, self.recurrent_scale,
                           self.bias, zmask)
         return self._time_major(h[1:]), self._final_state(h, lengths)
@@ -635,7 +645,7 @@ class LayerNormIndRNN(_RNNBase):
             y, h = _LayerNormIndRNNFunction.apply(self.training, self.zoneout, wanted, x.contiguous(), h0,
                                                   self.kernel.contiguous(), self.recurrent_scale.contiguous(),
                                                   self.bias.contiguous(), self.gamma.contiguous(), zmask)
-            return self._time_major(y), self._fused_state(h)
+            return self._time_major(y), self._fused_state(h, y)
         h = _eager_indrnn(self.training, self.zoneout, x, h0, self.kernel, self.recurrent_scale,
                           self.bias, zmask, gamma=self.gamma)
         return self._time_major(h[1:]), self._final_state(h, lengths)
@@ -683,7 +693,7 @@ class LayerNormLSTM(_RNNBase):
                                                    self.kernel.contiguous(), R.contiguous(),
                                                    self.bias.contiguous(), self.gamma.contiguous(),
                                                    self.gamma_h.contiguous(), self.beta_h.contiguous(), zmask)
-            return self._time_major(y), (self._fused_state(h), self._fused_state(c))
+            return self._time_major(y), (self._fused_state(h, y), self._fused_state(c))
         h, c = _eager_lstm(self.training, self.zoneout, x, h0, c0, self.kernel, R, self.bias, zmask,
                            gamma=self.gamma, gamma_h=self.gamma_h, beta_h=self.beta_h)
         return self._time_major(h[1:]), (self._final_state(h, lengths), self._final_state(c, lengths))
@@ -725,7 +735,7 @@ class LayerNormGRU(_RNNBase):
                                                self.kernel.contiguous(), R.contiguous(),
                                                self.bias.contiguous(), self.recurrent_bias.contiguous(),
                                                self.gamma.contiguous(), zmask)
-            return self._time_major(y), self._fused_state(h)
+            return self._time_major(y), self._fused_state(h, y)
         h = _eager_gru(self.training, self.zoneout, x, h0, self.kernel, R, self.bias,
                        self.recurrent_bias, zmask, gamma=self.gamma)
         return self._time_major(h[1:]), self._final_state(h, lengths)

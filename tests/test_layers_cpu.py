@@ -372,3 +372,27 @@ def test_autograd_is_told_of_every_fused_pass(fused_lstm_on_cpu, grad):
             layer(forward_ad.make_dual(x, torch.ones_like(x)))
         with pytest.raises(RuntimeError, match="vmap"):
             torch.func.vmap(layer)(x.expand(2, 5, 3, 4))
+
+
+@pytest.mark.parametrize("how", ["frozen", "no_grad", "trained"])
+@pytest.mark.parametrize("wanted", ["last", "lengths", "all"])
+def test_a_state_that_was_saved_survives_changes_of_the_output(fused_lstm_on_cpu, how, wanted):
+    """A head behind the layer saves h_n; masking y in place afterwards must not change what the head's
+    gradient is computed from without autograd saying so."""
+    torch.manual_seed(7)
+    layer = fused_lstm_on_cpu(4, 6, return_state_sequence=wanted == "all", batch_first=wanted == "all")
+    layer.requires_grad_(how == "trained")
+    with torch.set_grad_enabled(how != "no_grad"):
+        y, (h, _) = layer(torch.randn(5, 3, 4), lengths=[5, 1, 3] if wanted == "lengths" else None)
+    w = torch.randn_like(h).requires_grad_()
+    want = h.detach().clone()
+    assert torch.equal(want[0] if wanted == "all" else want[0, 0], y if wanted == "all" else y[-1, 0])
+    loss = (h * w).sum()
+    with torch.no_grad():
+        y.mul_(0.0)
+    try:
+        (grad,) = torch.autograd.grad(loss, w)
+    except RuntimeError as e:
+        assert "modified by an inplace operation" in str(e)
+    else:
+        assert torch.equal(grad, want)
