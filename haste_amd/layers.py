@@ -93,9 +93,9 @@ def _upstream(like, grad_steps, grad_wanted, wanted):
     if grad_steps is not None:
         full[1:] = grad_steps
         full[0].zero_()
-    # one entry per batch row: nothing is indexed twice
     cols = torch.arange(like.size(1), device=like.device)
-    full[wanted, cols] = full[wanted, cols] + grad_wanted
+    # several steps of a row may be asked for, the same one twice among them
+    full.index_put_((wanted, cols), grad_wanted, accumulate=True)
     return full, None
 
 

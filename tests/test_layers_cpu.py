@@ -396,3 +396,23 @@ def test_a_state_that_was_saved_survives_changes_of_the_output(fused_lstm_on_cpu
         assert "modified by an inplace operation" in str(e)
     else:
         assert torch.equal(grad, want)
+
+
+@pytest.mark.parametrize("lengths", [[[5, 1, 3], [5, 2, 3]], 4, [2]])
+def test_lengths_of_any_shape_that_indexing_takes(fused_lstm_on_cpu, lengths):
+    """Several steps per row (one of them twice), one step for all rows: states and gradients of the plain loop."""
+    torch.manual_seed(8)
+    layer = fused_lstm_on_cpu(4, 6).double()
+    plain = haste_amd.LSTM(4, 6).double()
+    plain.load_state_dict(layer.state_dict())
+    plain._is_cuda = lambda: False
+    x = torch.randn(5, 3, 4, dtype=torch.float64)
+    results = []
+    for net in (layer, plain):
+        y, (h, c) = net(x, lengths=lengths)
+        gen = torch.Generator().manual_seed(9)
+        loss = sum((s * torch.randn(s.shape, generator=gen, dtype=s.dtype)).sum() for s in (y, h, c))
+        loss.backward()
+        results.append([h, c] + [p.grad for p in net.parameters()])
+    for got, want in zip(*results):
+        assert got.shape == want.shape and torch.allclose(got, want, rtol=1e-12, atol=1e-12)
