@@ -294,23 +294,30 @@ int open_scratch(hipStream_t stream, size_t own_bytes, size_t gemm_bytes, Scratc
   return HASTE_HIP_OK;
 }
 
-// Scratch for the exchange tiles of a recurrence in one launch (recurrent_f64.hip), 0 when the
+// *bytes: scratch for the exchange tiles of a recurrence in one launch (recurrent_f64.hip), 0 when the
 // call runs step by step: always for float (its persistent kernels are the callers of this file),
 // and for double when the shape does not fit the chip, while the stream is being captured (a
 // persistent launch needs a control block that replays wipe, and these calls never had one in
-// their graphs), and in memory lent by the caller that is too small for the tiles.
+// their graphs), and in memory lent by the caller that is too small for the tiles.  An error of the
+// workspace is the call's: get_workspace() is also what reports, once, that an earlier launch timed out.
 template <typename T>
-size_t one_launch_bytes(hipStream_t, int, int, int, int, int, size_t) { return 0; }
+int one_launch_bytes(hipStream_t, int, int, int, int, int, size_t, size_t* bytes) {
+  *bytes = 0;
+  return HASTE_HIP_OK;
+}
 template <>
-size_t one_launch_bytes<double>(hipStream_t stream, int in_gates, int out_gates, int steps, int N, int H, size_t others) {
-  const size_t bytes = padded(recurrence64_scratch_bytes(in_gates, out_gates, steps, N, H));
-  if (bytes == 0) return 0;
+int one_launch_bytes<double>(hipStream_t stream, int in_gates, int out_gates, int steps, int N, int H, size_t others,
+                             size_t* bytes) {
+  *bytes = 0;
+  const size_t tiles = padded(recurrence64_scratch_bytes(in_gates, out_gates, steps, N, H));
+  if (tiles == 0) return HASTE_HIP_OK;
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &capture) != hipSuccess) (void)hipGetLastError();
-  if (capture != hipStreamCaptureStatusNone) return 0;
+  if (capture != hipStreamCaptureStatusNone) return HASTE_HIP_OK;
   Workspace ws;
-  if (get_workspace(stream, 0, &ws) != HASTE_HIP_OK) return 0;
-  return ws.caller_owned && ws.scratch_bytes < others + bytes + 256 ? 0 : bytes;
+  HASTE_HIP_PROPAGATE(get_workspace(stream, 0, &ws));
+  if (!ws.caller_owned || ws.scratch_bytes >= others + tiles + 256) *bytes = tiles;
+  return HASTE_HIP_OK;
 }
 
 // ---- small kernels ------------------------------------------------------------------
@@ -820,7 +827,8 @@ int lstm_forward_steps(hipStream_t stream, int training, int steps, int N, int C
   const size_t NH = (size_t)N * H, N4H = NH * 4, r_count = (size_t)H * 4 * H;
   size_t own = padded(N4H * sizeof(T)) + (dc_mask ? padded(r_count * sizeof(T)) : 0);
   const size_t room = max2(gemm_room<T>(steps * N, 4 * H, C), gemm_room<T>(N, 4 * H, H));
-  const size_t tiles = one_launch_bytes<T>(stream, 1, 4, steps, N, H, own + room);
+  size_t tiles = 0;
+  HASTE_HIP_PROPAGATE(one_launch_bytes<T>(stream, 1, 4, steps, N, H, own + room, &tiles));
   own += tiles;
   Scratch sc;
   HASTE_HIP_PROPAGATE(open_scratch(stream, own, room, &sc));
@@ -856,7 +864,8 @@ int lstm_backward_steps(hipStream_t stream, int steps, int N, int C, int H, cons
   const size_t sums = column_sum_bytes<T>((size_t)TN, 4 * H);
   size_t room = max2(gemm_room<T>(N, H, 4 * H), gemm_room<T>(C, 4 * H, TN));
   room = max2(room, max2(gemm_room<T>(H, 4 * H, TN), gemm_room<T>(TN, C, 4 * H)));
-  const size_t tiles = one_launch_bytes<T>(stream, 4, 1, steps, N, H, sums + room);
+  size_t tiles = 0;
+  HASTE_HIP_PROPAGATE(one_launch_bytes<T>(stream, 4, 1, steps, N, H, sums + room, &tiles));
   Scratch sc;
   HASTE_HIP_PROPAGATE(open_scratch(stream, sums + tiles, room, &sc));
   void* partial = sc.take<char>(sums);
@@ -893,7 +902,8 @@ int gru_forward_steps(hipStream_t stream, int training, int steps, int N, int C,
   const size_t NH = (size_t)N * H, N3H = NH * 3, N4H = NH * 4, r_count = (size_t)H * 3 * H;
   size_t own = padded(N3H * sizeof(T)) + (dc_mask ? padded(r_count * sizeof(T)) : 0);
   const size_t room = max2(gemm_room<T>(steps * N, 3 * H, C), gemm_room<T>(N, 3 * H, H));
-  const size_t tiles = one_launch_bytes<T>(stream, 1, 3, steps, N, H, own + room);
+  size_t tiles = 0;
+  HASTE_HIP_PROPAGATE(one_launch_bytes<T>(stream, 1, 3, steps, N, H, own + room, &tiles));
   own += tiles;
   Scratch sc;
   HASTE_HIP_PROPAGATE(open_scratch(stream, own, room, &sc));
@@ -928,7 +938,8 @@ int gru_backward_steps(hipStream_t stream, int steps, int N, int C, int H, const
   const size_t sums = column_sum_bytes<T>((size_t)TN, 3 * H);
   size_t room = max2(gemm_room<T>(N, H, 3 * H), gemm_room<T>(C, 3 * H, TN));
   room = max2(room, max2(gemm_room<T>(H, 3 * H, TN), gemm_room<T>(TN, C, 3 * H)));
-  const size_t tiles = one_launch_bytes<T>(stream, 3, 1, steps, N, H, sums + room);
+  size_t tiles = 0;
+  HASTE_HIP_PROPAGATE(one_launch_bytes<T>(stream, 3, 1, steps, N, H, sums + room, &tiles));
   Scratch sc;
   HASTE_HIP_PROPAGATE(open_scratch(stream, sums + tiles, room, &sc));
   void* partial = sc.take<char>(sums);
