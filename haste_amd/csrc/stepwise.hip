@@ -300,6 +300,8 @@ int open_scratch(hipStream_t stream, size_t own_bytes, size_t gemm_bytes, Scratc
 // persistent launch needs a control block that replays wipe, and these calls never had one in
 // their graphs), and in memory lent by the caller that is too small for the tiles.  An error of the
 // workspace is the call's: get_workspace() is also what reports, once, that an earlier launch timed out.
+// The callers ask for the tiles on top of what the steps take: a call made ahead of a capture then leaves
+// the captured one, which runs step by step, a buffer that need not grow.
 template <typename T>
 int one_launch_bytes(hipStream_t, int, int, int, int, int, size_t, size_t* bytes) {
   *bytes = 0;
