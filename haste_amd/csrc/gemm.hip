@@ -354,12 +354,15 @@ __device__ __forceinline__ void split_tile(int M, int N, int K, const float* __r
   // neighbours, and neighbour i goes to MFMA tile i: writes to LDS stay consecutive, and a lane
   // ends up with two neighbouring columns of C.
   float a_raw[MI][8], b_raw[2][8];
+  // Where row k of a panel starts; rows from K on are beyond every panel (with few of them and a long
+  // stride their own offset need not be: it wraps at 2^32).  Scalar arithmetic: a wavefront's k are its own.
+  const int wave_k = 8 * __builtin_amdgcn_readfirstlane(wave);
+  auto row_at = [&](int k, int ld) { return k < K ? (unsigned)k * (unsigned)ld * 4u : 0x80000000u; };
   auto load_global = [&](int kk) {
     if constexpr (TRANS_A) {
-      const unsigned int base = ((unsigned)(kk + 8 * wave) * (unsigned)lda + (unsigned)(lane * MI)) * 4u;
 #pragma unroll
       for (int r = 0; r < 8; ++r) {
-        const unsigned int off = base + (unsigned)(r * lda) * 4u;
+        const unsigned int off = row_at(kk + wave_k + r, lda) + (unsigned)(lane * MI) * 4u;
         if constexpr (MI == 2) {
           const auto u = __builtin_amdgcn_raw_buffer_load_b64(a_panel, off, 0, 0);
           a_raw[0][r] = __uint_as_float(u[0]);
@@ -382,10 +385,9 @@ __device__ __forceinline__ void split_tile(int M, int N, int K, const float* __r
         }
       }
     }
-    const unsigned int base = ((unsigned)(kk + 8 * wave) * (unsigned)ldb + (unsigned)(lane * 2)) * 4u;
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
-      const auto u = __builtin_amdgcn_raw_buffer_load_b64(b_panel, base + (unsigned)(r * ldb) * 4u, 0, 0);
+      const auto u = __builtin_amdgcn_raw_buffer_load_b64(b_panel, row_at(kk + wave_k + r, ldb) + (unsigned)(lane * 2) * 4u, 0, 0);
       b_raw[0][r] = __uint_as_float(u[0]);
       b_raw[1][r] = __uint_as_float(u[1]);
     }

@@ -158,6 +158,28 @@ def test_gemm_edges_and_range(trans_a, M, N, K, scale_a, scale_b):
     assert np.all(np.abs(out - a64 @ b64) <= _bound(a64, b64, K) + K * 2.0 ** -149)
 
 
+@pytest.mark.parametrize("K", [1, 4, 6])
+def test_gemm_few_rows_of_a_long_stride(K):
+    """Rows 2^26 floats apart: the byte offset of rows that a stage of 32 k looks at beyond the last one
+    wraps at 2^32, to the panel's first rows."""
+    import torch
+    from haste_amd import lib
+    M, N, ld = 130, 70, 1 << 26
+    r = np.random.default_rng(K)
+    a, b = (r.standard_normal((K, n)).astype(np.float32) for n in (M, N))
+    views = []
+    for m in (a, b):
+        t = torch.empty((K - 1) * ld + m.shape[1], device="cuda")
+        views.append(t.as_strided(m.shape, (ld, 1)))
+        views[-1].copy_(torch.from_numpy(m))
+    out = torch.empty(M, N, device="cuda")
+    print("gemm long stride", K, ld, flush=True)
+    lib.call("haste_hip_gemm_f32", 1, M, N, K, views[0], ld, views[1], ld, out, N, 0)
+    torch.cuda.synchronize()
+    a64, b64 = a.T.astype(np.float64), b.astype(np.float64)
+    assert np.all(np.abs(host(out) - a64 @ b64) <= _bound(a64, b64, K))
+
+
 @pytest.mark.parametrize("trans_a", [False, True])
 def test_gemm_operands_that_are_not_finite(trans_a):
     """Infinities, NaNs and values beyond the largest bfloat16 give what float arithmetic gives, and
