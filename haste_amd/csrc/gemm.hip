@@ -12,9 +12,10 @@
 // three left out are below 2^-24 of the largest.  The five small products have an accumulator
 // of their own, so that the large one is rounded once per 16 k where the fp32 instruction
 // (32x32x2) rounds eight times.  Measured against float64, normal operands: 0.3 - 0.4 of the
-// fp32 instruction's error (2-norm, K = 75 .. 160000).  A tile in which that does not work --
-// infinities, NaNs, values within 0.4 % of the largest float, results so small that the third
-// parts fall below the smallest bfloat16 -- is computed again with the fp32 instruction.
+// fp32 instruction's error (2-norm, K = 75 .. 160000).  Operands are scaled by a power of two, so
+// that the parts of the smallest floats are bfloat16 too; a tile in which that does not work --
+// infinities, NaNs, operands from 2^104 or results from 2^80 on -- is computed again with the fp32
+// instruction.
 //
 // Design: 128x128 output tile per 256-thread workgroup (4 wavefronts, each a 64x64 quadrant =
 // 2x2 v_mfma_f32_32x32x16_bf16 tiles), K consumed 32 at a time.  A stage is read as float,
@@ -286,12 +287,18 @@ __device__ __forceinline__ unsigned int pack_bf16(float a, float b) {
 __device__ __forceinline__ float bf16_low(unsigned int u) { return __uint_as_float(u << 16); }
 __device__ __forceinline__ float bf16_high(unsigned int u) { return __uint_as_float(u & 0xffff0000u); }
 
-// Eight consecutive k of one row, split into three bf16 each and stored into the three planes.
+// What operands are multiplied with before they are split, and the product's scale that comes of it.  A
+// bfloat16 holds nothing below 2^-133, a float goes down to 2^-149: unscaled, operands below 2^-110 would
+// lose their last part and those below 2^-134 all three.  Scaled, every part of every float is a normal
+// bfloat16; in exchange operands from 2^104 and results from 2^80 on are infinite, which split_tile() sees.
+constexpr float kSplitScale = 0x1p24f, kProductScale = 0x1p-48f;
+
+// Eight consecutive k of one row, scaled, split into three bf16 each and stored into the three planes.
 __device__ __forceinline__ void split_store(const float (&f)[8], char* at, int plane_bytes) {
   uint4_t p[3];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    float a = f[2 * j], b = f[2 * j + 1];
+    float a = f[2 * j] * kSplitScale, b = f[2 * j + 1] * kSplitScale;
     const unsigned int hi = pack_bf16(a, b);
     a -= bf16_low(hi);
     b -= bf16_high(hi);
@@ -305,11 +312,6 @@ __device__ __forceinline__ void split_store(const float (&f)[8], char* at, int p
 #pragma unroll
   for (int q = 0; q < 3; ++q) *reinterpret_cast<uint4_t*>(at + q * plane_bytes) = p[q];
 }
-
-// A bfloat16 cannot hold what lies below 2^-133.  When everything a wavefront computed is smaller
-// than this, that may be visible (the loss is at most 2^-134 per operand element): 2^-90 leaves
-// it below a float's rounding for partners up to 2^7 and K up to 2^13.
-constexpr float kTinyTile = 0x1p-90f;
 
 // One BM x 128 output tile, BM = 64 * MI, over the K range [k_begin, k_end): MI = 2 (each
 // wavefront a 64x64 quadrant) or 1 (each a 32x64 quadrant) for outputs of at most 64 rows.
@@ -457,21 +459,17 @@ __device__ __forceinline__ void split_tile(int M, int N, int K, const float* __r
 #pragma unroll
   for (int i = 0; i < MI; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] += low[i][j];
-  // An operand that is not finite, or rounds to infinity as a bfloat16, gives NaNs here, and parts
-  // below the smallest bfloat16 are lost: such tiles are computed again on the float matrix cores.
-  float finite = 0.f, largest = 0.f;
+    for (int j = 0; j < 2; ++j) acc[i][j] = (acc[i][j] + low[i][j]) * kProductScale;
+  // An operand that is not finite, or is not once it is scaled, gives infinities or NaNs here, and so do
+  // results that scaled are beyond the largest float: such tiles are computed again on the float matrix cores.
+  float finite = 0.f;
 #pragma unroll
   for (int i = 0; i < MI; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        finite = fmaf(acc[i][j][e], 0.f, finite);
-        largest = fmaxf(largest, fabsf(acc[i][j][e]));
-      }
-  const bool tiny = __all(largest < kTinyTile) && __any(largest > 0.f);
-  if (__syncthreads_or(!(finite == 0.f) || tiny)) {
+      for (int e = 0; e < 16; ++e) finite = fmaf(acc[i][j][e], 0.f, finite);
+  if (__syncthreads_or(!(finite == 0.f))) {
     float_tile<TRANS_A, BM>(M, N, K, A, lda, B, ldb, C, ldc, accumulate, tm, tn, k_begin, k_end, part,
                            reinterpret_cast<float*>(smem));
     return;

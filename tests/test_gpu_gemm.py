@@ -142,7 +142,8 @@ def _bound(a64, b64, K):
 @pytest.mark.parametrize("M,N,K", [
     (1, 1, 1), (63, 127, 31), (64, 128, 32), (65, 129, 33), (127, 2, 63), (128, 130, 64), (129, 255, 65),
     (66, 3, 7), (192, 257, 1029), (70, 70, 4099)])
-@pytest.mark.parametrize("scale_a,scale_b", [(1.0, 1.0), (1e-37, 1.0), (1e-20, 1e-18), (1e30, 1e-30), (1e18, 1e18)])
+@pytest.mark.parametrize("scale_a,scale_b", [(1.0, 1.0), (1e-37, 1.0), (1e-20, 1e-18), (1e30, 1e-30), (1e18, 1e18),
+                                             (1e-37, 1e18), (1e-36, 1e10), (1e-41, 1e30), (1e30, 1e-43), (1e-22, 1e-22)])
 def test_gemm_edges_and_range(trans_a, M, N, K, scale_a, scale_b):
     """Every edge of the 64 / 128 x 128 tiles and of the 32 k of a stage, operands from the smallest
     to the largest floats (what a float cannot represent of the result excepted)."""
@@ -155,6 +156,24 @@ def test_gemm_edges_and_range(trans_a, M, N, K, scale_a, scale_b):
     out = host(ops.gemm(dev(a), dev(b), trans_a=trans_a)).astype(np.float64)
     torch.cuda.synchronize()
     a64, b64 = (a.T if trans_a else a).astype(np.float64), b.astype(np.float64)
+    assert np.all(np.abs(out - a64 @ b64) <= _bound(a64, b64, K) + K * 2.0 ** -149)
+
+
+@pytest.mark.parametrize("trans_a", [False, True])
+@pytest.mark.parametrize("M,N,K", [(150, 140, 512), (40, 130, 75), (512, 256, 2080)])
+def test_gemm_operands_of_all_sizes_in_a_tile(trans_a, M, N, K):
+    """Rows of A and columns of B from the smallest floats to large ones side by side: every result as
+    accurate as its own operands allow, whatever lies beside it."""
+    import torch
+    from haste_amd import ops
+    r = np.random.default_rng(M + N + K)
+    rows, cols = 10.0 ** r.uniform(-44, 10, (M, 1)), 10.0 ** r.uniform(-44, 10, (1, N))
+    rows[::5], cols[:, ::5] = 1.0, 1.0
+    a = (r.standard_normal((M, K)) * rows).astype(np.float32)
+    b = (r.standard_normal((K, N)) * cols).astype(np.float32)
+    out = host(ops.gemm(dev(a.T if trans_a else a), dev(b), trans_a=trans_a)).astype(np.float64)
+    torch.cuda.synchronize()
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
     assert np.all(np.abs(out - a64 @ b64) <= _bound(a64, b64, K) + K * 2.0 ** -149)
 
 
