@@ -460,6 +460,11 @@ __device__ __forceinline__ void split_tile(int M, int N, int K, const float* __r
   for (int i = 0; i < MI; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = (acc[i][j] + low[i][j]) * kProductScale;
+  const int col = wc * 64 + 2 * (lane & 31);
+  auto row_of = [&](int i, int e) {
+    const int q = 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
+    return TRANS_A ? wr * WM + MI * q + i : wr * WM + 32 * i + q;
+  };
   // An operand that is not finite, or is not once it is scaled, gives infinities or NaNs here, and so do
   // results that scaled are beyond the largest float: such tiles are computed again on the float matrix cores.
   float finite = 0.f;
@@ -468,22 +473,24 @@ __device__ __forceinline__ void split_tile(int M, int N, int K, const float* __r
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) finite = fmaf(acc[i][j][e], 0.f, finite);
+      for (int e = 0; e < 16; ++e) {
+        // what lies beside the matrices (between rows of a longer stride) is nobody's to judge by
+        const bool inside = row_of(i, e) < rows_here && col + j < cols_here;
+        finite = fmaf(inside ? acc[i][j][e] : 0.f, 0.f, finite);
+      }
   if (__syncthreads_or(!(finite == 0.f))) {
     float_tile<TRANS_A, BM>(M, N, K, A, lda, B, ldb, C, ldc, accumulate, tm, tn, k_begin, k_end, part,
                            reinterpret_cast<float*>(smem));
     return;
   }
 
-  const int col = wc * 64 + 2 * (lane & 31);
   // Whole tiles with 8-byte aligned rows: a lane's two columns in one store.
   const bool wide = cols_here == BN && (ldc & 1) == 0 && (reinterpret_cast<uintptr_t>(C) & 7) == 0;
 #pragma unroll
   for (int i = 0; i < MI; ++i)
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
-      const int q = 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
-      const int row = TRANS_A ? wr * WM + MI * q + i : wr * WM + 32 * i + q;
+      const int row = row_of(i, e);
       if (part != nullptr) {
         const float2_t v = {acc[i][0][e], acc[i][1][e]};
         *reinterpret_cast<float2_t*>(part + row * BN + col) = v;

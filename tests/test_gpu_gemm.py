@@ -177,6 +177,29 @@ def test_gemm_operands_of_all_sizes_in_a_tile(trans_a, M, N, K):
     assert np.all(np.abs(out - a64 @ b64) <= _bound(a64, b64, K) + K * 2.0 ** -149)
 
 
+@pytest.mark.parametrize("trans_a", [False, True])
+@pytest.mark.parametrize("M,N,K", [(130, 104, 512), (60, 200, 100)])
+def test_gemm_memory_beside_the_matrices_does_not_matter(trans_a, M, N, K):
+    """Operands that are columns of wider matrices: bit for bit the same product whatever the other columns hold."""
+    import torch
+    from haste_amd import lib
+    gen = torch.Generator().manual_seed(M)
+    wide = [torch.randn(K if trans_a else M, 260, generator=gen), torch.randn(K, 260, generator=gen)]
+    wide = [m.cuda() for m in wide] if trans_a else [torch.randn(M, K, generator=gen).cuda(), wide[1].cuda()]
+    outs = []
+    for beside in (0.0, float("nan"), float("inf"), 3e38, 1e-40):
+        if trans_a:
+            wide[0][:, M:] = beside
+        wide[1][:, N:] = beside
+        out = torch.empty(M, N, device="cuda")
+        lib.call("haste_hip_gemm_f32", int(trans_a), M, N, K, wide[0], wide[0].stride(0), wide[1], 260, out, N, 0)
+        outs.append(out)
+    assert all(torch.equal(out, outs[0]) for out in outs)
+    a = wide[0][:, :M].t() if trans_a else wide[0]
+    a64, b64 = a.cpu().double().numpy(), wide[1][:, :N].cpu().double().numpy()
+    assert np.all(np.abs(host(outs[0]) - a64 @ b64) <= _bound(a64, b64, K))
+
+
 @pytest.mark.parametrize("K", [1, 4, 6])
 def test_gemm_few_rows_of_a_long_stride(K):
     """Rows 2^26 floats apart: the byte offset of rows that a stage of 32 k looks at beyond the last one
