@@ -35,17 +35,19 @@ void gather_states_kernel(int T, int N, int H, StateJobs<V> jobs, const long lon
 }
 
 // out[t][n] = grad[t][n] (0 without grad) + last[n] where t + 1 is the row's length; length 0 names
-// the initial state, which is no step's.
+// the initial state, which is no step's.  A row whose length names no step had NaNs for a state: so are
+// its gradients.
 template <typename V>
 __global__ __launch_bounds__(kStateThreads)
 void state_gradients_kernel(int T, int N, int H, const V* __restrict__ grad, size_t step_stride, size_t row_stride,
                             const V* __restrict__ last, const long long* __restrict__ lengths, V* __restrict__ out) {
   const int t = blockIdx.x / N, n = blockIdx.x % N;
-  const bool here = step_of(lengths[n], T) == t + 1;
+  const long long s = step_of(lengths[n], T);
   const V* from = grad + t * step_stride + n * row_stride;
   for (int j = threadIdx.x; j < H; j += kStateThreads) {
     V v = grad != nullptr ? from[j] : V(0);
-    if (here) v = v + last[(size_t)n * H + j];
+    if (s == t + 1) v = v + last[(size_t)n * H + j];
+    if (s < 0) v = V(__builtin_nanf(""));
     out[(size_t)blockIdx.x * H + j] = v;
   }
 }

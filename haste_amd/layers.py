@@ -395,13 +395,20 @@ class _RNNBase(nn.Module):
                                  % (shape, list(s.shape) if torch.is_tensor(s) else type(s)))
         return tuple(s[0].contiguous() for s in states)
 
-    def _wanted(self, lengths, device):
-        """Which states the fused functions are to return (see _wanted_states)."""
+    def _wanted(self, lengths, x):
+        """Which states the fused functions are to return (see _wanted_states).  Lengths beyond x are an
+        error where the host knows them; on the GPU they give NaNs, for the states and the gradients of their rows."""
         if self.return_state_sequence:
             return "all"
         if lengths is None:
             return "last" if torch.is_grad_enabled() else "last of y"
-        return torch.as_tensor(lengths, device=device, dtype=torch.long)
+        lengths = torch.as_tensor(lengths, dtype=torch.long)
+        steps = x.shape[0]
+        if not lengths.is_cuda and lengths.numel():
+            for length in lengths.aminmax():
+                if not -steps - 1 <= length <= steps:
+                    raise IndexError("length %d is out of bounds for sequences of %d steps" % (length, steps))
+        return lengths.to(x.device)
 
     def _fused_state(self, states, y=None):
         """A state as the layer returns it, from what the fused functions return of it (None: y holds it)."""
@@ -512,7 +519,7 @@ class LSTM(_RNNBase):
         zmask = self._zoneout_mask(x)
         if fused:
             self._check_fused(x)
-            wanted = self._wanted(lengths, x.device)
+            wanted = self._wanted(lengths, x)
             y, h, c = _LSTMFunction.apply(self.training, self.zoneout, wanted, x.contiguous(), h0, c0,
                                           self.kernel.contiguous(), self.recurrent_kernel.contiguous(),
                                           self.bias.contiguous(), zmask, dmask, dscale)
@@ -564,7 +571,7 @@ class GRU(_RNNBase):
         zmask = self._zoneout_mask(x)
         if fused:
             self._check_fused(x)
-            wanted = self._wanted(lengths, x.device)
+            wanted = self._wanted(lengths, x)
             y, h = _GRUFunction.apply(self.training, self.zoneout, wanted, x.contiguous(), h0,
                                       self.kernel.contiguous(), self.recurrent_kernel.contiguous(),
                                       self.bias.contiguous(), self.recurrent_bias.contiguous(),
@@ -603,7 +610,7 @@ class IndRNN(_RNNBase):
         zmask = self._zoneout_mask(x)
         if fused:
             self._check_fused(x)
-            wanted = self._wanted(lengths, x.device)
+            wanted = self._wanted(lengths, x)
             y, h = _IndRNNFunction.apply(self.training, self.zoneout, wanted, x.contiguous(), h0,
                                          self.kernel.contiguous(), self.recurrent_scale.contiguous(),
                                          self.bias.contiguous(), zmask)
@@ -641,7 +648,7 @@ class LayerNormIndRNN(_RNNBase):
         zmask = self._zoneout_mask(x)
         if fused:
             self._check_fused(x)
-            wanted = self._wanted(lengths, x.device)
+            wanted = self._wanted(lengths, x)
             y, h = _LayerNormIndRNNFunction.apply(self.training, self.zoneout, wanted, x.contiguous(), h0,
                                                   self.kernel.contiguous(), self.recurrent_scale.contiguous(),
                                                   self.bias.contiguous(), self.gamma.contiguous(), zmask)
@@ -688,7 +695,7 @@ class LayerNormLSTM(_RNNBase):
         zmask = self._zoneout_mask(x)
         if fused:
             self._check_fused(x)
-            wanted = self._wanted(lengths, x.device)
+            wanted = self._wanted(lengths, x)
             y, h, c = _LayerNormLSTMFunction.apply(self.training, self.zoneout, wanted, x.contiguous(), h0, c0,
                                                    self.kernel.contiguous(), R.contiguous(),
                                                    self.bias.contiguous(), self.gamma.contiguous(),
@@ -730,7 +737,7 @@ class LayerNormGRU(_RNNBase):
         zmask = self._zoneout_mask(x)
         if fused:
             self._check_fused(x)
-            wanted = self._wanted(lengths, x.device)
+            wanted = self._wanted(lengths, x)
             y, h = _LayerNormGRUFunction.apply(self.training, self.zoneout, wanted, x.contiguous(), h0,
                                                self.kernel.contiguous(), R.contiguous(),
                                                self.bias.contiguous(), self.recurrent_bias.contiguous(),

@@ -145,10 +145,10 @@ int haste_hip_transpose3_f32(int rows0, int cols0, const float* in0, float* out0
 /* Batches whose sequences have lengths of their own (reference frameworks/pytorch/base_rnn.py:54-61).
  * lengths: N 64-bit integers on the device, steps 0 (the initial state) .. T of a sequence
  * [T+1,N,H], counted from the end when negative.
- * gather_states: out0[n] = seq0[length of n][n], [N,H], and the same for seq1 unless it is NULL;
- * a length that names no step gives NaNs.
+ * gather_states: out0[n] = seq0[length of n][n], [N,H], and the same for seq1 unless it is NULL.
  * state_gradients: out[T,N,H] = grad (zeros when NULL; rows of H elements, the strides between
- * steps and batch rows in elements) + last[N,H] at each row's last step (none for length 0). */
+ * steps and batch rows in elements) + last[N,H] at each row's last step (none for length 0).
+ * A length that names no step gives NaNs for its row, in both. */
 int haste_hip_gather_states_f32(int T, int N, int H, const float* seq0, const float* seq1,
                                 const void* lengths, float* out0, float* out1, void* stream);
 int haste_hip_state_gradients_f32(int T, int N, int H, const float* grad, size_t step_stride,

@@ -375,3 +375,19 @@ def test_states_at_lengths_match_indexing(dtype, T, N, H):
             full[1:] = grad
         full[lengths, rows] = full[lengths, rows] + last
         assert torch.equal(ops.state_gradients(seqs[0], grad, last, lengths), full[1:])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64, torch.float16])
+def test_lengths_beyond_the_sequence_give_nans(dtype):
+    """Lengths that only the GPU knows: a row without such a step has NaNs for its state, and the gradients
+    that come through it are NaNs too."""
+    T, N, H = 4, 5, 70
+    lengths = torch.tensor([4, 5, -5, -6, 1], device="cuda")
+    layer = haste_amd.GRU(8, H).cuda().to(dtype)
+    x = torch.randn(T, N, 8, device="cuda").to(dtype).requires_grad_()
+    y, h = layer(x, lengths=lengths)
+    h.sum().backward()
+    wrong = torch.tensor([False, True, False, True, False], device="cuda")
+    assert torch.equal(h[0].isnan(), wrong[:, None].expand(N, H)) and not y.isnan().any()
+    assert torch.equal(x.grad.isnan(), wrong[None, :, None].expand(T, N, 8))
+    assert layer.kernel.grad.isnan().all()

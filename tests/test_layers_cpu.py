@@ -416,3 +416,13 @@ def test_lengths_of_any_shape_that_indexing_takes(fused_lstm_on_cpu, lengths):
         results.append([h, c] + [p.grad for p in net.parameters()])
     for got, want in zip(*results):
         assert got.shape == want.shape and torch.allclose(got, want, rtol=1e-12, atol=1e-12)
+
+
+@pytest.mark.parametrize("wrong", [6, -7])
+def test_lengths_beyond_the_sequence_are_refused(fused_lstm_on_cpu, wrong):
+    layer = fused_lstm_on_cpu(4, 6)
+    x = torch.randn(5, 3, 4)
+    for lengths in ([1, wrong, 2], torch.tensor([1, wrong, 2])):
+        with pytest.raises(IndexError, match="out of bounds for sequences of 5 steps"):
+            layer(x, lengths=lengths)
+    layer(x, lengths=[5, -6, 0])
