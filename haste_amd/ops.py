@@ -143,13 +143,21 @@ def _first_states(T, N, H, first, opts):
     return seqs
 
 
-def _upstream(grad, T):
+def _upstream(grad, T, like):
     """The address a backward entry point takes for the gradients of the states: it expects
     [T+1,N,H] and reads slots 1 .. T, so gradients [T,N,H] of the states after each step are handed
-    over as they are, with the address of the slot before them."""
-    if grad is None or grad.shape[0] == T + 1:
+    over as they are, with the address of the slot before them.  like: one state, [N,H]."""
+    if grad is None:
+        return None
+    if grad.dtype != like.dtype or grad.device != like.device:
+        raise ValueError("all tensors of a call must have the same dtype and device, got %s on %s and %s on %s"
+                         % (grad.dtype, grad.device, like.dtype, like.device))
+    if grad.numel() >= (T + 1) * like.numel():
         return grad
-    return grad.data_ptr() - grad[0].numel() * grad.element_size()
+    if grad.numel() != T * like.numel():
+        raise ValueError("gradients of the states must be [%d,%d,%d] or [%d,%d,%d], got %s"
+                         % (T + 1, *like.shape, T, *like.shape, list(grad.shape)))
+    return grad.data_ptr() - like.numel() * like.element_size()
 
 
 def _carried(opts, *pairs):
@@ -207,9 +215,20 @@ def transpose3(a, b, c):
     return tuple(outs)
 
 
+def _check_lengths(lengths, like):
+    """The kernels read like.shape[1] 64-bit integers at the address of `lengths`."""
+    if lengths.dtype != torch.int64 or lengths.device != like.device or not lengths.is_contiguous() \
+            or tuple(lengths.shape) != (like.shape[1],):
+        raise ValueError("lengths must be a contiguous int64 tensor [%d] on %s, got %s %s on %s"
+                         % (like.shape[1], like.device, lengths.dtype, list(lengths.shape), lengths.device))
+
+
 def gather_states(seqs, lengths):
     """The states [N,H] of one or two sequences [T+1,N,H] at the steps lengths[N] (int64)."""
     _check(*seqs)
+    _check_lengths(lengths, seqs[0])
+    if any(s.shape != seqs[0].shape or s.device != seqs[0].device for s in seqs[1:]) or len(seqs) > 2:
+        raise ValueError("one or two state sequences of one shape are gathered")
     T1, N, H = seqs[0].shape
     outs = [torch.empty(N, H, device=s.device, dtype=s.dtype) for s in seqs]
     second = seqs[1:] or (None,)
@@ -222,10 +241,15 @@ def state_gradients(like, grad, last, lengths):
     """Gradients [T,N,H] of the steps of a sequence `like` [T+1,N,H]: grad [T,N,H] (None: zeros) plus
     last [N,H] at the steps lengths[N] (int64; step 0, the initial state, gets none)."""
     T1, N, H = like.shape
+    _check_lengths(lengths, like)
+    if tuple(last.shape) != (N, H) or (grad is not None and tuple(grad.shape) != (T1 - 1, N, H)):
+        raise ValueError("gradients of %s states must be [%d,%d,%d] and [%d,%d]" % (list(like.shape), T1 - 1, N, H, N, H))
     if grad is not None and grad.stride(2) != 1:
         grad = grad.contiguous()
     last = last.contiguous()
     _check(last)
+    if grad is not None and grad.device != like.device:
+        raise ValueError("gradients must be on %s" % like.device)
     out = torch.empty(T1 - 1, N, H, device=like.device, dtype=like.dtype)
     step, row = (0, 0) if grad is None else grad.stride()[:2]
     _call("haste_hip_state_gradients", T1 - 1, N, H, grad, step, row, last, lengths.data_ptr(), out)
@@ -268,7 +292,7 @@ def lstm_backward(x_t, kernel_t, recurrent_kernel_t, bias, zoneout_mask, h, c, c
     dW, dR, db, dh, dc = _carried(opts, ((C, 4 * H), None), ((H, 4 * H), None), ((4 * H,), None),
                                   ((N, H), dh_last), ((N, H), dc_last))
     _call("haste_hip_lstm_backward", T, N, C, H, kernel_t, recurrent_kernel_t, bias, x_t,
-             h, c, _upstream(dh_new, T), _upstream(dc_new, T), dx, dW, dR, db, dh, dc, cache,
+             h, c, _upstream(dh_new, T, dh), _upstream(dc_new, T, dh), dx, dW, dR, db, dh, dc, cache,
              _mask_or_none(has_zoneout, zoneout_mask))
     return dx, dh, dc, dW, dR, db
 
@@ -375,7 +399,7 @@ def gru_backward(x_t, kernel_t, recurrent_kernel_t, bias, recurrent_bias, zoneou
     dp = torch.empty(T, N, 3 * H, **opts)
     dq = torch.empty(T, N, 3 * H, **opts)
     _call("haste_hip_gru_backward", T, N, C, H, kernel_t, recurrent_kernel_t, bias,
-             recurrent_bias, x_t, h, cache, _upstream(dh_new, T), dx, dW, dR, dbx, dbr, dh, dp, dq,
+             recurrent_bias, x_t, h, cache, _upstream(dh_new, T, dh), dx, dW, dR, dbx, dbr, dh, dp, dq,
              _mask_or_none(has_zoneout, zoneout_mask))
     return dx, dh, dW, dR, dbx, dbr
 
@@ -425,7 +449,7 @@ def indrnn_backward(x_t, kernel_t, recurrent_scale, bias, zoneout_mask, h, dh_ne
     dW, du, db, dh = _carried(opts, ((C, H), None), ((H,), None), ((H,), None), ((N, H), dh_last))
     workspace = torch.empty(T, N, H, **opts)
     _call("haste_hip_indrnn_backward", T, N, C, H, kernel_t, recurrent_scale, bias, x_t, h,
-             _upstream(dh_new, T), dx, dW, du, db, dh, workspace, _mask_or_none(has_zoneout, zoneout_mask))
+             _upstream(dh_new, T, dh), dx, dW, du, db, dh, workspace, _mask_or_none(has_zoneout, zoneout_mask))
     return dx, dh, dW, du, db
 
 
@@ -459,7 +483,7 @@ def layer_norm_indrnn_backward(x_t, kernel_t, recurrent_scale, bias, gamma, zone
     workspace = torch.empty(T, N, H, **opts)
     dgamma = torch.zeros_like(gamma)
     _call("haste_hip_layer_norm_indrnn_backward", T, N, C, H, kernel_t, recurrent_scale, bias,
-             x_t, h, _upstream(dh_new, T), dx, dW, du, db, dh, workspace, act_Wx, gamma[0], dgamma[0],
+             x_t, h, _upstream(dh_new, T, dh), dx, dW, du, db, dh, workspace, act_Wx, gamma[0], dgamma[0],
              _mask_or_none(has_zoneout, zoneout_mask))
     return dx, dh, dW, du, db, dgamma
 
@@ -505,7 +529,7 @@ def layer_norm_lstm_backward(x_t, kernel_t, recurrent_kernel_t, bias, gamma, gam
         opts, ((C, 4 * H), None), ((H, 4 * H), None), ((4 * H,), None), (tuple(gamma.shape), None),
         ((H,), None), ((H,), None), ((N, H), dh_last), ((N, H), dc_last))
     _call("haste_hip_layer_norm_lstm_backward", T, N, C, H, kernel_t, recurrent_kernel_t,
-             bias, x_t, h, c, _upstream(dh_new, T), _upstream(dc_new, T), dx, dW, dR, db, dh, dc,
+             bias, x_t, h, c, _upstream(dh_new, T, dh), _upstream(dc_new, T, dh), dx, dW, dR, db, dh, dc,
              act_Wx, gamma[0], dgamma[0], act_Wx_norm, act_Rh, gamma[1], dgamma[1],
              act_Rh_norm_cache, gamma_h, beta_h, dgamma_h, dbeta_h, act_c_norm_cache, act_c_norm,
              _mask_or_none(has_zoneout, zoneout_mask))
@@ -550,7 +574,7 @@ def layer_norm_gru_backward(x_t, kernel_t, recurrent_kernel_t, bias, recurrent_b
     dp = torch.empty(T, N, 3 * H, **opts)
     dq = torch.empty(T, N, 3 * H, **opts)
     _call("haste_hip_layer_norm_gru_backward", T, N, C, H, kernel_t, recurrent_kernel_t, bias,
-             recurrent_bias, x_t, h, cache, _upstream(dh_new, T), dx, dW, dR, dbx, dbr, dh, dp, dq,
+             recurrent_bias, x_t, h, cache, _upstream(dh_new, T, dh), dx, dW, dR, dbx, dbr, dh, dp, dq,
              act_Wx, gamma[0], dgamma[0], act_Rh, gamma[1], dgamma[1], act_Rh_norm_cache,
              _mask_or_none(has_zoneout, zoneout_mask))
     return dx, dh, dW, dR, dbx, dbr, dgamma

@@ -426,3 +426,26 @@ def test_lengths_beyond_the_sequence_are_refused(fused_lstm_on_cpu, wrong):
         with pytest.raises(IndexError, match="out of bounds for sequences of 5 steps"):
             layer(x, lengths=lengths)
     layer(x, lengths=[5, -6, 0])
+
+
+def test_addresses_of_gradients_and_lengths_are_checked():
+    """What reaches the entry points as a bare address is what they read there."""
+    from haste_amd import ops
+    T, N, H = 4, 3, 5
+    like = torch.zeros(N, H)
+    full = torch.zeros(T + 1, N, H)
+    assert ops._upstream(None, T, like) is None
+    assert ops._upstream(full, T, like) is full
+    flat = full.view((T + 1) * N, H)
+    assert ops._upstream(flat, T, like) is flat
+    steps = torch.zeros(T, N, H)
+    assert ops._upstream(steps, T, like) == steps.data_ptr() - 4 * N * H
+    for wrong in (steps.double(), steps[:, :2], torch.zeros(T - 1, N, H), steps.to("meta")):
+        with pytest.raises(ValueError):
+            ops._upstream(wrong, T, like)
+    lengths = torch.zeros(N, dtype=torch.int64)
+    ops._check_lengths(lengths, full)
+    for wrong in (lengths.int(), lengths.double(), lengths[:2], torch.zeros(2 * N, dtype=torch.int64)[::2],
+                  lengths.view(N, 1), lengths.to("meta")):
+        with pytest.raises(ValueError, match="lengths must be"):
+            ops._check_lengths(wrong, full)
