@@ -12,6 +12,8 @@ namespace haste_hip {
 namespace {
 
 constexpr int kStateThreads = 256;
+// A launch has fewer than 2^32 threads: more rows than this are looped over.
+constexpr int kMaxStateBlocks = 1 << 20;
 
 // Step of the sequence [T+1,...] a length means: counted from the end when negative, -1 when there
 // is no such step.
@@ -23,15 +25,16 @@ __device__ __forceinline__ long long step_of(long long length, int T) {
 template <typename V>
 struct StateJobs { const V* seq[2]; V* out[2]; };
 
-// blockIdx.x: batch row, blockIdx.y: sequence.
+// blockIdx.x: batch row (and those a grid further on), blockIdx.y: sequence.
 template <typename V>
 __global__ __launch_bounds__(kStateThreads)
 void gather_states_kernel(int T, int N, int H, StateJobs<V> jobs, const long long* __restrict__ lengths) {
-  const int n = blockIdx.x;
-  const long long s = step_of(lengths[n], T);
-  const V* from = jobs.seq[blockIdx.y] + ((size_t)(s < 0 ? 0 : s) * N + n) * H;
-  V* to = jobs.out[blockIdx.y] + (size_t)n * H;
-  for (int j = threadIdx.x; j < H; j += kStateThreads) to[j] = s < 0 ? V(__builtin_nanf("")) : from[j];
+  for (unsigned n = blockIdx.x; n < (unsigned)N; n += gridDim.x) {
+    const long long s = step_of(lengths[n], T);
+    const V* from = jobs.seq[blockIdx.y] + ((size_t)(s < 0 ? 0 : s) * N + n) * H;
+    V* to = jobs.out[blockIdx.y] + (size_t)n * H;
+    for (int j = threadIdx.x; j < H; j += kStateThreads) to[j] = s < 0 ? V(__builtin_nanf("")) : from[j];
+  }
 }
 
 // out[t][n] = grad[t][n] (0 without grad) + last[n] where t + 1 is the row's length; length 0 names
@@ -41,22 +44,26 @@ template <typename V>
 __global__ __launch_bounds__(kStateThreads)
 void state_gradients_kernel(int T, int N, int H, const V* __restrict__ grad, size_t step_stride, size_t row_stride,
                             const V* __restrict__ last, const long long* __restrict__ lengths, V* __restrict__ out) {
-  const int t = blockIdx.x / N, n = blockIdx.x % N;
-  const long long s = step_of(lengths[n], T);
-  const V* from = grad + t * step_stride + n * row_stride;
-  for (int j = threadIdx.x; j < H; j += kStateThreads) {
-    V v = grad != nullptr ? from[j] : V(0);
-    if (s == t + 1) v = v + last[(size_t)n * H + j];
-    if (s < 0) v = V(__builtin_nanf(""));
-    out[(size_t)blockIdx.x * H + j] = v;
+  for (unsigned row = blockIdx.x; row < (unsigned)T * (unsigned)N; row += gridDim.x) {
+    const int t = row / (unsigned)N, n = row % (unsigned)N;
+    const long long s = step_of(lengths[n], T);
+    const V* from = grad + t * step_stride + n * row_stride;
+    for (int j = threadIdx.x; j < H; j += kStateThreads) {
+      V v = grad != nullptr ? from[j] : V(0);
+      if (s == t + 1) v = v + last[(size_t)n * H + j];
+      if (s < 0) v = V(__builtin_nanf(""));
+      out[(size_t)row * H + j] = v;
+    }
   }
 }
+
+unsigned state_blocks(long long rows) { return (unsigned)(rows < kMaxStateBlocks ? rows : kMaxStateBlocks); }
 
 template <typename V>
 int gather_states(int T, int N, int H, const V* seq0, const V* seq1, const void* lengths, V* out0, V* out1, void* stream) {
   HASTE_HIP_REQUIRE(T > 0 && N > 0 && H > 0 && seq0 && out0 && lengths && (seq1 == nullptr) == (out1 == nullptr));
   const StateJobs<V> jobs = {{seq0, seq1}, {out0, out1}};
-  gather_states_kernel<V><<<dim3((unsigned)N, seq1 != nullptr ? 2u : 1u), dim3(kStateThreads), 0, as_stream(stream)>>>(
+  gather_states_kernel<V><<<dim3(state_blocks(N), seq1 != nullptr ? 2u : 1u), dim3(kStateThreads), 0, as_stream(stream)>>>(
       T, N, H, jobs, static_cast<const long long*>(lengths));
   HASTE_HIP_TRY(hipGetLastError());
   return HASTE_HIP_OK;
@@ -66,7 +73,7 @@ template <typename V>
 int state_gradients(int T, int N, int H, const V* grad, size_t step_stride, size_t row_stride, const V* last,
                     const void* lengths, V* out, void* stream) {
   HASTE_HIP_REQUIRE(T > 0 && N > 0 && H > 0 && last && lengths && out && (long long)T * N < (1ll << 31));
-  state_gradients_kernel<V><<<dim3((unsigned)(T * N)), dim3(kStateThreads), 0, as_stream(stream)>>>(
+  state_gradients_kernel<V><<<dim3(state_blocks((long long)T * N)), dim3(kStateThreads), 0, as_stream(stream)>>>(
       T, N, H, grad, step_stride, row_stride, last, static_cast<const long long*>(lengths), out);
   HASTE_HIP_TRY(hipGetLastError());
   return HASTE_HIP_OK;

@@ -391,3 +391,19 @@ def test_lengths_beyond_the_sequence_give_nans(dtype):
     assert torch.equal(h[0].isnan(), wrong[:, None].expand(N, H)) and not y.isnan().any()
     assert torch.equal(x.grad.isnan(), wrong[None, :, None].expand(T, N, 8))
     assert layer.kernel.grad.isnan().all()
+
+
+def test_states_at_lengths_of_more_rows_than_a_launch_has_blocks():
+    from haste_amd import ops
+    T, N, H = 2, (1 << 23) + 5, 1  # T * N beyond 2^24 blocks of 256 threads
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    seq = torch.randn(T + 1, N, H, device="cuda", generator=gen)
+    lengths = torch.randint(0, T + 1, (N,), device="cuda", generator=gen)
+    rows = torch.arange(N, device="cuda")
+    (got,) = ops.gather_states([seq], lengths)
+    assert torch.equal(got, seq[lengths, rows])
+    last = torch.randn(N, H, device="cuda", generator=gen)
+    want = torch.zeros_like(seq)
+    want[lengths, rows] = last
+    assert torch.equal(ops.state_gradients(seq, None, last, lengths), want[1:])
+    assert torch.equal(ops.state_gradients(seq, seq[1:], last, lengths), seq[1:] + want[1:])
