@@ -59,7 +59,8 @@ _entries = {}
 def entry(name):
     """Entry point `name` with the argument types its declaration in include/haste_hip.h has: the
     arguments of a call are then converted by ctypes itself (a wrapper object per argument, made in
-    Python, costs more than the rest of a short call).  None when the library has no such entry."""
+    Python, costs more than the rest of a short call; a package without the header does that).  None
+    when the library has no such entry."""
     fn = _entries.get(name)
     if fn is None:
         try:
@@ -67,17 +68,29 @@ def entry(name):
         except AttributeError:
             return None
         fn.restype = ctypes.c_int
-        fn.argtypes = [ctypes.c_void_p if "*" in p else _TYPES[p.split()[-2]] for p in _parameters()[name]]
+        parameters = _parameters().get(name)
+        if parameters is not None:
+            fn.argtypes = [ctypes.c_void_p if "*" in p else _TYPES[p.split()[-2]] for p in parameters]
         _entries[name] = fn
     return fn
 
 
 @functools.lru_cache(maxsize=None)
 def _parameters():
+    if not os.path.exists(HEADER_PATH):
+        return {}
     with open(HEADER_PATH) as f:
         text = re.sub(r"/\*.*?\*/", "", f.read(), flags=re.S)
     found = re.findall(r"\b(haste_hip_[a-z0-9_]+)\s*\(([^()]*)\)", text)
     return {name: [p.strip() for p in params.split(",")] for name, params in found}
+
+
+def _wrapped(a):
+    """An argument of an entry point whose declaration is not at hand.  Whole numbers go as 64 bits: the
+    callee reads as many of them as its parameter has, and addresses need all."""
+    if a is None or isinstance(a, float):
+        return ctypes.c_void_p(a) if a is None else ctypes.c_float(a)
+    return ctypes.c_longlong(a)
 
 
 def call(name, *args, stream=None):
@@ -87,6 +100,7 @@ def call(name, *args, stream=None):
         raise AttributeError("libhaste_hip.so has no entry point " + name)
     if stream is None:
         stream = torch.cuda.current_stream().cuda_stream
-    rc = fn(*[a.data_ptr() if isinstance(a, torch.Tensor) else a for a in args], stream)
+    args = [a.data_ptr() if isinstance(a, torch.Tensor) else a for a in args] + [stream]
+    rc = fn(*args) if fn.argtypes is not None else fn(*map(_wrapped, args))
     if rc != 0:
         raise HasteHipError(rc, name)

@@ -96,3 +96,43 @@ def test_cpp_headers_declare_the_reference_class_surface():
         assert re.search(r"namespace %s \{" % ns, text)
         assert "class ForwardPass" in text and "class BackwardPass" in text
         assert "void Run(" in text
+
+
+@pytest.fixture
+def no_header(lib, monkeypatch, tmp_path):
+    monkeypatch.setattr(hlib, "HEADER_PATH", str(tmp_path / "haste_hip.h"))
+    monkeypatch.setattr(hlib, "_entries", {})
+    hlib._parameters.cache_clear()
+    yield
+    hlib._parameters.cache_clear()
+
+
+def test_calls_without_the_header(no_header):
+    """A package whose C header was left out: bad arguments come back as the library's error."""
+    with pytest.raises(hlib.HasteHipError) as e:
+        hlib.call("haste_hip_lstm_forward_f32", True, 3, 2, 2, 2, *([None] * 8), 0.0, None, stream=0)
+    assert e.value.code == 1
+    with pytest.raises(AttributeError):
+        hlib.call("haste_hip_no_such_entry", 1, stream=0)
+
+
+@pytest.mark.gpu
+def test_passes_without_the_header(no_header):
+    """Whole numbers, strides, addresses and floats arrive as they are."""
+    import torch
+    import haste_amd
+    torch.manual_seed(0)
+    results = []
+    layer = haste_amd.LSTM(8, 24, zoneout=0.25).cuda().eval()
+    x = torch.randn(5, 3, 8, device="cuda", requires_grad=True)
+    train = haste_amd.LSTM(8, 24).cuda()
+    for path in (hlib.HEADER_PATH, os.path.join(ROOT, "include", "haste_hip.h")):
+        hlib.HEADER_PATH = path
+        hlib._entries.clear()
+        hlib._parameters.cache_clear()
+        y, (h, c) = layer(x.detach())
+        y2, (h2, _) = train(x, lengths=[5, 1, 3])
+        grads = torch.autograd.grad([y2, h2], [x, *train.parameters()], [torch.ones_like(y2), torch.ones_like(h2)])
+        assert (hlib.entry("haste_hip_lstm_forward_f32").argtypes is None) == (not os.path.exists(path))
+        results.append([y, h, c, *grads])
+    assert all(torch.equal(a, b) for a, b in zip(*results))
