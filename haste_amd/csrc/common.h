@@ -135,6 +135,10 @@ int xcd_layout_ready(hipStream_t stream);
 // kernel just enqueued on `stream` as the one to wait for.
 int order_persistent_launches(hipStream_t stream, bool before);
 
+// Whether a persistent launch has been recorded into a graph on the current device: its replays are
+// ordered with nothing, so that another persistent launch beside one could starve both.
+bool persistent_launch_recorded();
+
 // Holds the process-wide order of persistent launches from before the wait for the previous
 // launch until this launch has been recorded as the last one: two host threads that launch
 // on different streams would otherwise both wait for the launch before theirs and then run

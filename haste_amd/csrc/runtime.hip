@@ -79,6 +79,7 @@ struct LastPersistent {
   hipEvent_t event = nullptr;
   hipStream_t stream = nullptr;
   bool valid = false;
+  bool recorded = false;  // a graph with persistent kernels exists, or has existed
 };
 std::map<int, LastPersistent> g_last_persistent;
 }  // namespace
@@ -100,7 +101,10 @@ int order_persistent_launches(hipStream_t stream, bool before) {
   // persistent kernels replays, the caller keeps other persistent launches off the device.)
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &capture) != hipSuccess) (void)hipGetLastError();
-  if (capture != hipStreamCaptureStatusNone) return HASTE_HIP_OK;
+  if (capture != hipStreamCaptureStatusNone) {
+    lp.recorded = true;
+    return HASTE_HIP_OK;
+  }
   if (before) {
     if (lp.valid && lp.stream != stream) HASTE_HIP_TRY(hipStreamWaitEvent(stream, lp.event, 0));
     return HASTE_HIP_OK;
@@ -110,6 +114,14 @@ int order_persistent_launches(hipStream_t stream, bool before) {
   lp.stream = stream;
   lp.valid = true;
   return HASTE_HIP_OK;
+}
+
+bool persistent_launch_recorded() {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return false;
+  std::lock_guard<std::mutex> lock(g_mutex);
+  auto it = g_last_persistent.find(dev);
+  return it != g_last_persistent.end() && it->second.recorded;
 }
 
 namespace {

@@ -298,7 +298,9 @@ int open_scratch(hipStream_t stream, size_t own_bytes, size_t gemm_bytes, Scratc
 // call runs step by step: always for float (its persistent kernels are the callers of this file),
 // and for double when the shape does not fit the chip, while the stream is being captured (a
 // persistent launch needs a control block that replays wipe, and these calls never had one in
-// their graphs), and in memory lent by the caller that is too small for the tiles.  An error of the
+// their graphs), once a persistent launch of another cell has been recorded into a graph on the device
+// (these calls may run beside its replays, which persistent launches must not), and in memory lent by
+// the caller that is too small for the tiles.  An error of the
 // workspace is the call's: get_workspace() is also what reports, once, that an earlier launch timed out.
 // The callers ask for the tiles on top of what the steps take: a call made ahead of a capture then leaves
 // the captured one, which runs step by step, a buffer that need not grow.
@@ -315,7 +317,7 @@ int one_launch_bytes<double>(hipStream_t stream, int in_gates, int out_gates, in
   if (tiles == 0) return HASTE_HIP_OK;
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &capture) != hipSuccess) (void)hipGetLastError();
-  if (capture != hipStreamCaptureStatusNone) return HASTE_HIP_OK;
+  if (capture != hipStreamCaptureStatusNone || persistent_launch_recorded()) return HASTE_HIP_OK;
   Workspace ws;
   HASTE_HIP_PROPAGATE(get_workspace(stream, 0, &ws));
   if (!ws.caller_owned || ws.scratch_bytes >= others + tiles + 256) *bytes = tiles;

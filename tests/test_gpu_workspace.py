@@ -208,13 +208,53 @@ def child_timeout_double():
     print("timeout reported", flush=True)
 
 
-def _run_child(name):
-    env = dict(os.environ, HASTE_HIP_TEST_HOOKS="1", HASTE_HIP_SPIN_LIMIT="512", HASTE_HIP_TEST_ABSENT_WORKGROUP="1",
-               PYTHONPATH=os.pathsep.join([ROOT, os.path.join(ROOT, "tests")]))
+def child_double_beside_graphs():
+    """Once a graph holds a persistent launch, double passes must not be one: its replays wait for nobody."""
+    sys.path.insert(0, ROOT)
+    import ctypes
+    from haste_amd import lib, ops
+    dev = torch.device("cuda:0")
+    a = _inputs(4, 4, 32, 64, dev)
+    d = {k: v.double() for k, v in a.items()}
+    handle = lib.load()
+    handle.haste_hip_profile_enable(1)
+
+    def launches():
+        h, _, _ = ops.lstm_forward(True, 0.0, d["x"], d["h0"], d["h0"], d["W"], d["R"], d["b"], d["mask"])
+        torch.cuda.synchronize()
+        counts = []
+        for name in (b"lstm_forward_recurrence64", b"lstm_forward_steps"):
+            ms, n = ctypes.c_double(0.0), ctypes.c_int(0)
+            assert handle.haste_hip_profile_read(name, ctypes.byref(ms), ctypes.byref(n)) == 0
+            counts.append(n.value)
+        handle.haste_hip_profile_reset()
+        return h, counts
+
+    before, counts = launches()
+    assert counts == [1, 0], counts
+    handle.haste_hip_profile_enable(0)  # its events are not for a capture
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        ops.lstm_forward(True, 0.0, a["x"], a["h0"], a["h0"], a["W"], a["R"], a["b"], a["mask"])
+        stream.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            ops.lstm_forward(True, 0.0, a["x"], a["h0"], a["h0"], a["W"], a["R"], a["b"], a["mask"])
+    handle.haste_hip_profile_enable(1)
+    after, counts = launches()
+    assert counts == [0, 1], counts
+    assert torch.allclose(before, after, rtol=1e-13, atol=1e-14)
+    print("ends as expected", flush=True)
+
+
+def _run_child(name, says="timeout reported"):
+    env = dict(os.environ, PYTHONPATH=os.pathsep.join([ROOT, os.path.join(ROOT, "tests")]))
+    if name.startswith("timeout"):
+        env.update(HASTE_HIP_TEST_HOOKS="1", HASTE_HIP_SPIN_LIMIT="512", HASTE_HIP_TEST_ABSENT_WORKGROUP="1")
     res = subprocess.run([sys.executable, os.path.abspath(__file__), name], env=env,
                          capture_output=True, text=True, timeout=110)
     assert res.returncode == 0, res.stdout + res.stderr
-    assert "timeout reported" in res.stdout
+    assert says in res.stdout
 
 
 def test_a_wait_that_runs_out_is_reported_by_stream_status():
@@ -225,8 +265,14 @@ def test_a_wait_that_runs_out_is_reported_by_the_next_double_call():
     _run_child("timeout_double")
 
 
+def test_double_passes_run_step_by_step_where_graphs_hold_persistent_launches():
+    _run_child("double_beside_graphs", "ends as expected")
+
+
 if __name__ == "__main__":
     if sys.argv[1:] == ["timeout"]:
         child_timeout()
     if sys.argv[1:] == ["timeout_double"]:
         child_timeout_double()
+    if sys.argv[1:] == ["double_beside_graphs"]:
+        child_double_beside_graphs()
