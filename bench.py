@@ -18,6 +18,10 @@ import numpy as np
 
 PEAK_FP32_MFMA_TFLOPS = 157.3
 PEAK_FP64_MFMA_TFLOPS = 78.6
+PEAK_HALF_MFMA_TFLOPS = 2500.0  # bf16 and f16, dense
+# The fp32 GEMM runs on the bf16 matrix cores, six bf16 products to one fp32 product; the fp32
+# recurrences run on the fp32 matrix instruction.
+PEAK_SPLIT_TFLOPS = PEAK_HALF_MFMA_TFLOPS / 6.0
 PEAK_HBM_GBS = 8000.0
 
 # HBM bytes per launch at the metric workload, from two rocprofv3 --pmc runs (FETCH_SIZE, then
@@ -26,11 +30,17 @@ PEAK_HBM_GBS = 8000.0
 # of the step's three products (dx; dW and dR, which share a launch that counts as two), each with
 # its split reduce; the forward recurrence includes the input projection it computes itself.
 TRAFFIC_SOURCE = "profiles/lstm_fwd_bwd_N64_T100_H512_hbm_traffic_pmc.txt (a constant from that profile, not measured in this run)"
-MEASURED_TRAFFIC_BYTES = {"gemm_f32": 143.2e6, "lstm_forward_recurrence": 161.3e6,
+MEASURED_TRAFFIC_BYTES = {"gemm_f32": 111.7e6, "lstm_forward_recurrence": 161.3e6,
                           "lstm_backward_recurrence": 196.1e6,
                           # at N=1 C=512 H=4096 (--workload stepwise): 131558.5 FETCH_SIZE units
                           # + 192 WRITE_SIZE units per launch of the streaming kernel
                           "gemm_f32_skinny": 269.6e6}
+
+
+def mixed_peak(*parts):
+    """The rate at which work that several units share is bound by them one after the other; parts of
+    (flops, that unit's TFLOP/s)."""
+    return sum(f for f, _ in parts) / sum(f / peak for f, peak in parts)
 
 
 def parse():
@@ -155,41 +165,44 @@ def run_metric(args, torch, lib, ops, dev):
     # three GEMM products instead of four and the forward kernel does the flops of two.
     fused_input = round(gemm_count / args.steps) == 3
     kernels = {}
-    for name, flops in (("gemm_f32", f_gemm),
-                        ("lstm_forward_recurrence", f_rec + (f_gemm if fused_input else 0.0)),
-                        ("lstm_backward_recurrence", f_rec)):
+    f_forward = f_rec + (f_gemm if fused_input else 0.0)
+    for name, flops, peak in (("gemm_f32", f_gemm, PEAK_SPLIT_TFLOPS),
+                              ("lstm_forward_recurrence", f_forward, PEAK_FP32_MFMA_TFLOPS),
+                              ("lstm_backward_recurrence", f_rec, PEAK_FP32_MFMA_TFLOPS)):
         total_ms, count = profile_read(lib, name)
         avg_ms = total_ms / max(count, 1)
         tf = flops / (avg_ms * 1e-3) / 1e12 if avg_ms > 0 else 0.0
         kernels[name] = {"launches_per_step": count / args.steps, "avg_ms": round(avg_ms, 5),
                          "ms_per_step": round(total_ms / args.steps, 5),
                          "flops_per_launch": flops, "tflops": round(tf, 3),
-                         "frac_of_fp32_mfma_peak": round(tf / PEAK_FP32_MFMA_TFLOPS, 4)}
+                         "peak_tflops": round(peak, 1), "frac_of_mfma_peak": round(tf / peak, 4)}
     if fused_input:
         kernels["lstm_forward_recurrence"]["computes_input_projection"] = True
     lib.haste_hip_profile_reset()
     # The roofline entry is the kernel with the longest single launch (a recurrence), with the
     # whole step beside it: all six products of the step, 2*T*N*4H*(3C + 3H) flops, over the
-    # step's wall time.
+    # step's wall time, against what the units that they run on deliver together.
     total_flops = 3.0 * (f_gemm + f_rec)
+    step_peak = mixed_peak((f_forward + f_rec, PEAK_FP32_MFMA_TFLOPS),
+                           (total_flops - f_forward - f_rec, PEAK_SPLIT_TFLOPS))
     tflops_whole = total_flops / (ms_per_step * 1e-3) / 1e12
     dominant = max(kernels, key=lambda k: kernels[k]["avg_ms"])
     dom = kernels[dominant]
     roofline = {"kernel": dominant, "bound": "mfma", "achieved": dom["tflops"],
-                "peak": PEAK_FP32_MFMA_TFLOPS, "unit": "TFLOP/s",
-                "frac": round(dom["tflops"] / PEAK_FP32_MFMA_TFLOPS, 4),
+                "peak": dom["peak_tflops"], "unit": "TFLOP/s",
+                "frac": dom["frac_of_mfma_peak"],
                 "traffic": MEASURED_TRAFFIC_BYTES.get(dominant),
                 "traffic_source": TRAFFIC_SOURCE,
                 "us_per_launch": round(dom["avg_ms"] * 1e3, 2),
                 "whole_step_tflops": round(tflops_whole, 3),
-                "whole_step_frac": round(tflops_whole / PEAK_FP32_MFMA_TFLOPS, 4)}
+                "whole_step_peak": round(step_peak, 1), "whole_step_frac": round(tflops_whole / step_peak, 4)}
     return dict(ms_per_step=ms_per_step, ms_per_ops_step=ms_per_ops_step, kernels=kernels, roofline=roofline,
                 tflops_whole_step=tflops_whole, host=(W, R, b, x, dy))
 
 
-def run_measured_peak(args, torch, lib, ops, dev):
-    """What the fp32 matrix cores deliver on this box on a long, square product (the library's
-    own GEMM at 8192^3), beside the nominal 157.3 TFLOP/s the fractions are quoted against."""
+def run_gemm_rate(args, torch, lib, ops, dev):
+    """What the library's fp32 GEMM delivers on this box on a long, square product (8192^3), beside the
+    nominal rate of six bf16 products for each fp32 one."""
     n = 8192
     a = torch.randn(n, n, device=dev)
     b = torch.randn(n, n, device=dev)
@@ -206,7 +219,7 @@ def run_measured_peak(args, torch, lib, ops, dev):
     torch.cuda.synchronize()
     tf = 2.0 * n ** 3 / (e0.elapsed_time(e1) / reps * 1e-3) / 1e12
     return {"workload": "gemm_f32 8192 x 8192 x 8192", "tflops": round(tf, 2),
-            "frac_of_nominal": round(tf / PEAK_FP32_MFMA_TFLOPS, 4)}
+            "peak_tflops": round(PEAK_SPLIT_TFLOPS, 1), "frac_of_mfma_peak": round(tf / PEAK_SPLIT_TFLOPS, 4)}
 
 
 def run_iterate(args, torch, lib, ops, dev):
@@ -475,19 +488,26 @@ def run_hbm_kernels(args, torch, lib, ops, dev):
 
 
 def run_configs(args, torch, lib, ops, dev):
-    """The other BASELINE.json configurations (parity-test cases; timed here for the record):
+    """The other configurations (parity-test cases; timed here for the record):
     forward (+ backward with the caller-side transposes) in ms per call, with the algorithmic
     flops of the matrix products (2*T*N*G*H*(C + H) forward, three times that forward +
-    backward) and the fraction of the matrix cores' peak for the arithmetic type.  Also the
+    backward) and the fraction of the matrix cores' peak: fp32 passes that of the fp32 instruction for
+    the recurrences' products and of the split bf16 ones for the others.  Also the
     other instantiations of the reference at the metric shape: the double LSTM (all steps of
-    a recurrence in one launch, products on the fp64 matrix cores) and the half GRU (fp32 recurrences on widened
+    a recurrence in one launch, products on the fp64 matrix cores) and the half GRU (recurrences on widened
     tensors, products on the half matrix cores)."""
     details = {}
 
-    def note(key, ms, flops, peak=PEAK_FP32_MFMA_TFLOPS, dtype="f32"):
+    def note(key, ms, gates, training, rows=None, peak=None, dtype="f32"):
+        per_feature = 2.0 * T * (rows or N) * gates * H
+        in_recurrence = per_feature * H * (2 if training else 1)  # h*R, and dv*R^T
+        around = per_feature * (3 * C + H if training else C)     # x*W, dx, dW, dR
+        flops = in_recurrence + around
+        if peak is None:
+            peak = mixed_peak((in_recurrence, PEAK_FP32_MFMA_TFLOPS), (around, PEAK_SPLIT_TFLOPS))
         tf = flops / (ms * 1e-3) / 1e12
         details[key] = {"ms": ms, "flops": flops, "tflops": round(tf, 3), "dtype": dtype,
-                        "peak_tflops": peak, "frac_of_mfma_peak": round(tf / peak, 4)}
+                        "peak_tflops": round(peak, 1), "frac_of_mfma_peak": round(tf / peak, 4)}
 
     def timed(fn, reps):
         # untimed calls first: the allocator's pools, the library's scratch buffer and the clocks
@@ -519,8 +539,7 @@ def run_configs(args, torch, lib, ops, dev):
     z = torch.zeros(N, H, device=dev)
     out["lstm_inference_N16_T100_C128_H256_ms"] = timed(
         lambda: ops.lstm_forward(False, 0.0, x, z, z, W, R, b, no_mask), 50)
-    note("lstm_inference_N16_T100_C128_H256", out["lstm_inference_N16_T100_C128_H256_ms"],
-         2.0 * T * N * 4 * H * (C + H))
+    note("lstm_inference_N16_T100_C128_H256", out["lstm_inference_N16_T100_C128_H256_ms"], 4, False)
 
     T, N, C, H = 100, 64, 512, 512  # config 2: GRU training, zoneout 0.1, DropConnect 0.05
     k = H ** -0.5
@@ -536,7 +555,7 @@ def run_configs(args, torch, lib, ops, dev):
         return ops.gru_backward(ops.transpose(x), ops.transpose(W), Reff_t, bx, br, zm, h, cache, dh_new)
     out["gru_fwd_bwd_N64_T100_H512_zoneout_dropconnect_ms"] = timed(gru_step, 30)
     note("gru_fwd_bwd_N64_T100_H512_zoneout_dropconnect", out["gru_fwd_bwd_N64_T100_H512_zoneout_dropconnect_ms"],
-         3 * 2.0 * T * N * 3 * H * (C + H))
+         3, True)
 
     # the half GRU of the reference (lib/gru_forward_gpu.cu.cc:373) at the same shape
     xh, Wh, Rh, bxh, brh, zh, zmh, dhh = (a.half() for a in (x, W, R, bx, br, z, zm, dh_new))
@@ -546,10 +565,10 @@ def run_configs(args, torch, lib, ops, dev):
         return ops.gru_backward(ops.transpose(xh), ops.transpose(Wh), ops.transpose(Rh), bxh, brh, zmh, h, cache, dhh)
     ms = timed(gru_half_step, 20)
     out["gru_f16_fwd_bwd_N64_T100_H512_zoneout_ms"] = ms
-    # half tensors; the recurrences (half of the flops) run in fp32 on widened copies, the
-    # products around them on the half matrix cores: quoted against the fp32 peak, like the rest
-    note("gru_f16_fwd_bwd_N64_T100_H512_zoneout", ms, 3 * 2.0 * T * N * 3 * H * (C + H), PEAK_FP32_MFMA_TFLOPS,
-         "f16 tensors, f32 recurrences, f16 products with f32 accumulation")
+    # half tensors, every product on the half matrix cores (at this shape the recurrences' too), the
+    # state and the pointwise math in fp32
+    note("gru_f16_fwd_bwd_N64_T100_H512_zoneout", ms, 3, True, peak=PEAK_HALF_MFMA_TFLOPS,
+         dtype="f16 tensors and products with f32 accumulation, f32 state")
 
     T, N, C, H = 100, 128, 512, 512  # config 3: LSTM training, N=128
     x, W, R = rnd(T, N, C), uni(k, C, 4 * H), uni(k, H, 4 * H)
@@ -563,7 +582,7 @@ def run_configs(args, torch, lib, ops, dev):
         return ops.lstm_backward(*ops.transpose3(x, W, R), b, no_mask, h, c,
                                  cache, dh_new, dc_new)
     out["lstm_fwd_bwd_N128_T100_H512_ms"] = timed(lstm_step, 30)
-    note("lstm_fwd_bwd_N128_T100_H512", out["lstm_fwd_bwd_N128_T100_H512_ms"], 3 * 2.0 * T * N * 4 * H * (C + H))
+    note("lstm_fwd_bwd_N128_T100_H512", out["lstm_fwd_bwd_N128_T100_H512_ms"], 4, True)
 
     # the double LSTM of the reference (lib/lstm_forward_gpu.cu.cc:368-369) at the metric shape
     Nd = 64
@@ -576,7 +595,7 @@ def run_configs(args, torch, lib, ops, dev):
         return ops.lstm_backward(*ops.transpose3(xd_, Wd_, Rd_), bd_, no_mask64, h, c, cache, dhd_, dcd_)
     ms = timed(lstm_double_step, 10)
     out["lstm_f64_fwd_bwd_N64_T100_H512_ms"] = ms
-    note("lstm_f64_fwd_bwd_N64_T100_H512", ms, 3 * 2.0 * T * Nd * 4 * H * (C + H), PEAK_FP64_MFMA_TFLOPS, "f64")
+    note("lstm_f64_fwd_bwd_N64_T100_H512", ms, 4, True, rows=Nd, peak=PEAK_FP64_MFMA_TFLOPS, dtype="f64")
 
     T, N, C, H = 500, 32, 256, 256  # config 4: LayerNormLSTM training, zoneout 0.1
     k = H ** -0.5
@@ -594,7 +613,7 @@ def run_configs(args, torch, lib, ops, dev):
                                             gamma_h, beta_h, zm, *fwd, dh_new, dc_new)
     out["layer_norm_lstm_fwd_bwd_N32_T500_H256_zoneout_ms"] = timed(ln_lstm_step, 10)
     note("layer_norm_lstm_fwd_bwd_N32_T500_H256_zoneout", out["layer_norm_lstm_fwd_bwd_N32_T500_H256_zoneout_ms"],
-         3 * 2.0 * T * N * 4 * H * (C + H))
+         4, True)
     return out, details
 
 
@@ -641,7 +660,7 @@ def main():
         print(json.dumps(run_stepwise(args, torch, lib, ops, dev)))
         return
     if args.workload == "peak":
-        print(json.dumps(run_measured_peak(args, torch, lib, ops, dev)))
+        print(json.dumps(run_gemm_rate(args, torch, lib, ops, dev)))
         return
     if args.workload == "iterate":
         print(json.dumps(run_iterate(args, torch, lib, ops, dev)))
@@ -655,10 +674,8 @@ def main():
     stepwise = run_stepwise(args, torch, lib, ops, dev)
     hbm_kernels = run_hbm_kernels(args, torch, lib, ops, dev)
     configs, config_details = run_configs(args, torch, lib, ops, dev)
-    measured_peak = run_measured_peak(args, torch, lib, ops, dev)
+    gemm_rate = run_gemm_rate(args, torch, lib, ops, dev)
     iterate = run_iterate(args, torch, lib, ops, dev)
-    m["roofline"]["measured_peak"] = measured_peak["tflops"]
-    m["roofline"]["frac_of_measured_peak"] = round(m["roofline"]["achieved"] / measured_peak["tflops"], 4)
 
     # CPU baseline: torch.nn.LSTM fwd+bwd on the host cores (bounded sample).
     cpu = None
@@ -702,7 +719,7 @@ def main():
         "hbm_kernels": hbm_kernels,
         "other_configs_ms": configs,
         "other_configs": config_details,
-        "measured_fp32_mfma_peak": measured_peak,
+        "gemm_rate": gemm_rate,
         "iterate_n1": iterate,
         "cpu_baseline": cpu,
     }
