@@ -24,11 +24,13 @@
 // whose rows run along the output (B, and A stored transposed) are read 8 k deep per thread,
 // so that putting 8 k side by side is a choice of registers.  Two workgroups share a CU and one
 // splits while the other multiplies; the multiplying one has the higher wave priority (3-8 %).
-// What bounds it: the bf16 matrix cores, at the clock the chip's power allows (a bare loop of
-// these MFMAs on random data reaches 1700 TFLOP/s = 283 of fp32 product, 1430 with the splitting's
-// share of vector instructions beside them).  Measured, fp32 instruction before -> now:
-// 8192^3 140 -> 199 TFLOP/s; 6400 x 2048 x 512 110 -> 148; 6400 x 512 x 2048 113 -> 153;
-// 512 x 2048 x 6400 119 -> 170 (with the kernel that adds the K pieces).
+// What bounds it: the SIMDs' instructions.  At 8192^3 the bf16 matrix cores execute for 66 % of the time and the
+// other vector instructions, nearly all of them the splitting's 6.5 per element, take 38 % of a SIMD's cycles; the two
+// hardly overlap (counters).  A bare loop of these MFMAs on random data reaches 1700 TFLOP/s = 283 of fp32 product,
+// 1430 with the splitting's share of vector instructions beside them.  Measured, fp32 instruction before -> now:
+// 8192^3 140 -> 193 TFLOP/s; 6400 x 2048 x 512 110 -> 155; 6400 x 512 x 2048 113 -> 153;
+// 512 x 2048 x 6400 119 -> 166 (with the kernel that adds the K pieces).  Before operands were scaled (see kSplitScale)
+// 8192^3 ran at 199; against that:
 // One accumulator instead of two leaves registers for three workgroups per CU: 213 TFLOP/s at
 // 8192^3 and 0-5 % on the other shapes, with 2.5 times the error.  256x128 tiles (8 wavefronts, two LDS
 // stages) 195; 16x16x32 instructions 197 with one accumulator.
@@ -291,6 +293,7 @@ __device__ __forceinline__ float bf16_high(unsigned int u) { return __uint_as_fl
 // bfloat16 holds nothing below 2^-133, a float goes down to 2^-149: unscaled, operands below 2^-110 would
 // lose their last part and those below 2^-134 all three.  Scaled, every part of every float is a normal
 // bfloat16; in exchange operands from 2^104 and results from 2^80 on are infinite, which split_tile() sees.
+// It is one vector instruction more per element: 8192^3 5.42 -> 5.55 ms, 6400 x 512 x 2048 85.6 -> 87.5 us.
 constexpr float kSplitScale = 0x1p24f, kProductScale = 0x1p-48f;
 
 // Eight consecutive k of one row, scaled, split into three bf16 each and stored into the three planes.

@@ -408,8 +408,10 @@ int haste_hip_layer_norm_indrnn_backward_f32(int steps, int batch_size, int inpu
  * what haste::v0::<cell>::ForwardPass<double>::Run / BackwardPass<double>::Run (and Iterate)
  * bind to: same arguments, shapes and semantics as the *_f32 entry points above, tensors in
  * double; zoneout_prob and dropconnect_scale stay float as in the reference's signatures.
- * Every step is a GEMM on the fp64 matrix cores plus row-wise / pointwise kernels, for any
- * hidden size. */
+ * The LSTM and the GRU run all steps of a recurrence in one launch on the fp64 matrix cores where the
+ * weights fit the chip, from four steps on; otherwise (also while the stream is being captured and once
+ * a persistent launch has been recorded into a graph on the device), and in the other cells, every step
+ * is a GEMM plus row-wise / pointwise kernels, for any hidden size. */
 int haste_hip_gemm_f64(int trans_a, int M, int N, int K,
                        const double* A, int lda, const double* B, int ldb,
                        double* C, int ldc, int accumulate, void* stream);
