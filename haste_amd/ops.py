@@ -170,7 +170,9 @@ def _carried(opts, *pairs):
             raise ValueError("gradient of the last state must be %s, %s on %s, got %s, %s on %s"
                              % (list(shape), opts["dtype"], opts["device"], list(start.shape), start.dtype, start.device))
     out = _zeros(opts, *[shape for shape, start in pairs if start is None])
-    return [out.pop(0) if start is None else start.clone(memory_format=torch.contiguous_format)
+    # detached: the kernels write into the copies, which a pass that is itself differentiated
+    # (create_graph) would otherwise take for copies still
+    return [out.pop(0) if start is None else start.detach().clone(memory_format=torch.contiguous_format)
             for _, start in pairs]
 
 

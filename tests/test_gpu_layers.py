@@ -407,3 +407,16 @@ def test_states_at_lengths_of_more_rows_than_a_launch_has_blocks():
     want[lengths, rows] = last
     assert torch.equal(ops.state_gradients(seq, None, last, lengths), want[1:])
     assert torch.equal(ops.state_gradients(seq, seq[1:], last, lengths), seq[1:] + want[1:])
+
+
+def test_gradients_of_a_pass_are_not_differentiated_again():
+    """The backward passes are kernels: what they return is a constant to create_graph, all of it."""
+    layer = haste_amd.LSTM(4, 8).cuda()
+    h0, c0 = (torch.randn(1, 2, 8, device="cuda", requires_grad=True) for _ in range(2))
+    x = torch.randn(3, 2, 4, device="cuda", requires_grad=True)
+    _, (h, c) = layer(x, (h0, c0))
+    grads = torch.autograd.grad(h.square().sum() + c.square().sum(), [x, *layer.parameters()], create_graph=True)
+    assert not any(g.requires_grad for g in grads)
+    _, (h, c) = layer(x, (h0, c0))
+    grads = torch.autograd.grad(h.square().sum() + c.square().sum(), [h0, c0], create_graph=True)
+    assert not any(g.requires_grad for g in grads)
