@@ -1,4 +1,4 @@
-"""fp32 MFMA GEMM vs fp64 NumPy matmul, through the C-ABI (haste_hip_gemm_f32)."""
+"""fp32 GEMM vs fp64 NumPy matmul, through the C-ABI (haste_hip_gemm_f32)."""
 import numpy as np
 import pytest
 
@@ -15,13 +15,12 @@ SHAPES = [
     (True, 512, 2048, 6400),    # dR: split along K, A = h^T
     (False, 6400, 512, 2048),   # dx
     (False, 96, 96, 5000),      # split-K with ragged tiles
-    # M <= 64 with a long enough K: the kernel that streams B into the MFMA operands
+    # a step's products: up to 32 rows in the kernel that streams B into the MFMA operands, more in K pieces
     (False, 64, 1024, 4096), (False, 47, 6144, 1536), (False, 33, 772, 3000), (False, 128, 1024, 4096),
     (False, 100, 768, 3072),
     (False, 1, 2048, 512), (False, 16, 6144, 1536), (False, 5, 1300, 5200), (False, 32, 768, 3072),
     (False, 17, 4100, 332), (False, 3, 64, 1024), (False, 32, 16384, 1000),
-    # whole tiles beside edge tiles, K pieces that are and are not multiples of 16: the unmasked
-    # and the masked loop in one launch
+    # whole tiles beside edge tiles, K pieces whose last stage is and is not whole
     (False, 300, 260, 250), (True, 384, 1000, 1600), (False, 640, 192, 2048), (True, 800, 512, 1000),
     (False, 1024, 1024, 17),
 ]
