@@ -1,6 +1,6 @@
 """Benchmark of the hot path on one MI355X.
 
-Metric (BASELINE.json): LSTM forward + backward, ms per batch, at N=64, T=100,
+Metric: LSTM forward + backward, ms per batch, at N=64, T=100,
 C=H=512, fp32; plus microseconds per timestep of streaming inference at N=1, T=2000.
 
 One step = ForwardPass::Run (training) + the caller-side transposes of x, W, R +
@@ -379,7 +379,7 @@ def run_stepwise(args, torch, lib, ops, dev):
 
 def run_hbm_kernels(args, torch, lib, ops, dev):
     """The HBM-bound kernels of the path against the 8 TB/s roof: stand-alone layer norm
-    (rows = T*N of BASELINE configuration 4, D = 4H), IndRNN recurrences and the transpose
+    (rows = T*N of the layer-norm configuration, D = 4H), IndRNN recurrences and the transpose
     helper.  Algorithmic bytes: each distinct tensor element read or written once."""
     out = {}
 
