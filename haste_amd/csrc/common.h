@@ -77,6 +77,10 @@ struct Workspace {
 // it is too small.
 int get_workspace(hipStream_t stream, size_t scratch_bytes, Workspace* out);
 
+// Whether the stream's workspace holds `bytes` of scratch or can be made to: not where the caller lent
+// less, nor where it would have to grow while the stream is captured.
+int workspace_has_room(hipStream_t stream, size_t bytes, bool* room);
+
 // While one of these is alive on a host thread, get_workspace() on that thread hands out the
 // scratch area behind the first `bytes` bytes (a multiple of 256) of the stream's scratch
 // buffer: an entry point that stages tensors of its own there and then calls other entry

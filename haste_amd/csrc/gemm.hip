@@ -42,6 +42,7 @@
 // depend on scheduling.  Whole tiles are numbered so that each XCD (one L2) works on a
 // contiguous run of them; the pieces follow, dealt round-robin over the XCDs.
 #include "common.h"
+#include "split_bf16.h"
 
 namespace haste_hip {
 namespace {
@@ -271,46 +272,24 @@ __device__ __forceinline__ void float_tile(int M, int N, int K,
 
 
 // ---- the product on the bf16 matrix cores ------------------------------------------------
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float float2_t __attribute__((ext_vector_type(2)));
-
 constexpr int SK = 32;  // k of one LDS stage
 // Bytes of one group of 8 k of `rows` rows in one plane (the padding puts the groups that a
 // wavefront writes side by side on different banks), and of an operand's three planes.
 constexpr int split_group_bytes(int rows) { return rows * 16 + 64; }
 constexpr int split_operand_bytes(int rows) { return 3 * (SK / 8) * split_group_bytes(rows); }
 
-__device__ __forceinline__ unsigned int pack_bf16(float a, float b) {
-  const float2_t v = {a, b};
-  return __builtin_bit_cast(unsigned int, __builtin_convertvector(v, bf16x2_t));
-}
-
-__device__ __forceinline__ float bf16_low(unsigned int u) { return __uint_as_float(u << 16); }
-__device__ __forceinline__ float bf16_high(unsigned int u) { return __uint_as_float(u & 0xffff0000u); }
-
-// What operands are multiplied with before they are split, and the product's scale that comes of it.  A
-// bfloat16 holds nothing below 2^-133, a float goes down to 2^-149: unscaled, operands below 2^-110 would
-// lose their last part and those below 2^-134 all three.  Scaled, every part of every float is a normal
-// bfloat16; in exchange operands from 2^104 and results from 2^80 on are infinite, which split_tile() sees.
-// It is one vector instruction more per element: 8192^3 5.42 -> 5.55 ms, 6400 x 512 x 2048 85.6 -> 87.5 us.
-constexpr float kSplitScale = 0x1p24f, kProductScale = 0x1p-48f;
-
+// The scaling (split_bf16.h) is one vector instruction more per element: 8192^3 5.42 -> 5.55 ms, 6400 x 512 x 2048
+// 85.6 -> 87.5 us.
 // Eight consecutive k of one row, scaled, split into three bf16 each and stored into the three planes.
 __device__ __forceinline__ void split_store(const float (&f)[8], char* at, int plane_bytes) {
   uint4_t p[3];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    float a = f[2 * j] * kSplitScale, b = f[2 * j + 1] * kSplitScale;
-    const unsigned int hi = pack_bf16(a, b);
-    a -= bf16_low(hi);
-    b -= bf16_high(hi);
-    const unsigned int mid = pack_bf16(a, b);
-    a -= bf16_low(mid);
-    b -= bf16_high(mid);
+    unsigned int hi, mid, lo;
+    split_pair(f[2 * j] * kSplitScale, f[2 * j + 1] * kSplitScale, hi, mid, lo);
     p[0][j] = hi;
     p[1][j] = mid;
-    p[2][j] = pack_bf16(a, b);
+    p[2][j] = lo;
   }
 #pragma unroll
   for (int q = 0; q < 3; ++q) *reinterpret_cast<uint4_t*>(at + q * plane_bytes) = p[q];

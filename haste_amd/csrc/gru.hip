@@ -6,6 +6,7 @@
 // Arithmetic follows reference lib/gru_forward_gpu.cu.cc:46-84 and
 // lib/gru_backward_gpu.cu.cc:45-95; orchestration replaces :314-371 and :321-409.
 #include "scatter_backward.h"
+#include "split_forward.h"
 
 namespace haste_hip {
 namespace {
@@ -277,6 +278,54 @@ void gru_forward_kernel(GruFwdParams p) {
     }
   }
 }
+
+// The GRU's pointwise forward step for the recurrence on the bf16 matrix cores (split_forward.h):
+// arithmetic as in gru_forward_kernel.
+struct GruForwardCell {
+  using Params = GruFwdParams;
+  static constexpr int kGates = 3;
+  static constexpr int kOut = 5, kStates = 1;  // h, what the backward pass needs (4)
+  float h, bxv[3], brv[3], saved[4];
+
+  __device__ __forceinline__ void load_state(const Params& p, size_t row, size_t unit, bool mine) {
+    h = mine ? p.h[row * p.H + unit] : 0.f;
+#pragma unroll
+    for (int g = 0; g < 3; ++g) {
+      bxv[g] = p.bx[(size_t)g * p.H + unit];
+      brv[g] = p.br[(size_t)g * p.H + unit];
+    }
+  }
+  __device__ __forceinline__ static bool aligned(const Params& p) {
+    return ((reinterpret_cast<uintptr_t>(p.Wx) | reinterpret_cast<uintptr_t>(p.v) | reinterpret_cast<uintptr_t>(p.h_out) |
+             reinterpret_cast<uintptr_t>(p.zoneout_mask)) & 15u) == 0;
+  }
+  __device__ __forceinline__ static const float* in_row(const Params& p, int gate, size_t row) {
+    return p.Wx + (row * 3 + gate) * p.H;
+  }
+  __device__ __forceinline__ static size_t in_stride(const Params& p) { return (size_t)p.N * 3 * p.H; }
+  __device__ __forceinline__ static float* out_row(const Params& p, int i, size_t row) {
+    return i == 0 ? p.h_out + row * p.H : p.v + (row * 4 + i - 1) * p.H;
+  }
+  __device__ __forceinline__ static size_t out_stride(const Params& p, int i) { return (size_t)p.N * p.H * (i < 1 ? 1 : 4); }
+  __device__ __forceinline__ float out(int i) const { return i == 0 ? h : saved[i - 1]; }
+  __device__ __forceinline__ void step(const Params& p, const float4_t& in, float mask, const float4_t& rh, bool zoneout) {
+    const float a[2] = {in[0] + rh[0] + bxv[0] + brv[0], in[1] + rh[1] + bxv[1] + brv[1]};
+    float zr[2];
+    gates_f<2, 0>(a, zr);
+    const float z = zr[0], r = zr[1], qg = rh[2] + brv[2];
+    const float g = tanh_f(in[2] + r * qg + bxv[2]);
+    saved[0] = z;
+    saved[1] = r;
+    saved[2] = g;
+    saved[3] = qg;
+    float h_new = z * h + (1.0f - z) * g;
+    if (zoneout) {
+      if (p.training) h_new = (h_new - h) * mask + h;
+      else h_new = p.zoneout_prob * h + (1.0f - p.zoneout_prob) * h_new;
+    }
+    h = h_new;
+  }
+};
 
 // The forward pass of a single batch row (see "one batch row" in recurrent.h): 16 hidden units
 // x 3 gates per workgroup (the fourth 16 columns of the 64 are idle), the recurrent weights in
@@ -847,6 +896,11 @@ int gru_forward_impl(hipStream_t stream, int training, int T, int N, int C, int 
                      tile.reg_groups == 0 && C <= 512 && C % 4 == 0 &&
                      (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
   if (fused) HASTE_HIP_PROPAGATE(input_projection_in_recurrence(stream, T, N, C, H, 3 * H, &fused));
+  // The recurrence on the bf16 matrix cores, where it is the faster one (split_forward.h).
+  int split_rows = 0;
+  if (!half_product)
+    HASTE_HIP_PROPAGATE(split_forward_rule(stream, T, N, C, H, 3 * H, wx_ready, fused, &split_rows));
+  if (split_rows > 0) fused = false;
   const int xsg = C <= 256 ? 1 : 2;
   size_t lds_bytes = paired ? paired_lds : tile.lds_bytes;
   if (fused)
@@ -857,7 +911,8 @@ int gru_forward_impl(hipStream_t stream, int training, int T, int N, int C, int 
   // Taken after the GEMM, which may replace the stream's scratch buffer with a larger one.
   Workspace ws;
   HASTE_HIP_PROPAGATE(get_workspace(
-      stream, exchange_floats(H, tile.nb, tile.gy, kPolledTiles) * sizeof(float), &ws));
+      stream, split_rows > 0 ? split_forward_tile_bytes(N, H, split_rows)
+                             : exchange_floats(H, tile.nb, tile.gy, kPolledTiles) * sizeof(float), &ws));
   HASTE_HIP_PROPAGATE(check_and_clear_abort(stream, &ws));
 
   GruFwdParams p;
@@ -867,6 +922,8 @@ int gru_forward_impl(hipStream_t stream, int training, int T, int N, int C, int 
   p.zoneout_prob = zoneout_prob; p.zoneout_mask = zoneout_mask;
   p.dc_mask = dc_mask; p.dc_scale = dc_scale;
   p.xh = ws.scratch;
+  if (split_rows > 0)
+    return launch_split_forward<GruForwardCell>("gru_forward_recurrence", stream, ws, split_rows, p);
   LaunchPlan plan;
   HASTE_HIP_PROPAGATE(plan_launch(stream, ws, tile.gx, tile.gy, tile.nb, lds_bytes, (unsigned)T + 1, &plan));
   p.ls = plan.shape;

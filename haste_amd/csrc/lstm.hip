@@ -6,6 +6,7 @@
 // Arithmetic follows reference lib/lstm_forward_gpu.cu.cc:55-86 and
 // lib/lstm_backward_gpu.cu.cc:47-95; orchestration replaces :313-366 and :319-405.
 #include "scatter_backward.h"
+#include "split_forward.h"
 
 namespace haste_hip {
 namespace {
@@ -273,6 +274,49 @@ void lstm_forward_kernel(LstmFwdParams p) {
     }
   }
 }
+
+// The LSTM's pointwise forward step for the recurrence on the bf16 matrix cores (split_forward.h):
+// arithmetic as in lstm_forward_kernel.
+struct LstmForwardCell {
+  using Params = LstmFwdParams;
+  static constexpr int kGates = 4;
+  static constexpr int kOut = 6, kStates = 2;  // h, c, activations (4 gates)
+  float h, c, bias[4], gate[4];
+
+  __device__ __forceinline__ void load_state(const Params& p, size_t row, size_t unit, bool mine) {
+    const size_t e = row * p.H + unit;
+    h = mine ? p.h[e] : 0.f;
+    c = mine ? p.c[e] : 0.f;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) bias[g] = p.b[(size_t)g * p.H + unit];
+  }
+  __device__ __forceinline__ static bool aligned(const Params& p) {
+    return ((reinterpret_cast<uintptr_t>(p.v) | reinterpret_cast<uintptr_t>(p.h_out) | reinterpret_cast<uintptr_t>(p.c_out) |
+             reinterpret_cast<uintptr_t>(p.zoneout_mask)) & 15u) == 0;
+  }
+  __device__ __forceinline__ static const float* in_row(const Params& p, int gate, size_t row) {
+    return p.v + (row * 4 + gate) * p.H;
+  }
+  __device__ __forceinline__ static size_t in_stride(const Params& p) { return (size_t)p.N * 4 * p.H; }
+  __device__ __forceinline__ static float* out_row(const Params& p, int i, size_t row) {
+    return i == 0 ? p.h_out + row * p.H : (i == 1 ? p.c_out + row * p.H : p.v + (row * 4 + i - 2) * p.H);
+  }
+  __device__ __forceinline__ static size_t out_stride(const Params& p, int i) { return (size_t)p.N * p.H * (i < 2 ? 1 : 4); }
+  __device__ __forceinline__ float out(int i) const { return i == 0 ? h : (i == 1 ? c : gate[i - 2]); }
+  __device__ __forceinline__ void step(const Params& p, const float4_t& in, float mask, const float4_t& rh, bool zoneout) {
+    float a[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) a[g] = in[g] + rh[g] + bias[g];
+    gates_f<4, 0b0010>(a, gate);
+    c = gate[2] * c + gate[0] * gate[1];
+    float h_new = gate[3] * tanh_f(c);
+    if (zoneout) {
+      if (p.training) h_new = (h_new - h) * mask + h;
+      else h_new = p.zoneout_prob * h + (1.0f - p.zoneout_prob) * h_new;
+    }
+    h = h_new;
+  }
+};
 
 // The forward pass of a single batch row (see "one batch row" in recurrent.h): 16 hidden units
 // x 4 gates per workgroup, the recurrent weights in registers.
@@ -848,13 +892,18 @@ int lstm_forward_impl(hipStream_t stream, int training, int T, int N, int C, int
   bool fused = (paired || tile.nb == 4) && H > 192 && C <= 512 && C % 4 == 0 &&
                      (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
   if (fused) HASTE_HIP_PROPAGATE(input_projection_in_recurrence(stream, T, N, C, H, 4 * H, &fused));
+  // The recurrence on the bf16 matrix cores, where it is the faster one (split_forward.h).
+  int split_rows = 0;
+  HASTE_HIP_PROPAGATE(split_forward_rule(stream, T, N, C, H, 4 * H, false, fused, &split_rows));
+  if (split_rows > 0) fused = false;
   if (!fused)
     HASTE_HIP_PROPAGATE(gemm_f32(stream, false, T * N, 4 * H, C, x, C, W, 4 * H, v, 4 * H, false));
 
   // Taken after the GEMM, which may replace the stream's scratch buffer with a larger one.
   Workspace ws;
   HASTE_HIP_PROPAGATE(get_workspace(
-      stream, exchange_floats(H, tile.nb, tile.gy, kPolledTiles) * sizeof(float), &ws));
+      stream, split_rows > 0 ? split_forward_tile_bytes(N, H, split_rows)
+                             : exchange_floats(H, tile.nb, tile.gy, kPolledTiles) * sizeof(float), &ws));
   HASTE_HIP_PROPAGATE(check_and_clear_abort(stream, &ws));
 
   LstmFwdParams p;
@@ -864,6 +913,8 @@ int lstm_forward_impl(hipStream_t stream, int training, int T, int N, int C, int
   p.dc_mask = dc_mask; p.dc_scale = dc_scale;
   p.xh = ws.scratch;
   p.x = x; p.W = W; p.C = C;
+  if (split_rows > 0)
+    return launch_split_forward<LstmForwardCell>("lstm_forward_recurrence", stream, ws, split_rows, p);
   LaunchPlan plan;
   HASTE_HIP_PROPAGATE(plan_launch(stream, ws, tile.gx, tile.gy, tile.nb,
                                   paired ? paired_lds : tile.lds_bytes, (unsigned)T + 1, &plan));

@@ -35,12 +35,43 @@ __device__ __forceinline__ float sigmoid_f(float x) {
 }
 // Small arguments use the odd series (truncation below 1e-7 for |x| < 0.25), which keeps
 // the relative accuracy that 1 - 2/(exp(2x)+1) loses to cancellation there.
-__device__ __forceinline__ float tanh_f(float x) {
+constexpr float kTanhSeries = 0.25f;
+__device__ __forceinline__ float tanh_series_f(float x) {
   const float x2 = x * x;
-  const float series =
-      x * (1.0f + x2 * (-0.333333333f + x2 * (0.133333333f + x2 * -0.0539682540f)));
+  return x * (1.0f + x2 * (-0.333333333f + x2 * (0.133333333f + x2 * -0.0539682540f)));
+}
+__device__ __forceinline__ float tanh_f(float x) {
+  const float series = tanh_series_f(x);
   const float wide = 1.0f - 2.0f * __builtin_amdgcn_rcpf(1.0f + exp_f(2.0f * x));
-  return fabsf(x) < 0.25f ? series : wide;
+  return fabsf(x) < kTanhSeries ? series : wide;
+}
+// Several at once, tanh where TANH has a bit set: one operation for all of them after the other (a wavefront that has
+// its SIMD to itself waits twice as long for an operation that needs the result of the one before it).
+template <int N, unsigned int TANH>
+__device__ __forceinline__ void gates_f(const float (&a)[N], float (&y)[N]) {
+  constexpr float kLog2e = 1.44269504088896341f;
+  float e[N], series[N];
+  auto keep = [&] {
+#pragma unroll
+    for (int i = 0; i < N; ++i) asm volatile("" : "+v"(e[i]));
+  };
+#pragma unroll
+  for (int i = 0; i < N; ++i) e[i] = (TANH >> i & 1 ? 2.0f * a[i] : -a[i]) * kLog2e;
+  keep();
+#pragma unroll
+  for (int i = 0; i < N; ++i) e[i] = __builtin_amdgcn_exp2f(e[i]);
+  keep();
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    series[i] = TANH >> i & 1 ? tanh_series_f(a[i]) : 0.f;
+    e[i] = 1.0f + e[i];
+  }
+  keep();
+#pragma unroll
+  for (int i = 0; i < N; ++i) e[i] = __builtin_amdgcn_rcpf(e[i]);
+  keep();
+#pragma unroll
+  for (int i = 0; i < N; ++i) y[i] = !(TANH >> i & 1) ? e[i] : (fabsf(a[i]) < kTanhSeries ? series[i] : 1.0f - 2.0f * e[i]);
 }
 __device__ __forceinline__ float d_sigmoid_f(float y) { return y * (1.0f - y); }
 __device__ __forceinline__ float d_tanh_f(float y) { return 1.0f - y * y; }

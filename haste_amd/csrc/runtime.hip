@@ -286,17 +286,24 @@ bool fused_input_enabled() {
   return enabled;
 }
 
+int workspace_has_room(hipStream_t stream, size_t bytes, bool* room) {
+  Workspace ws;
+  HASTE_HIP_PROPAGATE(get_workspace(stream, 0, &ws));
+  *room = true;
+  if (ws.scratch_bytes < bytes) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &capture) != hipSuccess) (void)hipGetLastError();
+    *room = !ws.caller_owned && capture == hipStreamCaptureStatusNone;
+  }
+  return HASTE_HIP_OK;
+}
+
 int input_projection_in_recurrence(hipStream_t stream, int T, int N, int C, int H, int columns, bool* fused) {
   *fused = fused_input_enabled();
   if (!*fused || N > 32 || (long long)C * H < (1 << 16) || (long long)T * C * H < (1ll << 24)) return HASTE_HIP_OK;
-  Workspace ws;
-  HASTE_HIP_PROPAGATE(get_workspace(stream, 0, &ws));
-  if (ws.scratch_bytes < gemm_f32_scratch_bytes(T * N, columns, C)) {
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &capture) != hipSuccess) (void)hipGetLastError();
-    if (ws.caller_owned || capture != hipStreamCaptureStatusNone) return HASTE_HIP_OK;
-  }
-  *fused = false;
+  bool room = false;
+  HASTE_HIP_PROPAGATE(workspace_has_room(stream, gemm_f32_scratch_bytes(T * N, columns, C), &room));
+  *fused = !room;
   return HASTE_HIP_OK;
 }
 
