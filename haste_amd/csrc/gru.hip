@@ -6,6 +6,7 @@
 // Arithmetic follows reference lib/gru_forward_gpu.cu.cc:46-84 and
 // lib/gru_backward_gpu.cu.cc:45-95; orchestration replaces :314-371 and :321-409.
 #include "scatter_backward.h"
+#include "split_backward.h"
 #include "split_forward.h"
 
 namespace haste_hip {
@@ -811,6 +812,25 @@ struct GruScatterCell {
     if (col < 3 * p.H) p.dbx[col] += s;
     else p.dbr[col - 3 * p.H] += s;
   }
+
+  // For split_backward_kernel.
+  static constexpr int kOut = 6;  // dp, dq
+  __device__ __forceinline__ static int out_value(int i) { return i < 3 ? (i == 2 ? 3 : i) : i - 3; }
+  __device__ __forceinline__ static bool aligned(const Params& p) {
+    return ((reinterpret_cast<uintptr_t>(p.v) | reinterpret_cast<uintptr_t>(p.h) | reinterpret_cast<uintptr_t>(p.dh_next) |
+             reinterpret_cast<uintptr_t>(p.dp) | reinterpret_cast<uintptr_t>(p.dq) |
+             reinterpret_cast<uintptr_t>(p.zoneout_mask)) & 15u) == 0;
+  }
+  __device__ __forceinline__ static bool in_used(const Params&, int i, bool zoneout) { return i < 6 || zoneout; }
+  __device__ __forceinline__ static const float* in_row(const Params& p, int i, size_t row) {
+    if (i < 4) return p.v + (row * 4 + i) * p.H;
+    return (i == 4 ? p.h : (i == 5 ? p.dh_next : p.zoneout_mask)) + row * p.H;
+  }
+  __device__ __forceinline__ static size_t in_stride(const Params& p, int i) { return (size_t)p.N * p.H * (i < 4 ? 4 : 1); }
+  __device__ __forceinline__ static float* out_row(const Params& p, int i, size_t row) {
+    return i < 3 ? p.dp + (row * 3 + i) * p.H : p.dq + (row * 3 + i - 3) * p.H;
+  }
+  __device__ __forceinline__ static size_t out_stride(const Params& p, int) { return (size_t)p.N * p.H * 3; }
 };
 
 }  // namespace
@@ -1006,10 +1026,17 @@ int gru_backward_impl(hipStream_t stream, int T, int N, int C, int H,
                               : tile.nb == 8 && paired_lds <= kMaxLdsBytes;
   const int sets = paired ? 2 : 1;
 
+  // Tiles of 8 and 16 rows: on the bf16 matrix cores (split_backward.h).
+  int split_rows = 0;
+  size_t split_sums = 0, split_floats = 0;
+  if (!half_product)
+    HASTE_HIP_PROPAGATE(split_backward_rule(stream, N, H, 6, &split_rows, &split_sums, &split_floats));
+
   Workspace ws;
-  const size_t db_floats = ((size_t)tile.gy * sets * 6 * H + 3) / 4 * 4;
+  const size_t db_floats = split_rows > 0 ? split_sums : ((size_t)tile.gy * sets * 6 * H + 3) / 4 * 4;
   const size_t xdq_floats =
-      scatter ? (size_t)tile.gy * sets * kScatterTiles * scatter_tile_floats(tile.gx, H <= 256 ? 1 : 2)
+      split_rows > 0 ? split_floats - split_sums
+      : scatter ? (size_t)tile.gy * sets * kScatterTiles * scatter_tile_floats(tile.gx, H <= 256 ? 1 : 2)
               : exchange_floats(gru_backward_k(H), tile.nb, tile.gy, kPolledTiles);
   HASTE_HIP_PROPAGATE(get_workspace(stream, (db_floats + xdq_floats) * sizeof(float), &ws));
   HASTE_HIP_PROPAGATE(check_and_clear_abort(stream, &ws));
@@ -1021,15 +1048,17 @@ int gru_backward_impl(hipStream_t stream, int T, int N, int C, int H,
   p.db_partial = ws.scratch;
   p.xdq = ws.scratch + db_floats;
   LaunchPlan plan;
-  HASTE_HIP_PROPAGATE(plan_launch(stream, ws, tile.gx, tile.gy, tile.nb,
-                                  scatter ? sets * kScatterSetFloats * sizeof(float)
-                                          : (paired ? paired_lds : tile.lds_bytes),
-                                  (unsigned)T + 1, &plan));
+  if (split_rows == 0)
+    HASTE_HIP_PROPAGATE(plan_launch(stream, ws, tile.gx, tile.gy, tile.nb,
+                                    scatter ? sets * kScatterSetFloats * sizeof(float)
+                                            : (paired ? paired_lds : tile.lds_bytes),
+                                    (unsigned)T + 1, &plan));
   p.ls = plan.shape;
   if (paired) plan.threads = 512;
   int rc = HASTE_HIP_ERROR_UNSUPPORTED_SIZE;
   const char* name = "gru_backward_recurrence";
-  if (scatter && half_product) rc = launch_scatter_backward<GruScatterCell, true>(name, H, sets, plan, p, stream);
+  if (split_rows > 0) rc = launch_split_backward<GruScatterCell>(name, stream, ws, split_rows, p);
+  else if (scatter && half_product) rc = launch_scatter_backward<GruScatterCell, true>(name, H, sets, plan, p, stream);
   else if (scatter) rc = launch_scatter_backward<GruScatterCell>(name, H, sets, plan, p, stream);
   else
 #define HASTE_LAUNCH_BWD_RESIDENT(NB_)                                                           \

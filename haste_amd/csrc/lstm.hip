@@ -6,6 +6,7 @@
 // Arithmetic follows reference lib/lstm_forward_gpu.cu.cc:55-86 and
 // lib/lstm_backward_gpu.cu.cc:47-95; orchestration replaces :313-366 and :319-405.
 #include "scatter_backward.h"
+#include "split_backward.h"
 #include "split_forward.h"
 
 namespace haste_hip {
@@ -823,6 +824,25 @@ struct LstmScatterCell {
     for (int g = 0; g < 4; ++g) vt[g * (size_t)p.H] = a[g];
   }
   __device__ __forceinline__ static void add_sums(const Params& p, int col, float s) { p.db[col] += s; }
+
+  // For split_backward_kernel.
+  static constexpr int kOut = 4;
+  __device__ __forceinline__ static int out_value(int i) { return i; }
+  __device__ __forceinline__ static bool aligned(const Params& p) {
+    return ((reinterpret_cast<uintptr_t>(p.v) | reinterpret_cast<uintptr_t>(p.c) | reinterpret_cast<uintptr_t>(p.c_next) |
+             reinterpret_cast<uintptr_t>(p.dh_next) | reinterpret_cast<uintptr_t>(p.dc_next) |
+             reinterpret_cast<uintptr_t>(p.zoneout_mask)) & 15u) == 0;
+  }
+  __device__ __forceinline__ static bool in_used(const Params& p, int i, bool zoneout) {
+    return i < 7 || (i == 7 ? p.dc_given != 0 : zoneout);
+  }
+  __device__ __forceinline__ static const float* in_row(const Params& p, int i, size_t row) {
+    if (i < 4) return p.v + (row * 4 + i) * p.H;
+    return (i == 4 ? p.c : (i == 5 ? p.c_next : (i == 6 ? p.dh_next : (i == 7 ? p.dc_next : p.zoneout_mask)))) + row * p.H;
+  }
+  __device__ __forceinline__ static size_t in_stride(const Params& p, int i) { return (size_t)p.N * p.H * (i < 4 ? 4 : 1); }
+  __device__ __forceinline__ static float* out_row(const Params& p, int i, size_t row) { return p.v + (row * 4 + i) * p.H; }
+  __device__ __forceinline__ static size_t out_stride(const Params& p, int) { return (size_t)p.N * p.H * 4; }
 };
 
 }  // namespace
@@ -988,9 +1008,14 @@ int lstm_backward_impl(hipStream_t stream, int T, int N, int C, int H,
   const int sets = paired ? 2 : 1;
   const int ctn = H <= 256 ? 1 : 2;  // column tiles of 64 per wavefront
 
+  // Tiles of 8 and 16 rows: on the bf16 matrix cores (split_backward.h).
+  int split_rows = 0;
+  size_t split_sums = 0, split_floats = 0;
+  HASTE_HIP_PROPAGATE(split_backward_rule(stream, N, H, 4, &split_rows, &split_sums, &split_floats));
+
   Workspace ws;
-  const size_t db_floats = (size_t)tile.gy * sets * 4 * H;
-  const size_t xdv_floats = scatter ? (size_t)tile.gy * sets * kScatterTiles * scatter_tile_floats(tile.gx, ctn)
+  const size_t db_floats = split_rows > 0 ? split_sums : (size_t)tile.gy * sets * 4 * H;
+  const size_t xdv_floats = split_rows > 0 ? split_floats - split_sums : scatter ? (size_t)tile.gy * sets * kScatterTiles * scatter_tile_floats(tile.gx, ctn)
                                     : exchange_floats(64 * tile.gx, tile.nb, tile.gy, kPolledTiles);
   HASTE_HIP_PROPAGATE(get_workspace(stream, ((db_floats + 3) / 4 * 4 + xdv_floats) * sizeof(float), &ws));
   HASTE_HIP_PROPAGATE(check_and_clear_abort(stream, &ws));
@@ -1004,13 +1029,16 @@ int lstm_backward_impl(hipStream_t stream, int T, int N, int C, int H,
   p.db_partial = ws.scratch;
   p.xdv = ws.scratch + (db_floats + 3) / 4 * 4;
   LaunchPlan plan;
-  HASTE_HIP_PROPAGATE(plan_launch(stream, ws, tile.gx, tile.gy, tile.nb,
-                                  scatter ? sets * kScatterSetFloats * sizeof(float) : (paired ? paired_lds : tile.lds_bytes), (unsigned)T + 1, &plan));
+  if (split_rows == 0)
+    HASTE_HIP_PROPAGATE(plan_launch(stream, ws, tile.gx, tile.gy, tile.nb,
+                                    scatter ? sets * kScatterSetFloats * sizeof(float) : (paired ? paired_lds : tile.lds_bytes), (unsigned)T + 1, &plan));
   p.ls = plan.shape;
   if (paired) plan.threads = 512;
   int rc = HASTE_HIP_ERROR_UNSUPPORTED_SIZE;
   const char* name = "lstm_backward_recurrence";
-  if (scatter) {
+  if (split_rows > 0) {
+    rc = launch_split_backward<LstmScatterCell>(name, stream, ws, split_rows, p);
+  } else if (scatter) {
     rc = launch_scatter_backward<LstmScatterCell>(name, H, sets, plan, p, stream);
   } else
 #define HASTE_LAUNCH_BWD_RESIDENT(NB_)                                                            \

@@ -292,15 +292,17 @@ void scatter_backward_kernel(typename Cell::Params p) {
 }
 
 
-// Launches the kernel for `sets` sets per workgroup and hidden size H <= 512.
+// Launches the kernel for `sets` sets per workgroup and hidden size H <= 512 (two sets of fp32 products: H <= 256, beyond
+// that split_backward.h's kernel runs).
 template <class Cell, bool HALF = false>
 int launch_scatter_backward(const char* name, int H, int sets, const LaunchPlan& plan, typename Cell::Params& p,
                             hipStream_t stream) {
   if (H <= 256)
     return sets == 2 ? launch_persistent(name, scatter_backward_kernel<Cell, 1, 2, HALF>, plan, p, stream)
                      : launch_persistent(name, scatter_backward_kernel<Cell, 1, 1, HALF>, plan, p, stream);
-  return sets == 2 ? launch_persistent(name, scatter_backward_kernel<Cell, 2, 2, HALF>, plan, p, stream)
-                   : launch_persistent(name, scatter_backward_kernel<Cell, 2, 1, HALF>, plan, p, stream);
+  if (sets == 1) return launch_persistent(name, scatter_backward_kernel<Cell, 2, 1, HALF>, plan, p, stream);
+  if constexpr (HALF) return launch_persistent(name, scatter_backward_kernel<Cell, 2, 2, HALF>, plan, p, stream);
+  return HASTE_HIP_ERROR_UNSUPPORTED_SIZE;
 }
 
 }  // namespace haste_hip

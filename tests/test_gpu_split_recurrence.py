@@ -1,4 +1,4 @@
-"""The forward recurrences on the bf16 matrix cores (h and R as sums of three bfloat16):
+"""The recurrences on the bf16 matrix cores (h, the gate gradients and R as sums of three bfloat16):
 the edges of their tiles against the fp64 oracle, and values whose parts would overflow or are not finite."""
 import numpy as np
 import pytest
@@ -86,3 +86,65 @@ def test_dropconnect(N):
     a = ops.lstm_forward(False, 0.0, *first, dev(p["R"]), dev(p["b"]), none, dev(keep), scale)
     b = ops.lstm_forward(False, 0.0, *first, dev(p["R"] * keep * scale), dev(p["b"]), none)
     assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+
+
+def backward(cell, p, states):
+    """Gradients for the states and activations of the reference's forward pass, by name."""
+    from haste_amd import ops
+    x_t = dev(p["x"]).permute(2, 0, 1).contiguous()
+    W_t, R_t = dev(p["W"]).t().contiguous(), dev(p["R"]).t().contiguous()
+    if cell == "lstm":
+        h, c, v = (dev(a) for a in states)
+        out = ops.lstm_backward(x_t, W_t, R_t, dev(p["b"]), dev(p["mask"]), h, c, v, dev(p["dh_new"]), dev(p["dc_new"]))
+        return dict(zip(("dx", "dh0", "dc0", "dW", "dR", "db", "dv"), map(host, out + (v,))))
+    h, v = (dev(a) for a in states)
+    out = ops.gru_backward(x_t, W_t, R_t, dev(p["b"]), dev(p["b2"]), dev(p["mask"]), h, v, dev(p["dh_new"]))
+    return dict(zip(("dx", "dh0", "dW", "dR", "dbx", "dbr"), map(host, out)))
+
+
+def backward_reference(cell, p, states):
+    states = tuple(np.float64(np.float32(a)) for a in states)
+    if cell == "lstm":
+        out = O.lstm_backward(p["W"], p["R"], p["b"], p["x"], *states, p["dh_new"], p["dc_new"], p["mask"])
+        return dict(zip(("dx", "dW", "dR", "db", "dh0", "dc0", "dv"), out))
+    out = O.gru_backward(p["W"], p["R"], p["b"], p["b2"], p["x"], *states, p["dh_new"], p["mask"])
+    return dict(zip(("dx", "dW", "dR", "dbx", "dbr", "dh0"), out))
+
+
+@pytest.mark.parametrize("T,N,H", [(1, 33, 33), (3, 64, 16), (6, 40, 128), (4, 39, 257), (5, 64, 384), (2, 41, 385), (7, 50, 511),
+                                   (9, 64, 512), (1, 65, 32), (5, 65, 31), (4, 128, 256), (3, 127, 258), (6, 96, 384),
+                                   (2, 113, 400), (7, 66, 510), (9, 128, 512)])
+@pytest.mark.parametrize("zoneout", [0.0, 0.2])
+@pytest.mark.parametrize("cell", ["lstm", "gru"])
+def test_backward_tiles(cell, zoneout, T, N, H):
+    print("split backward recurrence", cell, zoneout, T, N, H, flush=True)
+    p = problem(T + N + H, T, N, 12, H, 4 if cell == "lstm" else 3, zoneout)
+    states = reference(cell, p, True, zoneout)
+    # The partial sums give their last bit (2^-24) to the exchange at every step, the gradients of the weights add up
+    # T * N terms: 2^-18 of the largest value holds both.
+    ours, theirs = backward(cell, p, states), backward_reference(cell, p, states)
+    for name in ours:
+        assert relerr(ours[name], theirs[name]) < 2.0 ** -18, name
+
+
+@pytest.mark.parametrize("what", ["gradient", "gradient_inf", "weight", "weight_inf", "nan"])
+@pytest.mark.parametrize("N", [40, 100])
+@pytest.mark.parametrize("cell", ["lstm", "gru"])
+def test_backward_values_that_do_not_split(cell, N, what):
+    """What reaches the initial state: finite, infinite and not a number where the reference is, and equal where finite."""
+    print("split backward recurrence, extreme values", cell, N, what, flush=True)
+    T, H = 4, 70
+    p = problem(9 + N, T, N, 8, H, 4 if cell == "lstm" else 3)
+    states = reference(cell, p, True, 0.0)
+    p["dh_new"][3, 5, 6], p["R"][9, 11] = {"gradient": (2.0 ** 60, 0.01), "gradient_inf": (np.inf, 0.01),
+                                           "weight": (1.0, 2.0 ** 40), "weight_inf": (1.0, np.inf),
+                                           "nan": (np.nan, 0.01)}[what]
+    with np.errstate(all="ignore"):
+        dh0, expected = backward(cell, p, states)["dh0"], backward_reference(cell, p, states)["dh0"]
+    rows = np.arange(N) != 5
+    assert np.array_equal(np.isnan(dh0), np.isnan(expected))
+    assert np.array_equal(np.isfinite(dh0), np.isfinite(expected))
+    finite = np.isfinite(expected)
+    for mask in (finite & rows[:, None], finite & ~rows[:, None]):
+        if np.any(mask):
+            assert np.max(np.abs(dh0[mask] - expected[mask])) <= 1e-5 * np.max(np.abs(expected[mask]))
