@@ -5,16 +5,17 @@
 // Bound: MFMA (fp64 peak 78.6 TFLOP/s), algorithmic flops 2*M*N*K.  A workgroup of four
 // wavefronts owns a 64 x 64 tile of C; a wavefront owns 32 x 32 of it as 2 x 2 MFMA tiles.
 // Operand panels of 32 k go through LDS k-major ([k][m], [k][n]): the lanes of one MFMA
-// operand read 16 consecutive doubles of one k row.  Measured, panels loaded in runs of 256 - 512
-// bytes and requested three ahead (one ahead and in runs of 16 bytes before): 512 x 2048 x 6400
-// 359 -> 312 us, with A transposed 405 -> 295 (45 TFLOP/s, one workgroup per CU); products of many
-// tiles were and are bound by the matrix cores, 64 - 75 % busy: 6400 x 2048 x 512 300, 4096^3 56
-// TFLOP/s.  A product with few tiles and a long
-// contraction (the product of one step over 70 rows: 128 x 512 x 2048 is 16 tiles) is cut along K
-// into pieces, each a workgroup of its own, which park partial results in the stream's scratch
-// buffer; a second kernel adds a tile's pieces in index order.  How a product is cut depends
-// on its shape only, so results are reproducible.  Lane layout of the instruction (checked on
-// the hardware): a = A[i = lane%16][k = lane/16], b = B[k = lane/16][j = lane%16],
+// operand read 16 consecutive doubles of one k row.  Panels are loaded in runs of 256 - 512
+// bytes and requested three ahead.  Two workgroups share a CU (256 registers a lane, accumulators and
+// operands alike: given 512, the compiler computed in one half of the file and kept the accumulators in the other,
+// 64 moves and a wait for the matrix cores every two panels), and the tiles that would fill a last round of
+// workgroups only partly are cut along K, as is a product of few tiles and a long contraction (the product of one step
+// over 70 rows: 128 x 512 x 2048 is 16 tiles): each piece a workgroup of its own, which parks partial results in the
+// stream's scratch buffer; a second kernel adds a tile's pieces in index order.  Measured, before and after those
+// two and the branch-free loop below: 6400 x 2048 x 512 273 -> 255 us, 6400 x 512 x 2048 307 -> 222,
+// 512 x 2048 x 6400 295 -> 238, with A transposed 278 -> 221 (61 TFLOP/s), 4096^3 59 -> 64 TFLOP/s (the library: 72).
+// How a product is cut depends on its shape only (and on whether the scratch buffer has room for the pieces), so
+// results are reproducible.  Lane layout of the instruction (checked on the hardware): a = A[i = lane%16][k = lane/16], b = B[k = lane/16][j = lane%16],
 // d[r] = D[i = 4*r + lane/16][j = lane%16].
 #include "common.h"
 
@@ -37,23 +38,45 @@ __device__ __forceinline__ int panel_at(int k, int i) {
   return k * 64 + (i ^ (((k >> 1) & 3) << 2) ^ (((k >> 3) ^ k) & 1) << 4);
 }
 
+// How a product is cut: the first `whole` tiles (row by row) are not, the others into `pieces` of k_per_piece each.
+struct F64Plan {
+  int whole, pieces, k_per_piece;
+};
+constexpr int kXcds = 8;
+
+// How a workgroup's operands are loaded: pairs in whole panels, pairs with a ragged last panel, or single elements.
+enum { kWhole, kPairs, kSingle };
+
 template <bool TRANS_A>
-__global__ __launch_bounds__(256)
+__global__ __launch_bounds__(256, 2)
 void gemm_f64_kernel(int M, int N, int K, const double* __restrict__ A, int lda,
                      const double* __restrict__ B, int ldb, double* __restrict__ C, int ldc,
-                     int accumulate, int k_per_piece, double* __restrict__ part, int panels_ok) {
+                     int accumulate, F64Plan plan, int tiles_n, double* __restrict__ part, int chunks, int panels_ok) {
   __shared__ double2_t panels[2][2][DK * 64 / 2];  // [buffer][A, B]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int m0 = blockIdx.y * DM, n0 = blockIdx.x * DN;
+  // Workgroups [0, whole) take a tile each, the others a piece of one of the remaining tiles.  Ids go to the XCDs
+  // round-robin; an XCD (one L2) gets a contiguous run of the whole tiles, and of the pieces.
+  int tile, piece = 0;
+  {
+    const int id = blockIdx.x, first = id < plan.whole ? 0 : plan.whole;
+    const int count = id < plan.whole ? plan.whole : (int)gridDim.x - plan.whole;
+    const int xcd = (id - first) % kXcds, q = count / kXcds, r = count % kXcds;
+    const int at = xcd * q + (xcd < r ? xcd : r) + (id - first) / kXcds;
+    tile = first == 0 && id < plan.whole ? at : plan.whole + at / plan.pieces;
+    piece = id < plan.whole ? 0 : at % plan.pieces;
+  }
+  const int m0 = tile / tiles_n * DM, n0 = tile % tiles_n * DN;
   const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
-  // A workgroup whose columns (and, with A stored transposed, rows) are all inside the problem
-  // and whose piece of K is whole panels loads through buffer resources, 16 bytes at a time and
-  // without a branch: rows of A beyond M lie beyond the resource's range and read as zero.
-  // Otherwise every element is loaded under its own bounds check (one branch each).
-  const int piece_begin = blockIdx.z * k_per_piece;
-  const int piece_end = piece_begin + k_per_piece < K ? piece_begin + k_per_piece : K;
-  const bool fast = panels_ok != 0 && (piece_end - piece_begin) % DK == 0 && n0 + DN <= N &&
-                    (!TRANS_A || m0 + DM <= M);
+  // Loads go through buffer resources, 16 bytes at a time and without a branch: pairs beyond the problem take an offset
+  // beyond the resource's range and read as zero, as do rows of A beyond M.  A pair must lie inside or outside as a
+  // whole: a piece of K (A not transposed), a last tile's columns or transposed rows of odd number load every element
+  // under its own bounds check (one branch each).  (Ragged pieces took that path too: 768 x 3072 x 2000, A
+  // transposed, 272 -> 164 us, 300 x 1200 x 3071 87 -> 54.)
+  const bool cut = tile >= plan.whole;
+  const int piece_begin = cut ? piece * plan.k_per_piece : 0;
+  const int piece_end = cut && piece_begin + plan.k_per_piece < K ? piece_begin + plan.k_per_piece : K;
+  const bool fast = panels_ok != 0 && (n0 + DN <= N || N % 2 == 0) &&
+                    (TRANS_A ? m0 + DM <= M || M % 2 == 0 : (piece_end - piece_begin) % 2 == 0);
   const __amdgpu_buffer_rsrc_t pa = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<double*>(A), 0,
       fast ? (int)((TRANS_A ? (long long)(K - 1) * lda + M : (long long)(M - 1) * lda + K) * 8) : 0, 0x00020000);
@@ -64,10 +87,10 @@ void gemm_f64_kernel(int M, int N, int K, const double* __restrict__ A, int lda,
   // wavefront's load is runs of 256 or 512 bytes.
   const int rrow = tid >> 4, rk = (tid & 15) * 2;
   const int ck = tid >> 5, ci = (tid & 31) * 2;
-  const unsigned int a_voff = TRANS_A ? (unsigned int)((ck * lda + m0 + ci) * 8)
+  const unsigned int a_voff = TRANS_A ? m0 + ci < M ? (unsigned int)((ck * lda + m0 + ci) * 8) : kNowhere
                                       : (unsigned int)(((m0 + rrow) * lda + rk) * 8);
   const unsigned int a_step = (unsigned int)((TRANS_A ? 8 : 16) * lda) * 8u, b_step = (unsigned int)ldb * 64u;
-  const unsigned int b_voff = (unsigned int)((ck * ldb + n0 + ci) * 8);
+  const unsigned int b_voff = n0 + ci < N ? (unsigned int)((ck * ldb + n0 + ci) * 8) : kNowhere;
   double4_t acc[2][2];
 #pragma unroll
   for (int a = 0; a < 2; ++a)
@@ -78,13 +101,16 @@ void gemm_f64_kernel(int M, int N, int K, const double* __restrict__ A, int lda,
   // (two in registers, one in LDS): a product with one workgroup per CU has nothing else to do
   // while it waits for memory.
   double2_t ra[2][4], rb[2][4];
-  auto request = [&](int set, int k0) {
-    if (fast) {
+  auto request = [&](auto fast_c, int set, int k0) {
+    if constexpr (decltype(fast_c)::value != kSingle) {
       const int sa = TRANS_A ? k0 * lda * 8 : k0 * 8, sb = k0 * ldb * 8;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        ra[set][i] = __builtin_bit_cast(double2_t, __builtin_amdgcn_raw_buffer_load_b128(pa, a_voff + i * a_step, sa, 0));
-        rb[set][i] = __builtin_bit_cast(double2_t, __builtin_amdgcn_raw_buffer_load_b128(pb, b_voff + i * b_step, sb, 0));
+        const bool whole = decltype(fast_c)::value == kWhole;
+        const bool b_in = whole || k0 + ck + 8 * i < K, a_in = TRANS_A ? b_in : whole || k0 + rk < K;
+        const unsigned int ao = a_in ? a_voff + i * a_step : kNowhere, bo = b_in ? b_voff + i * b_step : kNowhere;
+        ra[set][i] = __builtin_bit_cast(double2_t, __builtin_amdgcn_raw_buffer_load_b128(pa, ao, sa, 0));
+        rb[set][i] = __builtin_bit_cast(double2_t, __builtin_amdgcn_raw_buffer_load_b128(pb, bo, sb, 0));
       }
       return;
     }
@@ -122,70 +148,131 @@ void gemm_f64_kernel(int M, int N, int K, const double* __restrict__ A, int lda,
   // this workgroup's piece of the contraction; request() and the loop below see its end as K
   const int k_begin = piece_begin;
   K = piece_end;
-  if (part != nullptr) {  // piece z parks [M][N] at part + z * M * N
-    C = part + (size_t)blockIdx.z * M * N;
+  int row0 = m0, col0 = n0, rows = M, cols = N;
+  if (cut && chunks) {  // piece z parks [M][N] at part + z * M * N
+    C = part + (size_t)piece * M * N;
     ldc = N;
     accumulate = 0;
+  } else if (cut) {  // a tile's pieces park [64][64] one behind the other
+    C = part + ((size_t)(tile - plan.whole) * plan.pieces + piece) * DM * DN;
+    ldc = DN;
+    row0 = col0 = accumulate = 0;
+    rows = DM;
+    cols = DN;
   }
-  // Panel p lies in buffer p % 2; at its turn the panel behind it is parked in the other buffer,
-  // which everybody has finished with, and the one three behind requested.
-  auto panel = [&](auto parity, int k0) {
-    constexpr int P = decltype(parity)::value;
-    if (k0 + DK < K) park(P ^ 1, P ^ 1);
-    if (k0 + 3 * DK < K) request(P ^ 1, k0 + 3 * DK);
-    const double* as = reinterpret_cast<const double*>(panels[P][0]);
-    const double* bs = reinterpret_cast<const double*>(panels[P][1]);
+  // The operands of an instruction group are read one group ahead: a wavefront issues in order, so a read behind the
+  // group before it comes back when the matrix cores have run dry.  between(g): what is issued behind group g.
+  auto multiply = [&](int buffer, auto&& between) {
+    const double* as = reinterpret_cast<const double*>(panels[buffer][0]);
+    const double* bs = reinterpret_cast<const double*>(panels[buffer][1]);
+    double a[2][2], b[2][2];
+    auto read = [&](int g) {
+      const int k = 4 * g + (lane >> 4), o = lane & 15;
 #pragma unroll
-    for (int kk = 0; kk < DK; kk += 4) {
-      const int k = kk + (lane >> 4), o = lane & 15;
-      const double a0 = as[panel_at(k, wm + o)], a1 = as[panel_at(k, wm + 16 + o)];
-      const double b0 = bs[panel_at(k, wn + o)], b1 = bs[panel_at(k, wn + 16 + o)];
-      acc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b0, acc[0][0], 0, 0, 0);
-      acc[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b1, acc[0][1], 0, 0, 0);
-      acc[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b0, acc[1][0], 0, 0, 0);
-      acc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b1, acc[1][1], 0, 0, 0);
+      for (int i = 0; i < 2; ++i) {
+        a[g & 1][i] = as[panel_at(k, wm + 16 * i + o)];
+        b[g & 1][i] = bs[panel_at(k, wn + 16 * i + o)];
+      }
+    };
+    read(0);
+#pragma unroll
+    for (int g = 0; g < DK / 4; ++g) {
+      if (g + 1 < DK / 4) read(g + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[g & 1][i], b[g & 1][j], acc[i][j], 0, 0, 0);
+      between(g);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    __syncthreads();
   };
-  request(0, k_begin);
-  if (k_begin + DK < K) request(1, k_begin + DK);
-  park(0, 0);
-  if (k_begin + 2 * DK < K) request(0, k_begin + 2 * DK);
-  __syncthreads();
-  for (int k0 = k_begin; k0 < K; k0 += 2 * DK) {
-    panel(std::integral_constant<int, 0>{}, k0);
-    if (k0 + DK < K) panel(std::integral_constant<int, 1>{}, k0 + DK);
-  }
+  // Panel p lies in buffer p % 2; at its turn the panel behind it is parked in the other buffer,
+  // which everybody has finished with, and the one three behind requested.  Without a branch (behind the last panel
+  // that one is read again, for nobody): with one the compiler cannot tell which loads a panel waits for, and waited
+  // for all of them, and read the operands of a group when its instructions were due.
+  // (6400 x 2048 x 512 271 -> 262 us, 512 x 2048 x 6400 296 -> 277, with A transposed 278 -> 258.)
+  auto run = [&](auto fast_c) {
+    const int last = k_begin + (K - k_begin - 1) / DK * DK;
+    auto panel = [&](auto parity, int k0) {
+      constexpr int P = decltype(parity)::value;
+      multiply(P, [&](int g) {
+        if (g == 1) park(P ^ 1, P ^ 1);
+        if (g == 3) request(fast_c, P ^ 1, k0 + 3 * DK < last ? k0 + 3 * DK : last);
+      });
+      __syncthreads();
+    };
+    request(fast_c, 0, k_begin);
+    request(fast_c, 1, k_begin + DK < last ? k_begin + DK : last);
+    park(0, 0);
+    request(fast_c, 0, k_begin + 2 * DK < last ? k_begin + 2 * DK : last);
+    __syncthreads();
+    int k0 = k_begin;
+    for (; k0 + DK < K; k0 += 2 * DK) {
+      panel(std::integral_constant<int, 0>{}, k0);
+      panel(std::integral_constant<int, 1>{}, k0 + DK);
+    }
+    if (k0 < K) multiply(0, [](int) {});
+  };
+  if (!fast) run(std::integral_constant<int, kSingle>{});
+  else if ((K - k_begin) % DK == 0) run(std::integral_constant<int, kWhole>{});
+  else run(std::integral_constant<int, kPairs>{});
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
     for (int b = 0; b < 2; ++b)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int gm = m0 + wm + 16 * a + 4 * r + (lane >> 4);
-        const int gn = n0 + wn + 16 * b + (lane & 15);
-        if (gm < M && gn < N) {
+        const int gm = row0 + wm + 16 * a + 4 * r + (lane >> 4);
+        const int gn = col0 + wn + 16 * b + (lane & 15);
+        if (gm < rows && gn < cols) {
           double* p = C + (size_t)gm * ldc + gn;
           *p = accumulate ? *p + acc[a][b][r] : acc[a][b][r];
         }
       }
 }
 
-// C (+)= the pieces of every element, added in index order.
+// C (+)= the pieces of every element of the cut tiles, added in index order.  A workgroup takes 16 rows of a tile, a
+// thread four columns.
 __global__ __launch_bounds__(256)
-void gemm_f64_reduce_kernel(int M, int N, int pieces, const double* __restrict__ part,
+void gemm_f64_reduce_kernel(int M, int N, F64Plan plan, int tiles_n, const double* __restrict__ part,
                             double* __restrict__ C, int ldc, int accumulate) {
-  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= (size_t)M * N) return;
-  double s = part[i];
-  for (int z = 1; z < pieces; ++z) s += part[(size_t)z * M * N + i];
-  double* out = C + (i / N) * ldc + i % N;
-  *out = accumulate ? *out + s : s;
+  const int tile = plan.whole + blockIdx.x;
+  const int r = blockIdx.y * 16 + (threadIdx.x >> 4), c = (threadIdx.x & 15) * 4;
+  const int row = tile / tiles_n * DM + r, col = tile % tiles_n * DN + c;
+  if (row >= M || col >= N) return;
+  const double* p = part + (size_t)blockIdx.x * plan.pieces * DM * DN + r * DN + c;
+  double4_t s = *reinterpret_cast<const double4_t*>(p);
+  for (int z = 1; z < plan.pieces; ++z) s += *reinterpret_cast<const double4_t*>(p + (size_t)z * DM * DN);
+  double* out = C + (size_t)row * ldc + col;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (col + i < N) out[i] = accumulate ? out[i] + s[i] : s[i];
 }
 
-// Pieces a product is cut into along K: as many as fill about one workgroup per CU, a piece
-// keeping at least 4 panels of the contraction; products of 128 tiles and more are not cut.
-void plan_f64(int M, int N, int K, int* pieces, int* k_per_piece) {
+// Whole tiles for full rounds of one per CU (a CU holds two workgroups, which share its matrix cores); the tiles of the
+// last, partial round are cut along K into pieces that make about two per CU, a piece keeping at least 8 panels of the
+// contraction (its first panel's load and its 64 KiB of partial results show below that).  A last round of more than
+// three quarters of the CUs has too little to give: stays whole.  A product of no more tiles than CUs is all cut, to
+// pieces of at least 4 panels: with one workgroup per CU its barriers and first loads show (512 x 2048 x 6400, 256
+// tiles: 258 us whole, 238 in two pieces; 6400 x 512 x 2048, 800 tiles: 295 whole, 222 with the last 32 in 8).
+F64Plan plan_f64(int M, int N, int K) {
+  const long long tiles = (long long)((M + DM - 1) / DM) * ((N + DN - 1) / DN);
+  const long long cus = device_cu_count() > 0 ? device_cu_count() : 256;
+  long long whole = tiles > cus ? tiles / cus * cus : 0;
+  const long long rest = tiles - whole;
+  long long s = rest > 0 ? 2 * cus / rest : 1;
+  const long long most = K / ((whole > 0 ? 8 : 4) * DK);
+  s = s < most ? s : most;
+  s = s < 64 ? s : 64;
+  if (s <= 1 || (whole > 0 && 4 * rest > 3 * cus)) return F64Plan{(int)tiles, 1, K};
+  int per = (int)((K + s - 1) / s);
+  per = (per + DK - 1) / DK * DK;
+  return F64Plan{(int)whole, (K + per - 1) / per, per};
+}
+// The same for a consumer that adds the pieces itself: all tiles, about one piece per CU.
+F64Plan plan_f64_chunks(int M, int N, int K) {
   const long long tiles = (long long)((M + DM - 1) / DM) * ((N + DN - 1) / DN);
   int s = 1;
   if (tiles < 128) {
@@ -197,8 +284,11 @@ void plan_f64(int M, int N, int K, int* pieces, int* k_per_piece) {
   }
   int per = (K + s - 1) / s;
   per = (per + DK - 1) / DK * DK;
-  *k_per_piece = per;
-  *pieces = (K + per - 1) / per;
+  return F64Plan{0, (K + per - 1) / per, per};
+}
+size_t f64_piece_bytes(const F64Plan& plan, int M, int N) {
+  const long long tiles = (long long)((M + DM - 1) / DM) * ((N + DN - 1) / DN);
+  return plan.pieces > 1 ? (size_t)(tiles - plan.whole) * plan.pieces * DM * DN * sizeof(double) : 0;
 }
 
 // ---- The product of one step of the step-wise regime: at most 64 rows (the batch), a few
@@ -346,17 +436,20 @@ bool skinny_f64_applies(int M, int N, int K, int lda, int ldb) {
 
 }  // namespace
 
-size_t gemm_f64_scratch_bytes(int M, int N, int K) {
-  if (M <= 0 || N <= 0 || K <= 0) return 0;
-  int pieces, per;
-  plan_f64(M, N, K, &pieces, &per);
-  size_t tiled = pieces > 1 ? (size_t)pieces * M * N * sizeof(double) : 0;
+// *need: what a product takes at least (its chunks, where a consumer adds them); *wish: with the pieces of a cut one.
+void gemm_f64_scratch_bytes(int M, int N, int K, size_t* need, size_t* wish) {
+  *need = *wish = 0;
+  if (M <= 0 || N <= 0 || K <= 0) return;
+  const F64Plan chunked = plan_f64_chunks(M, N, K);
+  if (chunked.pieces > 1) *need = (size_t)chunked.pieces * M * N * sizeof(double);
   if (M <= 64) {
+    int pieces, per;
     plan_skinny_f64(M, N, K, &pieces, &per);
     const size_t skinny = (size_t)pieces * M * N * sizeof(double);
-    tiled = tiled > skinny ? tiled : skinny;
+    *need = *need > skinny ? *need : skinny;
   }
-  return tiled;
+  const size_t cut = f64_piece_bytes(plan_f64(M, N, K), M, N);
+  *wish = *need > cut ? *need : cut;
 }
 
 // The partial results of a cut product lie `scratch_offset` bytes (a multiple of 16) into the
@@ -365,28 +458,33 @@ int gemm_f64(hipStream_t stream, bool trans_a, int M, int N, int K, const double
              const double* B, int ldb, double* C, int ldc, bool accumulate, size_t scratch_offset) {
   HASTE_HIP_REQUIRE(M > 0 && N > 0 && K > 0 && A && B && C);
   HASTE_HIP_REQUIRE(lda >= (trans_a ? M : K) && ldb >= N && ldc >= N);
-  int pieces, per;
-  plan_f64(M, N, K, &pieces, &per);
-  const dim3 grid((unsigned)((N + DN - 1) / DN), (unsigned)((M + DM - 1) / DM), (unsigned)pieces);
-  HASTE_HIP_REQUIRE(grid.y < 65536u);
+  const int tiles_n = (N + DN - 1) / DN;
+  const long long tiles = (long long)((M + DM - 1) / DM) * tiles_n;
+  HASTE_HIP_REQUIRE(tiles < (1ll << 30));
+  F64Plan plan = plan_f64(M, N, K);
   double* part = nullptr;
-  if (pieces > 1) {
+  if (plan.pieces > 1) {  // not cut without room for the pieces (a caller's own buffer, a capture, a buffer in use)
+    const size_t bytes = scratch_offset + f64_piece_bytes(plan, M, N);
+    bool room;
+    HASTE_HIP_PROPAGATE(workspace_has_room(stream, bytes, &room));
     Workspace ws;
-    HASTE_HIP_PROPAGATE(get_workspace(stream, scratch_offset + (size_t)pieces * M * N * sizeof(double), &ws));
-    part = reinterpret_cast<double*>(reinterpret_cast<char*>(ws.scratch) + scratch_offset);
+    HASTE_HIP_PROPAGATE(get_workspace(stream, room && scratch_offset == 0 ? bytes : 0, &ws));
+    if (ws.scratch_bytes >= bytes) part = reinterpret_cast<double*>(reinterpret_cast<char*>(ws.scratch) + scratch_offset);
+    else plan = F64Plan{(int)tiles, 1, K};
   }
+  const int rest = (int)(tiles - plan.whole);
+  const dim3 grid((unsigned)(plan.whole + (long long)rest * plan.pieces));
   ScopedKernelTimer timer("gemm_f64", stream);
   if (trans_a)
-    gemm_f64_kernel<true><<<grid, dim3(256), 0, stream>>>(M, N, K, A, lda, B, ldb, C, ldc, accumulate, per, part,
+    gemm_f64_kernel<true><<<grid, dim3(256), 0, stream>>>(M, N, K, A, lda, B, ldb, C, ldc, accumulate, plan, tiles_n, part, 0,
                                                           panels_fit(true, M, N, K, lda, ldb));
   else
-    gemm_f64_kernel<false><<<grid, dim3(256), 0, stream>>>(M, N, K, A, lda, B, ldb, C, ldc, accumulate, per, part,
+    gemm_f64_kernel<false><<<grid, dim3(256), 0, stream>>>(M, N, K, A, lda, B, ldb, C, ldc, accumulate, plan, tiles_n, part, 0,
                                                            panels_fit(false, M, N, K, lda, ldb));
   HASTE_HIP_TRY(hipGetLastError());
-  if (pieces > 1) {
-    const size_t n = (size_t)M * N;
-    gemm_f64_reduce_kernel<<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream>>>(M, N, pieces, part, C, ldc,
-                                                                                         accumulate ? 1 : 0);
+  if (rest > 0) {
+    gemm_f64_reduce_kernel<<<dim3((unsigned)rest, DM / 16), dim3(256), 0, stream>>>(M, N, plan, tiles_n, part, C, ldc,
+                                                                                     accumulate ? 1 : 0);
     HASTE_HIP_TRY(hipGetLastError());
   }
   return HASTE_HIP_OK;
@@ -401,10 +499,11 @@ int gemm_f64_chunks(hipStream_t stream, int M, int N, int K, const double* A, in
   *chunks = 0;
   HASTE_HIP_REQUIRE(M > 0 && N > 0 && K > 0 && A && B);
   HASTE_HIP_REQUIRE(lda >= K && ldb >= N);
-  int pieces, per;
+  int pieces, per = 0;
   const bool skinny = skinny_f64_applies(M, N, K, lda, ldb);
+  const F64Plan plan = plan_f64_chunks(M, N, K);
   if (skinny) plan_skinny_f64(M, N, K, &pieces, &per);
-  else plan_f64(M, N, K, &pieces, &per);
+  else pieces = plan.pieces;
   if (!skinny && pieces <= 1) return HASTE_HIP_OK;
   Workspace ws;
   HASTE_HIP_PROPAGATE(get_workspace(stream, scratch_offset + (size_t)pieces * M * N * sizeof(double), &ws));
@@ -417,10 +516,10 @@ int gemm_f64_chunks(hipStream_t stream, int M, int N, int K, const double* A, in
     else skinny_f64_kernel<4><<<grid, dim3(256), 0, stream>>>(M, N, K, A, lda, B, ldb, part, per);
     HASTE_HIP_TRY(hipGetLastError());
   } else {
-    const dim3 grid((unsigned)((N + DN - 1) / DN), (unsigned)((M + DM - 1) / DM), (unsigned)pieces);
-    HASTE_HIP_REQUIRE(grid.y < 65536u);
+    const int tiles_n = (N + DN - 1) / DN;
+    const dim3 grid((unsigned)((M + DM - 1) / DM * tiles_n * pieces));
     ScopedKernelTimer timer("gemm_f64", stream);
-    gemm_f64_kernel<false><<<grid, dim3(256), 0, stream>>>(M, N, K, A, lda, B, ldb, nullptr, 0, 0, per, part,
+    gemm_f64_kernel<false><<<grid, dim3(256), 0, stream>>>(M, N, K, A, lda, B, ldb, nullptr, 0, 0, plan, tiles_n, part, 1,
                                                            panels_fit(false, M, N, K, lda, ldb));
     HASTE_HIP_TRY(hipGetLastError());
   }

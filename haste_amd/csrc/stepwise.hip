@@ -26,7 +26,7 @@ namespace haste_hip {
 
 int gemm_f64(hipStream_t stream, bool trans_a, int M, int N, int K, const double* A, int lda,
              const double* B, int ldb, double* C, int ldc, bool accumulate, size_t scratch_offset);
-size_t gemm_f64_scratch_bytes(int M, int N, int K);
+void gemm_f64_scratch_bytes(int M, int N, int K, size_t* need, size_t* wish);
 int gemm_f64_chunks(hipStream_t stream, int M, int N, int K, const double* A, int lda, const double* B,
                     int ldb, size_t scratch_offset, const double** partial, int* chunks);
 // recurrent_f64.hip: all steps of the double LSTM and GRU in one launch.
@@ -96,10 +96,24 @@ inline int gemm(hipStream_t s, bool ta, int M, int N, int K, const half_t* A, in
                 const half_t* B, int ldb, half_t* C, int ldc, bool acc, size_t) {
   return gemm_f16(s, ta, M, N, K, A, lda, B, ldb, C, ldc, acc);
 }
-template <typename T> size_t gemm_room(int M, int N, int K);
-template <> size_t gemm_room<float>(int M, int N, int K) { return gemm_f32_scratch_bytes(M, N, K); }
-template <> size_t gemm_room<double>(int M, int N, int K) { return gemm_f64_scratch_bytes(M, N, K); }
-template <> size_t gemm_room<half_t>(int, int, int) { return 0; }
+// Scratch of a product: what it takes, and what it is faster with.
+struct Room {
+  size_t need, wish;
+};
+inline Room max2(Room a, Room b) {
+  return Room{a.need > b.need ? a.need : b.need, a.wish > b.wish ? a.wish : b.wish};
+}
+template <typename T> Room gemm_room(int M, int N, int K);
+template <> Room gemm_room<float>(int M, int N, int K) {
+  const size_t bytes = gemm_f32_scratch_bytes(M, N, K);
+  return Room{bytes, bytes};
+}
+template <> Room gemm_room<double>(int M, int N, int K) {
+  Room room;
+  gemm_f64_scratch_bytes(M, N, K, &room.need, &room.wish);
+  return room;
+}
+template <> Room gemm_room<half_t>(int, int, int) { return Room{0, 0}; }
 
 // A step's product as its consumer reads it: either one finished matrix (chunks == 1,
 // stride == 0) or the K chunks of the small-batch streaming kernel, which the consumer adds in
@@ -285,9 +299,11 @@ struct Scratch {
 };
 inline size_t padded(size_t bytes) { return (bytes + 255) / 256 * 256; }
 
-int open_scratch(hipStream_t stream, size_t own_bytes, size_t gemm_bytes, Scratch* sc) {
+int open_scratch(hipStream_t stream, size_t own_bytes, Room gemm, Scratch* sc) {
   Workspace ws;
-  HASTE_HIP_PROPAGATE(get_workspace(stream, own_bytes + gemm_bytes + 256, &ws));
+  bool room;
+  HASTE_HIP_PROPAGATE(workspace_has_room(stream, own_bytes + gemm.wish + 256, &room));
+  HASTE_HIP_PROPAGATE(get_workspace(stream, own_bytes + (room ? gemm.wish : gemm.need) + 256, &ws));
   sc->base = reinterpret_cast<char*>(ws.scratch);
   sc->used = 0;
   sc->own = own_bytes;
@@ -821,7 +837,6 @@ int effective_r(hipStream_t stream, size_t n, const T* R, const T* dc_mask, floa
   return HASTE_HIP_OK;
 }
 
-inline size_t max2(size_t a, size_t b) { return a > b ? a : b; }
 
 template <typename T>
 int lstm_forward_steps(hipStream_t stream, int training, int steps, int N, int C, int H,
@@ -830,9 +845,9 @@ int lstm_forward_steps(hipStream_t stream, int training, int steps, int N, int C
                        const T* dc_mask, float dc_scale) {
   const size_t NH = (size_t)N * H, N4H = NH * 4, r_count = (size_t)H * 4 * H;
   size_t own = padded(N4H * sizeof(T)) + (dc_mask ? padded(r_count * sizeof(T)) : 0);
-  const size_t room = max2(gemm_room<T>(steps * N, 4 * H, C), gemm_room<T>(N, 4 * H, H));
+  const Room room = max2(gemm_room<T>(steps * N, 4 * H, C), gemm_room<T>(N, 4 * H, H));
   size_t tiles = 0;
-  HASTE_HIP_PROPAGATE(one_launch_bytes<T>(stream, 1, 4, steps, N, H, own + room, &tiles));
+  HASTE_HIP_PROPAGATE(one_launch_bytes<T>(stream, 1, 4, steps, N, H, own + room.need, &tiles));
   own += tiles;
   Scratch sc;
   HASTE_HIP_PROPAGATE(open_scratch(stream, own, room, &sc));
@@ -866,10 +881,10 @@ int lstm_backward_steps(hipStream_t stream, int steps, int N, int C, int H, cons
   const size_t NH = (size_t)N * H, N4H = NH * 4;
   const int TN = steps * N;
   const size_t sums = column_sum_bytes<T>((size_t)TN, 4 * H);
-  size_t room = max2(gemm_room<T>(N, H, 4 * H), gemm_room<T>(C, 4 * H, TN));
+  Room room = max2(gemm_room<T>(N, H, 4 * H), gemm_room<T>(C, 4 * H, TN));
   room = max2(room, max2(gemm_room<T>(H, 4 * H, TN), gemm_room<T>(TN, C, 4 * H)));
   size_t tiles = 0;
-  HASTE_HIP_PROPAGATE(one_launch_bytes<T>(stream, 4, 1, steps, N, H, sums + room, &tiles));
+  HASTE_HIP_PROPAGATE(one_launch_bytes<T>(stream, 4, 1, steps, N, H, sums + room.need, &tiles));
   Scratch sc;
   HASTE_HIP_PROPAGATE(open_scratch(stream, sums + tiles, room, &sc));
   void* partial = sc.take<char>(sums);
@@ -905,9 +920,9 @@ int gru_forward_steps(hipStream_t stream, int training, int steps, int N, int C,
                       float dc_scale) {
   const size_t NH = (size_t)N * H, N3H = NH * 3, N4H = NH * 4, r_count = (size_t)H * 3 * H;
   size_t own = padded(N3H * sizeof(T)) + (dc_mask ? padded(r_count * sizeof(T)) : 0);
-  const size_t room = max2(gemm_room<T>(steps * N, 3 * H, C), gemm_room<T>(N, 3 * H, H));
+  const Room room = max2(gemm_room<T>(steps * N, 3 * H, C), gemm_room<T>(N, 3 * H, H));
   size_t tiles = 0;
-  HASTE_HIP_PROPAGATE(one_launch_bytes<T>(stream, 1, 3, steps, N, H, own + room, &tiles));
+  HASTE_HIP_PROPAGATE(one_launch_bytes<T>(stream, 1, 3, steps, N, H, own + room.need, &tiles));
   own += tiles;
   Scratch sc;
   HASTE_HIP_PROPAGATE(open_scratch(stream, own, room, &sc));
@@ -940,10 +955,10 @@ int gru_backward_steps(hipStream_t stream, int steps, int N, int C, int H, const
   const size_t NH = (size_t)N * H, N3H = NH * 3, N4H = NH * 4;
   const int TN = steps * N;
   const size_t sums = column_sum_bytes<T>((size_t)TN, 3 * H);
-  size_t room = max2(gemm_room<T>(N, H, 3 * H), gemm_room<T>(C, 3 * H, TN));
+  Room room = max2(gemm_room<T>(N, H, 3 * H), gemm_room<T>(C, 3 * H, TN));
   room = max2(room, max2(gemm_room<T>(H, 3 * H, TN), gemm_room<T>(TN, C, 3 * H)));
   size_t tiles = 0;
-  HASTE_HIP_PROPAGATE(one_launch_bytes<T>(stream, 3, 1, steps, N, H, sums + room, &tiles));
+  HASTE_HIP_PROPAGATE(one_launch_bytes<T>(stream, 3, 1, steps, N, H, sums + room.need, &tiles));
   Scratch sc;
   HASTE_HIP_PROPAGATE(open_scratch(stream, sums + tiles, room, &sc));
   void* partial = sc.take<char>(sums);
@@ -1018,7 +1033,7 @@ int ln_lstm_backward_steps(hipStream_t stream, int steps, int N, int C, int H, c
   const int TN = steps * N;
   const size_t part_bytes = column_sum_bytes<T>((size_t)TN, (size_t)N, 4 * H);
   const size_t own = part_bytes + padded((size_t)TN * 2 * sizeof(T));
-  size_t room = max2(gemm_room<T>(N, H, 4 * H), gemm_room<T>(C, 4 * H, TN));
+  Room room = max2(gemm_room<T>(N, H, 4 * H), gemm_room<T>(C, 4 * H, TN));
   room = max2(room, max2(gemm_room<T>(H, 4 * H, TN), gemm_room<T>(TN, C, 4 * H)));
   Scratch sc;
   HASTE_HIP_PROPAGATE(open_scratch(stream, own, room, &sc));
@@ -1099,7 +1114,7 @@ int ln_gru_backward_steps(hipStream_t stream, int steps, int N, int C, int H, co
   const int TN = steps * N;
   const size_t part_bytes = column_sum_bytes<T>((size_t)TN, (size_t)N, 3 * H);
   const size_t own = part_bytes + padded((size_t)TN * 2 * sizeof(T));
-  size_t room = max2(gemm_room<T>(N, H, 3 * H), gemm_room<T>(C, 3 * H, TN));
+  Room room = max2(gemm_room<T>(N, H, 3 * H), gemm_room<T>(C, 3 * H, TN));
   room = max2(room, max2(gemm_room<T>(H, 3 * H, TN), gemm_room<T>(TN, C, 3 * H)));
   Scratch sc;
   HASTE_HIP_PROPAGATE(open_scratch(stream, own, room, &sc));
@@ -1228,7 +1243,7 @@ int layer_norm_backward_wide(hipStream_t stream, int rows, int dim, const float*
                              float* dbeta) {
   const size_t part_bytes = column_sum_bytes<float>((size_t)rows, dim);
   Scratch sc;
-  HASTE_HIP_PROPAGATE(open_scratch(stream, part_bytes + padded((size_t)rows * 2 * sizeof(float)), 0, &sc));
+  HASTE_HIP_PROPAGATE(open_scratch(stream, part_bytes + padded((size_t)rows * 2 * sizeof(float)), Room{0, 0}, &sc));
   void* partial = sc.take<char>(part_bytes);
   float* stats = sc.take<float>((size_t)rows * 2);
   HASTE_HIP_PROPAGATE(ln_forward_rows<float>(stream, (size_t)rows, dim, gamma, nullptr, x, nullptr, stats));
@@ -1454,7 +1469,7 @@ int haste_hip_layer_norm_backward_f64(int rows, int dim, const double* gamma, co
   hipStream_t stream = as_stream(stream_);
   const size_t part_bytes = column_sum_bytes<double>((size_t)rows, dim);
   Scratch sc;
-  HASTE_HIP_PROPAGATE(open_scratch(stream, part_bytes + padded((size_t)rows * 2 * sizeof(double)), 0, &sc));
+  HASTE_HIP_PROPAGATE(open_scratch(stream, part_bytes + padded((size_t)rows * 2 * sizeof(double)), Room{0, 0}, &sc));
   void* partial = sc.take<char>(part_bytes);
   double* stats = sc.take<double>((size_t)rows * 2);
   ScopedKernelTimer timer("layer_norm_backward_f64", stream);

@@ -107,6 +107,39 @@ def test_f64_gemm_and_transpose(trans_a, M, N, K, accumulate):
     assert torch.equal(t, dev64(a).t().contiguous())
 
 
+@pytest.mark.parametrize("trans_a,M,N,K", [
+    # the last tiles cut behind whole ones, loads in pairs of whole and ragged panels and single
+    (False, 1100, 1024, 512), (True, 1030, 1022, 770), (False, 1041, 1021, 515), (True, 1088, 1021, 516),
+    # all tiles cut; a last round that fills the chip and is not; pairs in a panel of less than 32
+    (True, 512, 2048, 512), (False, 1920, 1024, 512), (False, 70, 66, 2), (True, 66, 70, 30)])
+@pytest.mark.parametrize("room", [True, False])
+def test_f64_gemm_in_pieces(trans_a, M, N, K, room):
+    """Error of a sum of K products in double, in any order: below K * 2^-53 of the sum of their magnitudes.  Without
+    room for the pieces (a lent buffer of 128 KiB) a product is not cut, and is right."""
+    from haste_amd import ops
+    import torch
+    r = np.random.default_rng(M + N + K)
+    a = r.standard_normal((K, M) if trans_a else (M, K))
+    b = r.standard_normal((K, N))
+    c0 = r.standard_normal((M, N))
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        lent = None if room else torch.empty(128 * 1024, dtype=torch.uint8, device="cuda")
+        ops.set_workspace(lent)
+        try:
+            wide = torch.full((M, N + 3), 7.0, dtype=torch.float64, device="cuda")   # what lies beside C stays
+            wide[:, :N] = dev64(c0)
+            ops.gemm(dev64(a), dev64(b), out=wide[:, :N], trans_a=trans_a, accumulate=True)
+        finally:
+            s.synchronize()
+            ops.set_workspace(None)
+    at = a.T if trans_a else a
+    out = host(wide)
+    bound = K * 2.0 ** -53 * (np.abs(at) @ np.abs(b) + np.abs(c0))
+    assert (np.abs(out[:, :N] - (at @ b + c0)) <= 2 * bound).all()   # twice: the reference's own sum
+    assert (out[:, N:] == 7.0).all()
+
+
 def test_f64_layers_match_torch_nn():
     """haste_amd.LSTM / GRU in double against torch.nn.LSTM / GRU in double on the CPU."""
     import torch
