@@ -4,32 +4,36 @@
 // most of its time is theirs: at N = 64, H = 512 the pair takes 15 us, and 9.3 us are left when
 // its product loads no operand at all; the fp64 matrix cores need 1.7 us.  Here a workgroup keeps
 // its columns of the weights in registers for the whole launch, and what the steps exchange goes
-// through two alternating tiles in memory behind the group's step barrier.
-//   * A group is 16 batch rows (one v_mfma_f64_16x16x4_f64 row tile); its workgroups own HS hidden
-//     units each.  Forward: all gates of 8 units (16 when the chip would not hold the grid), the
+// through tiles in memory, behind the group's step barrier or polled (polled64).
+//   * A group is 8 or 16 batch rows; its workgroups own HS hidden units each.  Forward: all gates of 8 or 16 units, the
 //     contraction runs over h.  Backward: 16 units of dh, the contraction over all gate gradients.
+//   * 16 rows: v_mfma_f64_16x16x4_f64.  8 rows: twice v_mfma_f64_4x4x4_4b_f64, four blocks of 4 x 4 at the same rate
+//     (16.7 cycles for 512 flops, 70 for 2048), so that twice the groups share the work and 64 rows fill the eight
+//     XCDs with a group each.  Forward the blocks are 16 columns and read the same A; backward, where A is the larger
+//     part, they are 16 k, and the blocks' sums are added once a step.
 //   * The four wavefronts take a quarter of the contraction each: at most KS instructions of four k,
 //     a lane holding B[k = lane / 16][column = lane % 16] of every one of them and column tile.
-//   * Exchange tile: A operand of instruction s at ((s / 2) * 64 + lane) * 2 + s % 2, so that a
-//     wavefront's loads are consecutive 16-byte words.  k = gate * Hp + unit, Hp = H rounded up to 4.
+//   * Exchange tile: what a lane needs next lies in one 16-byte word (two instructions of 16 rows, rows r and r + 4 of
+//     8), a wavefront's loads are consecutive.  k = gate * Hp + unit, Hp = H rounded up to 4.
 //   * The wavefronts' partial tiles are added through LDS in wavefront order; a thread then owns one
 //     (row, unit), whose state stays in its registers.
 //   * The inputs of the next step are requested behind the last operand load of a product, so that
 //     they neither delay an operand nor a look at the barrier's flags.
-// Bound: the chain barrier - operand load - product - pointwise math of a step.  The matrix cores need
-// 1.9 us of a forward step and, with only 128 workgroups of 16 columns, 3.9 us of a backward one.
-// Measured per step at N = 64, H = 512, LSTM, step-wise -> here: forward 14.7 -> 6.1 us, backward
-// 14.9 -> 8.4 us.  Whole training passes, T = 100: LSTM 4.30 -> 2.72 ms (with gemm_f64's change), GRU
-// 4.23 -> 2.37; LSTM N = 16, H = 256 1.54 -> 1.01; N = 32, H = 768 4.22 -> 3.68; LSTM inference N = 1 0.83 -> 0.64.
+// Bound: the chain exchange - operand load - product - pointwise math of a step (a tanh takes 0.3 us, two follow each
+// other).  The matrix cores need 1.9 us of a step.
+// Measured per step at N = 64, H = 512, LSTM, step-wise -> 16 rows -> 8 rows: forward 14.7 -> 6.1 -> 5.3 us, backward
+// 14.9 -> 8.4 -> 5.5 us.  Whole training passes, 16 rows behind barriers -> now (with gemm_f64's changes), T = 100: LSTM
+// N = 64, H = 512 2.70 -> 2.27 ms, GRU 2.33 -> 1.85; N = 64, H = 128 0.81 -> 0.67; GRU N = 5, H = 64 0.52 -> 0.44;
+// T = 50: N = 32, H = 768 1.77 -> 1.49, N = 40, H = 700 2.52 -> 1.59.
 #include "recurrent.h"
 
 namespace haste_hip {
 namespace {
 
+typedef unsigned int uint2_t __attribute__((ext_vector_type(2)));
 typedef double double2_t __attribute__((ext_vector_type(2)));
 typedef double double4_t __attribute__((ext_vector_type(4)));
 constexpr unsigned int kNowhere64 = 0x7ffffff0u;  // beyond any buffer resource's range: the load returns zeros
-constexpr int kRows64 = 16;
 constexpr int kChunk64 = 8;  // instructions whose operands are requested together
 constexpr int kAgentScope64 = 16;  // the sc1 bit of a load's cache policy
 
@@ -44,8 +48,28 @@ __device__ __forceinline__ void store_exchanged_d(const GroupSync& g, double* p,
                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Polled tiles (recurrent.h): what has not been published holds a bit pattern that no producer stores.  An element's
+// eight bytes arrive together: they are one aligned store.
+__device__ __forceinline__ double unwritten_d() { return __builtin_bit_cast(double, ~0ull); }
+__device__ __forceinline__ double publishable_d(double v) {
+  return __builtin_bit_cast(unsigned long long, v) == ~0ull ? __builtin_bit_cast(double, 0x7ff8000000000000ull) : v;
+}
+__device__ __forceinline__ bool written_d(double2_t a) {
+  const double x = a[0], y = a[1];  // bit_cast of an element itself takes the vector's first
+  return __builtin_bit_cast(unsigned long long, x) != ~0ull && __builtin_bit_cast(unsigned long long, y) != ~0ull;
+}
+template <int N>
+__device__ __forceinline__ bool all_written_d(const double2_t (&a)[N]) {
+  bool written = true;
+#pragma unroll
+  for (int i = 0; i < N; ++i) written = written && written_d(a[i]);
+  return __all(written) != 0;
+}
+
 // Where the A operand for contraction index k and batch row `row` of a group lies in its tile.
+template <int ROWS>
 __device__ __forceinline__ int exchange_index(int k, int row) {
+  if (ROWS == 8) return (k * 4 + (row & 3)) * 2 + (row >> 2);
   const int s = k >> 2;
   return ((s >> 1) * 64 + (k & 3) * 16 + row) * 2 + (s & 1);
 }
@@ -55,11 +79,11 @@ struct RecurrenceShape {
   int T, N, H;
   int kw;                 // instructions of a wavefront per step and column tile, a multiple of kChunk64
   const double* weights;  // [kIn * H][kOut * H]
-  double* exchange;       // [groups][2][4 * kw * 64]
+  double* exchange;       // [groups][kPolledTiles][16 * kw * rows of a group]
 };
 
 // A cell: its parameters, what a step reads of the caller's memory (Inputs, requested a step
-// ahead), what a thread carries from step to step, and the arithmetic of stepwise.hip's kernels.
+// ahead; prepare() does what needs nothing else while the workgroup waits for the others), what a thread carries from step to step, and the arithmetic of stepwise.hip's kernels.
 struct LstmForward64 {
   static constexpr bool kForward = true;
   static constexpr int kIn = 1, kOut = 4;
@@ -79,6 +103,7 @@ struct LstmForward64 {
     for (int g = 0; g < 4; ++g) bias[g] = p.b[g * p.H + j];
   }
   __device__ double initial(int) const { return h; }
+  __device__ void prepare(const Inputs&) {}
   __device__ static void request(const Params& p, int s, int n, int j, Inputs& in) {
     const size_t row = (size_t)s * p.N + n;
 #pragma unroll
@@ -134,6 +159,7 @@ struct GruForward64 {
     }
   }
   __device__ double initial(int) const { return h; }
+  __device__ void prepare(const Inputs&) {}
   __device__ static void request(const Params& p, int s, int n, int j, Inputs& in) {
     const size_t row = (size_t)s * p.N + n;
 #pragma unroll
@@ -173,13 +199,14 @@ struct LstmBackward64 {
     double *dh, *dc, *v;
   };
   struct Inputs { double gate[4], c, c_next, dh, dc, m; };
-  double dh, dc, grad[4];
+  double dh, dc, c_tanh, grad[4];
 
   __device__ void begin(const Params& p, size_t idx, int) {
     dh = p.dh[idx];
     dc = p.dc[idx];
   }
   __device__ double initial(int) const { return 0.0; }
+  __device__ void prepare(const Inputs& in) { c_tanh = tanh(in.c_next); }
   __device__ static void request(const Params& p, int s, int n, int j, Inputs& in) {
     const size_t row = (size_t)(p.T - 1 - s) * p.N + n, at = row * p.H + j;
 #pragma unroll
@@ -193,7 +220,6 @@ struct LstmBackward64 {
   __device__ void step(const Params& p, const Inputs& in, const double (&sum)[1]) {
     double dc_total = (p.dc_next != nullptr ? in.dc : 0.0) + dc;
     double dh_total = in.dh + (dh + sum[0]);
-    const double c_tanh = tanh(in.c_next);
     dh = 0.0;
     if (p.mask != nullptr) {
       dh = (1.0 - in.m) * dh_total;
@@ -233,6 +259,7 @@ struct GruBackward64 {
 
   __device__ void begin(const Params& p, size_t idx, int) { dh = p.dh[idx]; }
   __device__ double initial(int) const { return 0.0; }
+  __device__ void prepare(const Inputs&) {}
   __device__ static void request(const Params& p, int s, int n, int j, Inputs& in) {
     const size_t row = (size_t)(p.T - 1 - s) * p.N + n, at = row * p.H + j;
 #pragma unroll
@@ -281,26 +308,59 @@ constexpr int column_tiles64(int gates, int units) { return (gates * units + 15)
 // Of a wavefront's ks instructions per column tile, those whose weights lie in LDS: what leaves at
 // most 64 doubles per lane in registers (with all 128 of a backward step at H = 512 there, four chunks
 // of operands in flight are spilled: 12.7 us per step, two chunks 9.5, this 8.4), as far as LDS reaches beside the partial tiles.
-constexpr int lds_steps64(int ks, int ct) {
+constexpr int lds_steps64(int ks, int ct, int rows) {
   int steps = 0;
-  while ((ks - steps) * ct > 64 && (steps + kChunk64) * ct * 2048 + ct * 8192 + 16 <= (int)kMaxLdsBytes) steps += kChunk64;
+  while ((ks - steps) * ct > 64 && (steps + kChunk64) * ct * 2048 + ct * rows * 512 + 16 <= (int)kMaxLdsBytes) steps += kChunk64;
   return steps;
 }
-constexpr bool fits64(int ks, int ct) { return (ks - lds_steps64(ks, ct)) * ct <= 128; }
+constexpr bool fits64(int ks, int ct, int rows) { return (ks - lds_steps64(ks, ct, rows)) * ct <= 128; }
 // Partial tiles of the four wavefronts, one word for the role, the weights in LDS.
-constexpr size_t recurrence64_lds_bytes(int ks, int ct) { return (size_t)ct * 8192 + 16 + (size_t)lds_steps64(ks, ct) * ct * 2048; }
+constexpr size_t recurrence64_lds_bytes(int ks, int ct, int rows) {
+  return (size_t)ct * rows * 512 + 16 + (size_t)lds_steps64(ks, ct, rows) * ct * 2048;
+}
 
-template <class Cell, int HS, int KS>
+// Lanes of a row of 16: the value of the lane 4 * BLOCKS before (in a circle), BLOCKS = 1 only for lanes whose bit 2 is
+// set, the others the lane 4 behind: the neighbour block.
+template <int CTRL, int BANKS>
+__device__ __forceinline__ unsigned int moved(unsigned int old, unsigned int v) {
+  return (unsigned int)__builtin_amdgcn_update_dpp((int)old, (int)v, CTRL, 0xf, BANKS, false);
+}
+__device__ __forceinline__ double from_block(double v, bool two) {
+  const uint2_t x = __builtin_bit_cast(uint2_t, v);
+  uint2_t y;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    y[i] = two ? moved<0x128, 0xf>(x[i], x[i])                               // row_ror:8
+               : moved<0x12c, 0x5>(moved<0x124, 0xf>(x[i], x[i]), x[i]);     // row_ror:4, in blocks 0 and 2 row_ror:12
+  return __builtin_bit_cast(double, y);
+}
+
+// Polled tiles or the step barrier.  A look at a tile costs more the longer a wavefront's share of it is, and its chunks
+// arrive one after the other; the barrier costs a store's acknowledgement and a flag's round trip, more across XCDs.
+// Training passes, barrier / polled, ms: 8 rows, T = 100: N = 64 H = 128 0.785 / 0.670, N = 20 H = 256 (GRU) 0.744 / 0.691,
+// N = 37 H = 300 1.149 / 1.167, N = 64 H = 512 2.25 / 2.30 (inference 0.811 / 0.900); 16 rows: N = 128 H = 256
+// 1.29 / 1.25, T = 50 N = 32 H = 768 1.78 / 1.49, but inference with H = 768 0.462 / 0.492.
+constexpr bool polled64(bool forward, int ks, int rows) {
+  return rows == 16 ? !forward || ks <= 32 : ks <= (forward ? 16 : 64);
+}
+
+template <class Cell, int HS, int KS, int ROWS>
 __global__ __launch_bounds__(256, 1)
 void recurrence64_kernel(typename Cell::Params p) {
   constexpr int CT = column_tiles64(Cell::kOut, HS);
   constexpr int CHAINS = CT == 1 ? 2 : 1;  // accumulators per column tile: no instruction waits for the one before
-  constexpr int KL = lds_steps64(KS, CT), KR = KS - KL;
-  constexpr int RING = KS >= 4 * kChunk64 && CT == 1 ? 4 : 2;  // chunks of operands in registers (CT > 1: no gain)
+  constexpr int KL = lds_steps64(KS, CT, ROWS), KR = KS - KL;
+  constexpr bool kShort = ROWS == 8;
+  // Short tiles, blocks over k: "instruction" i stands for columns 4 * (i % 4) .. +3 and 16 k.
+  constexpr bool kBlocksOverK = kShort && CT == 1;
+  constexpr int LOADS = kBlocksOverK ? kChunk64 / 4 : kShort ? kChunk64 : kChunk64 / 2;  // 16-byte operand loads of a chunk
+  // chunks of operands in registers (CT > 1: no gain)
+  constexpr int RING = KS >= 4 * kChunk64 && CT == 1 ? (kShort && KS >= 8 * kChunk64 ? 8 : 4) : 2;
+  constexpr bool kPolled = polled64(Cell::kForward, KS, ROWS);
   // The chunk behind whose request those of the inputs go: the last that every kw served by this KS has.
   constexpr int kInputsBehind = smaller_steps64(KS) / kChunk64;
   extern __shared__ double partial[];
-  const Role role = take_role(p.ls, reinterpret_cast<unsigned int*>(partial + 4 * CT * 256));
+  const Role role = take_role(p.ls, reinterpret_cast<unsigned int*>(partial + CT * ROWS * 64));
   if (!role.active) return;
   GroupSync gs;
   group_sync_init(gs, p.ls, role);
@@ -309,17 +369,18 @@ void recurrence64_kernel(typename Cell::Params p) {
   const int H = p.H, Hp = rounded_up(H, 4), kw = p.kw;
 
   double w[KR][CT];
-  double2_t* w_lds = reinterpret_cast<double2_t*>(partial + 4 * CT * 256 + 2) + (size_t)wave * (KL / 2) * CT * 64 + lane;
+  double2_t* w_lds = reinterpret_cast<double2_t*>(partial + CT * ROWS * 64 + 2) + (size_t)wave * (KL / 2) * CT * 64 + lane;
   {
     const int row_len = Cell::kOut * H;
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<double*>(p.weights), 0, Cell::kIn * H * row_len * 8, 0x00020000);
 #pragma unroll
     for (int i = 0; i < KS; ++i) {
-      const int k = 4 * (wave * kw + i) + q, gate = k / Hp, unit = k % Hp;
+      const int k = kBlocksOverK ? 4 * wave * kw + 16 * (i / 4) + (lane >> 2) : 4 * (wave * kw + i) + q;
+      const int gate = k / Hp, unit = k % Hp;
 #pragma unroll
       for (int ct = 0; ct < CT; ++ct) {
-        const int col = 16 * ct + c, out = col / HS, owned = role.cw * HS + col % HS;
+        const int col = kBlocksOverK ? 4 * (i % 4) + (lane & 3) : 16 * ct + c, out = col / HS, owned = role.cw * HS + col % HS;
         const bool there = i < kw && gate < Cell::kIn && unit < H && out < Cell::kOut && owned < H;
         const unsigned int off = there ? (unsigned int)(((gate * H + unit) * row_len + out * H + owned) * 8) : kNowhere64;
         const double v = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rw, off, 0, 0));
@@ -329,15 +390,15 @@ void recurrence64_kernel(typename Cell::Params p) {
     }
   }
 
-  const int tile = 4 * kw * 64;
-  double* exchange = p.exchange + (size_t)role.bt * 2 * tile;
-  for (int i = role.cw * 256 + tid; i < 2 * tile; i += p.ls.gx * 256) store_exchanged_d(gs, exchange + i, 0.0);
+  const int tile = 16 * kw * ROWS;
+  double* exchange = p.exchange + (size_t)role.bt * kPolledTiles * tile;
+  for (int i = role.cw * 256 + tid; i < kPolledTiles * tile; i += p.ls.gx * 256) store_exchanged_d(gs, exchange + i, 0.0);
   group_arrive(gs);
   group_wait(gs);
 
   const int u = tid % HS, row = tid / HS;
-  const int n = role.bt * kRows64 + row, j = role.cw * HS + u;
-  const bool owner = row < kRows64 && n < p.N && j < H;
+  const int n = role.bt * ROWS + row, j = role.cw * HS + u;
+  const bool owner = row < ROWS && n < p.N && j < H;
   const size_t idx = (size_t)n * H + j;
   // Requests are unconditional (a branch would make every wait behind it a wait for all loads: 9.5
   // instead of 8.4 us per backward step): threads without an element read the last one's.
@@ -348,63 +409,125 @@ void recurrence64_kernel(typename Cell::Params p) {
   Cell::request(p, 0, n_read, j_read, in);
   if (owner) {
     cell.begin(p, idx, j);
-    if (Cell::kForward) store_exchanged_d(gs, exchange + exchange_index(j, row), cell.initial(0));
+    // Tile 0 receives the initial state; the others' elements that steps will publish start out unwritten.
+    for (int g = 0; g < Cell::kIn; ++g)
+      for (int b = 0; b < kPolledTiles; ++b)
+        store_exchanged_d(gs, exchange + b * tile + exchange_index<ROWS>(g * Hp + j, row),
+                          Cell::kForward && b == 0 ? publishable_d(cell.initial(0)) : unwritten_d());
   }
   group_arrive(gs);
+  if constexpr (kPolled) group_wait(gs);
 
   for (int s = 0; s <= p.T; ++s) {
     if (Cell::kForward && s == p.T) break;
     double sum[Cell::kOut] = {};
+    if (owner) cell.prepare(in);
     if (Cell::kForward || s > 0) {
-      group_wait(gs);
-      const __amdgpu_buffer_rsrc_t ra =
-          __builtin_amdgcn_make_buffer_rsrc(exchange + (size_t)(s & 1) * tile, 0, tile * 8, 0x00020000);
-      const unsigned int base = (unsigned int)(wave * kw / 2 * 64 + lane) * 16u;
-      double4_t acc[CT][CHAINS];
-#pragma unroll
-      for (int ct = 0; ct < CT; ++ct)
-#pragma unroll
-        for (int e = 0; e < CHAINS; ++e) acc[ct][e] = double4_t{0.0, 0.0, 0.0, 0.0};
-      double2_t a[RING][kChunk64 / 2];
+      const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
+          exchange + (size_t)(s % kPolledTiles) * tile, 0, tile * 8, 0x00020000);
+      // Short tiles: rows r and r + 4 of a k side by side, 256 bytes per 4 k; with blocks over columns every block
+      // reads the same.
+      const unsigned int base = kBlocksOverK ? (unsigned int)(wave * kw * 256 + lane * 16)
+                                : kShort     ? (unsigned int)(wave * kw * 256 + (q * 4 + (lane & 3)) * 16)
+                                             : (unsigned int)(wave * kw / 2 * 64 + lane) * 16u;
+      constexpr int kStride = kShort && !kBlocksOverK ? 256 : 1024;
+      double2_t a[RING][LOADS];
+      auto request_one = [&](int set, int first, int i) {
+        a[set][i] = __builtin_bit_cast(double2_t, __builtin_amdgcn_raw_buffer_load_b128(
+                                                      ra, base, (first / kChunk64 * LOADS + i) * kStride, kAgentScope64));
+      };
       auto request = [&](int set, int first) {
         if (first >= kw) first = 0;  // nobody uses it; a load that is always there keeps the waits exact
 #pragma unroll
-        for (int i = 0; i < kChunk64 / 2; ++i)
-          a[set][i] = __builtin_bit_cast(double2_t, __builtin_amdgcn_raw_buffer_load_b128(
-                                                        ra, base, (first / 2 + i) * 1024, kAgentScope64));
+        for (int i = 0; i < LOADS; ++i) request_one(set, first, i);
       };
+      // Waits for a chunk: what is missing is asked for again.  The loop is apart from the first look, so that this one
+      // waits for its chunk only.
+      auto arrive = [&](int set, int first) {
+        if (kPolled && !all_written_d(a[set]))
+          poll_until_written(gs, [&] {
 #pragma unroll
-      for (int ch = 0; ch < RING - 1; ++ch) request(ch, ch * kChunk64);
+            for (int i = 0; i < LOADS; ++i)
+              if (__all(written_d(a[set][i])) == 0) request_one(set, first, i);
+          }, [&] { return all_written_d(a[set]); });
+      };
+      if constexpr (!kPolled) group_wait(gs);
+      request(0, 0);
+      arrive(0, 0);  // the first chunk tells when the others are worth asking for: most of what is to come arrives at one time
 #pragma unroll
-      for (int ch = 0; ch < KS / kChunk64; ++ch) {
-        if (ch * kChunk64 >= kw) break;
-        if (ch + RING - 1 < KS / kChunk64) request((ch + RING - 1) % RING, (ch + RING - 1) * kChunk64);
-        if (ch == kInputsBehind) Cell::request(p, s < last_step ? s + 1 : last_step, n_read, j_read, next);
+      for (int ch = 1; ch < RING - 1; ++ch) request(ch, ch * kChunk64);
+      auto chunks = [&](auto&& multiply) {
 #pragma unroll
-        for (int i = 0; i < kChunk64; i += 2)
+        for (int ch = 0; ch < KS / kChunk64; ++ch) {
+          if (ch * kChunk64 >= kw) break;
+          if (ch > 0) arrive(ch % RING, ch * kChunk64);
+          if (ch + RING - 1 < KS / kChunk64) request((ch + RING - 1) % RING, (ch + RING - 1) * kChunk64);
+          if (ch == kInputsBehind) Cell::request(p, s < last_step ? s + 1 : last_step, n_read, j_read, next);
 #pragma unroll
-          for (int ct = 0; ct < CT; ++ct) {
-            const int k = ch * kChunk64 + i;
-            const double2_t b = k < KR ? double2_t{w[k < KR ? k : 0][ct], w[k < KR ? k + 1 : 0][ct]}
-                                       : w_lds[((k - KR) / 2 * CT + ct) * 64];
-            acc[ct][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[ch % RING][i / 2][0], b[0], acc[ct][0], 0, 0, 0);
-            acc[ct][CHAINS - 1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[ch % RING][i / 2][1], b[1], acc[ct][CHAINS - 1], 0, 0, 0);
+          for (int i = 0; i < kChunk64; i += 2)
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) {
+              const int k = ch * kChunk64 + i;
+              const double2_t b = k < KR ? double2_t{w[k < KR ? k : 0][ct], w[k < KR ? k + 1 : 0][ct]}
+                                         : w_lds[((k - KR) / 2 * CT + ct) * 64];
+              multiply(a[ch % RING], i, ct, b);
+            }
+        }
+      };
+      if constexpr (kShort) {
+        constexpr int OUTS = kBlocksOverK ? 4 : CT;
+        double acc[OUTS][2];
+#pragma unroll
+        for (int g = 0; g < OUTS; ++g) acc[g][0] = acc[g][1] = 0.0;
+        chunks([&](const double2_t (&x)[LOADS], int i, int ct, double2_t b) {
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            const int g = kBlocksOverK ? (i + e) % 4 : ct, load = kBlocksOverK ? (i + e) / 4 : i + e;
+#pragma unroll
+            for (int r = 0; r < 2; ++r) acc[g][r] = __builtin_amdgcn_mfma_f64_4x4x4f64(x[load][r], b[e], acc[g][r], 0, 0, 0);
+          }
+        });
+        if constexpr (kBlocksOverK) {
+          // The four blocks' sums are added where the columns belong: block b keeps columns 4 b .. 4 b + 3.
+          const bool upper = (lane & 8) != 0, odd = (lane & 4) != 0;
+#pragma unroll
+          for (int r = 0; r < 2; ++r) {
+            const double a0 = (upper ? acc[2][r] : acc[0][r]) + from_block(upper ? acc[0][r] : acc[2][r], true);
+            const double a1 = (upper ? acc[3][r] : acc[1][r]) + from_block(upper ? acc[1][r] : acc[3][r], true);
+            partial[wave * ROWS * 16 + (4 * r + q) * 16 + c] = (odd ? a1 : a0) + from_block(odd ? a0 : a1, false);
+          }
+        } else {
+#pragma unroll
+          for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+            for (int r = 0; r < 2; ++r) partial[(wave * CT + ct) * ROWS * 16 + (4 * r + q) * 16 + c] = acc[ct][r];
+        }
+      } else {
+        double4_t acc[CT][CHAINS];
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+          for (int e = 0; e < CHAINS; ++e) acc[ct][e] = double4_t{0.0, 0.0, 0.0, 0.0};
+        chunks([&](const double2_t (&x)[LOADS], int i, int ct, double2_t b) {
+          acc[ct][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[i / 2][0], b[0], acc[ct][0], 0, 0, 0);
+          acc[ct][CHAINS - 1] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[i / 2][1], b[1], acc[ct][CHAINS - 1], 0, 0, 0);
+        });
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            double v = acc[ct][0][r];
+            if (CHAINS == 2) v += acc[ct][CHAINS - 1][r];
+            partial[(wave * CT + ct) * 256 + (4 * r + q) * 16 + c] = v;
           }
       }
-#pragma unroll
-      for (int ct = 0; ct < CT; ++ct)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          double v = acc[ct][0][r];
-          if (CHAINS == 2) v += acc[ct][CHAINS - 1][r];
-          partial[(wave * CT + ct) * 256 + (4 * r + q) * 16 + c] = v;
-        }
       __syncthreads();
-      if (row < kRows64) {
+      if (row < ROWS) {
 #pragma unroll
         for (int g = 0; g < Cell::kOut; ++g) {
-          const int col = g * HS + u, at = (col / 16) * 256 + row * 16 + col % 16;
-          sum[g] = ((partial[at] + partial[CT * 256 + at]) + partial[2 * CT * 256 + at]) + partial[3 * CT * 256 + at];
+          constexpr int TILE = ROWS * 16, WAVE = CT * TILE;
+          const int col = g * HS + u, at = (col / 16) * TILE + row * 16 + col % 16;
+          sum[g] = ((partial[at] + partial[WAVE + at]) + partial[2 * WAVE + at]) + partial[3 * WAVE + at];
         }
       }
     } else {
@@ -414,70 +537,91 @@ void recurrence64_kernel(typename Cell::Params p) {
       if (owner) cell.finish(p, idx, sum);
       break;
     }
-    if (owner) {
-      cell.step(p, in, sum);
-      double* to = exchange + (size_t)((s + 1) & 1) * tile;
+    if (owner) cell.step(p, in, sum);
+    // What this wavefront stored during the step before (its resets among it) has landed before the step is visible.
+    if constexpr (kPolled) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (owner && (!Cell::kForward || s + 1 < p.T)) {
+      double* to = exchange + (size_t)((s + 1) % kPolledTiles) * tile;
+      double* done = exchange + (size_t)((s + 3) % kPolledTiles) * tile;  // read at step s - 1: nobody needs it any more
 #pragma unroll
-      for (int g = 0; g < Cell::kIn; ++g)
-        store_exchanged_d(gs, to + exchange_index(g * Hp + j, row), cell.published(g));
+      for (int g = 0; g < Cell::kIn; ++g) {
+        const int e = exchange_index<ROWS>(g * Hp + j, row);
+        store_exchanged_d(gs, to + e, kPolled ? publishable_d(cell.published(g)) : cell.published(g));
+        if constexpr (kPolled) store_exchanged_d(gs, done + e, unwritten_d());
+      }
     }
-    group_arrive(gs);
+    if constexpr (kPolled) __syncthreads();  // the partial tiles may be overwritten
+    else group_arrive(gs);
     if (owner) cell.store(p, s, n, j);
     in = next;
   }
 }
 
-// The geometry: HS units per workgroup, what a wavefront does per step.
-struct Plan64 { int hs, gx, gy, kw; };
+// The geometry: rows of a group, HS units per workgroup, what a wavefront does per step.
+struct Plan64 { int rows, hs, gx, gy, kw; };
 
 // The kernel's KS for kw instructions per wavefront and column tile, 0 when its weights fit neither
 // registers nor LDS.
-constexpr int variant64(int kw, int ct) {
+constexpr int variant64(int kw, int ct, int rows) {
   for (int ks : kSteps64)
-    if (kw <= ks) return fits64(ks, ct) ? ks : 0;
+    if (kw <= ks) return fits64(ks, ct, rows) ? ks : 0;
   return 0;
 }
 
-// 16 hidden units per workgroup unless 8 are offered and fit the chip; the weights of a wavefront
-// must fit its registers and its part of LDS.
+// Groups of 8 rows where each has an XCD of its own (32 CUs, 8 XCDs), otherwise of 16 rows, which need half the
+// workgroups, or 8 across XCDs where those are the only ones whose weights fit; 16 hidden units per workgroup unless 8
+// are offered and fit.  The weights of a wavefront must fit its registers and its part of LDS.
 bool plan_recurrence64(int in_gates, int out_gates, int N, int H, bool eight_units, Plan64* plan) {
   const int steps = in_gates * rounded_up(H, 4) / 4;
   plan->kw = rounded_up((steps + 3) / 4, kChunk64);
-  plan->gy = (N + kRows64 - 1) / kRows64;
-  for (int hs : {8, 16}) {
-    if (hs == 8 && !eight_units) continue;
-    plan->hs = hs;
-    plan->gx = (H + hs - 1) / hs;
-    if (variant64(plan->kw, column_tiles64(out_gates, hs)) > 0 && plan->gy <= kMaxGroups &&
-        (long long)plan->gx * plan->gy <= device_cu_count() && plan->gx * plan->gy <= kMaxWorkgroups)
-      return true;
-  }
+  for (int choice = 0; choice < 3; ++choice)
+    for (int hs : {8, 16}) {
+      if (hs == 8 && (!eight_units || choice == 2)) continue;
+      plan->rows = choice == 1 ? 16 : 8;
+      plan->hs = hs;
+      plan->gx = (H + hs - 1) / hs;
+      plan->gy = (N + plan->rows - 1) / plan->rows;
+      if (choice == 0 && (plan->gx > 32 || plan->gy > 8)) continue;
+      if (choice == 2 && in_gates > 1) continue;
+      if (variant64(plan->kw, column_tiles64(out_gates, hs), plan->rows) > 0 && plan->gy <= kMaxGroups &&
+          (long long)plan->gx * plan->gy <= device_cu_count() && plan->gx * plan->gy <= kMaxWorkgroups)
+        return true;
+    }
   return false;
 }
 
 size_t exchange64_bytes(const Plan64& plan) {
-  return (size_t)plan.gy * 2 * 4 * plan.kw * 64 * sizeof(double);
+  return (size_t)plan.gy * kPolledTiles * 16 * plan.kw * plan.rows * sizeof(double);
 }
 
-template <class Cell, int HS>
+template <class Cell, int HS, int ROWS>
 int launch_recurrence64(const char* name, hipStream_t stream, const Plan64& plan, typename Cell::Params& p) {
   constexpr int CT = column_tiles64(Cell::kOut, HS);
   Workspace ws;
   HASTE_HIP_PROPAGATE(get_workspace(stream, 0, &ws));
   HASTE_HIP_PROPAGATE(check_and_clear_abort(stream, &ws));
   LaunchPlan launch;
-  const int variant = variant64(plan.kw, CT);
-  HASTE_HIP_PROPAGATE(plan_launch(stream, ws, plan.gx, plan.gy, kRows64, recurrence64_lds_bytes(variant, CT),
+  const int variant = variant64(plan.kw, CT, ROWS);
+  HASTE_HIP_PROPAGATE(plan_launch(stream, ws, plan.gx, plan.gy, ROWS, recurrence64_lds_bytes(variant, CT, ROWS),
                                   (unsigned)p.T + 3, &launch));
   p.ls = launch.shape;
   p.kw = plan.kw;
 #define HASTE_LAUNCH_64(KS_)                                                             \
-  if constexpr (fits64(KS_, CT))                                                         \
-    if (variant == KS_) return launch_persistent(name, recurrence64_kernel<Cell, HS, KS_>, launch, p, stream);
+  if constexpr (fits64(KS_, CT, ROWS) && (ROWS == 16 || KS_ <= (Cell::kForward ? (HS == 16 ? 48 : 16) : 128))) \
+    if (variant == KS_) return launch_persistent(name, recurrence64_kernel<Cell, HS, KS_, ROWS>, launch, p, stream);
   HASTE_LAUNCH_64(8) HASTE_LAUNCH_64(16) HASTE_LAUNCH_64(32) HASTE_LAUNCH_64(48) HASTE_LAUNCH_64(64)
   HASTE_LAUNCH_64(96) HASTE_LAUNCH_64(128) HASTE_LAUNCH_64(160) HASTE_LAUNCH_64(192)
 #undef HASTE_LAUNCH_64
   return HASTE_HIP_ERROR_UNSUPPORTED_SIZE;
+}
+
+template <class Cell>
+int launch_recurrence64(const char* name, hipStream_t stream, const Plan64& plan, typename Cell::Params& p) {
+  if constexpr (Cell::kForward)
+    if (plan.hs == 8) return plan.rows == 8 ? launch_recurrence64<Cell, 8, 8>(name, stream, plan, p)
+                                            : launch_recurrence64<Cell, 8, 16>(name, stream, plan, p);
+  return plan.rows == 8 ? launch_recurrence64<Cell, 16, 8>(name, stream, plan, p)
+                        : launch_recurrence64<Cell, 16, 16>(name, stream, plan, p);
 }
 
 }  // namespace
@@ -501,8 +645,7 @@ int lstm_forward_recurrence64(hipStream_t stream, int training, int T, int N, in
   p.training = training; p.zoneout_prob = zoneout_prob; p.mask = mask;
   p.b = b; p.h = h; p.c = c; p.h_out = h_out; p.c_out = c_out; p.v = v;
   const char* name = "lstm_forward_recurrence64";
-  return plan.hs == 8 ? launch_recurrence64<LstmForward64, 8>(name, stream, plan, p)
-                      : launch_recurrence64<LstmForward64, 16>(name, stream, plan, p);
+  return launch_recurrence64<LstmForward64>(name, stream, plan, p);
 }
 
 int gru_forward_recurrence64(hipStream_t stream, int training, int T, int N, int H, const double* R, const double* bx,
@@ -515,8 +658,7 @@ int gru_forward_recurrence64(hipStream_t stream, int training, int T, int N, int
   p.training = training; p.zoneout_prob = zoneout_prob; p.mask = mask;
   p.bx = bx; p.br = br; p.h = h; p.wx = wx; p.h_out = h_out; p.v = v;
   const char* name = "gru_forward_recurrence64";
-  return plan.hs == 8 ? launch_recurrence64<GruForward64, 8>(name, stream, plan, p)
-                      : launch_recurrence64<GruForward64, 16>(name, stream, plan, p);
+  return launch_recurrence64<GruForward64>(name, stream, plan, p);
 }
 
 int lstm_backward_recurrence64(hipStream_t stream, int T, int N, int H, const double* R_t, const double* c,
@@ -528,7 +670,7 @@ int lstm_backward_recurrence64(hipStream_t stream, int T, int N, int H, const do
   p.T = T; p.N = N; p.H = H; p.weights = R_t; p.exchange = static_cast<double*>(exchange);
   p.c = c; p.c_next = c_next; p.dh_next = dh_next; p.dc_next = dc_next; p.mask = mask;
   p.dh = dh; p.dc = dc; p.v = v;
-  return launch_recurrence64<LstmBackward64, 16>("lstm_backward_recurrence64", stream, plan, p);
+  return launch_recurrence64<LstmBackward64>("lstm_backward_recurrence64", stream, plan, p);
 }
 
 int gru_backward_recurrence64(hipStream_t stream, int T, int N, int H, const double* R_t, const double* h,
@@ -540,7 +682,7 @@ int gru_backward_recurrence64(hipStream_t stream, int T, int N, int H, const dou
   p.T = T; p.N = N; p.H = H; p.weights = R_t; p.exchange = static_cast<double*>(exchange);
   p.h = h; p.v = v; p.dh_next = dh_next; p.mask = mask;
   p.dh = dh; p.dp = dp; p.dq = dq;
-  return launch_recurrence64<GruBackward64, 16>("gru_backward_recurrence64", stream, plan, p);
+  return launch_recurrence64<GruBackward64>("gru_backward_recurrence64", stream, plan, p);
 }
 
 }  // namespace haste_hip

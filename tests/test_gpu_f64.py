@@ -195,6 +195,35 @@ def test_f64_recurrence_in_one_launch(double_precision, T, N, C, H, zoneout):
     test_gpu_gru.test_gru_training_forward_backward(T, N, C, H, zoneout)
 
 
+# Enough steps for every exchange tile to be written twice.  Groups of 8 rows: one workgroup; 8 units per workgroup up to
+# 32 of them, 16 from there; polled up to 64 backward steps' worth of k, behind the barrier above; 8 rows across XCDs.
+# Groups of 16 rows from 65 rows or 513 units on.
+@pytest.mark.parametrize("T,N,C,H", [(9, 8, 4, 16), (9, 9, 4, 256), (9, 64, 4, 257), (10, 61, 4, 340), (9, 65, 4, 128),
+                                     (9, 37, 4, 520), (9, 3, 4, 513)])
+def test_f64_recurrence_tiles(double_precision, T, N, C, H):
+    test_gpu_lstm.test_lstm_training_forward_backward(T, N, C, H, 0.3)
+    test_gpu_gru.test_gru_training_forward_backward(T, N, C, H, 0.3)
+
+
+@pytest.mark.parametrize("N,H", [(8, 64), (64, 512), (70, 64)])
+def test_f64_recurrence_carries_every_nan(N, H):
+    """A state whose bits mark unwritten elements: its row turns to NaN, the others do not, nobody waits for it."""
+    import torch
+    from haste_amd import layers, ops
+    torch.manual_seed(1)
+    layer = layers.GRU(16, H).cuda().double()
+    x = torch.randn(9, N, 16, device="cuda", dtype=torch.float64)
+    h0 = torch.zeros(1, N, H, device="cuda", dtype=torch.float64)
+    with torch.no_grad():
+        expected, _ = layer(x, h0)
+        h0[0, 2].view(torch.int64).fill_(-1)
+        y, _ = layer(x, h0)
+    ops.stream_status()
+    assert torch.isnan(y[:, 2]).all()
+    others = [n for n in range(N) if n != 2]
+    assert torch.equal(y[:, others], expected[:, others])
+
+
 @pytest.mark.parametrize("T,N,C,H", ONE_LAUNCH_SHAPES[1:5])
 def test_f64_inference_in_one_launch(double_precision, T, N, C, H):
     test_gpu_lstm.test_lstm_inference_forward(0.25, T, N, C, H)
