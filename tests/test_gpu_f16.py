@@ -62,6 +62,13 @@ def test_f16_gru_training_forward_backward(T, N, C, H, zoneout):
         assert relerr(host(ours), theirs) < TOL16, name
 
 
+# The transposes of a pass on the half matrix cores: tiles of 64 with remainders of whole 16-byte pieces, and an input
+# width that is not one (its matrix is transposed element by element).
+@pytest.mark.parametrize("T,N,C,H", [(8, 9, 72, 40), (5, 8, 20, 64), (24, 5, 33, 24)])
+def test_f16_gru_transposed_operands(T, N, C, H):
+    test_f16_gru_training_forward_backward(T, N, C, H, 0.3)
+
+
 def test_f16_gru_inference_and_iterate():
     from haste_amd import ops
     import torch
