@@ -19,7 +19,8 @@ import numpy as np
 PEAK_FP32_MFMA_TFLOPS = 157.3
 PEAK_FP64_MFMA_TFLOPS = 78.6
 PEAK_HALF_MFMA_TFLOPS = 2500.0  # bf16 and f16, dense
-# The fp32 GEMM runs on the bf16 matrix cores, six bf16 products to one fp32 product; the fp32
+# The fp32 GEMM runs on the bf16 matrix cores, six bf16 products to one fp32 product, and so do the LSTM's and
+# the GRU's recurrences where they are fastest that way (H = 512 from 64 rows on, both passes); the other fp32
 # recurrences run on the fp32 matrix instruction.
 PEAK_SPLIT_TFLOPS = PEAK_HALF_MFMA_TFLOPS / 6.0
 PEAK_HBM_GBS = 8000.0
@@ -27,11 +28,11 @@ PEAK_HBM_GBS = 8000.0
 # HBM bytes per launch at the metric workload, from two rocprofv3 --pmc runs (FETCH_SIZE, then
 # WRITE_SIZE) scaled by what the same counters read for a 1 GiB device copy (--workload copy):
 # one FETCH_SIZE unit = 2.000 KiB, one WRITE_SIZE unit = 1.000 KiB.  A GEMM "launch" is the mean
-# of the step's three products (dx; dW and dR, which share a launch that counts as two), each with
-# its split reduce; the forward recurrence includes the input projection it computes itself.
+# of the step's four products (x*W; dx; dW and dR, which share a launch that counts as two), each with
+# its split reduce.
 TRAFFIC_SOURCE = "profiles/lstm_fwd_bwd_N64_T100_H512_hbm_traffic_pmc.txt (a constant from that profile, not measured in this run)"
-MEASURED_TRAFFIC_BYTES = {"gemm_f32": 111.7e6, "lstm_forward_recurrence": 161.3e6,
-                          "lstm_backward_recurrence": 196.1e6,
+MEASURED_TRAFFIC_BYTES = {"gemm_f32": 117.8e6, "lstm_forward_recurrence": 167.9e6,
+                          "lstm_backward_recurrence": 196.5e6,
                           # at N=1 C=512 H=4096 (--workload stepwise): 131558.5 FETCH_SIZE units
                           # + 192 WRITE_SIZE units per launch of the streaming kernel
                           "gemm_f32_skinny": 269.6e6}
@@ -161,14 +162,15 @@ def run_metric(args, torch, lib, ops, dev):
     f_gemm = 2.0 * T * N * C * 4 * H  # each of the 4 products x*W, dx, dW, dR (C == H)
     f_rec = 2.0 * T * N * H * 4 * H   # h*R over all steps, forward or backward
     gemm_ms, gemm_count = profile_read(lib, "gemm_f32")
-    # With 4-row batch tiles the forward recurrence computes x*W itself: the step then has
-    # three GEMM products instead of four and the forward kernel does the flops of two.
+    # A forward recurrence that computes x*W itself (on the fp32 instruction) leaves the step three GEMM
+    # products instead of four and does the flops of two.
     fused_input = round(gemm_count / args.steps) == 3
+    recurrence_peak = PEAK_FP32_MFMA_TFLOPS if fused_input else PEAK_SPLIT_TFLOPS
     kernels = {}
     f_forward = f_rec + (f_gemm if fused_input else 0.0)
     for name, flops, peak in (("gemm_f32", f_gemm, PEAK_SPLIT_TFLOPS),
-                              ("lstm_forward_recurrence", f_forward, PEAK_FP32_MFMA_TFLOPS),
-                              ("lstm_backward_recurrence", f_rec, PEAK_FP32_MFMA_TFLOPS)):
+                              ("lstm_forward_recurrence", f_forward, recurrence_peak),
+                              ("lstm_backward_recurrence", f_rec, PEAK_SPLIT_TFLOPS)):
         total_ms, count = profile_read(lib, name)
         avg_ms = total_ms / max(count, 1)
         tf = flops / (avg_ms * 1e-3) / 1e12 if avg_ms > 0 else 0.0
@@ -183,8 +185,7 @@ def run_metric(args, torch, lib, ops, dev):
     # whole step beside it: all six products of the step, 2*T*N*4H*(3C + 3H) flops, over the
     # step's wall time, against what the units that they run on deliver together.
     total_flops = 3.0 * (f_gemm + f_rec)
-    step_peak = mixed_peak((f_forward + f_rec, PEAK_FP32_MFMA_TFLOPS),
-                           (total_flops - f_forward - f_rec, PEAK_SPLIT_TFLOPS))
+    step_peak = mixed_peak((f_forward, recurrence_peak), (total_flops - f_forward, PEAK_SPLIT_TFLOPS))
     tflops_whole = total_flops / (ms_per_step * 1e-3) / 1e12
     dominant = max(kernels, key=lambda k: kernels[k]["avg_ms"])
     dom = kernels[dominant]
@@ -491,20 +492,20 @@ def run_configs(args, torch, lib, ops, dev):
     """The other configurations (parity-test cases; timed here for the record):
     forward (+ backward with the caller-side transposes) in ms per call, with the algorithmic
     flops of the matrix products (2*T*N*G*H*(C + H) forward, three times that forward +
-    backward) and the fraction of the matrix cores' peak: fp32 passes that of the fp32 instruction for
-    the recurrences' products and of the split bf16 ones for the others.  Also the
+    backward) and the fraction of the matrix cores' peak: fp32 passes that of the split bf16 products, but
+    of the fp32 instruction for the products of recurrences that run on it.  Also the
     other instantiations of the reference at the metric shape: the double LSTM (all steps of
     a recurrence in one launch, products on the fp64 matrix cores) and the half GRU (recurrences on widened
     tensors, products on the half matrix cores)."""
     details = {}
 
-    def note(key, ms, gates, training, rows=None, peak=None, dtype="f32"):
+    def note(key, ms, gates, training, rows=None, peak=None, dtype="f32", recurrence_peak=PEAK_FP32_MFMA_TFLOPS):
         per_feature = 2.0 * T * (rows or N) * gates * H
         in_recurrence = per_feature * H * (2 if training else 1)  # h*R, and dv*R^T
         around = per_feature * (3 * C + H if training else C)     # x*W, dx, dW, dR
         flops = in_recurrence + around
         if peak is None:
-            peak = mixed_peak((in_recurrence, PEAK_FP32_MFMA_TFLOPS), (around, PEAK_SPLIT_TFLOPS))
+            peak = mixed_peak((in_recurrence, recurrence_peak), (around, PEAK_SPLIT_TFLOPS))
         tf = flops / (ms * 1e-3) / 1e12
         details[key] = {"ms": ms, "flops": flops, "tflops": round(tf, 3), "dtype": dtype,
                         "peak_tflops": round(peak, 1), "frac_of_mfma_peak": round(tf / peak, 4)}
@@ -555,7 +556,7 @@ def run_configs(args, torch, lib, ops, dev):
         return ops.gru_backward(ops.transpose(x), ops.transpose(W), Reff_t, bx, br, zm, h, cache, dh_new)
     out["gru_fwd_bwd_N64_T100_H512_zoneout_dropconnect_ms"] = timed(gru_step, 30)
     note("gru_fwd_bwd_N64_T100_H512_zoneout_dropconnect", out["gru_fwd_bwd_N64_T100_H512_zoneout_dropconnect_ms"],
-         3, True)
+         3, True, recurrence_peak=PEAK_SPLIT_TFLOPS)
 
     # the half GRU of the reference (lib/gru_forward_gpu.cu.cc:373) at the same shape
     xh, Wh, Rh, bxh, brh, zh, zmh, dhh = (a.half() for a in (x, W, R, bx, br, z, zm, dh_new))
@@ -582,7 +583,8 @@ def run_configs(args, torch, lib, ops, dev):
         return ops.lstm_backward(*ops.transpose3(x, W, R), b, no_mask, h, c,
                                  cache, dh_new, dc_new)
     out["lstm_fwd_bwd_N128_T100_H512_ms"] = timed(lstm_step, 30)
-    note("lstm_fwd_bwd_N128_T100_H512", out["lstm_fwd_bwd_N128_T100_H512_ms"], 4, True)
+    note("lstm_fwd_bwd_N128_T100_H512", out["lstm_fwd_bwd_N128_T100_H512_ms"], 4, True,
+         recurrence_peak=PEAK_SPLIT_TFLOPS)
 
     # the double LSTM of the reference (lib/lstm_forward_gpu.cu.cc:368-369) at the metric shape
     Nd = 64
