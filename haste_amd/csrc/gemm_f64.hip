@@ -153,12 +153,14 @@ void gemm_f64_kernel(int M, int N, int K, const double* __restrict__ A, int lda,
     C = part + (size_t)piece * M * N;
     ldc = N;
     accumulate = 0;
-  } else if (cut) {  // a tile's pieces park [64][64] one behind the other
+  } else if (cut) {
+    // A tile's pieces park [64][64] one behind the other, what there is of them: with few rows, zeros written for the
+    // others cost more than the product (4 x 768 x 3072: 9.4 MB, 15.4 us in place of 14.2).
     C = part + ((size_t)(tile - plan.whole) * plan.pieces + piece) * DM * DN;
     ldc = DN;
     row0 = col0 = accumulate = 0;
-    rows = DM;
-    cols = DN;
+    rows = M - m0;
+    cols = N - n0;
   }
   // The operands of an instruction group are read one group ahead: a wavefront issues in order, so a read behind the
   // group before it comes back when the matrix cores have run dry.  between(g): what is issued behind group g.
@@ -244,6 +246,7 @@ void gemm_f64_reduce_kernel(int M, int N, F64Plan plan, int tiles_n, const doubl
   if (row >= M || col >= N) return;
   const double* p = part + (size_t)blockIdx.x * plan.pieces * DM * DN + r * DN + c;
   double4_t s = *reinterpret_cast<const double4_t*>(p);
+#pragma unroll 8  // (eight pieces' loads in flight: 24 pieces of 4 x 768 4.5 -> 4.0 us)
   for (int z = 1; z < plan.pieces; ++z) s += *reinterpret_cast<const double4_t*>(p + (size_t)z * DM * DN);
   double* out = C + (size_t)row * ldc + col;
 #pragma unroll
@@ -256,7 +259,9 @@ void gemm_f64_reduce_kernel(int M, int N, F64Plan plan, int tiles_n, const doubl
 // contraction (its first panel's load and its 64 KiB of partial results show below that).  A last round of more than
 // three quarters of the CUs has too little to give: stays whole.  A product of no more tiles than CUs is all cut, to
 // pieces of at least 4 panels: with one workgroup per CU its barriers and first loads show (512 x 2048 x 6400, 256
-// tiles: 258 us whole, 238 in two pieces; 6400 x 512 x 2048, 800 tiles: 295 whole, 222 with the last 32 in 8).
+// tiles: 258 us whole, 238 in two pieces; 6400 x 512 x 2048, 800 tiles: 295 whole, 222 with the last 32 in 8).  Where the
+// shortest piece keeps that to little more than one per CU, the CUs with two hold up the others, and it is one per CU (4 x
+// 768 x 3072: 288 pieces of 4 panels 14.2 us, 240 of 5 10.4).
 F64Plan plan_f64(int M, int N, int K) {
   const long long tiles = (long long)((M + DM - 1) / DM) * ((N + DN - 1) / DN);
   const long long cus = device_cu_count() > 0 ? device_cu_count() : 256;
@@ -267,9 +272,14 @@ F64Plan plan_f64(int M, int N, int K) {
   s = s < most ? s : most;
   s = s < 64 ? s : 64;
   if (s <= 1 || (whole > 0 && 4 * rest > 3 * cus)) return F64Plan{(int)tiles, 1, K};
-  int per = (int)((K + s - 1) / s);
-  per = (per + DK - 1) / DK * DK;
-  return F64Plan{(int)whole, (K + per - 1) / per, per};
+  auto cut = [&](long long pieces) {
+    const int per = ((int)((K + pieces - 1) / pieces) + DK - 1) / DK * DK;
+    return F64Plan{(int)whole, (K + per - 1) / per, per};
+  };
+  auto turns = [&](const F64Plan& p) { return (rest * p.pieces + cus - 1) / cus * p.k_per_piece; };
+  const F64Plan two = cut(s), one = cut(s < cus / rest ? s : cus / rest);
+  if (whole > 0 || turns(two) <= turns(one)) return two;
+  return one.pieces > 1 ? one : F64Plan{(int)tiles, 1, K};
 }
 // The same for a consumer that adds the pieces itself: all tiles, about one piece per CU.
 F64Plan plan_f64_chunks(int M, int N, int K) {
@@ -473,6 +483,7 @@ int gemm_f64(hipStream_t stream, bool trans_a, int M, int N, int K, const double
     else plan = F64Plan{(int)tiles, 1, K};
   }
   const int rest = (int)(tiles - plan.whole);
+  HASTE_HIP_REQUIRE(rest == 0 || part != nullptr);  // a tile that is not whole is parked
   const dim3 grid((unsigned)(plan.whole + (long long)rest * plan.pieces));
   ScopedKernelTimer timer("gemm_f64", stream);
   if (trans_a)

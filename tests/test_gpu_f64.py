@@ -111,7 +111,11 @@ def test_f64_gemm_and_transpose(trans_a, M, N, K, accumulate):
     # the last tiles cut behind whole ones, loads in pairs of whole and ragged panels and single
     (False, 1100, 1024, 512), (True, 1030, 1022, 770), (False, 1041, 1021, 515), (True, 1088, 1021, 516),
     # all tiles cut; a last round that fills the chip and is not; pairs in a panel of less than 32
-    (True, 512, 2048, 512), (False, 1920, 1024, 512), (False, 70, 66, 2), (True, 66, 70, 30)])
+    (True, 512, 2048, 512), (False, 1920, 1024, 512), (False, 70, 66, 2), (True, 66, 70, 30),
+    # pieces of fewer rows and columns than a tile
+    (False, 4, 130, 1030), (True, 67, 5, 1031), (False, 1, 1, 4096),
+    # two pieces of whole panels are longer than the product: not cut
+    (True, 520, 1560, 333)])
 @pytest.mark.parametrize("room", [True, False])
 def test_f64_gemm_in_pieces(trans_a, M, N, K, room):
     """Error of a sum of K products in double, in any order: below K * 2^-53 of the sum of their magnitudes.  Without
