@@ -115,6 +115,20 @@ int reserve_tickets(hipStream_t stream, unsigned int count, unsigned int* base);
 // returns HASTE_HIP_ERROR_STEP_BARRIER once.
 int check_and_clear_abort(hipStream_t stream, Workspace* ws);
 
+// A pass that is planned and not run (haste_hip_plan_recurrence): while one is set on a host thread, its entry points
+// go through the same choices as ever, on a device and a workspace that are assumed, and launch nothing; the
+// recurrence's launch is written down here instead.
+enum { kPlanSteps, kPlanSingleStep, kPlanFloat, kPlanSplit, kPlanDouble };
+struct PlannedPass {
+  size_t lent;       // scratch the assumed workspace offers, not to be grown; 0: as much as is asked for
+  size_t asked = 0;  // the most that was asked for
+  int kernel = 0;    // what runs the recurrence: see haste_hip_plan_recurrence
+  int rows = 0, sets = 0, gx = 0, gy = 0, xcd_local = 0;
+};
+PlannedPass* planned_pass();
+// Plans a pass of the LSTM (4 gates) or GRU (3); the caller has set the thread's PlannedPass (plan.hip).
+int plan_recurrence(int gates, int element_bytes, bool backward, int T, int N, int C, int H);
+
 int device_cu_count();
 
 // XCDs of the current device on which a launch of one workgroup per CU puts equally many

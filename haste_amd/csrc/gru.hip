@@ -900,7 +900,7 @@ int gru_forward_impl(hipStream_t stream, int training, int T, int N, int C, int 
   const ForwardTile tile = pick_forward_tile(3, N, H, 0, kWorkgroupLdsBytes, false, 3);
   // No slice of R fits a CU: stream R from HBM every step instead.
   if (!tile.ok)
-    return gru_forward_streamed(stream, training, T, N, C, H, W, R, bx, br, x, h, h_out, v, tmp_Wx,
+    return planned_pass() != nullptr ? HASTE_HIP_OK : gru_forward_streamed(stream, training, T, N, C, H, W, R, bx, br, x, h, h_out, v, tmp_Wx,
                                 zoneout_prob, zoneout_mask, dc_mask, dc_scale);
   // An 8-row tile is run as two sets of 4 rows when the partial tiles of both fit beside the
   // slice (exchange tiles: one per set, together as large as the tile's).
@@ -1011,15 +1011,16 @@ int gru_backward_impl(hipStream_t stream, int T, int N, int C, int H,
   // per row: the partial tiles or the 6 bias-gradient columns of 16 floats
   const BackwardTile tile = pick_backward_tile(gru_backward_k(H), N, H, 6 * 16, 0, true);
   if (!tile.ok)
-    return gru_backward_streamed(stream, T, N, C, H, W_t, R_t, x_t, h, v, dh_next, dx, dW, dR, dbx,
+    return planned_pass() != nullptr ? HASTE_HIP_OK : gru_backward_streamed(stream, T, N, C, H, W_t, R_t, x_t, h, v, dh_next, dx, dW, dR, dbx,
                                  dbr, dh, dp, dq, zoneout_mask);
 
   // An 8-row tile is run as two sets of 4 rows (see gru_forward_impl).
   const size_t paired_lds = paired_lds_bytes((gru_backward_k(H) + 63) / 64 * 64, 1);
   // 4-row tiles (8 rows: two sets of 4) with H <= 512 take the scattered form: partial sums of
   // dh go to their owners instead of the gate gradients to everybody.
-  // (Measured over H = 64 ... 512, T = 100: with two sets per workgroup it is 5-15 % faster
-  // at every H, with one set from H = 384 on; below, one set is 5-20 % faster the other way.)
+  // (Measured against the other form over H = 64 ... 512, T = 100: with two sets per workgroup it is 5-15 % faster
+  // at every H, with one set from H = 384 on; below, one set is 5-20 % faster the other way.  Two sets run where
+  // split_backward_rule() below declines.)
   const bool scatter = tile.reg_groups == 0 && H <= 512 &&
                        (tile.nb == 8 || (tile.nb == 4 && H > 320));
   const bool paired = scatter ? tile.nb == 8

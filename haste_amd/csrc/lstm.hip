@@ -895,7 +895,7 @@ int lstm_forward_impl(hipStream_t stream, int training, int T, int N, int C, int
   const ForwardTile tile = pick_forward_tile(4, N, H, 0, kWorkgroupLdsBytes, false, 2);
   // No slice of R fits a CU: stream R from HBM every step instead.
   if (!tile.ok)
-    return lstm_forward_streamed(stream, training, T, N, C, H, W, R, b, x, h, c, h_out, c_out, v,
+    return planned_pass() != nullptr ? HASTE_HIP_OK : lstm_forward_streamed(stream, training, T, N, C, H, W, R, b, x, h, c, h_out, c_out, v,
                                  zoneout_prob, zoneout_mask, dc_mask, dc_scale);
   // An 8-row tile is run as two sets of 4 rows when the partial tiles of both fit beside the
   // slice (exchange tiles: one per set, together as large as the tile's).  Measured at
@@ -991,7 +991,7 @@ int lstm_backward_impl(hipStream_t stream, int T, int N, int C, int H,
   HASTE_HIP_REQUIRE(dx && dW && dR && db && dh && dc && v);
   const BackwardTile tile = pick_backward_tile(4 * H, N, H, 4 * 16, 0, true);
   if (!tile.ok)
-    return lstm_backward_streamed(stream, T, N, C, H, W_t, R_t, x_t, h, c, c_next, dh_next, dc_next,
+    return planned_pass() != nullptr ? HASTE_HIP_OK : lstm_backward_streamed(stream, T, N, C, H, W_t, R_t, x_t, h, c, c_next, dh_next, dc_next,
                                   dx, dW, dR, db, dh, dc, v, zoneout_mask);
 
   // An 8-row tile is run as two sets of 4 rows (see lstm_forward_impl): four polled areas of
@@ -999,8 +999,9 @@ int lstm_backward_impl(hipStream_t stream, int T, int N, int C, int H,
   const size_t paired_lds = paired_lds_bytes(64 * tile.gx, 1);
   // 4-row tiles (8 rows: two sets of 4) with H <= 512 take the scattered form: partial sums of
   // dh go to their owners instead of the gate gradients to everybody.
-  // (Measured over H = 64 ... 512, T = 100: with two sets per workgroup it is 5-15 % faster
-  // at every H, with one set from H = 384 on; below, one set is 5-20 % faster the other way.)
+  // (Measured against the other form over H = 64 ... 512, T = 100: with two sets per workgroup it is 5-15 % faster
+  // at every H, with one set from H = 384 on; below, one set is 5-20 % faster the other way.  Two sets run where
+  // split_backward_rule() below declines.)
   const bool scatter = tile.reg_groups == 0 && H <= 512 &&
                        (tile.nb == 8 || (tile.nb == 4 && H > 320));
   const bool paired = scatter ? tile.nb == 8

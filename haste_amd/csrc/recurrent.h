@@ -1583,6 +1583,7 @@ struct LaunchPlan {
   size_t lds_bytes;
   LaunchShape shape;
   int threads = 256;  // 512: two 256-thread sets per workgroup
+  int kernel = kPlanFloat;  // for a pass that is planned only
 };
 
 inline bool xcd_local_fits(int gx, int gy) {
@@ -1638,6 +1639,18 @@ constexpr size_t kMaxLdsBytes = kWorkgroupLdsBytes - 256;
 template <typename KernelT, typename ParamsT>
 int launch_persistent(const char* name, KernelT kernel, const LaunchPlan& plan, ParamsT& params,
                       hipStream_t stream) {
+  if (PlannedPass* pass = planned_pass()) {
+    // one workgroup per CU, as the geometry searches have it
+    if (plan.lds_bytes > kWorkgroupLdsBytes || (long long)plan.grid.x * plan.grid.y > device_cu_count())
+      return HASTE_HIP_ERROR_UNSUPPORTED_SIZE;
+    pass->kernel = plan.kernel;
+    pass->rows = plan.shape.tile_rows;
+    pass->sets = plan.threads == 512 ? 2 : 1;
+    pass->gx = plan.shape.gx;
+    pass->gy = plan.shape.gy;
+    pass->xcd_local = plan.shape.xcd_local;
+    return HASTE_HIP_OK;
+  }
   // The kernel's LDS limit and its occupancy at this request are looked up once per process
   // and device: single-step callers (Iterate) launch the same kernel over and over.  The
   // limit is a property of the kernel, not of the launch, and is only ever raised.

@@ -605,6 +605,7 @@ int launch_recurrence64(const char* name, hipStream_t stream, const Plan64& plan
   HASTE_HIP_PROPAGATE(plan_launch(stream, ws, plan.gx, plan.gy, ROWS, recurrence64_lds_bytes(variant, CT, ROWS),
                                   (unsigned)p.T + 3, &launch));
   p.ls = launch.shape;
+  launch.kernel = kPlanDouble;
   p.kw = plan.kw;
 #define HASTE_LAUNCH_64(KS_)                                                             \
   if constexpr (fits64(KS_, CT, ROWS) && (ROWS == 16 || KS_ <= (Cell::kForward ? (HS == 16 ? 48 : 16) : 128))) \

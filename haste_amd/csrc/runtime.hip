@@ -208,6 +208,7 @@ XcdLayout& xcd_layout_locked(int dev) {
 }  // namespace
 
 int xcd_layout_ready(hipStream_t stream) {
+  if (planned_pass() != nullptr) return HASTE_HIP_OK;
   int dev = 0;
   HASTE_HIP_TRY(hipGetDevice(&dev));
   {
@@ -229,7 +230,10 @@ int xcd_layout_ready(hipStream_t stream) {
 namespace {
 // A device shape assumed by this thread instead of the current device's (haste_hip_plan_tiles).
 thread_local int t_assumed_cus = 0, t_assumed_xcds = 0;
+thread_local PlannedPass* t_planned = nullptr;
 }  // namespace
+
+PlannedPass* planned_pass() { return t_planned; }
 
 int device_xcd_count() {
   if (t_assumed_cus > 0) return t_assumed_xcds;
@@ -240,6 +244,7 @@ int device_xcd_count() {
 }
 
 unsigned long long device_xcc_logical_map() {
+  if (planned_pass() != nullptr) return 0;
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return 0;
   std::lock_guard<std::mutex> lock(g_mutex);
@@ -292,7 +297,7 @@ int workspace_has_room(hipStream_t stream, size_t bytes, bool* room) {
   *room = true;
   if (ws.scratch_bytes < bytes) {
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &capture) != hipSuccess) (void)hipGetLastError();
+    if (planned_pass() == nullptr && hipStreamIsCapturing(stream, &capture) != hipSuccess) (void)hipGetLastError();
     *room = !ws.caller_owned && capture == hipStreamCaptureStatusNone;
   }
   return HASTE_HIP_OK;
@@ -398,6 +403,15 @@ ScratchPrefix::ScratchPrefix(size_t bytes) : saved_(t_scratch_prefix) { t_scratc
 ScratchPrefix::~ScratchPrefix() { t_scratch_prefix = saved_; }
 
 int get_workspace(hipStream_t stream, size_t scratch_bytes, Workspace* out) {
+  if (PlannedPass* pass = planned_pass()) {
+    if (pass->lent > 0 && scratch_bytes > pass->lent) return HASTE_HIP_ERROR_UNSUPPORTED_SIZE;
+    pass->asked = pass->asked > scratch_bytes ? pass->asked : scratch_bytes;
+    *out = Workspace();
+    out->scratch = reinterpret_cast<float*>(uintptr_t(256));  // never read: nothing is launched
+    out->scratch_bytes = pass->lent > 0 ? pass->lent : pass->asked;
+    out->caller_owned = pass->lent > 0;
+    return HASTE_HIP_OK;
+  }
   int dev = 0;
   HASTE_HIP_TRY(hipGetDevice(&dev));
   const size_t prefix = t_scratch_prefix;
@@ -456,6 +470,8 @@ int get_workspace(hipStream_t stream, size_t scratch_bytes, Workspace* out) {
 constexpr unsigned int kEpochLimit = 0xe0000000u;
 
 int reserve_epochs(hipStream_t stream, unsigned int count, unsigned int* base) {
+  *base = 0;
+  if (planned_pass() != nullptr) return HASTE_HIP_OK;
   int dev = 0;
   HASTE_HIP_TRY(hipGetDevice(&dev));
   std::lock_guard<std::mutex> lock(g_mutex);
@@ -483,6 +499,8 @@ int reserve_epochs(hipStream_t stream, unsigned int count, unsigned int* base) {
 }
 
 int reserve_tickets(hipStream_t stream, unsigned int count, unsigned int* base) {
+  *base = 0;
+  if (planned_pass() != nullptr) return HASTE_HIP_OK;
   int dev = 0;
   HASTE_HIP_TRY(hipGetDevice(&dev));
   std::lock_guard<std::mutex> lock(g_mutex);
@@ -572,6 +590,28 @@ int haste_hip_plan_tiles(int cus, int xcds, int gates, int batch_size, int hidde
                        b.ok, b.nb, 16, 1, b.gx, b.gy, b.reg_groups, (k_back + 63) / 64};
   for (int i = 0; i < 16; ++i) plan[i] = (i % 8 == 0 || out[i - i % 8]) ? out[i] : 0;
   return HASTE_HIP_OK;
+}
+
+int haste_hip_plan_recurrence(int cus, int xcds, int gates, int element_bytes, int backward, int time_steps,
+                              int batch_size, int input_size, int hidden_size, size_t workspace_bytes, int* plan) {
+  using namespace haste_hip;
+  HASTE_HIP_REQUIRE(plan != nullptr && (gates == 3 || gates == 4) && (element_bytes == 4 || element_bytes == 8));
+  HASTE_HIP_REQUIRE(cus >= 0 && xcds >= 0 && (cus > 0 || xcds == 0));
+  HASTE_HIP_REQUIRE(time_steps > 0 && batch_size > 0 && input_size > 0 && hidden_size > 0);
+  HASTE_HIP_REQUIRE(workspace_bytes == 0 || workspace_bytes > kControlBytes);
+  PlannedPass pass;
+  pass.lent = workspace_bytes == 0 ? 0 : workspace_bytes - kControlBytes;
+  t_assumed_cus = cus;
+  t_assumed_xcds = xcds;
+  t_planned = &pass;
+  const int rc = plan_recurrence(gates, element_bytes, backward != 0, time_steps, batch_size, input_size, hidden_size);
+  t_planned = nullptr;
+  t_assumed_cus = 0;
+  t_assumed_xcds = 0;
+  const int out[8] = {pass.kernel, pass.rows, pass.sets, pass.gx, pass.gy, pass.xcd_local,
+                      (int)((pass.asked + kControlBytes + 1023) / 1024), 0};
+  for (int i = 0; i < 8; ++i) plan[i] = rc == HASTE_HIP_OK ? out[i] : 0;
+  return rc;
 }
 
 int haste_hip_stream_status(void* stream_) {

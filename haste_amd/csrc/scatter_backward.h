@@ -292,17 +292,16 @@ void scatter_backward_kernel(typename Cell::Params p) {
 }
 
 
-// Launches the kernel for `sets` sets per workgroup and hidden size H <= 512 (two sets of fp32 products: H <= 256, beyond
-// that split_backward.h's kernel runs).
+// Launches the kernel for `sets` sets per workgroup and hidden size H <= 512.  (Two sets of fp32 products beyond H = 256 are
+// what runs where split_backward_rule() declines: groups across XCDs, fewer than eight XCDs, too small a workspace.)
 template <class Cell, bool HALF = false>
 int launch_scatter_backward(const char* name, int H, int sets, const LaunchPlan& plan, typename Cell::Params& p,
                             hipStream_t stream) {
   if (H <= 256)
     return sets == 2 ? launch_persistent(name, scatter_backward_kernel<Cell, 1, 2, HALF>, plan, p, stream)
                      : launch_persistent(name, scatter_backward_kernel<Cell, 1, 1, HALF>, plan, p, stream);
-  if (sets == 1) return launch_persistent(name, scatter_backward_kernel<Cell, 2, 1, HALF>, plan, p, stream);
-  if constexpr (HALF) return launch_persistent(name, scatter_backward_kernel<Cell, 2, 2, HALF>, plan, p, stream);
-  return HASTE_HIP_ERROR_UNSUPPORTED_SIZE;
+  return sets == 2 ? launch_persistent(name, scatter_backward_kernel<Cell, 2, 2, HALF>, plan, p, stream)
+                   : launch_persistent(name, scatter_backward_kernel<Cell, 2, 1, HALF>, plan, p, stream);
 }
 
 }  // namespace haste_hip

@@ -275,6 +275,10 @@ int launch_step(hipStream_t stream, StepParams<T>& p, const char* name) {
   const bool in_place = p.h_out < p.h + state_floats && p.h < p.h_out + state_floats;
   Workspace ws;
   HASTE_HIP_PROPAGATE(get_workspace(stream, partial_bytes + (in_place ? state_floats * sizeof(float) : 0) + 256, &ws));
+  if (PlannedPass* pass = planned_pass()) {
+    pass->kernel = kPlanSingleStep;
+    return HASTE_HIP_OK;
+  }
   p.partial = ws.scratch;
   p.h_stage = in_place ? ws.scratch + partial_bytes / sizeof(float) : nullptr;
   p.cb = ws.control;

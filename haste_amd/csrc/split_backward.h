@@ -482,6 +482,7 @@ int launch_split_backward_rows(const char* name, hipStream_t stream, const Works
   HASTE_HIP_PROPAGATE(plan_launch(stream, ws, gx, (p.N + NB - 1) / NB, NB, sizeof(SplitBackwardLds<Cell, NB>),
                                   (unsigned)p.T + 1, &plan));
   p.ls = plan.shape;
+  plan.kernel = kPlanSplit;
   if (ctw == 4) return launch_persistent(name, split_backward_kernel<Cell, NB, 4>, plan, p, stream);
   if (ctw == 6) return launch_persistent(name, split_backward_kernel<Cell, NB, 6>, plan, p, stream);
   return launch_persistent(name, split_backward_kernel<Cell, NB, 8>, plan, p, stream);

@@ -512,6 +512,7 @@ int launch_split_forward_tile(const char* name, hipStream_t stream, const Worksp
   HASTE_HIP_PROPAGATE(plan_launch(stream, ws, (p.H + 15) / 16, (p.N + NB - 1) / NB, NB, sizeof(SplitForwardLds<NB>),
                                   (unsigned)p.T + 1, &plan));
   p.ls = plan.shape;
+  plan.kernel = kPlanSplit;
   return launch_persistent(name, split_forward_kernel<Cell, NB, KST>, plan, p, stream);
 }
 template <class Cell, int NB>

@@ -56,6 +56,18 @@ int haste_hip_max_hidden_size(int gates, int batch_size);
  * for tests of the geometry search. */
 int haste_hip_plan_tiles(int cus, int xcds, int gates, int batch_size, int hidden_size, int* plan);
 
+/* What runs the recurrence of a forward or backward pass of the LSTM (4 gates) or GRU (3), in float
+ * (element_bytes 4) or double (8): the pass's own choices, on the device that is described as for
+ * haste_hip_plan_tiles and with a workspace of `workspace_bytes` lent with haste_hip_set_workspace
+ * (0: the library's own, which grows); nothing is launched, and no device touched when cus > 0.
+ * plan[0]: 0 step by step, the recurrent matrix streamed; 1 a single step in one kernel; 2 one
+ * launch on the fp32 matrix instruction; 3 on the bf16 matrix cores, operands as sums of three;
+ * 4 in double.  plan[1..5], of the one launch: batch rows per tile, tiles a workgroup works on side by
+ * side, column workgroups, batch tiles, whether each tile's workgroups share an XCD.  plan[6]: KiB
+ * of workspace that were asked for.  plan[7]: 0.  Returns what the pass would. */
+int haste_hip_plan_recurrence(int cus, int xcds, int gates, int element_bytes, int backward, int time_steps,
+                              int batch_size, int input_size, int hidden_size, size_t workspace_bytes, int* plan);
+
 /* Drops this thread's cached per-stream workspaces on the current device (frees
  * device memory; the caller must have synchronized the streams that used them). */
 int haste_hip_release_workspaces(void);

@@ -56,3 +56,33 @@ def test_plan_tiles_refuses_bad_arguments():
     assert lib.haste_hip_plan_tiles(256, 8, 4, 0, 64, out) != 0
     assert lib.haste_hip_plan_tiles(256, 8, 4, 4, 64, None) != 0
     assert lib.haste_hip_plan_tiles(0, 8, 4, 4, 64, out) != 0
+
+
+PASSES = [(gates, size, backward) for gates in (3, 4) for size in (4,) for backward in (0, 1)]
+
+
+def _plan_pass(lib, cus, xcds, gates, size, backward, T, N, C, H, workspace=0):
+    out = (ctypes.c_int * 8)()
+    rc = lib.haste_hip_plan_recurrence(cus, xcds, gates, size, backward, T, N, C, H, ctypes.c_size_t(workspace), out)
+    return rc, list(out)
+
+
+@pytest.mark.parametrize("cus,xcds", DEVICES + [(128, 0), (64, 2), (32, 1)])
+@pytest.mark.parametrize("gates,size,backward", PASSES)
+def test_every_pass_has_a_kernel(cus, xcds, gates, size, backward):
+    """Whatever is chosen for a pass can be launched, on every device shape: with XCDs, without (the placement could not
+    be looked at, was switched off or turned out wrong) and with fewer of them."""
+    lib = hlib.load()
+    sizes = sorted(set(list(range(16, 1025, 16)) + [1, 5, 37, 100, 129, 257, 300, 321, 385, 500, 511, 770, 777, 800, 816, 1100, 2048, 4096]))
+    batches = sorted(set(BATCHES + list(range(1, 130, 4)) + [33, 40, 65, 72, 80]))
+    kernels = set()
+    for H in sizes:
+        for N in batches:
+            for T in (2, 30):
+                rc, plan = _plan_pass(lib, cus, xcds, gates, size, backward, T, N, 18, H)
+                assert rc == 0, (cus, xcds, gates, size, backward, T, N, H, rc)
+                kernels.add(plan[0])
+                if plan[0] > 1:
+                    assert plan[3] * plan[4] <= cus and plan[1] * plan[2] * plan[4] >= N
+    every = {0, 4} if size == 8 else {0, 2, 3}
+    assert kernels == every if (cus, xcds) == (256, 8) else kernels <= every if xcds else kernels <= every - {3}
