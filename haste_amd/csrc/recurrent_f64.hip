@@ -560,11 +560,15 @@ void recurrence64_kernel(typename Cell::Params p) {
 // The geometry: rows of a group, HS units per workgroup, what a wavefront does per step.
 struct Plan64 { int rows, hs, gx, gy, kw; };
 
-// The kernel's KS for kw instructions per wavefront and column tile, 0 when its weights fit neither
-// registers nor LDS.
-constexpr int variant64(int kw, int ct, int rows) {
+// The kernels there are: those whose weights fit registers and LDS, groups of 8 rows as far as the plan below has a use
+// for them.
+constexpr bool offered64(bool forward, int hs, int ks, int rows, int ct) {
+  return fits64(ks, ct, rows) && (rows == 16 || ks <= (forward ? (hs == 16 ? 48 : 16) : 128));
+}
+// The kernel's KS for kw instructions per wavefront and column tile, 0 when there is none.
+constexpr int variant64(bool forward, int hs, int kw, int rows, int ct) {
   for (int ks : kSteps64)
-    if (kw <= ks) return fits64(ks, ct, rows) ? ks : 0;
+    if (kw <= ks) return offered64(forward, hs, ks, rows, ct) ? ks : 0;
   return 0;
 }
 
@@ -583,7 +587,7 @@ bool plan_recurrence64(int in_gates, int out_gates, int N, int H, bool eight_uni
       plan->gy = (N + plan->rows - 1) / plan->rows;
       if (choice == 0 && (plan->gx > 32 || plan->gy > 8)) continue;
       if (choice == 2 && in_gates > 1) continue;
-      if (variant64(plan->kw, column_tiles64(out_gates, hs), plan->rows) > 0 && plan->gy <= kMaxGroups &&
+      if (variant64(out_gates > 1, hs, plan->kw, plan->rows, column_tiles64(out_gates, hs)) > 0 && plan->gy <= kMaxGroups &&
           (long long)plan->gx * plan->gy <= device_cu_count() && plan->gx * plan->gy <= kMaxWorkgroups)
         return true;
     }
@@ -601,14 +605,14 @@ int launch_recurrence64(const char* name, hipStream_t stream, const Plan64& plan
   HASTE_HIP_PROPAGATE(get_workspace(stream, 0, &ws));
   HASTE_HIP_PROPAGATE(check_and_clear_abort(stream, &ws));
   LaunchPlan launch;
-  const int variant = variant64(plan.kw, CT, ROWS);
+  const int variant = variant64(Cell::kForward, HS, plan.kw, ROWS, CT);
   HASTE_HIP_PROPAGATE(plan_launch(stream, ws, plan.gx, plan.gy, ROWS, recurrence64_lds_bytes(variant, CT, ROWS),
                                   (unsigned)p.T + 3, &launch));
   p.ls = launch.shape;
   launch.kernel = kPlanDouble;
   p.kw = plan.kw;
-#define HASTE_LAUNCH_64(KS_)                                                             \
-  if constexpr (fits64(KS_, CT, ROWS) && (ROWS == 16 || KS_ <= (Cell::kForward ? (HS == 16 ? 48 : 16) : 128))) \
+#define HASTE_LAUNCH_64(KS_)                                   \
+  if constexpr (offered64(Cell::kForward, HS, KS_, ROWS, CT))  \
     if (variant == KS_) return launch_persistent(name, recurrence64_kernel<Cell, HS, KS_, ROWS>, launch, p, stream);
   HASTE_LAUNCH_64(8) HASTE_LAUNCH_64(16) HASTE_LAUNCH_64(32) HASTE_LAUNCH_64(48) HASTE_LAUNCH_64(64)
   HASTE_LAUNCH_64(96) HASTE_LAUNCH_64(128) HASTE_LAUNCH_64(160) HASTE_LAUNCH_64(192)

@@ -201,9 +201,9 @@ def test_f64_recurrence_in_one_launch(double_precision, T, N, C, H, zoneout):
 
 # Enough steps for every exchange tile to be written twice.  Groups of 8 rows: one workgroup; 8 units per workgroup up to
 # 32 of them, 16 from there; polled up to 64 backward steps' worth of k, behind the barrier above; 8 rows across XCDs.
-# Groups of 16 rows from 65 rows or 513 units on.
+# Groups of 16 rows from 65 rows or 513 units on; none, where the GRU's forward pass finds no kernel (37 rows, 800 units).
 @pytest.mark.parametrize("T,N,C,H", [(9, 8, 4, 16), (9, 9, 4, 256), (9, 64, 4, 257), (10, 61, 4, 340), (9, 65, 4, 128),
-                                     (9, 37, 4, 520), (9, 3, 4, 513)])
+                                     (9, 37, 4, 520), (9, 3, 4, 513), (5, 37, 4, 800)])
 def test_f64_recurrence_tiles(double_precision, T, N, C, H):
     test_gpu_lstm.test_lstm_training_forward_backward(T, N, C, H, 0.3)
     test_gpu_gru.test_gru_training_forward_backward(T, N, C, H, 0.3)

@@ -58,7 +58,7 @@ def test_plan_tiles_refuses_bad_arguments():
     assert lib.haste_hip_plan_tiles(0, 8, 4, 4, 64, out) != 0
 
 
-PASSES = [(gates, size, backward) for gates in (3, 4) for size in (4,) for backward in (0, 1)]
+PASSES = [(gates, size, backward) for gates in (3, 4) for size in (4, 8) for backward in (0, 1)]
 
 
 def _plan_pass(lib, cus, xcds, gates, size, backward, T, N, C, H, workspace=0):
