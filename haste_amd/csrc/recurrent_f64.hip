@@ -572,7 +572,7 @@ constexpr int variant64(bool forward, int hs, int kw, int rows, int ct) {
   return 0;
 }
 
-// Groups of 8 rows where each has an XCD of its own (32 CUs, 8 XCDs), otherwise of 16 rows, which need half the
+// Groups of 8 rows where each has an XCD of its own, otherwise of 16 rows, which need half the
 // workgroups, or 8 across XCDs where those are the only ones whose weights fit; 16 hidden units per workgroup unless 8
 // are offered and fit.  The weights of a wavefront must fit its registers and its part of LDS.
 bool plan_recurrence64(int in_gates, int out_gates, int N, int H, bool eight_units, Plan64* plan) {
@@ -585,7 +585,7 @@ bool plan_recurrence64(int in_gates, int out_gates, int N, int H, bool eight_uni
       plan->hs = hs;
       plan->gx = (H + hs - 1) / hs;
       plan->gy = (N + plan->rows - 1) / plan->rows;
-      if (choice == 0 && (plan->gx > 32 || plan->gy > 8)) continue;
+      if (choice == 0 && !xcd_local_fits(plan->gx, plan->gy)) continue;
       if (choice == 2 && in_gates > 1) continue;
       if (variant64(out_gates > 1, hs, plan->kw, plan->rows, column_tiles64(out_gates, hs)) > 0 && plan->gy <= kMaxGroups &&
           (long long)plan->gx * plan->gy <= device_cu_count() && plan->gx * plan->gy <= kMaxWorkgroups)
@@ -594,8 +594,10 @@ bool plan_recurrence64(int in_gates, int out_gates, int N, int H, bool eight_uni
   return false;
 }
 
-size_t exchange64_bytes(const Plan64& plan) {
-  return (size_t)plan.gy * kPolledTiles * 16 * plan.kw * plan.rows * sizeof(double);
+// Room for groups of 8 rows and of 16: which of them run is asked again at the launch, and another thread may have found
+// the placement on XCDs wrong in between.
+size_t exchange64_bytes(const Plan64& plan, int N) {
+  return (size_t)rounded_up(N, 16) * kPolledTiles * 16 * plan.kw * sizeof(double);
 }
 
 template <class Cell, int HS, int ROWS>
@@ -637,7 +639,7 @@ int launch_recurrence64(const char* name, hipStream_t stream, const Plan64& plan
 size_t recurrence64_scratch_bytes(int in_gates, int out_gates, int steps, int N, int H) {
   Plan64 plan;
   if (steps < 4 || !plan_recurrence64(in_gates, out_gates, N, H, out_gates > 1, &plan)) return 0;
-  return exchange64_bytes(plan);
+  return exchange64_bytes(plan, N);
 }
 
 int lstm_forward_recurrence64(hipStream_t stream, int training, int T, int N, int H, const double* R, const double* b,

@@ -86,3 +86,23 @@ def test_every_pass_has_a_kernel(cus, xcds, gates, size, backward):
                     assert plan[3] * plan[4] <= cus and plan[1] * plan[2] * plan[4] >= N
     every = {0, 4} if size == 8 else {0, 2, 3}
     assert kernels == every if (cus, xcds) == (256, 8) else kernels <= every if xcds else kernels <= every - {3}
+
+
+def test_double_groups_of_8_rows_have_an_xcd_each():
+    """Groups of 8 rows rather than 16 pay where a group's workgroups share an XCD: with XCDs, as far as there are, and not
+    without."""
+    lib = hlib.load()
+    for gates in (3, 4):
+        for N, H in [(64, 512), (40, 256), (8, 64)]:
+            for backward in (0, 1):
+                rows = {}
+                for cus, xcds in [(256, 8), (256, 0), (128, 4), (256, 16)]:
+                    rc, plan = _plan_pass(lib, cus, xcds, gates, 8, backward, 30, N, 18, H)
+                    assert rc == 0
+                    rows[cus, xcds] = (plan[1], plan[5])
+                assert rows[256, 8] == (8, 1), (gates, N, H, backward)
+                assert rows[256, 0] == (16, 0), (gates, N, H, backward)
+                # four XCDs of 32 CUs: four groups
+                assert rows[128, 4] == ((8, 1) if N <= 32 else (16, 1 if N <= 64 and H <= 512 else 0)), (gates, N, H, backward)
+                # sixteen XCDs of 16 CUs: 256 units
+                assert (rows[256, 16][0] == 8) == (H <= 256), (gates, N, H, backward)
