@@ -77,8 +77,9 @@ struct Workspace {
 // it is too small.
 int get_workspace(hipStream_t stream, size_t scratch_bytes, Workspace* out);
 
-// Whether the stream's workspace holds `bytes` of scratch or can be made to: not where the caller lent
-// less, nor where it would have to grow while the stream is captured.
+// Whether the stream's workspace holds `bytes` of scratch or can be made to: not where the caller lent less, nor where it
+// would have to grow while the stream is captured or beneath a ScratchPrefix.  Where a kernel is chosen by it, a workspace of
+// haste_hip_workspace_bytes() holds every one, so that results depend on it in smaller ones only.
 int workspace_has_room(hipStream_t stream, size_t bytes, bool* room);
 
 // While one of these is alive on a host thread, get_workspace() on that thread hands out the

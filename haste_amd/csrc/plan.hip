@@ -36,7 +36,8 @@ int plan_recurrence(int gates, int element_bytes, bool backward, int T, int N, i
   const bool lstm = gates == 4;
   if (element_bytes == 8) {
     const size_t bytes = recurrence64_scratch_bytes(backward ? gates : 1, backward ? 1 : gates, T, N, H);
-    if (bytes == 0) return HASTE_HIP_OK;  // step by step
+    const size_t lent = planned_pass()->lent;
+    if (bytes == 0 || (lent > 0 && lent < bytes)) return HASTE_HIP_OK;  // step by step
     Workspace ws;
     HASTE_HIP_PROPAGATE(get_workspace(nullptr, bytes, &ws));
     double* a = reinterpret_cast<double*>(ws.scratch);  // an address for every tensor: none is read

@@ -231,6 +231,7 @@ namespace {
 // A device shape assumed by this thread instead of the current device's (haste_hip_plan_tiles).
 thread_local int t_assumed_cus = 0, t_assumed_xcds = 0;
 thread_local PlannedPass* t_planned = nullptr;
+thread_local size_t t_scratch_prefix = 0;
 }  // namespace
 
 PlannedPass* planned_pass() { return t_planned; }
@@ -298,7 +299,7 @@ int workspace_has_room(hipStream_t stream, size_t bytes, bool* room) {
   if (ws.scratch_bytes < bytes) {
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     if (planned_pass() == nullptr && hipStreamIsCapturing(stream, &capture) != hipSuccess) (void)hipGetLastError();
-    *room = !ws.caller_owned && capture == hipStreamCaptureStatusNone;
+    *room = !ws.caller_owned && capture == hipStreamCaptureStatusNone && t_scratch_prefix == 0;
   }
   return HASTE_HIP_OK;
 }
@@ -393,10 +394,6 @@ int recover_from_abort_locked(int dev, hipStream_t stream, Workspace& ws, unsign
   return HASTE_HIP_ERROR_STEP_BARRIER;
 }
 
-}  // namespace
-
-namespace {
-thread_local size_t t_scratch_prefix = 0;
 }  // namespace
 
 ScratchPrefix::ScratchPrefix(size_t bytes) : saved_(t_scratch_prefix) { t_scratch_prefix = saved_ + bytes; }

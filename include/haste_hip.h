@@ -64,7 +64,8 @@ int haste_hip_plan_tiles(int cus, int xcds, int gates, int batch_size, int hidde
  * launch on the fp32 matrix instruction; 3 on the bf16 matrix cores, operands as sums of three;
  * 4 in double.  plan[1..5], of the one launch: batch rows per tile, tiles a workgroup works on side by
  * side, column workgroups, batch tiles, whether each tile's workgroups share an XCD.  plan[6]: KiB
- * of workspace that were asked for.  plan[7]: 0.  Returns what the pass would. */
+ * of workspace that were asked for (in double: for the one launch alone).  plan[7]: 0.  Returns what
+ * the pass would. */
 int haste_hip_plan_recurrence(int cus, int xcds, int gates, int element_bytes, int backward, int time_steps,
                               int batch_size, int input_size, int hidden_size, size_t workspace_bytes, int* plan);
 
@@ -102,7 +103,11 @@ int haste_hip_stream_status(void* stream);
  * (but for the half GRU, below) needs for (T, N, C, H) on the current device (for the stand-alone layer norm: T = 1,
  * N = rows, C = H = dim): 64 MiB for the partial tiles of split GEMMs plus terms in N*H,
  * H*H and T*N.  haste_hip_workspace_high_water: what the calls made on `stream` so far
- * have actually needed (after a rehearsal of the same calls, the exact size to lend). */
+ * have actually needed (after a rehearsal of the same calls, the exact size to lend).
+ * With at least either, and with the library's own workspace outside of captures, which kernels run
+ * depends on the call's sizes and the device only.  A smaller lent buffer, or the library's workspace
+ * where it would have to grow during a capture, may serve a call all the same, with kernels that
+ * need less and round the same sums in another order. */
 size_t haste_hip_workspace_bytes(int time_steps, int batch_size, int input_size, int hidden_size);
 
 /* The same bound for haste_hip_gru_{forward,forward_dropconnect,backward}_f16, which over more

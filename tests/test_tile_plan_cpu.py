@@ -106,3 +106,26 @@ def test_double_groups_of_8_rows_have_an_xcd_each():
                 assert rows[128, 4] == ((8, 1) if N <= 32 else (16, 1 if N <= 64 and H <= 512 else 0)), (gates, N, H, backward)
                 # sixteen XCDs of 16 CUs: 256 units
                 assert (rows[256, 16][0] == 8) == (H <= 256), (gates, N, H, backward)
+
+
+@pytest.mark.parametrize("gates,size,backward", PASSES)
+def test_a_workspace_of_the_stated_size_decides_nothing(gates, size, backward):
+    """A pass that was lent haste_hip_workspace_bytes(), or what a rehearsal asked for, runs what it runs with a workspace
+    that grows; one with less than it needs is refused or runs what needs less."""
+    lib = hlib.load()
+    lib.haste_hip_workspace_bytes.restype = ctypes.c_size_t
+    fewer = 0
+    for T in (1, 2, 30, 300):
+        for N in BATCHES + [20, 48, 96]:
+            for C, H in [(1, 1), (64, 128), (18, 257), (512, 300), (512, 512), (75, 512), (33, 800), (512, 1024), (2048, 1536)]:
+                where = (gates, size, backward, T, N, C, H)
+                own = _plan_pass(lib, 256, 8, gates, size, backward, T, N, C, H)
+                assert own[0] == 0, where
+                stated = lib.haste_hip_workspace_bytes(T, N, C, H)
+                assert own[1][6] * 1024 <= stated + 1024, where
+                for lent in (stated, own[1][6] * 1024):
+                    rc, plan = _plan_pass(lib, 256, 8, gates, size, backward, T, N, C, H, lent)
+                    assert rc == 0 and plan[:6] == own[1][:6], (where, lent)
+                rc, plan = _plan_pass(lib, 256, 8, gates, size, backward, T, N, C, H, own[1][6] * 512)
+                fewer += rc != 0 or plan[:6] != own[1][:6]
+    assert fewer > 0
