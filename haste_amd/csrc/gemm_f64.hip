@@ -11,11 +11,12 @@
 // 64 moves and a wait for the matrix cores every two panels), and the tiles that would fill a last round of
 // workgroups only partly are cut along K, as is a product of few tiles and a long contraction (the product of one step
 // over 70 rows: 128 x 512 x 2048 is 16 tiles): each piece a workgroup of its own, which parks partial results in the
-// stream's scratch buffer; a second kernel adds a tile's pieces in index order.  Measured, before and after those
-// two and the branch-free loop below: 6400 x 2048 x 512 273 -> 255 us, 6400 x 512 x 2048 307 -> 222,
-// 512 x 2048 x 6400 295 -> 238, with A transposed 278 -> 221 (61 TFLOP/s), 4096^3 59 -> 64 TFLOP/s (the library: 72).
-// How a product is cut depends on its shape only (and on whether the scratch buffer has room for the pieces), so
-// results are reproducible.  Lane layout of the instruction (checked on the hardware): a = A[i = lane%16][k = lane/16], b = B[k = lane/16][j = lane%16],
+// stream's scratch buffer; a second kernel adds a tile's pieces in index order.  Measured, launches back to back, before and
+// after those two, the loop and the order of tiles below: 6400 x 2048 x 512 255 -> 230 us, 6400 x 512 x 2048 306 -> 222,
+// 512 x 2048 x 6400 299 -> 237, with A transposed 281 -> 222 (60 TFLOP/s), 4096^3 59 -> 64 TFLOP/s (the library: 72);
+// a step's product 16 x 256 x 64 5.3 -> 5.2, 16 x 808 x 202 15.1 -> 12.2, 16 x 3072 x 768 13.1 -> 13.0.
+// How a product is cut depends on its shape and the device, and where the scratch buffer has no room for the pieces it is
+// not: the same call gives the same bits with any workspace that holds them.  Lane layout of the instruction (checked on the hardware): a = A[i = lane%16][k = lane/16], b = B[k = lane/16][j = lane%16],
 // d[r] = D[i = 4*r + lane/16][j = lane%16].
 #include "common.h"
 
@@ -58,12 +59,18 @@ void gemm_f64_kernel(int M, int N, int K, const double* __restrict__ A, int lda,
   // round-robin; an XCD (one L2) gets a contiguous run of the whole tiles, and of the pieces.
   int tile, piece = 0;
   {
-    const int id = blockIdx.x, first = id < plan.whole ? 0 : plan.whole;
-    const int count = id < plan.whole ? plan.whole : (int)gridDim.x - plan.whole;
-    const int xcd = (id - first) % kXcds, q = count / kXcds, r = count % kXcds;
-    const int at = xcd * q + (xcd < r ? xcd : r) + (id - first) / kXcds;
-    tile = first == 0 && id < plan.whole ? at : plan.whole + at / plan.pieces;
-    piece = id < plan.whole ? 0 : at % plan.pieces;
+    const int id = blockIdx.x;
+    auto mine = [](int at, int count) {
+      const int xcd = at % kXcds, q = count / kXcds, r = count % kXcds;
+      return xcd * q + (xcd < r ? xcd : r) + at / kXcds;
+    };
+    if (id < plan.whole) {
+      tile = mine(id, plan.whole);
+    } else {
+      const int at = mine(id - plan.whole, (int)gridDim.x - plan.whole);
+      tile = plan.whole + at / plan.pieces;
+      piece = at % plan.pieces;
+    }
   }
   const int m0 = tile / tiles_n * DM, n0 = tile % tiles_n * DN;
   const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
@@ -191,10 +198,10 @@ void gemm_f64_kernel(int M, int N, int K, const double* __restrict__ A, int lda,
     }
   };
   // Panel p lies in buffer p % 2; at its turn the panel behind it is parked in the other buffer,
-  // which everybody has finished with, and the one three behind requested.  Without a branch (behind the last panel
-  // that one is read again, for nobody): with one the compiler cannot tell which loads a panel waits for, and waited
-  // for all of them, and read the operands of a group when its instructions were due.
-  // (6400 x 2048 x 512 271 -> 262 us, 512 x 2048 x 6400 296 -> 277, with A transposed 278 -> 258.)
+  // which everybody has finished with, and the one three behind requested.  Without a branch: with one the compiler cannot
+  // tell which loads a panel waits for, and waited for all of them, and read the operands of a group when its instructions
+  // were due.  (6400 x 2048 x 512 271 -> 262 us, 512 x 2048 x 6400 296 -> 277, with A transposed 278 -> 258.)  The last
+  // one or two panels are written out: a turn of the barrier or a wait for nobody shows in the product of a step.
   auto run = [&](auto fast_c) {
     const int last = k_begin + (K - k_begin - 1) / DK * DK;
     auto panel = [&](auto parity, int k0) {
@@ -205,19 +212,53 @@ void gemm_f64_kernel(int M, int N, int K, const double* __restrict__ A, int lda,
       });
       __syncthreads();
     };
+    auto finish = [&](int k0) {
+      const bool two = k0 + DK < K;
+      multiply(0, [&](int g) {
+        if (g == 1 && two) park(1, 1);
+      });
+      if (!two) return;
+      __syncthreads();
+      multiply(1, [](int) {});
+    };
     request(fast_c, 0, k_begin);
-    request(fast_c, 1, k_begin + DK < last ? k_begin + DK : last);
+    if (K - k_begin <= 2 * DK) {
+      if (k_begin + DK < K) request(fast_c, 1, k_begin + DK);
+      park(0, 0);
+      __syncthreads();
+      return finish(k_begin);
+    }
+    request(fast_c, 1, k_begin + DK);
     park(0, 0);
-    request(fast_c, 0, k_begin + 2 * DK < last ? k_begin + 2 * DK : last);
+    request(fast_c, 0, k_begin + 2 * DK);
     __syncthreads();
     int k0 = k_begin;
-    for (; k0 + DK < K; k0 += 2 * DK) {
+    for (; k0 + 2 * DK < K; k0 += 2 * DK) {
       panel(std::integral_constant<int, 0>{}, k0);
       panel(std::integral_constant<int, 1>{}, k0 + DK);
     }
-    if (k0 < K) multiply(0, [](int) {});
+    finish(k0);
   };
-  if (!fast) run(std::integral_constant<int, kSingle>{});
+  // Element by element the loads are branches, many instructions each: all of them in front of a panel's product.
+  auto run_single = [&] {
+    const std::integral_constant<int, kSingle> single{};
+    auto panel = [&](int p, int k0) {
+      if (k0 + DK < K) park(p ^ 1, p ^ 1);
+      if (k0 + 3 * DK < K) request(single, p ^ 1, k0 + 3 * DK);
+      multiply(p, [](int) {});
+      __syncthreads();
+    };
+    request(single, 0, k_begin);
+    if (k_begin + DK < K) request(single, 1, k_begin + DK);
+    park(0, 0);
+    if (k_begin + 2 * DK < K) request(single, 0, k_begin + 2 * DK);
+    __syncthreads();
+    for (int k0 = k_begin; k0 < K; k0 += 2 * DK) {
+      panel(0, k0);
+      if (k0 + DK < K) panel(1, k0 + DK);
+    }
+  };
+  if (!fast) run_single();
   else if ((K - k_begin) % DK == 0) run(std::integral_constant<int, kWhole>{});
   else run(std::integral_constant<int, kPairs>{});
 #pragma unroll
@@ -235,22 +276,23 @@ void gemm_f64_kernel(int M, int N, int K, const double* __restrict__ A, int lda,
       }
 }
 
-// C (+)= the pieces of every element of the cut tiles, added in index order.  A workgroup takes 16 rows of a tile, a
-// thread four columns.
+// C (+)= the pieces of every element of the cut tiles, added in index order.  A workgroup takes kReduceRows rows of a tile, a
+// thread two columns.
+constexpr int kReduceRows = 8;
 __global__ __launch_bounds__(256)
 void gemm_f64_reduce_kernel(int M, int N, F64Plan plan, int tiles_n, const double* __restrict__ part,
                             double* __restrict__ C, int ldc, int accumulate) {
   const int tile = plan.whole + blockIdx.x;
-  const int r = blockIdx.y * 16 + (threadIdx.x >> 4), c = (threadIdx.x & 15) * 4;
+  const int r = blockIdx.y * kReduceRows + (threadIdx.x >> 5), c = (threadIdx.x & 31) * 2;
   const int row = tile / tiles_n * DM + r, col = tile % tiles_n * DN + c;
   if (row >= M || col >= N) return;
   const double* p = part + (size_t)blockIdx.x * plan.pieces * DM * DN + r * DN + c;
-  double4_t s = *reinterpret_cast<const double4_t*>(p);
+  double2_t s = *reinterpret_cast<const double2_t*>(p);
 #pragma unroll 8  // (eight pieces' loads in flight: 24 pieces of 4 x 768 4.5 -> 4.0 us)
-  for (int z = 1; z < plan.pieces; ++z) s += *reinterpret_cast<const double4_t*>(p + (size_t)z * DM * DN);
+  for (int z = 1; z < plan.pieces; ++z) s += *reinterpret_cast<const double2_t*>(p + (size_t)z * DM * DN);
   double* out = C + (size_t)row * ldc + col;
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < 2; ++i)
     if (col + i < N) out[i] = accumulate ? out[i] + s[i] : s[i];
 }
 
@@ -475,10 +517,10 @@ int gemm_f64(hipStream_t stream, bool trans_a, int M, int N, int K, const double
   double* part = nullptr;
   if (plan.pieces > 1) {  // not cut without room for the pieces (a caller's own buffer, a capture, a buffer in use)
     const size_t bytes = scratch_offset + f64_piece_bytes(plan, M, N);
-    bool room;
-    HASTE_HIP_PROPAGATE(workspace_has_room(stream, bytes, &room));
+    bool room = false;
+    if (scratch_offset == 0) HASTE_HIP_PROPAGATE(workspace_has_room(stream, bytes, &room));
     Workspace ws;
-    HASTE_HIP_PROPAGATE(get_workspace(stream, room && scratch_offset == 0 ? bytes : 0, &ws));
+    HASTE_HIP_PROPAGATE(get_workspace(stream, room ? bytes : 0, &ws));
     if (ws.scratch_bytes >= bytes) part = reinterpret_cast<double*>(reinterpret_cast<char*>(ws.scratch) + scratch_offset);
     else plan = F64Plan{(int)tiles, 1, K};
   }
@@ -494,7 +536,7 @@ int gemm_f64(hipStream_t stream, bool trans_a, int M, int N, int K, const double
                                                            panels_fit(false, M, N, K, lda, ldb));
   HASTE_HIP_TRY(hipGetLastError());
   if (rest > 0) {
-    gemm_f64_reduce_kernel<<<dim3((unsigned)rest, DM / 16), dim3(256), 0, stream>>>(M, N, plan, tiles_n, part, C, ldc,
+    gemm_f64_reduce_kernel<<<dim3((unsigned)rest, DM / kReduceRows), dim3(256), 0, stream>>>(M, N, plan, tiles_n, part, C, ldc,
                                                                                      accumulate ? 1 : 0);
     HASTE_HIP_TRY(hipGetLastError());
   }

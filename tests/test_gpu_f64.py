@@ -144,6 +144,14 @@ def test_f64_gemm_in_pieces(trans_a, M, N, K, room):
     assert (out[:, N:] == 7.0).all()
 
 
+# One to five panels of 32 k, whole, a pair and an element longer, the last ones written out: loads in whole panels, in pairs
+# (even sizes) and element by element (odd ones).
+@pytest.mark.parametrize("K", [1, 2, 31, 32, 33, 34, 64, 65, 66, 96, 97, 98, 128, 129, 130, 160, 161, 162])
+@pytest.mark.parametrize("trans_a,M,N", [(False, 70, 66), (True, 70, 66), (True, 67, 65)])
+def test_f64_gemm_short_contractions(trans_a, M, N, K):
+    test_f64_gemm_in_pieces(trans_a, M, N, K, True)
+
+
 def test_f64_layers_match_torch_nn():
     """haste_amd.LSTM / GRU in double against torch.nn.LSTM / GRU in double on the CPU."""
     import torch
