@@ -299,29 +299,43 @@ void gemm_f64_reduce_kernel(int M, int N, F64Plan plan, int tiles_n, const doubl
 // Whole tiles for full rounds of one per CU (a CU holds two workgroups, which share its matrix cores); the tiles of the
 // last, partial round are cut along K into pieces that make about two per CU, a piece keeping at least 8 panels of the
 // contraction (its first panel's load and its 64 KiB of partial results show below that).  A last round of more than
-// three quarters of the CUs has too little to give: stays whole.  A product of no more tiles than CUs is all cut, to
-// pieces of at least 4 panels: with one workgroup per CU its barriers and first loads show (512 x 2048 x 6400, 256
-// tiles: 258 us whole, 238 in two pieces; 6400 x 512 x 2048, 800 tiles: 295 whole, 222 with the last 32 in 8).  Where the
-// shortest piece keeps that to little more than one per CU, the CUs with two hold up the others, and it is one per CU (4 x
-// 768 x 3072: 288 pieces of 4 panels 14.2 us, 240 of 5 10.4).
+// three quarters of the CUs has too little to give: stays whole (6400 x 512 x 2048, 800 tiles: 295 us whole, 222 with the last
+// 32 in 8).  A product of no more tiles than CUs is cut into the number of pieces that is expected to be fastest, of at
+// least 4 panels.  Measured, in us: 5.5 and 1.25 a panel for whole tiles; 4.5 and 0.02 a workgroup for the pieces' way through
+// memory, 1.25 a panel again, 2 where two workgroups share a CU.  (512 x 2048 x 256 / 1024 / 6400, 256 tiles: 15.3 / 46.5 / 258
+// whole, 22.8 / 48.5 / 238 in two; 256 x 2048 x 1024: 45.7 whole, 31.3 in four; 64 x 2048 x 2048: 22.4 in 16, 19.4 in 8; 4 x
+// 768 x 3072: 14.2 in 24, 10.4 in 20.)
 F64Plan plan_f64(int M, int N, int K) {
   const long long tiles = (long long)((M + DM - 1) / DM) * ((N + DN - 1) / DN);
   const long long cus = device_cu_count() > 0 ? device_cu_count() : 256;
-  long long whole = tiles > cus ? tiles / cus * cus : 0;
+  const F64Plan uncut{(int)tiles, 1, K};
+  const long long whole = tiles > cus ? tiles / cus * cus : 0;
   const long long rest = tiles - whole;
-  long long s = rest > 0 ? 2 * cus / rest : 1;
-  const long long most = K / ((whole > 0 ? 8 : 4) * DK);
-  s = s < most ? s : most;
-  s = s < 64 ? s : 64;
-  if (s <= 1 || (whole > 0 && 4 * rest > 3 * cus)) return F64Plan{(int)tiles, 1, K};
+  if (rest == 0) return uncut;
   auto cut = [&](long long pieces) {
     const int per = ((int)((K + pieces - 1) / pieces) + DK - 1) / DK * DK;
     return F64Plan{(int)whole, (K + per - 1) / per, per};
   };
-  auto turns = [&](const F64Plan& p) { return (rest * p.pieces + cus - 1) / cus * p.k_per_piece; };
-  const F64Plan two = cut(s), one = cut(s < cus / rest ? s : cus / rest);
-  if (whole > 0 || turns(two) <= turns(one)) return two;
-  return one.pieces > 1 ? one : F64Plan{(int)tiles, 1, K};
+  long long most = K / ((whole > 0 ? 8 : 4) * DK);
+  most = most < 64 ? most : 64;
+  if (whole > 0) {
+    const long long pieces = 2 * cus / rest < most ? 2 * cus / rest : most;
+    if (pieces <= 1 || 4 * rest > 3 * cus) return uncut;
+    const F64Plan p = cut(pieces);
+    return p.pieces > 1 ? p : uncut;
+  }
+  F64Plan best = uncut;
+  long long best_cost = 275 + 62ll * ((K + DK - 1) / DK);  // 1/50 us
+  for (long long pieces = 2; pieces <= most && tiles * pieces <= 2 * cus; ++pieces) {
+    const F64Plan p = cut(pieces);
+    const long long workgroups = tiles * p.pieces;
+    const long long cost = 225 + workgroups + (workgroups > cus ? 100 : 62) * (p.k_per_piece / DK);
+    if (p.pieces > 1 && cost < best_cost) {
+      best = p;
+      best_cost = cost;
+    }
+  }
+  return best;
 }
 // The same for a consumer that adds the pieces itself: all tiles, about one piece per CU.
 F64Plan plan_f64_chunks(int M, int N, int K) {
