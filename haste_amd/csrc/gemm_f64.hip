@@ -42,6 +42,7 @@ __device__ __forceinline__ int panel_at(int k, int i) {
 // How a product is cut: the first `whole` tiles (row by row) are not, the others into `pieces` of k_per_piece each.
 struct F64Plan {
   int whole, pieces, k_per_piece;
+  int in_order = 0;
 };
 constexpr int kXcds = 8;
 
@@ -55,8 +56,8 @@ void gemm_f64_kernel(int M, int N, int K, const double* __restrict__ A, int lda,
                      int accumulate, F64Plan plan, int tiles_n, double* __restrict__ part, int chunks, int panels_ok) {
   __shared__ double2_t panels[2][2][DK * 64 / 2];  // [buffer][A, B]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  // Workgroups [0, whole) take a tile each, the others a piece of one of the remaining tiles.  Ids go to the XCDs
-  // round-robin; an XCD (one L2) gets a contiguous run of the whole tiles, and of the pieces.
+  // Workgroups [0, whole) take a tile each, in_order or with a contiguous run of them for every XCD (ids go to the XCDs
+  // round-robin; see tiles_in_order), the others a piece of one of the remaining tiles, an XCD a run of them.
   int tile, piece = 0;
   {
     const int id = blockIdx.x;
@@ -65,7 +66,7 @@ void gemm_f64_kernel(int M, int N, int K, const double* __restrict__ A, int lda,
       return xcd * q + (xcd < r ? xcd : r) + at / kXcds;
     };
     if (id < plan.whole) {
-      tile = mine(id, plan.whole);
+      tile = plan.in_order ? id : mine(id, plan.whole);
     } else {
       const int at = mine(id - plan.whole, (int)gridDim.x - plan.whole);
       tile = plan.whole + at / plan.pieces;
@@ -296,6 +297,21 @@ void gemm_f64_reduce_kernel(int M, int N, F64Plan plan, int tiles_n, const doubl
     if (col + i < N) out[i] = accumulate ? out[i] + s[i] : s[i];
 }
 
+// Whether the whole tiles go to the workgroups as they are numbered, so that XCD x (one L2) gets number x and every eighth
+// from there, rather than in a contiguous run per XCD: what reads fewer panels of A and B into an L2.  With a multiple of eight
+// columns of tiles an XCD's are the same in every row and only the tiles in flight count; with four they alternate; otherwise all
+// columns take turns.  (In order / in runs, us: 32 columns, 6400 x 2048 x 512 228 / 235, 768 x 2048 x 256 added to C 23.1 / 27.3;
+// 28 columns, 512 x 1792 x 256 15.1 / 18.4; 8 columns, 6400 x 512 x 2048 225 / 222; 13 columns, 6400 x 808 x 512 106 / 103,
+// 1500 x 808 x 128 added to C 17.8 / 15.0.)
+bool tiles_in_order(long long tiles_m, long long tiles_n, long long whole, long long cus) {
+  const int every = tiles_n % 8 == 0 ? 8 : (tiles_n % 4 == 0 ? 4 : 1);
+  if (every == 1) return false;
+  long long mine = whole / kXcds;
+  if (every == 8 && mine > 2 * cus / kXcds) mine = 2 * cus / kXcds;
+  const long long run_rows = (mine + tiles_n - 1) / tiles_n, order_rows = (mine * kXcds + tiles_n - 1) / tiles_n;
+  return (order_rows < tiles_m ? order_rows : tiles_m) + tiles_n / every < run_rows + (mine < tiles_n ? mine : tiles_n);
+}
+
 // Whole tiles for full rounds of one per CU (a CU holds two workgroups, which share its matrix cores); the tiles of the
 // last, partial round are cut along K into pieces that make about two per CU, a piece keeping at least 8 panels of the
 // contraction (its first panel's load and its 64 KiB of partial results show below that).  A last round of more than
@@ -306,15 +322,15 @@ void gemm_f64_reduce_kernel(int M, int N, F64Plan plan, int tiles_n, const doubl
 // whole, 22.8 / 48.5 / 238 in two; 256 x 2048 x 1024: 45.7 whole, 31.3 in four; 64 x 2048 x 2048: 22.4 in 16, 19.4 in 8; 4 x
 // 768 x 3072: 14.2 in 24, 10.4 in 20.)
 F64Plan plan_f64(int M, int N, int K) {
-  const long long tiles = (long long)((M + DM - 1) / DM) * ((N + DN - 1) / DN);
+  const long long tiles_m = (M + DM - 1) / DM, tiles_n = (N + DN - 1) / DN, tiles = tiles_m * tiles_n;
   const long long cus = device_cu_count() > 0 ? device_cu_count() : 256;
-  const F64Plan uncut{(int)tiles, 1, K};
+  const F64Plan uncut{(int)tiles, 1, K, tiles_in_order(tiles_m, tiles_n, tiles, cus)};
   const long long whole = tiles > cus ? tiles / cus * cus : 0;
   const long long rest = tiles - whole;
   if (rest == 0) return uncut;
   auto cut = [&](long long pieces) {
     const int per = ((int)((K + pieces - 1) / pieces) + DK - 1) / DK * DK;
-    return F64Plan{(int)whole, (K + per - 1) / per, per};
+    return F64Plan{(int)whole, (K + per - 1) / per, per, tiles_in_order(tiles_m, tiles_n, whole, cus)};
   };
   long long most = K / ((whole > 0 ? 8 : 4) * DK);
   most = most < 64 ? most : 64;

@@ -115,7 +115,9 @@ def test_f64_gemm_and_transpose(trans_a, M, N, K, accumulate):
     # pieces of fewer rows and columns than a tile
     (False, 4, 130, 1030), (True, 67, 5, 1031), (False, 1, 1, 4096),
     # two pieces of whole panels are longer than the product: not cut
-    (True, 520, 1560, 333)])
+    (True, 520, 1560, 333),
+    # whole tiles taken as they are numbered: 28 columns of tiles, 24 with the last tiles cut
+    (False, 520, 1792, 40), (True, 1100, 1536, 512)])
 @pytest.mark.parametrize("room", [True, False])
 def test_f64_gemm_in_pieces(trans_a, M, N, K, room):
     """Error of a sum of K products in double, in any order: below K * 2^-53 of the sum of their magnitudes.  Without
