@@ -129,3 +129,28 @@ def test_a_workspace_of_the_stated_size_decides_nothing(gates, size, backward):
                 rc, plan = _plan_pass(lib, 256, 8, gates, size, backward, T, N, C, H, own[1][6] * 512)
                 fewer += rc != 0 or plan[:6] != own[1][:6]
     assert fewer > 0
+
+
+def test_the_tests_of_the_split_recurrences_reach_them():
+    """The shapes that tests/test_gpu_split_recurrence.py means to run on the bf16 matrix cores do, on eight XCDs of 32 CUs."""
+    import test_gpu_split_recurrence as t
+    lib = hlib.load()
+
+    def kernel(gates, backward, T, N, H, C):
+        rc, plan = _plan_pass(lib, 256, 8, gates, 4, backward, T, N, C, H)
+        assert rc == 0
+        return plan[0], plan[1]
+    heights = set()
+    for gates in (3, 4):
+        for backward, shapes, C in ((0, t.FORWARD, 18), (0, t.EXTREME_FORWARD, 13), (1, t.BACKWARD, 12), (1, t.EXTREME_BACKWARD, 8),
+                                    (0, [(100, N, 512) for _, N in t.FP32_ERRORS], 512),
+                                    (1, [(100, N, 512) for _, N in t.FP32_ERRORS], 512)):
+            for T, N, H in shapes:
+                which, rows = kernel(gates, backward, T, N, H, C)
+                assert which == 3, (gates, backward, T, N, H)
+                heights.add((gates, backward, shapes is t.EXTREME_FORWARD or shapes is t.EXTREME_BACKWARD, rows))
+        for T, N, H in t.BESIDE_BACKWARD + t.EXTREME_BESIDE_BACKWARD:
+            assert kernel(gates, 1, T, N, H, 12)[0] == 2, (gates, T, N, H)
+    # every tile height, ordinary values and extreme ones
+    assert heights == {(gates, backward, extreme, rows) for gates in (3, 4) for extreme in (False, True)
+                       for backward, rows in ((0, 4), (0, 8), (0, 16), (1, 8), (1, 16))}
