@@ -21,9 +21,9 @@
 //     they neither delay an operand nor a look at the barrier's flags.
 // Bound: the chain exchange - operand load - product - pointwise math of a step (a tanh takes 0.3 us, two follow each
 // other).  The matrix cores need 1.9 us of a step.
-// Measured per step at N = 64, H = 512, LSTM, step-wise -> 16 rows -> 8 rows: forward 14.7 -> 6.1 -> 5.3 us, backward
-// 14.9 -> 8.4 -> 5.5 us.  Whole training passes, 16 rows behind barriers -> now (with gemm_f64's changes), T = 100: LSTM
-// N = 64, H = 512 2.70 -> 2.27 ms, GRU 2.33 -> 1.85; N = 64, H = 128 0.81 -> 0.67; GRU N = 5, H = 64 0.52 -> 0.44;
+// Measured per step at N = 64, H = 512, LSTM, step-wise -> 16 rows -> 8 rows (launches of 100 steps, set-up included): forward
+// 14.7 -> 6.1 -> 5.6 us, backward 14.9 -> 8.4 -> 6.4 us.  Whole training passes, 16 rows behind barriers -> now (with
+// gemm_f64's changes), T = 100: LSTM N = 64, H = 512 2.70 -> 2.20 ms, GRU 2.33 -> 1.85; N = 64, H = 128 0.81 -> 0.67; GRU N = 5, H = 64 0.52 -> 0.44;
 // T = 50: N = 32, H = 768 1.77 -> 1.49, N = 40, H = 700 2.52 -> 1.59.
 #include "recurrent.h"
 

@@ -45,7 +45,7 @@ const char* haste_hip_last_runtime_error(void);
 int haste_hip_max_hidden_size(int gates, int batch_size);
 
 /* How Run would lay the persistent recurrences of a cell with `gates` gate blocks (4 LSTM, 3 GRU)
- * out for this batch and hidden size on a device of `cus` compute units in `xcds` XCDs that take
+ * out on the fp32 matrix instruction (haste_hip_plan_recurrence: what a pass really takes) for this batch and hidden size on a device of `cus` compute units in `xcds` XCDs that take
  * workgroups evenly (cus == 0: the current device as the library found it; xcds == 0: no
  * placement by XCD).  Touches no device when cus > 0.  plan[0..7] describes the forward
  * recurrence, plan[8..15] the backward one: {found (0: the cell streams the recurrent matrix
