@@ -58,6 +58,18 @@ def test_plan_tiles_refuses_bad_arguments():
     assert lib.haste_hip_plan_tiles(0, 8, 4, 4, 64, out) != 0
 
 
+def test_plan_recurrence_refuses_bad_arguments():
+    lib = hlib.load()
+    good = (256, 8, 4, 4, 0, 30, 64, 512, 512)
+    assert _plan_pass(lib, *good)[0] == 0
+    for at, value in [(0, -1), (0, 0), (2, 5), (2, 2), (3, 2), (5, 0), (6, 0), (7, 0), (8, -3)]:
+        bad = list(good)
+        bad[at] = value
+        assert _plan_pass(lib, *bad)[0] != 0, bad
+    assert _plan_pass(lib, *good, workspace=64)[0] != 0
+    assert lib.haste_hip_plan_recurrence(*good, ctypes.c_size_t(0), None) != 0
+
+
 PASSES = [(gates, size, backward) for gates in (3, 4) for size in (4, 8) for backward in (0, 1)]
 
 
