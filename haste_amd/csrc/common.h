@@ -297,6 +297,25 @@ int layer_norm_gru_backward_streamed(hipStream_t stream, int T, int N, int C, in
                                      float* dgamma2, const float* cache2,
                                      const float* zoneout_mask);
 
+// The recurrence cut along the contraction and the columns (cut_recurrence.h), where it is the faster one: *taken.  Forward
+// with the product x * W (GRU: unless it is there), backward without the products around it.  beyond_lds: see cut_pays.
+int lstm_forward_cut(hipStream_t stream, int training, int T, int N, int C, int H, const float* W, const float* R,
+                     const float* b, const float* x, const float* h, const float* c, float* h_out, float* c_out, float* v,
+                     float zoneout_prob, const float* zoneout_mask, const float* dc_mask, float dc_scale, bool beyond_lds, bool* taken);
+int lstm_backward_cut(hipStream_t stream, int T, int N, int H, const float* R_t, const float* c, const float* c_next,
+                      const float* dh_next, const float* dc_next, float* db, float* dh, float* dc, float* v,
+                      const float* zoneout_mask, bool beyond_lds, bool* taken);
+int gru_forward_cut(hipStream_t stream, int training, int T, int N, int C, int H, const float* W, const float* R,
+                    const float* bx, const float* br, const float* x, const float* h, float* h_out, float* v,
+                    float* tmp_Wx, float zoneout_prob, const float* zoneout_mask, const float* dc_mask, float dc_scale,
+                    bool wx_ready, bool beyond_lds, bool* taken);
+int gru_backward_cut(hipStream_t stream, int T, int N, int H, const float* R_t, const float* h, const float* v,
+                     const float* dh_next, float* dbx, float* dbr, float* dh, float* dp, float* dq,
+                     const float* zoneout_mask, bool beyond_lds, bool* taken);
+
+// Bytes of scratch they may ask for on a device of `cus` compute units, whatever its XCDs.
+size_t cut_scratch_bound(int N, int H, int cus);
+
 // One forward step for a batch of at most 8 rows as a single kernel (single_step.hip): what the
 // Iterate entry points and one-step Run calls use.
 bool single_step_applies(int N, int C, int H);
@@ -321,6 +340,9 @@ int layer_norm_forward_wide(hipStream_t stream, int rows, int dim, const float* 
 int layer_norm_backward_wide(hipStream_t stream, int rows, int dim, const float* gamma,
                              const float* x, const float* dy, float* dx, float* dgamma,
                              float* dbeta);
+
+// out[i] = weights[i] * mask[i] * scale (stepwise.hip): the recurrent matrix under DropConnect.
+int scale_weights(hipStream_t stream, size_t n, const float* weights, const float* mask, float scale, float* out);
 
 // Row-wise layer norm kernels (rows x dim), used stand-alone and by the LN cells.
 int layer_norm_forward(hipStream_t stream, int rows, int dim, const float* gamma,

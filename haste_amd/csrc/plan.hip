@@ -1,5 +1,7 @@
 // What runs the recurrence of an LSTM or GRU pass, found by going through the pass's own choices without a launch.
-#include "recurrent.h"
+#include "cut_recurrence.h"
+#include "gru_cells.h"
+#include "lstm_cells.h"
 
 namespace haste_hip {
 
@@ -31,6 +33,22 @@ int lstm_backward_recurrence64(hipStream_t stream, int T, int N, int H, const do
 int gru_backward_recurrence64(hipStream_t stream, int T, int N, int H, const double* R_t, const double* h,
                               const double* v, const double* dh_next, double* dh, double* dp, double* dq,
                               const double* mask, void* exchange);
+
+size_t cut_scratch_bound(int N, int H, int cus) {
+  size_t most = 0;
+  for (int xcds = 1; xcds <= cus; ++xcds) {
+    if (cus % xcds != 0) continue;
+    auto ask = [&](const CutPlan& plan, size_t weights) {
+      if (plan.ok && plan.bytes() + weights > most) most = plan.bytes() + weights;
+    };
+    const size_t weights = ((size_t)4 * H * H + 64) * sizeof(float);
+    ask(cut_plan<LstmForwardCell, false>(N, H, cus, xcds), weights);
+    ask(cut_plan<LstmScatterCell, true>(N, H, cus, xcds), 0);
+    ask(cut_plan<GruForwardCell, false>(N, H, cus, xcds), weights);
+    ask(cut_plan<GruScatterCell, true>(N, H, cus, xcds), 0);
+  }
+  return most;
+}
 
 int plan_recurrence(int gates, int element_bytes, bool backward, int T, int N, int C, int H) {
   const bool lstm = gates == 4;

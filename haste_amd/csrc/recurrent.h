@@ -1584,6 +1584,7 @@ struct LaunchPlan {
   LaunchShape shape;
   int threads = 256;  // 512: two 256-thread sets per workgroup
   int kernel = kPlanFloat;  // for a pass that is planned only
+  int group_workgroups = 0, groups = 0, tiles_each = 0;  // the same, where a group is several XCDs: its workgroups and so on
 };
 
 inline bool xcd_local_fits(int gx, int gy) {
@@ -1649,6 +1650,12 @@ int launch_persistent(const char* name, KernelT kernel, const LaunchPlan& plan, 
     pass->gx = plan.shape.gx;
     pass->gy = plan.shape.gy;
     pass->xcd_local = plan.shape.xcd_local;
+    if (plan.groups > 0) {
+      pass->sets = plan.tiles_each;
+      pass->gx = plan.group_workgroups;
+      pass->gy = plan.groups;
+      pass->xcd_local = plan.group_workgroups == plan.shape.gx ? 1 : 0;
+    }
     return HASTE_HIP_OK;
   }
   // The kernel's LDS limit and its occupancy at this request are looked up once per process

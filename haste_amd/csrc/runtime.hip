@@ -696,6 +696,8 @@ size_t haste_hip_workspace_bytes(int time_steps, int batch_size, int input_size,
   // Backward recurrences of 4-row tiles in scattered form (H <= 512): two tiles of pieces per
   // tile of 4 rows, [owners][up to 32 producers][64].
   if (H <= 512) b += (N / 4 + 2) * 2 * (H / 16 + 1) * 32 * 64 * sizeof(float);
+  // Recurrences cut along the contraction and the columns.
+  if (H > 512 && H <= 8192 && N <= 4096) b += cut_scratch_bound(batch_size, hidden_size, (int)cus);
   // Step-wise regime (any scalar type up to 8 bytes): the step's product [N, 4H], a scaled
   // copy of R, column sums in at most 128 chunks, row statistics of all steps, two [N, H]
   // buffers; the stand-alone layer norm's column sums (two workgroups per CU, two rows each).

@@ -1201,6 +1201,12 @@ int indrnn_backward_steps(hipStream_t stream, int steps, int N, int C, int H, co
 }  // namespace
 
 // ---- float: what the persistent implementations fall back to -------------------------------
+int scale_weights(hipStream_t stream, size_t n, const float* weights, const float* mask, float scale, float* out) {
+  if (planned_pass() != nullptr) return HASTE_HIP_OK;
+  const float* scaled = nullptr;
+  return effective_r<float>(stream, n, weights, mask, scale, out, &scaled);
+}
+
 int lstm_forward_streamed(hipStream_t stream, int training, int T, int N, int C, int H,
                           const float* W, const float* R, const float* b, const float* x,
                           const float* h, const float* c, float* h_out, float* c_out, float* v,

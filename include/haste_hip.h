@@ -63,7 +63,7 @@ int haste_hip_plan_tiles(int cus, int xcds, int gates, int batch_size, int hidde
  * plan[0]: 0 step by step, the recurrent matrix streamed; 1 a single step in one kernel; 2 one
  * launch on the fp32 matrix instruction; 3 on the bf16 matrix cores, operands as sums of three;
  * 4 in double.  plan[1..5], of the one launch: batch rows per tile, tiles a workgroup works on side by
- * side, column workgroups, batch tiles, whether each tile's workgroups share an XCD.  plan[6]: KiB
+ * side or in turn, workgroups that share a tile, tiles (sets of them) at a time, whether each tile's workgroups share an XCD.  plan[6]: KiB
  * of workspace that were asked for (in double: for the one launch alone).  plan[7]: 0.  Returns what
  * the pass would. */
 int haste_hip_plan_recurrence(int cus, int xcds, int gates, int element_bytes, int backward, int time_steps,

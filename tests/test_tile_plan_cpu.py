@@ -166,3 +166,21 @@ def test_the_tests_of_the_split_recurrences_reach_them():
     # every tile height, ordinary values and extreme ones
     assert heights == {(gates, backward, extreme, rows) for gates in (3, 4) for extreme in (False, True)
                        for backward, rows in ((0, 4), (0, 8), (0, 16), (1, 8), (1, 16))}
+
+
+def test_the_tests_of_the_cut_recurrences_reach_them():
+    """The shapes that tests/test_gpu_cut_recurrence.py means to run on groups of several XCDs do, on eight XCDs of 32 CUs, where a
+    pass has enough steps; every number of XCDs per group and of batch tiles is among them."""
+    import test_gpu_cut_recurrence as t
+    lib = hlib.load()
+    seen = set()
+    for gates in (3, 4):
+        for backward in (0, 1):
+            for T, N, H in t.SHAPES + t.EXTREME + [t.MANY_NANS, (5, 50, 700), (5, 20, 1300), (4, 40, 1300)]:
+                rc, plan = _plan_pass(lib, 256, 8, gates, 4, backward, T, N, 12, H)
+                assert rc == 0 and plan[0] == 3 and plan[3] > 32, (gates, backward, T, N, H, plan)
+                seen.add((backward, plan[3] // 32, min(plan[2], 3)))
+                rc, few = _plan_pass(lib, 256, 8, gates, 4, backward, 3, N, 12, H)
+                assert rc == 0 and few[0] != 3, (gates, backward, N, H)
+    assert {(b, xcds) for b, xcds, _ in seen} == {(b, xcds) for b in (0, 1) for xcds in (2, 4, 8)}
+    assert {(b, tiles) for b, _, tiles in seen} == {(b, tiles) for b in (0, 1) for tiles in (1, 2, 3)}
