@@ -93,14 +93,28 @@ def _wrapped(a):
     return ctypes.c_longlong(a)
 
 
+def _current_stream():
+    """The address of torch's current stream: what torch.cuda.current_stream().cuda_stream is, without an object for it
+    (2.5 us of a call's 13)."""
+    if _raw_stream is None or not torch.cuda.is_initialized():
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(torch.cuda.current_device())
+
+
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
+def invoke(name, fn, values, stream=None):
+    """Calls the entry point `fn` (of that name) with ints, floats and addresses, plus the stream."""
+    values.append(_current_stream() if stream is None else stream)
+    rc = fn(*values) if fn.argtypes is not None else fn(*map(_wrapped, values))
+    if rc != 0:
+        raise HasteHipError(rc, name)
+
+
 def call(name, *args, stream=None):
     """Calls entry point `name` with ints/floats/tensors/addresses (None = NULL) plus the stream."""
     fn = entry(name)
     if fn is None:
         raise AttributeError("libhaste_hip.so has no entry point " + name)
-    if stream is None:
-        stream = torch.cuda.current_stream().cuda_stream
-    args = [a.data_ptr() if isinstance(a, torch.Tensor) else a for a in args] + [stream]
-    rc = fn(*args) if fn.argtypes is not None else fn(*map(_wrapped, args))
-    if rc != 0:
-        raise HasteHipError(rc, name)
+    invoke(name, fn, [a.data_ptr() if isinstance(a, torch.Tensor) else a for a in args], stream)

@@ -32,19 +32,24 @@ def _call(entry, *args):
     have one dtype (the reference's bindings dispatch the same way, AT_DISPATCH_FLOATING_TYPES,
     frameworks/pytorch/lstm.cc:65)."""
     dtype = None
-    for a in args:
-        if isinstance(a, torch.Tensor) and a.dtype is not dtype and a.numel():
-            if dtype is not None:
-                dtypes = {t.dtype for t in args if isinstance(t, torch.Tensor) and t.numel()}
-                raise ValueError("all tensors of a call must have the same dtype, got %s" % sorted(map(str, dtypes)))
-            dtype = a.dtype
+    values = []
+    for a in args:  # (one pass over them: a single step's call costs as much on the host as on the GPU)
+        if isinstance(a, torch.Tensor):
+            if a.dtype is not dtype and a.numel():
+                if dtype is not None:
+                    dtypes = {t.dtype for t in args if isinstance(t, torch.Tensor) and t.numel()}
+                    raise ValueError("all tensors of a call must have the same dtype, got %s" % sorted(map(str, dtypes)))
+                dtype = a.dtype
+            a = a.data_ptr()
+        values.append(a)
     if dtype is None:
         raise ValueError("all tensors of a call must have the same dtype, got []")
     name = entry + _SUFFIX[dtype]
-    if lib.entry(name) is None:
+    fn = lib.entry(name)
+    if fn is None:
         # as in the reference, half exists for the GRU only (lib/gru_forward_gpu.cu.cc:373)
         raise ValueError("%s is not implemented" % name)
-    lib.call(name, *args)
+    lib.invoke(name, fn, values)
 
 
 def stream_status(stream=None):
