@@ -316,9 +316,13 @@ int gru_backward_cut(hipStream_t stream, int T, int N, int H, const float* R_t, 
 // Bytes of scratch they may ask for on a device of `cus` compute units, whatever its XCDs.
 size_t cut_scratch_bound(int N, int H, int cus);
 
-// One forward step for a batch of at most 8 rows as a single kernel (single_step.hip): what the
-// Iterate entry points and one-step Run calls use.
-bool single_step_applies(int N, int C, int H);
+// One forward step as a single kernel (single_step.hip): what the Iterate entry points and one-step
+// Run calls use, for batches up to a size (single_step_rule: most_blocks blocks of 16 units, rows and
+// contraction indices) that depends on what the step would run on otherwise.
+constexpr long long kStepStreamed = 60 << 10, kStepResident = 128 << 10, kStepHalf = 1ll << 40;
+// staged_bytes: staged_state_bytes() of the call, scratch for a state that is updated in place.
+int single_step_rule(hipStream_t stream, int N, int C, int H, long long most_blocks, size_t staged_bytes, bool* applies);
+size_t staged_state_bytes(int N, int H, const void* h, const void* h_out, size_t element);
 int lstm_forward_single_step(hipStream_t stream, int training, int N, int C, int H, const float* W,
                              const float* R, const float* b, const float* x, const float* h,
                              const float* c, float* h_out, float* c_out, float* v,

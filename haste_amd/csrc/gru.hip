@@ -706,11 +706,18 @@ int gru_forward_impl(hipStream_t stream, int training, int T, int N, int C, int 
   HASTE_HIP_REQUIRE(R && bx && br && h && h_out && tmp_Wx && (wx_ready || (W && x)));
   HASTE_HIP_REQUIRE(!training || v != nullptr);
   HASTE_HIP_REQUIRE(!wx_ready || (T > 1 && gru_forward_resident(N, H)));
-  // A single step of a small batch (Iterate): one kernel, nothing kept on chip (tmp_Wx is
+  // A single step (Iterate): one kernel, nothing kept on chip (tmp_Wx is
   // scratch of the other paths and is left alone).
-  if (T == 1 && single_step_applies(N, C, H))
-    return gru_forward_single_step(stream, training, N, C, H, W, R, bx, br, x, h, h_out, v,
-                                   zoneout_prob, zoneout_mask, dc_mask, dc_scale);
+  if (T == 1) {
+    bool single = false;
+    const size_t staged = staged_state_bytes(N, H, h, h_out, sizeof(float));
+    HASTE_HIP_PROPAGATE(single_step_rule(stream, N, C, H, kStepStreamed, staged, &single));
+    if (!single && pick_forward_tile(3, N, H, 0, kWorkgroupLdsBytes, false, 3).ok)
+      HASTE_HIP_PROPAGATE(single_step_rule(stream, N, C, H, kStepResident, staged, &single));
+    if (single)
+      return gru_forward_single_step(stream, training, N, C, H, W, R, bx, br, x, h, h_out, v,
+                                     zoneout_prob, zoneout_mask, dc_mask, dc_scale);
+  }
   if (N == 1 && H <= 512 && xcd_local_fits((H + 15) / 16, 1))
     return gru_forward_single_row(stream, training, T, C, H, W, R, bx, br, x, h, h_out, v, tmp_Wx,
                                   zoneout_prob, zoneout_mask, dc_mask, dc_scale, wx_ready);

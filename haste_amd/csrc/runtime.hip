@@ -705,8 +705,9 @@ size_t haste_hip_workspace_bytes(int time_steps, int batch_size, int input_size,
   // ... and the K pieces of a double product's last tiles (at most two 64 x 64 pieces per CU)
   b += 2 * cus * 64 * 64 * 8;
   b += 2 * cus * 2 * widest * sizeof(float);
-  // Single forward steps: partial sums of at most 64 runs of the contraction, both sides, for 8
-  // rows and every gate column, and the staged state.
+  // Single forward steps: partial sums of every run of the contraction (four of 4 to 32 rows and 16 units a
+  // workgroup, at most four workgroups per CU and one per tile beyond: larger batches also use the room
+  // of the GEMM and the exchange tiles, which such a step does not touch), and the staged state.
   b += 64 * 2 * 8 * (H / 16 + 1) * 64 * sizeof(float) + 8 * H * sizeof(float) + 256;
   return kControlBytes + 4096 + (b + 255) / 256 * 256;
 }

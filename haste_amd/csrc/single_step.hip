@@ -1,14 +1,14 @@
-// One time step of an LSTM or GRU forward pass for a small batch, as one kernel: what
-// ForwardPass::Iterate (reference lib/haste/lstm.h:73-86, lib/haste/gru.h:72-84) is called for
-// in autoregressive decoding.  The all-steps kernels keep a slice of R on chip for a whole
+// One time step of an LSTM or GRU forward pass as one kernel: what ForwardPass::Iterate
+// (reference lib/haste/lstm.h:73-86, lib/haste/gru.h:72-84) is called for in autoregressive
+// decoding and streaming.  The all-steps kernels keep a slice of R on chip for a whole
 // sequence; for a single step there is nothing to keep -- every weight is used once -- and
 // their set-up (roles, exchange tiles, the slice, a group barrier) and the separate x * W
 // launch cost more than the step.  Here [x_t | h] (length C + H) is multiplied with the stacked
-// [W; R] straight from memory: a workgroup takes 16 hidden units (all their gate columns) and
-// a run of the contraction, parks its partial sums, and the last workgroup of a column block
-// to finish adds the runs in index order and does the pointwise step (gates, cell update,
-// zoneout) -- one launch, no float atomics, results independent of timing.  The GRU's half
-// entry points use the same kernel on half tensors (sums and pointwise step in float).
+// [W; R] straight from memory: a workgroup takes 16 hidden units (all their gate columns), 16 or
+// 32 batch rows and a run of the contraction, parks its partial sums, and the last workgroup of
+// an output tile to finish adds the runs in index order and does the pointwise step (gates, cell
+// update, zoneout) -- one launch, no float atomics, results independent of timing.  The GRU's
+// half entry points use the same kernel on half tensors (sums and pointwise step in float).
 //
 // Arithmetic: reference lib/lstm_forward_gpu.cu.cc:55-86, lib/gru_forward_gpu.cu.cc:46-84.
 #include "recurrent.h"
@@ -17,7 +17,11 @@ namespace haste_hip {
 namespace {
 
 constexpr int kStepUnits = 16;      // hidden units per workgroup
-constexpr int kStepMaxRun = 512;    // contraction indices per workgroup and side
+constexpr int kGroupRows = 16;      // contraction indices per group: four matrix instructions
+constexpr int kBatchGroups = 4;     // groups whose weights a wavefront has in flight
+constexpr int kStageGroups = 16;    // groups whose inputs are staged in LDS at a time
+constexpr int kStageStride = kStageGroups * kGroupRows + 4;  // floats a row: 16-byte reads of 16 rows meet all banks
+constexpr int kStepTiles = 4096;    // output tiles: the counters of the control block
 
 typedef _Float16 half_t;
 
@@ -40,26 +44,49 @@ struct StepParams {
   const T* dc_mask;           // DropConnect mask of R or null
   float dc_scale;
   float* h_stage;        // [N, H] when h_out overlaps h (state updated in place), else null
-  float* partial;        // [runs][2 sides][NB][column blocks * 64]; unused with one run
+  float* partial;        // [runs][output tiles][4 sums][quads of rows][64]; unused with one run
   ControlBlock* cb;
+  int runs, row_blocks, unit_blocks, quads;  // quads: of rows, in an output tile
 };
 
-// Unit j = 16 cw + u of row n: its pre-activations from x * W (wx) and h * R (rh), then the
-// pointwise step.
+// What the pointwise step of one unit of one row reads beside the sums.
+struct UnitInputs {
+  float h, c, b[4], mask;
+};
+
 template <int GATES, typename T>
-__device__ __forceinline__ void finish_unit(const StepParams<T>& p, int n, int j, const float (&wx)[GATES],
-                                            const float (&rh)[GATES]) {
+__device__ __forceinline__ UnitInputs unit_inputs(const StepParams<T>& p, int n, int j) {
+  UnitInputs u = {};
   const int H = p.H;
   const size_t e = (size_t)n * H + j;
-  const float h_old = (float)p.h[e];
+  u.h = (float)p.h[e];
+  if constexpr (GATES == 4) {
+    u.c = (float)p.c[e];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) u.b[g] = (float)p.b[g * H + j];
+  } else {
+    u.b[0] = (float)p.b[j] + (float)p.br[j];
+    u.b[1] = (float)p.b[H + j] + (float)p.br[H + j];
+    u.b[2] = (float)p.b[2 * H + j];
+    u.b[3] = (float)p.br[2 * H + j];
+  }
+  if (p.training && p.zoneout_prob != 0.f && p.zoneout_mask != nullptr) u.mask = (float)p.zoneout_mask[e];
+  return u;
+}
+
+// Unit j of row n from its sums a: LSTM the four gates of [x | h] * [W; R]; GRU the update and the
+// reset gate, x * W and h * R of the candidate gate.
+template <int GATES, typename T>
+__device__ __forceinline__ void finish_unit(const StepParams<T>& p, int n, int j, const float (&a)[4],
+                                            const UnitInputs& in) {
+  const int H = p.H;
+  const size_t e = (size_t)n * H + j;
   const bool zoneout = p.zoneout_prob != 0.f && p.zoneout_mask != nullptr;
   float h_new;
   if constexpr (GATES == 4) {
-    float a[4];
-#pragma unroll
-    for (int g = 0; g < 4; ++g) a[g] = wx[g] + rh[g] + (float)p.b[g * H + j];
-    const float gi = sigmoid_f(a[0]), gg = tanh_f(a[1]), gf = sigmoid_f(a[2]), go = sigmoid_f(a[3]);
-    const float c_new = gf * (float)p.c[e] + gi * gg;
+    const float gi = sigmoid_f(a[0] + in.b[0]), gg = tanh_f(a[1] + in.b[1]);
+    const float gf = sigmoid_f(a[2] + in.b[2]), go = sigmoid_f(a[3] + in.b[3]);
+    const float c_new = gf * in.c + gi * gg;
     h_new = go * tanh_f(c_new);
     p.c_out[e] = (T)c_new;
     if (p.training) {
@@ -67,19 +94,19 @@ __device__ __forceinline__ void finish_unit(const StepParams<T>& p, int n, int j
       vt[0] = (T)gi; vt[H] = (T)gg; vt[2 * H] = (T)gf; vt[3 * H] = (T)go;
     }
   } else {
-    const float z = sigmoid_f(wx[0] + rh[0] + (float)p.b[j] + (float)p.br[j]);
-    const float r = sigmoid_f(wx[1] + rh[1] + (float)p.b[H + j] + (float)p.br[H + j]);
-    const float qg = rh[2] + (float)p.br[2 * H + j];
-    const float g = tanh_f(wx[2] + r * qg + (float)p.b[2 * H + j]);
-    h_new = z * h_old + (1.0f - z) * g;
+    const float z = sigmoid_f(a[0] + in.b[0]);
+    const float r = sigmoid_f(a[1] + in.b[1]);
+    const float qg = a[3] + in.b[3];
+    const float g = tanh_f(a[2] + r * qg + in.b[2]);
+    h_new = z * in.h + (1.0f - z) * g;
     if (p.training && p.v != nullptr) {
       T* vt = p.v + (size_t)n * 4 * H + j;
       vt[0] = (T)z; vt[H] = (T)r; vt[2 * H] = (T)g; vt[3 * H] = (T)qg;
     }
   }
   if (zoneout) {
-    if (p.training) h_new = (h_new - h_old) * (float)p.zoneout_mask[e] + h_old;
-    else h_new = p.zoneout_prob * h_old + (1.0f - p.zoneout_prob) * h_new;
+    if (p.training) h_new = (h_new - in.h) * in.mask + in.h;
+    else h_new = p.zoneout_prob * in.h + (1.0f - p.zoneout_prob) * h_new;
   }
   if (p.h_stage == nullptr) p.h_out[e] = (T)h_new;
   else store_agent(&p.h_stage[e], h_new);
@@ -95,7 +122,7 @@ __device__ __forceinline__ void copy_staged_state(const StepParams<T>& p, unsign
   if (threadIdx.x == 0) {
     const unsigned int old = __hip_atomic_fetch_add(&p.cb->grid_exit_counter[0], 1u, __ATOMIC_RELAXED,
                                                     __HIP_MEMORY_SCOPE_AGENT);
-    const bool last = old == gridDim.x - 1;
+    const bool last = old == (unsigned)(p.row_blocks * p.unit_blocks) - 1u;
     if (last)
       __hip_atomic_store(&p.cb->grid_exit_counter[0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     *flag = last ? 1u : 0u;
@@ -106,200 +133,303 @@ __device__ __forceinline__ void copy_staged_state(const StepParams<T>& p, unsign
   for (int i = threadIdx.x; i < count; i += 256) p.h_out[i] = (T)load_exchanged(&p.h_stage[i]);
 }
 
-// GATES = 4: LSTM (i, g, f, o); GATES = 3: GRU (z, r, g).  NB: batch rows (N <= NB).
-// Workgroup (cw, run): columns of units 16 cw .. 16 cw + 15, run `run` of gridDim.y of the rows
-// of W and of the rows of R.  With a single run the workgroup finishes its units itself,
-// straight from LDS.
-template <int GATES, int NB, typename T>
+__device__ __forceinline__ void store_agent4(float* p, float4_t v) {
+  unsigned long long* q = reinterpret_cast<unsigned long long*>(p);
+  const unsigned long long lo = (unsigned long long)__float_as_uint(v.y) << 32 | __float_as_uint(v.x);
+  const unsigned long long hi = (unsigned long long)__float_as_uint(v.w) << 32 | __float_as_uint(v.z);
+  __hip_atomic_store(q, lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(q + 1, hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// GATES = 4: LSTM (i, g, f, o); GATES = 3: GRU (z, r, g).  RT: tiles of 16 batch rows a workgroup
+// takes.  [W; R] in groups of 16 rows, each side's last group filled up with zeros; a workgroup
+// takes run `run` of the groups.  Wavefront w sums gate w of its 16 units; for the GRU's
+// candidate gate, whose two sides meet the reset gate apart, wavefront 2 takes W and wavefront 3 R.
+// Every weight goes from memory to the register of the one lane that feeds it to the matrix unit
+// (fp32 instruction: 16 rows of a batch against 16 units cost a quarter of what the loads take);
+// the inputs are staged in LDS.  Lane (column l % 16, l / 16) of a group's i-th instruction holds
+// contraction index 4 (l / 16) + i, so that its inputs are one 16-byte read.
+template <int GATES, int RT, bool DROPCONNECT, typename T>
 __global__ __launch_bounds__(256)
 void forward_step_kernel(StepParams<T> p) {
-  constexpr int COLS = 64;  // 16 units x up to 4 gates (a GRU leaves the last 16 idle)
-  extern __shared__ float s_dyn[];
-  __shared__ float s_red[2][4][NB][COLS];
+  __shared__ __attribute__((aligned(16))) float s_in[RT * 16 * kStageStride];
   __shared__ unsigned int s_flag;
-  const int tid = threadIdx.x, col = tid & 63, q = tid >> 6;
-  const int cw = blockIdx.x, run = blockIdx.y, runs = gridDim.y;
-  const int N = p.N, H = p.H, GH = GATES * H;
-  const int gate = col / kStepUnits, unit = cw * kStepUnits + col % kStepUnits;
-  const bool col_ok = gate < GATES && unit < H;
-  const size_t col_off = (size_t)gate * H + unit;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int N = p.N, H = p.H;
+  // Workgroups go to the XCDs in turn: each XCD is given a range of the work, the row blocks and
+  // then the column blocks that share weights (and halves of 128-byte lines of them) side by side.
+  const int total = gridDim.x, xcd = blockIdx.x & 7, each = total >> 3, rest = total & 7;
+  const int work = xcd * each + (xcd < rest ? xcd : rest) + (blockIdx.x >> 3);
+  const int tiles = p.row_blocks * p.unit_blocks;
+  const int run = work / tiles, tile = work % tiles;
+  const int rb = tile % p.row_blocks, cw = tile / p.row_blocks;
+  const int n0 = rb * RT * 16, j0 = cw * kStepUnits;
 
-  const int len[2] = {p.C, H};
-  int per_run[2], kb[2], ke[2];
-#pragma unroll
-  for (int side = 0; side < 2; ++side) {
-    per_run[side] = ((len[side] + runs - 1) / runs + 3) / 4 * 4;
-    kb[side] = run * per_run[side];
-    ke[side] = kb[side] + per_run[side] < len[side] ? kb[side] + per_run[side] : len[side];
-  }
-  float* s_in[2] = {s_dyn, s_dyn + NB * per_run[0]};
+  const int len_w = p.C, len_r = H;
+  const int groups_w = (len_w + kGroupRows - 1) / kGroupRows;
+  const int groups = groups_w + (len_r + kGroupRows - 1) / kGroupRows;
+  const int first = (int)((long long)run * groups / p.runs), last = (int)((long long)(run + 1) * groups / p.runs);
+  // this wavefront's groups
+  const int my_first = GATES == 3 && wave == 3 && first < groups_w ? groups_w : first;
+  const int my_last = GATES == 3 && wave == 2 && last > groups_w ? groups_w : last;
+  const int gate = GATES == 3 && wave == 3 ? 2 : wave;
+  const int unit = j0 + (lane & 15) < H ? j0 + (lane & 15) : H - 1;  // columns beyond H are computed and dropped
+  const int k_lane = 4 * (lane >> 4);
+  const unsigned row_bytes = (unsigned)GATES * H * sizeof(T), column = ((unsigned)gate * H + unit) * sizeof(T);
+  const char *const W = reinterpret_cast<const char*>(p.W), *const R = reinterpret_cast<const char*>(p.R);
 
-  // Row k of side `side` (0: W, 1: R under DropConnect), this thread's column; rows beyond the
-  // run read row kb and are not used.
-  auto weight = [&](int side, int k) {
-    const T* M = side == 0 ? p.W : p.R;
-    const bool any = kb[side] < ke[side] && col_ok;
-    const size_t at = (size_t)(k < ke[side] ? k : kb[side]) * GH + col_off;
-    float w = any ? (float)M[at] : 0.f;
-    if (side == 1 && p.dc_mask != nullptr && any) w = w * (float)p.dc_mask[at] * p.dc_scale;
-    return w;
-  };
-  // The first eight rows of each side are requested before anything waits for the inputs.
-  float w0[2][8];
+  // The weights of kBatchGroups groups from group g on.  Nothing is read outside W and R: rows beyond a
+  // side's end are read from its last row, groups beyond the run from its last group (neither is used).
+  auto load_weights = [&](int g, T (&w)[kBatchGroups][4], T (&m)[kBatchGroups][4]) {
 #pragma unroll
-  for (int side = 0; side < 2; ++side)
+    for (int q = 0; q < kBatchGroups; ++q) {
+      const int gg = g + q < last ? g + q : last - 1;
+      const bool recurrent = gg >= groups_w;
+      const int k0 = (recurrent ? gg - groups_w : gg) * kGroupRows, left = (recurrent ? len_r : len_w) - k0;
+      const char* M = (recurrent ? R : W) + (size_t)k0 * row_bytes;
+      const unsigned end = (unsigned)(left - 1) * row_bytes + column;
 #pragma unroll
-    for (int u = 0; u < 8; ++u) w0[side][u] = weight(side, kb[side] + q + 4 * u);
-
-#pragma unroll
-  for (int side = 0; side < 2; ++side) {
-    const T* in = side == 0 ? p.x : p.h;
-    for (int i = tid; i < NB * per_run[side]; i += 256) {
-      const int n = i / per_run[side], k = kb[side] + i % per_run[side];
-      s_in[side][i] = (n < N && k < ke[side]) ? (float)in[(size_t)n * len[side] + k] : 0.f;
-    }
-  }
-  __syncthreads();
-
-#pragma unroll
-  for (int side = 0; side < 2; ++side) {
-    float acc[NB];
-#pragma unroll
-    for (int n = 0; n < NB; ++n) acc[n] = 0.f;
-    const float* sin = s_in[side];
-    const int pr = per_run[side], b0 = kb[side], e0 = ke[side];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int k = b0 + q + 4 * u;
-      if (k < e0) {  // the same for a whole wavefront
-#pragma unroll
-        for (int n = 0; n < NB; ++n) acc[n] = fmaf(w0[side][u], sin[n * pr + k - b0], acc[n]);
-      }
-    }
-    // the rest of the run, eight rows in flight per thread
-    for (int k0 = b0 + q + 32; k0 < e0; k0 += 32) {
-      float w[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) w[u] = weight(side, k0 + 4 * u);
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int k = k0 + 4 * u;
-        if (k < e0) {
-#pragma unroll
-          for (int n = 0; n < NB; ++n) acc[n] = fmaf(w[u], sin[n * pr + k - b0], acc[n]);
+      for (int i = 0; i < 4; ++i) {
+        const unsigned full = (unsigned)(k_lane + i) * row_bytes + column;
+        const unsigned at = left >= kGroupRows || full < end ? full : end;
+        w[q][i] = *reinterpret_cast<const T*>(M + at);
+        if constexpr (DROPCONNECT) {
+          // (for W: any value, not used)
+          const char* mask = reinterpret_cast<const char*>(p.dc_mask) + (recurrent ? (size_t)k0 * row_bytes : 0);
+          m[q][i] = *reinterpret_cast<const T*>(mask + (recurrent ? at : column));
         }
       }
     }
-#pragma unroll
-    for (int n = 0; n < NB; ++n) s_red[side][q][n][col] = acc[n];
-  }
-  __syncthreads();
-  auto quarter_sum = [&](int side, int n, int cc) {
-    return (s_red[side][0][n][cc] + s_red[side][1][n][cc]) + (s_red[side][2][n][cc] + s_red[side][3][n][cc]);
   };
-  const int n = tid / kStepUnits, u = tid % kStepUnits;
-  const int j = cw * kStepUnits + u;
-  const bool mine = n < N && j < H;  // thread (n, u) finishes unit u of row n
-  float wx[GATES], rh[GATES];
 
-  if (runs == 1) {
-    if (mine) {
+  const float4_t zero4 = {0.f, 0.f, 0.f, 0.f};
+  float4_t acc[RT];
 #pragma unroll
-      for (int g = 0; g < GATES; ++g) {
-        wx[g] = quarter_sum(0, n, g * kStepUnits + u);
-        rh[g] = quarter_sum(1, n, g * kStepUnits + u);
+  for (int rt = 0; rt < RT; ++rt) acc[rt] = zero4;
+  // Groups g .., staged from s0 on.  Every batch is summed by itself, in four sums side by side: short chains,
+  // whose rounding errors stay those of many small runs.
+  auto multiply = [&](int g, int s0, const T (&w)[kBatchGroups][4], const T (&m)[kBatchGroups][4]) {
+    float4_t part[RT][4];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) part[rt][i] = zero4;
+#pragma unroll
+    for (int q = 0; q < kBatchGroups; ++q) {
+      const int gg = g + q;
+      if (gg < my_first || gg >= my_last) continue;  // the same for a whole wavefront
+      const bool recurrent = gg >= groups_w;
+      const int left = (recurrent ? len_r : len_w) - (recurrent ? gg - groups_w : gg) * kGroupRows;
+      float4_t a[RT];
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt)
+        a[rt] = *reinterpret_cast<const float4_t*>(
+            &s_in[(rt * 16 + (lane & 15)) * kStageStride + (gg - s0) * kGroupRows + k_lane]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float weight = (float)w[q][i];
+        if constexpr (DROPCONNECT) weight = recurrent ? weight * (float)m[q][i] * p.dc_scale : weight;
+        weight = k_lane + i < left ? weight : 0.f;
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+          part[rt][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[rt][i], weight, part[rt][i], 0, 0, 0);
       }
-      finish_unit<GATES, T>(p, n, j, wx, rh);
     }
-    if (p.h_stage != nullptr) copy_staged_state(p, &s_flag);
-    return;
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) acc[rt] += (part[rt][0] + part[rt][1]) + (part[rt][2] + part[rt][3]);
+  };
+  // The inputs of groups s0 ..: lane l takes contraction index l of 64, a wavefront every fourth row.
+  auto stage = [&](int s0) {
+    if (s0 != first) __syncthreads();
+    const int s1 = s0 + kStageGroups < last ? s0 + kStageGroups : last;
+    for (int g = s0; g < s1; g += 4) {
+      const int mine = g + (lane >> 4) < last ? g + (lane >> 4) : last - 1;
+      const bool recurrent = mine >= groups_w;
+      const int len = recurrent ? len_r : len_w, k = (recurrent ? mine - groups_w : mine) * kGroupRows + (lane & 15);
+      const T* in = (recurrent ? p.h : p.x) + (k < len ? k : len - 1);
+      float value[4 * RT];
+#pragma unroll
+      for (int i = 0; i < 4 * RT; ++i) {
+        const int n = n0 + wave + 4 * i;
+        value[i] = (float)in[(size_t)(n < N ? n : N - 1) * len];
+      }
+#pragma unroll
+      for (int i = 0; i < 4 * RT; ++i)
+        s_in[(wave + 4 * i) * kStageStride + (g - s0) * kGroupRows + lane] =
+            k < len && n0 + wave + 4 * i < N ? value[i] : 0.f;
+    }
+    __syncthreads();
+  };
+  // Two batches of weights in turn: one is used while the next is on its way.
+  T w0[kBatchGroups][4], w1[kBatchGroups][4], m0[kBatchGroups][4], m1[kBatchGroups][4];
+  load_weights(first, w0, m0);
+  int s0 = first;
+  stage(s0);
+  if (first + kBatchGroups < last) load_weights(first + kBatchGroups, w1, m1);
+  multiply(first, s0, w0, m0);
+  for (int g = first + kBatchGroups; g < last;) {
+    load_weights(g + kBatchGroups, w0, m0);
+    if (g == s0 + kStageGroups) stage(s0 = g);
+    multiply(g, s0, w1, m1);
+    g += kBatchGroups;
+    if (g >= last) break;
+    load_weights(g + kBatchGroups, w1, m1);
+    if (g == s0 + kStageGroups) stage(s0 = g);
+    multiply(g, s0, w0, m0);
+    g += kBatchGroups;
   }
 
-  // Several runs: park this one's sums; the last workgroup of the column block to arrive adds
-  // the runs in index order (eight runs and all gates in flight per round trip).
-  const int slots = gridDim.x * COLS;
-  for (int i = tid; i < 2 * NB * COLS; i += 256) {
-    const int side = i / (NB * COLS), nn = (i / COLS) % NB, cc = i % COLS;
-    store_agent(&p.partial[(((size_t)run * 2 + side) * NB + nn) * slots + cw * COLS + cc], quarter_sum(side, nn, cc));
+  // Lane l of wavefront w holds sum w of rows 4 (l / 16) .. + 3 of each tile and unit l % 16.
+  // Thread t finishes row 4 (t / 64) + t % 4 and unit (t / 4) % 16 of each: its sums lie side by
+  // side with its neighbours'.
+  const int row = 4 * (tid >> 6) + (tid & 3), j = j0 + ((tid >> 2) & 15);
+  const unsigned slot = 64 * p.quads, run_stride = tiles * 4 * slot;  // floats of one sum of a tile, of a run
+  if (p.runs == 1) {
+    __syncthreads();
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+      *reinterpret_cast<float4_t*>(&s_in[(wave * RT + rt) * 256 + 4 * lane]) = acc[rt];
+  } else {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+      if (4 * rt + (lane >> 4) < p.quads)
+        store_agent4(p.partial + run * run_stride + (4 * tile + wave) * slot + rt * 256 + 4 * lane, acc[rt]);
   }
-  if (!column_last_arrival(p.cb, cw, runs, &s_flag)) return;
-  if (mine) {
+  // What the pointwise step reads is on its way while the sums are handed over.
+  UnitInputs in[RT];
 #pragma unroll
-    for (int g = 0; g < GATES; ++g) wx[g] = rh[g] = 0.f;
-    const size_t side_stride = (size_t)NB * slots, run_stride = 2 * side_stride;
-    const float* first = p.partial + (size_t)n * slots + cw * COLS + u;
-    for (int r0 = 0; r0 < runs; r0 += 8) {
-      float part[2][GATES][8];
+  for (int rt = 0; rt < RT; ++rt) {
+    in[rt] = UnitInputs{};
+    const int n = n0 + 16 * rt + row;
+    if (n < N && j < H) in[rt] = unit_inputs<GATES, T>(p, n, j);
+  }
+  if (p.runs == 1) __syncthreads();
+  else if (!column_last_arrival(p.cb, tile, p.runs, &s_flag)) return;
 #pragma unroll
-      for (int side = 0; side < 2; ++side)
+  for (int rt = 0; rt < RT; ++rt) {
+    const int n = n0 + 16 * rt + row;
+    if (n >= N || j >= H) continue;
+    float a[4] = {0.f, 0.f, 0.f, 0.f};
+    if (p.runs == 1) {
 #pragma unroll
-        for (int g = 0; g < GATES; ++g)
+      for (int g = 0; g < 4; ++g) a[g] = s_in[(g * RT + rt) * 256 + tid];
+    } else {
+      const unsigned at = 4 * tile * slot + rt * 256 + tid;
+      for (int r0 = 0; r0 < p.runs; r0 += 16) {  // 64 loads in flight
+        float run_sum[16][4];
 #pragma unroll
-          for (int i = 0; i < 8; ++i)
-            part[side][g][i] = r0 + i < runs ? load_exchanged(first + (size_t)(r0 + i) * run_stride +
-                                                              side * side_stride + g * kStepUnits)
-                                             : 0.f;
+        for (int i = 0; i < 16; ++i)
 #pragma unroll
-      for (int g = 0; g < GATES; ++g)
+          for (int g = 0; g < 4; ++g)
+            run_sum[i][g] = r0 + i < p.runs ? load_exchanged(p.partial + (at + (r0 + i) * run_stride + g * slot)) : 0.f;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          wx[g] += part[0][g][i];
-          rh[g] += part[1][g][i];
-        }
+        for (int width = 8; width > 0; width /= 2)
+#pragma unroll
+          for (int i = 0; i < width; ++i)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) run_sum[i][g] += run_sum[i + width][g];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) a[g] += run_sum[0][g];
+      }
     }
-    finish_unit<GATES, T>(p, n, j, wx, rh);
+    finish_unit<GATES, T>(p, n, j, a, in[rt]);
   }
   if (p.h_stage != nullptr) copy_staged_state(p, &s_flag);
 }
 
+// How a step is cut up.
+struct StepCut {
+  int rt, row_blocks, unit_blocks, runs, quads;
+  size_t partial_floats() const {
+    return runs > 1 ? (size_t)runs * row_blocks * unit_blocks * 4 * 64 * quads : 0;
+  }
+};
+
+// Blocks of 16 units, 16 rows and 16 contraction indices.
+long long step_blocks(int N, int C, int H) {
+  const long long groups = (C + kGroupRows - 1) / kGroupRows + (H + kGroupRows - 1) / kGroupRows;
+  return (long long)((N + 15) / 16) * ((H + kStepUnits - 1) / kStepUnits) * groups;
+}
+
+// A step of few rows is bound by the latency of its chain (loads, sums out, a counter, sums in): two
+// workgroups per CU, but runs of at least 8 groups, since every run's sums meet in memory (N = 1,
+// C = H = 512: 8 runs 8.3 us, 16 runs of half the length 9.0, 32 runs 13.7).  Where that leaves runs of
+// more than 32 groups, up to four workgroups per CU (GRU, N = 8, C = 64, H = 3776: 46.0 -> 44.5 us).
+// 32 rows a workgroup halve the reading of weights, once there are enough tiles for it (LSTM,
+// C = H = 512, us with 16 / 32 rows: N = 64, 128 tiles of 16, 12.2 / 14.2; N = 128, 256 tiles, 17.6 / 16.5).
+StepCut step_cut(int N, int C, int H) {
+  StepCut s;
+  const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
+  s.unit_blocks = (H + kStepUnits - 1) / kStepUnits;
+  s.rt = N > 16 && (N + 15) / 16 * (long long)s.unit_blocks >= cus ? 2 : 1;
+  s.row_blocks = (N + 16 * s.rt - 1) / (16 * s.rt);
+  s.quads = s.row_blocks > 1 ? 4 * s.rt : (N + 3) / 4;
+  const int groups = (C + kGroupRows - 1) / kGroupRows + (H + kGroupRows - 1) / kGroupRows;
+  const long long tiles = (long long)s.row_blocks * s.unit_blocks;
+  long long runs = (2 * cus + tiles - 1) / tiles;
+  if (runs > groups / 8) runs = groups / 8;
+  if (runs < groups / 32) {
+    runs = (4 * cus + tiles - 1) / tiles;
+    if (runs > groups / 32) runs = groups / 32;
+  }
+  s.runs = runs < 1 ? 1 : (int)runs;
+  return s;
+}
+
 template <int GATES, typename T>
 int launch_step(hipStream_t stream, StepParams<T>& p, const char* name) {
-  const int gx = (p.H + kStepUnits - 1) / kStepUnits;
-  // Runs of the contraction: enough workgroups for about two per CU, at most 64 runs, a run
-  // keeping at least 32 rows of the longer side.  The step is bound by memory latency, not
-  // bandwidth -- a thread has 8 to 16 loads of 4 bytes in flight -- so many small workgroups
-  // beat few large ones although their sums then meet in memory: at N = 1, C = H = 512 one run
-  // (32 workgroups streaming 256 KiB each, no second phase) takes 22 us, 16 runs 7 us.
-  const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
-  const int longest = p.C > p.H ? p.C : p.H;
-  int runs = (2 * cus + gx - 1) / gx;
-  if (runs > 64) runs = 64;
-  const int most = (longest + 31) / 32;
-  if (runs > most) runs = most;
-  if (runs < 1) runs = 1;
-  const int least = (longest + kStepMaxRun - 1) / kStepMaxRun;
-  if (runs < least) runs = least;
-  const int nb = p.N <= 1 ? 1 : (p.N <= 2 ? 2 : (p.N <= 4 ? 4 : 8));
-  const size_t partial_bytes = runs > 1 ? (size_t)runs * 2 * nb * gx * 64 * sizeof(float) : 0;
-  const size_t state_floats = (size_t)p.N * p.H;
-  const bool in_place = p.h_out < p.h + state_floats && p.h < p.h_out + state_floats;
+  StepCut cut = step_cut(p.N, p.C, p.H);
+  const size_t state_bytes = staged_state_bytes(p.N, p.H, p.h, p.h_out, sizeof(T));
+  for (bool room = false; !room && cut.runs > 1;) {
+    HASTE_HIP_PROPAGATE(workspace_has_room(stream, cut.partial_floats() * sizeof(float) + state_bytes + 256, &room));
+    if (!room) cut.runs = (cut.runs + 1) / 2;
+  }
+  const size_t partial_bytes = cut.partial_floats() * sizeof(float);
   Workspace ws;
-  HASTE_HIP_PROPAGATE(get_workspace(stream, partial_bytes + (in_place ? state_floats * sizeof(float) : 0) + 256, &ws));
+  HASTE_HIP_PROPAGATE(get_workspace(stream, partial_bytes + state_bytes + 256, &ws));
   if (PlannedPass* pass = planned_pass()) {
     pass->kernel = kPlanSingleStep;
     return HASTE_HIP_OK;
   }
   p.partial = ws.scratch;
-  p.h_stage = in_place ? ws.scratch + partial_bytes / sizeof(float) : nullptr;
+  p.h_stage = state_bytes > 0 ? ws.scratch + partial_bytes / sizeof(float) : nullptr;
   p.cb = ws.control;
-  const dim3 grid((unsigned)gx, (unsigned)runs);
-  auto padded_run = [&](int len) { return ((len + runs - 1) / runs + 3) / 4 * 4; };
-  const size_t lds = (size_t)nb * (padded_run(p.C) + padded_run(p.H)) * sizeof(float);
+  p.runs = cut.runs; p.row_blocks = cut.row_blocks; p.unit_blocks = cut.unit_blocks; p.quads = cut.quads;
+  const dim3 grid((unsigned)cut.row_blocks * cut.unit_blocks * cut.runs);
   ScopedKernelTimer timer(name, stream);
-  if (nb == 1) forward_step_kernel<GATES, 1, T><<<grid, dim3(256), lds, stream>>>(p);
-  else if (nb == 2) forward_step_kernel<GATES, 2, T><<<grid, dim3(256), lds, stream>>>(p);
-  else if (nb == 4) forward_step_kernel<GATES, 4, T><<<grid, dim3(256), lds, stream>>>(p);
-  else forward_step_kernel<GATES, 8, T><<<grid, dim3(256), lds, stream>>>(p);
+#define HASTE_LAUNCH_STEP(RT_)                                                                              \
+  if (cut.rt == RT_) {                                                                                      \
+    if (p.dc_mask != nullptr) forward_step_kernel<GATES, RT_, true, T><<<grid, dim3(256), 0, stream>>>(p);  \
+    else forward_step_kernel<GATES, RT_, false, T><<<grid, dim3(256), 0, stream>>>(p);                      \
+  }
+  HASTE_LAUNCH_STEP(1) HASTE_LAUNCH_STEP(2)
+#undef HASTE_LAUNCH_STEP
   HASTE_HIP_TRY(hipGetLastError());
   return HASTE_HIP_OK;
 }
 
 }  // namespace
 
-bool single_step_applies(int N, int C, int H) {
-  // per-run staging in LDS and the tile counters of the control block bound the sizes
-  // the tile counters of the control block and the 64 runs of at most kStepMaxRun bound the sizes
-  return N <= 8 && (H + kStepUnits - 1) / kStepUnits <= 4096 && C <= 64 * kStepMaxRun && H <= 64 * kStepMaxRun;
+// Whether a step of N rows is this kernel's.  Up to 8 rows always, as long as its tiles have counters.  Beyond, the other way is the
+// all-steps kernels, which fetch their slice of R in a single row of loads (kStepResident: they keep R on
+// chip; LSTM, us there / here: N = 43, C = 32, H = 128 13.6 / 5.7, N = 64, C = 64, H = 2048 82 / 52), or a GEMM
+// per side, faster from some size on because it keeps more of both operands on chip (kStepStreamed; N = 16,
+// C = 64, H = 4096, 66 560 blocks, 53 / 63; N = 128, C = 512, H = 1536, 98 304 blocks, 51 / 60; N = 128, C = 256,
+// H = 1024, 40 960 blocks, 48 / 30).  The half GRU's other way converts its weights: here at every size (N = 64,
+// C = 64, H = 2048 125 / 48, N = 128, C = 512, H = 4096 420 / 290).
+int single_step_rule(hipStream_t stream, int N, int C, int H, long long most_blocks, size_t staged_bytes, bool* applies) {
+  const StepCut cut = step_cut(N, C, H);
+  *applies = (long long)cut.row_blocks * cut.unit_blocks <= kStepTiles;
+  if (!*applies || N <= 8) return HASTE_HIP_OK;
+  *applies = step_blocks(N, C, H) <= most_blocks;
+  if (!*applies) return HASTE_HIP_OK;
+  return workspace_has_room(stream, cut.partial_floats() * sizeof(float) + staged_bytes + 256, applies);
+}
+
+size_t staged_state_bytes(int N, int H, const void* h, const void* h_out, size_t element) {
+  const uintptr_t from = reinterpret_cast<uintptr_t>(h), to = reinterpret_cast<uintptr_t>(h_out);
+  const size_t floats = (size_t)N * H;
+  return to < from + floats * element && from < to + floats * element ? floats * sizeof(float) : 0;
 }
 
 int lstm_forward_single_step(hipStream_t stream, int training, int N, int C, int H, const float* W,

@@ -1623,8 +1623,8 @@ int haste_hip_layer_norm_indrnn_backward_f64(int steps, int batch_size, int inpu
 // lib/gru_backward_gpu.cu.cc:411).  Tensors are IEEE binary16 passed as void*; products are
 // accumulated and the pointwise math is done in float, results rounded to half.  Passes over
 // more than one step run on the persistent fp32 kernels (gru_half.hip); a single step
-// (Iterate) of at most 8 rows is one kernel (single_step.hip), of more rows it runs here, one
-// product and one pointwise launch per side.
+// (Iterate) is one kernel (single_step.hip); where that has no counters or no scratch for a batch it
+// runs here, one product and one pointwise launch per side.
 static inline const half_t* hp(const void* p) { return static_cast<const half_t*>(p); }
 static inline half_t* hp(void* p) { return static_cast<half_t*>(p); }
 
@@ -1640,7 +1640,10 @@ int haste_hip_gru_forward_f16(int training, int steps, int batch_size, int input
   if (steps > 1)
     return gru_forward_half(as_stream(stream), training, steps, batch_size, input_size, hidden_size, W, R,
                             bx, br, x, h, v, zoneout_prob, zoneout_mask, nullptr, 1.f);
-  if (single_step_applies(batch_size, input_size, hidden_size))
+  bool single = false;
+  HASTE_HIP_PROPAGATE(single_step_rule(as_stream(stream), batch_size, input_size, hidden_size, kStepHalf,
+                                       staged_state_bytes(batch_size, hidden_size, h, hp(h) + NH, sizeof(half_t)), &single));
+  if (single)
     return gru_forward_single_step_half(as_stream(stream), training, batch_size, input_size, hidden_size,
                                         W, R, bx, br, x, h, hp(h) + NH, v, zoneout_prob, zoneout_mask,
                                         nullptr, 1.f);
@@ -1663,7 +1666,10 @@ int haste_hip_gru_forward_dropconnect_f16(int training, int steps, int batch_siz
     return gru_forward_half(as_stream(stream), training, steps, batch_size, input_size, hidden_size, W, R,
                             bx, br, x, h, v, zoneout_prob, zoneout_mask, dropconnect_mask,
                             dropconnect_scale);
-  if (single_step_applies(batch_size, input_size, hidden_size))
+  bool single = false;
+  HASTE_HIP_PROPAGATE(single_step_rule(as_stream(stream), batch_size, input_size, hidden_size, kStepHalf,
+                                       staged_state_bytes(batch_size, hidden_size, h, hp(h) + NH, sizeof(half_t)), &single));
+  if (single)
     return gru_forward_single_step_half(as_stream(stream), training, batch_size, input_size, hidden_size,
                                         W, R, bx, br, x, h, hp(h) + NH, v, zoneout_prob, zoneout_mask,
                                         dropconnect_mask, dropconnect_scale);
@@ -1701,7 +1707,10 @@ int haste_hip_gru_forward_iterate_f16(int training, int batch_size, int input_si
   (void)tmp_Rh;
   HASTE_HIP_REQUIRE(batch_size > 0 && input_size > 0 && hidden_size > 0);
   HASTE_HIP_REQUIRE(W && R && bx && br && x && h && h_out && tmp_Wx && (v || !training));
-  if (single_step_applies(batch_size, input_size, hidden_size))
+  bool single = false;
+  HASTE_HIP_PROPAGATE(single_step_rule(as_stream(stream), batch_size, input_size, hidden_size, kStepHalf,
+                                       staged_state_bytes(batch_size, hidden_size, h, h_out, sizeof(half_t)), &single));
+  if (single)
     return gru_forward_single_step_half(as_stream(stream), training, batch_size, input_size, hidden_size,
                                         W, R, bx, br, x, h, h_out, v, zoneout_prob, zoneout_mask, nullptr,
                                         1.f);

@@ -91,9 +91,10 @@ def test_f16_gru_inference_and_iterate():
     assert relerr(host(torch.stack(hs)), host(h)) < 4e-3
 
 
-@pytest.mark.parametrize("N,C,H", [(1, 512, 512), (3, 40, 100), (8, 24, 36), (5, 700, 16)])
+@pytest.mark.parametrize("N,C,H", [(1, 512, 512), (3, 40, 100), (8, 24, 36), (5, 700, 16), (9, 33, 31), (40, 60, 1500),
+                                   (128, 512, 512)])
 def test_f16_gru_single_step_of_a_small_batch(N, C, H):
-    """A step of at most 8 rows is one kernel on the half tensors: Iterate for training (gates
+    """A step is one kernel on the half tensors: Iterate for training (gates
     stored, zoneout by mask) and inference (zoneout by expectation), the state updated in place,
     and a one-step Run under DropConnect, each against the oracle's step."""
     from haste_amd import ops

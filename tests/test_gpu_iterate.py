@@ -133,7 +133,16 @@ def test_single_step_kernel(N, C, H, training, zoneout):
     assert torch.equal(gi, g1)
 
 
-@pytest.mark.parametrize("N,C,H", [(4, 48, 200), (8, 512, 512)])
+# Batches beyond 8 rows: tiles of 16 rows (the last one partly filled), of 32 rows (from 256 tiles of 16 on), runs that
+# end inside x * W, sides that are no multiple of a group, a single run.
+@pytest.mark.parametrize("N,C,H", [(9, 33, 31), (16, 16, 512), (17, 5, 47), (64, 300, 260), (128, 512, 512), (40, 60, 1500),
+                                   (300, 20, 1000), (128, 3, 1), (129, 1, 16)])
+@pytest.mark.parametrize("training,zoneout", [(True, 0.3), (False, 0.0)])
+def test_single_step_kernel_of_larger_batches(N, C, H, training, zoneout):
+    test_single_step_kernel(N, C, H, training, zoneout)
+
+
+@pytest.mark.parametrize("N,C,H", [(4, 48, 200), (8, 512, 512), (33, 48, 200), (70, 100, 1030)])
 def test_single_step_dropconnect_equals_premasked_weights(N, C, H):
     from haste_amd import ops
     import torch

@@ -100,6 +100,22 @@ def test_every_pass_has_a_kernel(cus, xcds, gates, size, backward):
     assert kernels == every if (cus, xcds) == (256, 8) else kernels <= every if xcds else kernels <= every - {3}
 
 
+@pytest.mark.parametrize("gates", [3, 4])
+def test_single_steps(gates):
+    """One kernel for a step of up to 8 rows of any size, and of more rows up to a size that depends on what else there
+    is; a workspace too small for its sums leaves larger batches what they ran on before."""
+    lib = hlib.load()
+    for N, C, H, single in [(1, 512, 512, 1), (8, 64, 4096, 1), (9, 512, 512, 1), (128, 512, 512, 1), (64, 64, 2048, 1),
+                            (16, 512, 4096, 0), (128, 64, 3000, 0), (1024, 512, 512, 0)]:
+        rc, plan = _plan_pass(lib, 256, 8, gates, 4, 0, 1, N, C, H)
+        assert rc == 0 and (plan[0] == 1) == bool(single), (N, C, H, rc, plan)
+    # the sums of a step of 64 rows take 2 MiB; its all-steps kernel asks for less
+    rc, plan = _plan_pass(lib, 256, 8, gates, 4, 0, 1, 64, 16, 512, workspace=(2 << 20) - 4096)
+    assert rc == 0 and plan[0] > 1, (rc, plan)
+    rc, plan = _plan_pass(lib, 256, 8, gates, 4, 0, 1, 8, 512, 512, workspace=100 << 10)
+    assert rc == 0 and plan[0] == 1, (rc, plan)
+
+
 def test_double_groups_of_8_rows_have_an_xcd_each():
     """Groups of 8 rows rather than 16 pay where a group's workgroups share an XCD: with XCDs, as far as there are, and not
     without."""
