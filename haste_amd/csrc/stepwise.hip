@@ -353,25 +353,40 @@ void scale_mask_kernel(size_t n, const T* __restrict__ w, const T* __restrict__ 
 
 // Column sums over rows in two deterministic stages.  MODE 0: a[r][col]; MODE 1: the gain
 // gradient of a layer norm, (x[r][col] - mean_r) * invstd_r * a[r][col] with (mean, invstd)
-// from cache[r].  Stage one: one thread per (column, chunk of rows); stage two adds the
-// chunks in index order into out (accumulating).  Sums are kept in the arithmetic type.
+// from cache[r].  MODE 2, 3: the same of a GRU's gradient of h * R before the norm, whose candidate
+// column is that of x * W (a) times the reset gate (in v: [rows][4H]).  Stage one: one thread per (column, chunk of rows); stage two adds the
+// chunks in a fixed order into out (accumulating).  Sums are kept in the arithmetic type.
 template <typename T, int MODE>
 __global__ __launch_bounds__(kThreads)
 void column_partial_kernel(size_t rows, int cols, size_t rows_per_chunk, const T* __restrict__ a,
                            const T* __restrict__ x, const T* __restrict__ cache,
-                           typename Acc<T>::type* __restrict__ partial) {
+                           typename Acc<T>::type* __restrict__ partial, const T* __restrict__ v) {
   using A = typename Acc<T>::type;
   const int col = blockIdx.x * kThreads + threadIdx.x;
   if (col >= cols) return;
+  const int H = cols / 3;
+  const bool reset = MODE >= 2 && col >= 2 * H;
   const size_t r0 = blockIdx.y * rows_per_chunk;
   size_t r1 = r0 + rows_per_chunk;
   if (r1 > rows) r1 = rows;
-  A s = A(0);
-  for (size_t r = r0; r < r1; ++r) {
+  auto term = [&](size_t r) {
     const size_t at = r * cols + col;
-    if (MODE == 0) s += A(a[at]);
-    else s += (A(x[at]) - A(cache[2 * r])) * A(cache[2 * r + 1]) * A(a[at]);
+    A g = A(a[at]);
+    if (reset) g = g * A(v[r * 4 * H + col - H]);
+    return MODE % 2 == 0 ? g : (A(x[at]) - A(cache[2 * r])) * A(cache[2 * r + 1]) * g;
+  };
+  // Four sums side by side: their loads are in flight together and their chains are short.
+  A sum[4] = {A(0), A(0), A(0), A(0)};
+  size_t r = r0;
+  for (; r + 4 <= r1; r += 4) {
+    A add[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) add[i] = term(r + i);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sum[i] += add[i];
   }
+  for (; r < r1; ++r) sum[0] += term(r);
+  const A s = (sum[0] + sum[1]) + (sum[2] + sum[3]);
   partial[(size_t)blockIdx.y * cols + col] = s;
 }
 
@@ -384,15 +399,16 @@ void column_finish_kernel(int chunks, int cols, const typename Acc<T>::type* __r
   if (col >= cols) return;
   constexpr int kInFlight = 32;
   A s = A(0);
-  int k = 0;
-  for (; k + kInFlight <= chunks; k += kInFlight) {
+  for (int k = 0; k < chunks; k += kInFlight) {
     A v[kInFlight];
 #pragma unroll
-    for (int u = 0; u < kInFlight; ++u) v[u] = partial[(size_t)(k + u) * cols + col];
+    for (int u = 0; u < kInFlight; ++u) v[u] = k + u < chunks ? partial[(size_t)(k + u) * cols + col] : A(0);
 #pragma unroll
-    for (int u = 0; u < kInFlight; ++u) s += v[u];
+    for (int width = kInFlight / 2; width > 0; width /= 2)
+#pragma unroll
+      for (int u = 0; u < width; ++u) v[u] += v[u + width];
+    s += v[0];
   }
-  for (; k < chunks; ++k) s += partial[(size_t)k * cols + col];
   out[col] = T(A(out[col]) + s);
 }
 
@@ -414,16 +430,16 @@ size_t column_sum_bytes(size_t all_rows, size_t step_rows, int cols) {
   return a > b ? a : b;
 }
 
-// out[col] += column sum (MODE 0) or gain gradient (MODE 1); `partial` holds
+// out[col] += column sum (MODE 0, 2) or gain gradient (MODE 1, 3); `partial` holds
 // column_sum_bytes() bytes.
 template <typename T, int MODE>
 int column_sum(hipStream_t stream, size_t rows, int cols, const T* a, const T* x, const T* cache,
-               void* partial_, T* out) {
+               void* partial_, T* out, const T* v = nullptr) {
   typename Acc<T>::type* partial = static_cast<typename Acc<T>::type*>(partial_);
   size_t rpc;
   const int chunks = column_chunks(rows, &rpc);
   const dim3 grid((unsigned)((cols + kThreads - 1) / kThreads), (unsigned)chunks);
-  column_partial_kernel<T, MODE><<<grid, dim3(kThreads), 0, stream>>>(rows, cols, rpc, a, x, cache, partial);
+  column_partial_kernel<T, MODE><<<grid, dim3(kThreads), 0, stream>>>(rows, cols, rpc, a, x, cache, partial, v);
   HASTE_LAUNCHED();
   column_finish_kernel<T><<<dim3(grid.x), dim3(kThreads), 0, stream>>>(chunks, cols, partial, out);
   HASTE_LAUNCHED();
@@ -773,6 +789,374 @@ void ln_lstm_gate_grad(int N, int H, const T* __restrict__ c, const T* __restric
   v_t[g0 + 2 * (size_t)H] = d_sigmoid(gf) * df;
 }
 
+// ---- a layer-norm cell's step in one launch: one workgroup per batch row ------------------------
+// Everything of a step but its product: the sum of the product's chunks, the norms, the gates and the
+// state, a row's units in registers (U a thread).  As launches of their own these were four to eleven small
+// kernels a step of 2 to 9 us each, bound by launches and memory round trips (LSTM, N = 8, H = 1152: 40 of the 46 us
+// of a reverse step).  What needs sums over the rows (gradients of gains, shifts and biases) is summed once after
+// the last step.
+constexpr int kRowThreads = 1024;
+constexpr int kRowUnits = 4;  // units a thread at most
+
+// Sums of K values over the workgroup, the same in every thread.
+template <typename T, int K>
+__device__ __forceinline__ void row_sums(T (&v)[K], T (*red)[K]) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+    for (int k = 0; k < K; ++k) v[k] += __shfl_xor(v[k], off, 64);
+  __syncthreads();  // red may still be read from the previous sums
+  if ((threadIdx.x & 63) == 0)
+#pragma unroll
+    for (int k = 0; k < K; ++k) red[threadIdx.x >> 6][k] = v[k];
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < K; ++k) v[k] = T(0);
+  for (int w = 0; w < (int)(blockDim.x >> 6); ++w)
+#pragma unroll
+    for (int k = 0; k < K; ++k) v[k] += red[w][k];
+}
+
+// Mean and 1 / sigma of a row of D values, of which a thread holds a[u][g] where on[u].
+template <typename T, int U, int G>
+__device__ __forceinline__ void held_moments(int D, const bool (&on)[U], const T (&a)[U][G], T* mean, T* invstd) {
+  __shared__ T red[kRowThreads / 64][1];
+  T s[1] = {T(0)};
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (on[u])
+#pragma unroll
+      for (int g = 0; g < G; ++g) s[0] += a[u][g];
+  row_sums<T, 1>(s, red);
+  const T m = s[0] / T(D);
+  T q[1] = {T(0)};
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (on[u])
+#pragma unroll
+      for (int g = 0; g < G; ++g) q[0] += (a[u][g] - m) * (a[u][g] - m);
+  row_sums<T, 1>(q, red);
+  *mean = m;
+  *invstd = Fn<T>::inv_sqrt(q[0] / T(D) + T(1e-5));
+}
+
+// The gradient through a norm (ln_backward_rows_kernel): x the normalised values, g gamma * dy; g becomes dx.
+template <typename T, int U, int G>
+__device__ __forceinline__ void held_norm_grad(int D, const bool (&on)[U], T mean, T invstd, const T (&x)[U][G],
+                                               T (&g)[U][G]) {
+  __shared__ T red[kRowThreads / 64][3];
+  T s[3] = {T(0), T(0), T(0)};
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (on[u])
+#pragma unroll
+      for (int i = 0; i < G; ++i) {
+        const T xc = x[u][i] - mean;
+        s[0] += xc * g[u][i];
+        s[1] += xc;
+        s[2] += g[u][i];
+      }
+  row_sums<T, 3>(s, red);
+  const T dsigma = T(-0.5) * s[0] * invstd * invstd * invstd;
+  const T dmu = (T(-2) * s[1] * dsigma / T(D)) - (s[2] * invstd);
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int i = 0; i < G; ++i)
+      g[u][i] = (T(2) * (x[u][i] - mean) * dsigma / T(D)) + (invstd * g[u][i]) + (dmu / T(D));
+}
+
+// The product's row n, summed; kept in `keep` (the row's h * R, which the reverse pass reads) unless it lies there.
+template <typename T, int U, int G>
+__device__ __forceinline__ void held_product(const StepProduct<T>& prod, size_t n, int H, T* keep, const bool (&on)[U],
+                                             const int (&j)[U], T (&a)[U][G]) {
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+#pragma unroll
+    for (int g = 0; g < G; ++g) a[u][g] = T(0);
+    if (!on[u]) continue;
+    const size_t g0 = n * G * H + j[u];
+    prod.template at<G>(g0, (size_t)H, a[u]);
+    if (prod.base != keep)
+#pragma unroll
+      for (int g = 0; g < G; ++g) keep[g0 + (size_t)g * H] = a[u][g];
+  }
+}
+
+#define HASTE_ROW_UNITS()                                                          \
+  const size_t n = blockIdx.x;                                                     \
+  int j[U];                                                                        \
+  bool on[U];                                                                      \
+  _Pragma("unroll") for (int u = 0; u < U; ++u) {                                  \
+    j[u] = (int)threadIdx.x + u * (int)blockDim.x;                                 \
+    on[u] = j[u] < H;                                                              \
+  }
+
+template <typename T>
+struct LnLstmForwardRow {
+  int training, H;
+  T* rh;             // [N, 4H], out (or in: the product itself)
+  const T* gamma2; T* cache2;
+  T* wxn;            // LN(x * W), out (training): the gates
+  const T *b, *c; T* c_out;
+  const T *gamma_h, *beta_h; T *cache3, *c_norm;
+  const T* h; T* h_out;
+  float zoneout_prob; const T* mask;
+};
+
+template <typename T, int U>
+__global__ __launch_bounds__(kRowThreads)
+void ln_lstm_forward_row(LnLstmForwardRow<T> p, StepProduct<T> prod) {
+  const int H = p.H;
+  HASTE_ROW_UNITS()
+  T a[U][4], mean, invstd;
+  held_product<T, U, 4>(prod, n, H, p.rh, on, j, a);
+  held_moments<T, U, 4>(4 * H, on, a, &mean, &invstd);
+  if (p.cache2 != nullptr && threadIdx.x == 0) {
+    p.cache2[2 * n] = mean;
+    p.cache2[2 * n + 1] = invstd;
+  }
+  T go[U], c_new[U][1];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    go[u] = c_new[u][0] = T(0);
+    if (!on[u]) continue;
+    const size_t g0 = n * 4 * H + j[u], e = n * H + j[u];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int col = g * H + j[u];
+      a[u][g] = p.wxn[g0 + (size_t)g * H] + (a[u][g] - mean) * invstd * p.gamma2[col] + p.b[col];
+    }
+    const T gi = Fn<T>::sigmoid(a[u][0]), gg = Fn<T>::tanh_(a[u][1]), gf = Fn<T>::sigmoid(a[u][2]);
+    go[u] = Fn<T>::sigmoid(a[u][3]);
+    if (p.training) {
+      p.wxn[g0] = gi;
+      p.wxn[g0 + H] = gg;
+      p.wxn[g0 + 2 * (size_t)H] = gf;
+      p.wxn[g0 + 3 * (size_t)H] = go[u];
+    }
+    c_new[u][0] = gf * p.c[e] + gi * gg;
+    p.c_out[e] = c_new[u][0];
+  }
+  held_moments<T, U, 1>(H, on, c_new, &mean, &invstd);
+  if (p.cache3 != nullptr && threadIdx.x == 0) {
+    p.cache3[2 * n] = mean;
+    p.cache3[2 * n + 1] = invstd;
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (!on[u]) continue;
+    const size_t e = n * H + j[u];
+    T cn = (c_new[u][0] - mean) * invstd * p.gamma_h[j[u]];
+    if (p.beta_h != nullptr) cn += p.beta_h[j[u]];
+    p.c_norm[e] = cn;
+    const T h_old = p.h[e];
+    T h_new = go[u] * Fn<T>::tanh_(cn);
+    if (p.zoneout_prob != 0.f && p.mask != nullptr) {
+      if (p.training) h_new = (h_new - h_old) * p.mask[e] + h_old;
+      else h_new = T(p.zoneout_prob) * h_old + (T(1) - T(p.zoneout_prob)) * h_new;
+    }
+    p.h_out[e] = h_new;
+  }
+}
+
+template <typename T>
+struct LnLstmBackwardRow {
+  int H, first;
+  const T* dh_next; T* dh; const T* mask;
+  T* c_norm;                          // LN(c'), out: its gradient
+  T* v;                               // the gates, out: their gradients
+  const T *gamma_h, *c_next, *cache3; // c_next: c'
+  const T *c, *dc_next; T* dc;
+  T* rh;                              // h * R, out: its gradient
+  const T *gamma2, *cache2;
+  T* dgamma2_rows;                    // [N, 4H]: each row's share of dgamma2, over the steps
+};
+
+template <typename T, int U>
+__global__ __launch_bounds__(kRowThreads)
+void ln_lstm_backward_row(LnLstmBackwardRow<T> p, StepProduct<T> pend) {
+  const int H = p.H;
+  HASTE_ROW_UNITS()
+  T dv[U][4], c_new[U][1], dcn[U][1], rh[U][4];
+  // through the output (ln_lstm_output_grad) and the norm of the cell state
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    c_new[u][0] = dcn[u][0] = T(0);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) dv[u][g] = rh[u][g] = T(0);
+    if (!on[u]) continue;
+    const size_t e = n * H + j[u], g0 = n * 4 * H + j[u];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      dv[u][g] = p.v[g0 + (size_t)g * H];
+      rh[u][g] = p.rh[g0 + (size_t)g * H];
+    }
+    c_new[u][0] = p.c_next[e];
+    T dh_total = p.dh_next[e] + (p.dh[e] + pend.at(e));
+    T dh_keep = T(0);
+    if (p.mask != nullptr) {
+      const T m = p.mask[e];
+      dh_keep = (T(1) - m) * dh_total;
+      dh_total = m * dh_total;
+    }
+    const T c_tanh = Fn<T>::tanh_(p.c_norm[e]);
+    const T go = dv[u][3];
+    dv[u][3] = d_sigmoid(go) * (c_tanh * dh_total);
+    dcn[u][0] = d_tanh(c_tanh) * (go * dh_total);
+    p.c_norm[e] = dcn[u][0];
+    dcn[u][0] = p.gamma_h[j[u]] * dcn[u][0];
+    p.dh[e] = dh_keep;
+  }
+  held_norm_grad<T, U, 1>(H, on, p.cache3[2 * n], p.cache3[2 * n + 1], c_new, dcn);
+  // through the gates (ln_lstm_gate_grad) and the norm of h * R
+  const T mean = p.cache2[2 * n], invstd = p.cache2[2 * n + 1];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (!on[u]) continue;
+    const size_t e = n * H + j[u], g0 = n * 4 * H + j[u];
+    const T gi = dv[u][0], gg = dv[u][1], gf = dv[u][2];
+    const T dc_total = (p.dc_next != nullptr ? p.dc_next[e] : T(0)) + p.dc[e] + dcn[u][0];
+    p.dc[e] = gf * dc_total;
+    dv[u][0] = d_sigmoid(gi) * (gg * dc_total);
+    dv[u][1] = d_tanh(gg) * (gi * dc_total);
+    dv[u][2] = d_sigmoid(gf) * (p.c[e] * dc_total);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const size_t at = g0 + (size_t)g * H;
+      p.v[at] = dv[u][g];
+      const T gain = (rh[u][g] - mean) * invstd * dv[u][g];
+      p.dgamma2_rows[at] = p.first ? gain : p.dgamma2_rows[at] + gain;
+      dv[u][g] = p.gamma2[g * H + j[u]] * dv[u][g];
+    }
+  }
+  held_norm_grad<T, U, 4>(4 * H, on, mean, invstd, rh, dv);
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (on[u])
+#pragma unroll
+      for (int g = 0; g < 4; ++g) p.rh[n * 4 * H + (size_t)g * H + j[u]] = dv[u][g];
+}
+
+template <typename T>
+struct LnGruForwardRow {
+  int training, H;
+  T* rh;             // [N, 3H], out (or in: the product itself)
+  const T* gamma2; T* cache2;
+  const T *wxn, *bx, *br, *h; T *h_out, *v;
+  float zoneout_prob; const T* mask;
+};
+
+template <typename T, int U>
+__global__ __launch_bounds__(kRowThreads)
+void ln_gru_forward_row(LnGruForwardRow<T> p, StepProduct<T> prod) {
+  const int H = p.H;
+  HASTE_ROW_UNITS()
+  T q[U][3], mean, invstd;
+  held_product<T, U, 3>(prod, n, H, p.rh, on, j, q);
+  held_moments<T, U, 3>(3 * H, on, q, &mean, &invstd);
+  if (p.cache2 != nullptr && threadIdx.x == 0) {
+    p.cache2[2 * n] = mean;
+    p.cache2[2 * n + 1] = invstd;
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (!on[u]) continue;
+    const size_t g0 = n * 3 * H + j[u], e = n * H + j[u];
+    T wx[3];
+#pragma unroll
+    for (int g = 0; g < 3; ++g) {
+      q[u][g] = (q[u][g] - mean) * invstd * p.gamma2[g * H + j[u]];
+      wx[g] = p.wxn[g0 + (size_t)g * H];
+    }
+    const T z = Fn<T>::sigmoid(wx[0] + q[u][0] + p.bx[j[u]] + p.br[j[u]]);
+    const T r = Fn<T>::sigmoid(wx[1] + q[u][1] + p.bx[H + j[u]] + p.br[H + j[u]]);
+    const T qg = q[u][2] + p.br[2 * H + j[u]];
+    const T g = Fn<T>::tanh_(wx[2] + r * qg + p.bx[2 * H + j[u]]);
+    if (p.training) {
+      const size_t v0 = n * 4 * H + j[u];
+      p.v[v0] = z;
+      p.v[v0 + H] = r;
+      p.v[v0 + 2 * (size_t)H] = g;
+      p.v[v0 + 3 * (size_t)H] = qg;
+    }
+    const T h_old = p.h[e];
+    T h_new = z * h_old + (T(1) - z) * g;
+    if (p.zoneout_prob != 0.f && p.mask != nullptr) {
+      if (p.training) h_new = (h_new - h_old) * p.mask[e] + h_old;
+      else h_new = T(p.zoneout_prob) * h_old + (T(1) - T(p.zoneout_prob)) * h_new;
+    }
+    p.h_out[e] = h_new;
+  }
+}
+
+template <typename T>
+struct LnGruBackwardRow {
+  int H;
+  const T *h, *v, *dh_next; T* dh; const T* mask;
+  T *dp, *dq;                       // dq: the gradient of h * R
+  const T *rh, *gamma2, *cache2;
+};
+
+template <typename T, int U>
+__global__ __launch_bounds__(kRowThreads)
+void ln_gru_backward_row(LnGruBackwardRow<T> p, StepProduct<T> pend) {
+  const int H = p.H;
+  HASTE_ROW_UNITS()
+  T dq[U][3], rh[U][3];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+#pragma unroll
+    for (int g = 0; g < 3; ++g) dq[u][g] = rh[u][g] = T(0);
+    if (!on[u]) continue;
+    const size_t e = n * H + j[u], v0 = n * 4 * H + j[u], g0 = n * 3 * H + j[u];
+    const T z = p.v[v0], r = p.v[v0 + H], g = p.v[v0 + 2 * (size_t)H], qg = p.v[v0 + 3 * (size_t)H];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) rh[u][i] = p.rh[g0 + (size_t)i * H];
+    T dh_total = p.dh_next[e] + (p.dh[e] + pend.at(e));
+    T dh_keep;
+    if (p.mask != nullptr) {
+      const T m = p.mask[e];
+      dh_keep = (T(1) - m) * dh_total;
+      dh_total = m * dh_total;
+      dh_keep += z * dh_total;
+    } else {
+      dh_keep = z * dh_total;
+    }
+    const T dp_g = d_tanh(g) * ((T(1) - z) * dh_total);
+    const T dp_r = d_sigmoid(r) * (dp_g * qg);
+    const T dp_z = d_sigmoid(z) * ((p.h[e] - g) * dh_total);
+    p.dh[e] = dh_keep;
+    p.dp[g0] = dp_z;
+    p.dp[g0 + H] = dp_r;
+    p.dp[g0 + 2 * (size_t)H] = dp_g;
+    dq[u][0] = p.gamma2[j[u]] * dp_z;
+    dq[u][1] = p.gamma2[H + j[u]] * dp_r;
+    dq[u][2] = p.gamma2[2 * H + j[u]] * (dp_g * r);
+  }
+  held_norm_grad<T, U, 3>(3 * H, on, p.cache2[2 * n], p.cache2[2 * n + 1], rh, dq);
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (on[u])
+#pragma unroll
+      for (int g = 0; g < 3; ++g) p.dq[n * 3 * H + (size_t)g * H + j[u]] = dq[u][g];
+}
+#undef HASTE_ROW_UNITS
+
+// Whether a step's rows are held by a workgroup each.
+inline bool rows_held(int H) { return H <= kRowThreads * kRowUnits; }
+
+// Launches KERNEL for rows of H units: as few units a thread as there can be.
+#define HASTE_LAUNCH_ROWS(KERNEL, T, N_, H_, ...)                                                         \
+  do {                                                                                                    \
+    const int units_ = (H_) <= kRowThreads ? 1 : (H_) <= 2 * kRowThreads ? 2 : 4;                         \
+    const dim3 threads_((unsigned)(((H_) + units_ - 1) / units_ + 63) / 64 * 64);                         \
+    if (units_ == 1) KERNEL<T, 1><<<dim3((unsigned)(N_)), threads_, 0, stream>>>(__VA_ARGS__);            \
+    else if (units_ == 2) KERNEL<T, 2><<<dim3((unsigned)(N_)), threads_, 0, stream>>>(__VA_ARGS__);       \
+    else KERNEL<T, 4><<<dim3((unsigned)(N_)), threads_, 0, stream>>>(__VA_ARGS__);                        \
+    HASTE_LAUNCHED();                                                                                     \
+  } while (0)
+
 // ---- IndRNN: one thread per (row, unit) walks the steps ---------------------------------
 template <typename T>
 __global__ __launch_bounds__(kThreads)
@@ -1005,6 +1389,21 @@ int ln_lstm_forward_steps(hipStream_t stream, int training, int steps, int N, in
   for (int t = 0; t < steps; ++t) {
     const T* h_t = h + (size_t)t * NH;
     T* rh_t = act_Rh + (size_t)t * N4H;
+    if (rows_held(H)) {
+      StepProduct<T> prod;
+      HASTE_HIP_PROPAGATE(step_product<T>(stream, N, 4 * H, H, h_t, R, rh_t, sc.gemm_offset(), &prod));
+      LnLstmForwardRow<T> row;
+      row.training = training; row.H = H;
+      row.rh = rh_t; row.gamma2 = gamma2; row.cache2 = cache2 ? cache2 + (size_t)t * N * 2 : nullptr;
+      row.wxn = act_Wx_norm + (size_t)t * N4H; row.b = b;
+      row.c = c + (size_t)t * NH; row.c_out = c + (size_t)(t + 1) * NH;
+      row.gamma_h = gamma_h; row.beta_h = beta_h; row.cache3 = cache3 ? cache3 + (size_t)t * N * 2 : nullptr;
+      row.c_norm = act_c_norm + (size_t)t * NH;
+      row.h = h_t; row.h_out = h + (size_t)(t + 1) * NH;
+      row.zoneout_prob = zoneout_prob; row.mask = zoneout_mask ? zoneout_mask + (size_t)t * NH : nullptr;
+      HASTE_LAUNCH_ROWS(ln_lstm_forward_row, T, N, H, row, prod);
+      continue;
+    }
     HASTE_HIP_PROPAGATE(gemm(stream, false, N, 4 * H, H, h_t, H, R, 4 * H, rh_t, 4 * H, false, sc.gemm_offset()));
     HASTE_HIP_PROPAGATE(ln_forward_rows<T>(stream, (size_t)N, 4 * H, gamma2, nullptr, rh_t, rhn,
                                            cache2 ? cache2 + (size_t)t * N * 2 : nullptr));
@@ -1032,13 +1431,19 @@ int ln_lstm_backward_steps(hipStream_t stream, int steps, int N, int C, int H, c
   const size_t NH = (size_t)N * H, N4H = NH * 4;
   const int TN = steps * N;
   const size_t part_bytes = column_sum_bytes<T>((size_t)TN, (size_t)N, 4 * H);
-  const size_t own = part_bytes + padded((size_t)TN * 2 * sizeof(T));
+  size_t own = part_bytes + padded((size_t)TN * 2 * sizeof(T));
   Room room = max2(gemm_room<T>(N, H, 4 * H), gemm_room<T>(C, 4 * H, TN));
   room = max2(room, max2(gemm_room<T>(H, 4 * H, TN), gemm_room<T>(TN, C, 4 * H)));
+  // Rows held by a workgroup each, where there is room for their sums of dgamma2.
+  const size_t sums_bytes = padded(N4H * sizeof(T));
+  bool held = rows_held(H);
+  if (held) HASTE_HIP_PROPAGATE(workspace_has_room(stream, own + sums_bytes + room.need + 256, &held));
+  if (held) own += sums_bytes;
   Scratch sc;
   HASTE_HIP_PROPAGATE(open_scratch(stream, own, room, &sc));
   void* partial = sc.take<char>(part_bytes);
   T* stats1 = sc.take<T>((size_t)TN * 2);
+  T* dgamma2_rows = held ? sc.take<T>(N4H) : nullptr;
   {
     ScopedKernelTimer timer("layer_norm_lstm_backward_steps", stream);
     StepProduct<T> pend;
@@ -1047,6 +1452,20 @@ int ln_lstm_backward_steps(hipStream_t stream, int steps, int N, int C, int H, c
       T* cn_t = act_c_norm + (size_t)t * NH;
       T* rh_t = act_Rh + (size_t)t * N4H;
       const T* mask_t = zoneout_mask ? zoneout_mask + (size_t)t * NH : nullptr;
+      if (held) {
+        LnLstmBackwardRow<T> row;
+        row.H = H; row.first = t == steps - 1;
+        row.dh_next = dh_new + (size_t)(t + 1) * NH; row.dh = dh; row.mask = mask_t;
+        row.c_norm = cn_t; row.v = v_t;
+        row.gamma_h = gamma_h; row.c_next = c + (size_t)(t + 1) * NH; row.cache3 = cache3 + (size_t)t * N * 2;
+        row.c = c + (size_t)t * NH; row.dc = dc;
+        row.dc_next = dc_new != nullptr ? dc_new + (size_t)(t + 1) * NH : nullptr;
+        row.rh = rh_t; row.gamma2 = gamma2; row.cache2 = cache2 + (size_t)t * N * 2;
+        row.dgamma2_rows = dgamma2_rows;
+        HASTE_LAUNCH_ROWS(ln_lstm_backward_row, T, N, H, row, pend);
+        HASTE_HIP_PROPAGATE(reverse_product<T>(stream, N, H, 4 * H, rh_t, R_t, dh, sc.gemm_offset(), &pend));
+        continue;
+      }
       ln_lstm_output_grad<T><<<blocks_for(NH), dim3(kThreads), 0, stream>>>(
           N, H, dh_new + (size_t)(t + 1) * NH, dh, pend, mask_t, cn_t, v_t);
       HASTE_LAUNCHED();
@@ -1062,6 +1481,12 @@ int ln_lstm_backward_steps(hipStream_t stream, int steps, int N, int C, int H, c
       HASTE_HIP_PROPAGATE(reverse_product<T>(stream, N, H, 4 * H, rh_t, R_t, dh, sc.gemm_offset(), &pend));
     }
     HASTE_HIP_PROPAGATE(flush_pending<T>(stream, NH, pend, dh));
+  }
+  if (held) {
+    HASTE_HIP_PROPAGATE((column_sum<T, 1>(stream, (size_t)TN, H, act_c_norm, c + NH, cache3, partial, dgamma_h)));
+    if (dbeta_h != nullptr)
+      HASTE_HIP_PROPAGATE((column_sum<T, 0>(stream, (size_t)TN, H, act_c_norm, nullptr, nullptr, partial, dbeta_h)));
+    HASTE_HIP_PROPAGATE((column_sum<T, 0>(stream, (size_t)N, 4 * H, dgamma2_rows, nullptr, nullptr, partial, dgamma2)));
   }
   HASTE_HIP_PROPAGATE((column_sum<T, 0>(stream, (size_t)TN, 4 * H, v, nullptr, nullptr, partial, db)));
   // through the norm of x*W, in place over act_Wx
@@ -1089,6 +1514,18 @@ int ln_gru_forward_steps(hipStream_t stream, int training, int steps, int N, int
   for (int t = 0; t < steps; ++t) {
     const T* h_t = h + (size_t)t * NH;
     T* rh_t = act_Rh + (size_t)t * N3H;
+    if (rows_held(H)) {
+      StepProduct<T> prod;
+      HASTE_HIP_PROPAGATE(step_product<T>(stream, N, 3 * H, H, h_t, R, rh_t, sc.gemm_offset(), &prod));
+      LnGruForwardRow<T> row;
+      row.training = training; row.H = H;
+      row.rh = rh_t; row.gamma2 = gamma2; row.cache2 = cache2 ? cache2 + (size_t)t * N * 2 : nullptr;
+      row.wxn = tmp_Wx_norm + (size_t)t * N3H; row.bx = bx; row.br = br;
+      row.h = h_t; row.h_out = h + (size_t)(t + 1) * NH; row.v = v ? v + (size_t)t * N4H : nullptr;
+      row.zoneout_prob = zoneout_prob; row.mask = zoneout_mask ? zoneout_mask + (size_t)t * NH : nullptr;
+      HASTE_LAUNCH_ROWS(ln_gru_forward_row, T, N, H, row, prod);
+      continue;
+    }
     HASTE_HIP_PROPAGATE(gemm(stream, false, N, 3 * H, H, h_t, H, R, 3 * H, rh_t, 3 * H, false, sc.gemm_offset()));
     HASTE_HIP_PROPAGATE(ln_forward_rows<T>(stream, (size_t)N, 3 * H, gamma2, nullptr, rh_t, rhn,
                                            cache2 ? cache2 + (size_t)t * N * 2 : nullptr));
@@ -1125,6 +1562,17 @@ int ln_gru_backward_steps(hipStream_t stream, int steps, int N, int C, int H, co
     StepProduct<T> pend;
     for (int t = steps - 1; t >= 0; --t) {
       T* dq_t = dq + (size_t)t * N3H;
+      if (rows_held(H)) {
+        LnGruBackwardRow<T> row;
+        row.H = H;
+        row.h = h + (size_t)t * NH; row.v = v + (size_t)t * N4H; row.dh_next = dh_new + (size_t)(t + 1) * NH;
+        row.dh = dh; row.mask = zoneout_mask ? zoneout_mask + (size_t)t * NH : nullptr;
+        row.dp = dp + (size_t)t * N3H; row.dq = dq_t;
+        row.rh = act_Rh + (size_t)t * N3H; row.gamma2 = gamma2; row.cache2 = cache2 + (size_t)t * N * 2;
+        HASTE_LAUNCH_ROWS(ln_gru_backward_row, T, N, H, row, pend);
+        HASTE_HIP_PROPAGATE(reverse_product<T>(stream, N, H, 3 * H, dq_t, R_t, dh, sc.gemm_offset(), &pend));
+        continue;
+      }
       gru_backward_pointwise<T><<<blocks_for(NH), dim3(kThreads), 0, stream>>>(
           N, H, h + (size_t)t * NH, v + (size_t)t * N4H, dh_new + (size_t)(t + 1) * NH, dh, pend,
           dp + (size_t)t * N3H, dq_t, zoneout_mask ? zoneout_mask + (size_t)t * NH : nullptr);
@@ -1136,6 +1584,10 @@ int ln_gru_backward_steps(hipStream_t stream, int steps, int N, int C, int H, co
       HASTE_HIP_PROPAGATE(reverse_product<T>(stream, N, H, 3 * H, dq_t, R_t, dh, sc.gemm_offset(), &pend));
     }
     HASTE_HIP_PROPAGATE(flush_pending<T>(stream, NH, pend, dh));
+  }
+  if (rows_held(H)) {
+    HASTE_HIP_PROPAGATE((column_sum<T, 2>(stream, (size_t)TN, 3 * H, dp, nullptr, nullptr, partial, dbr, v)));
+    HASTE_HIP_PROPAGATE((column_sum<T, 3>(stream, (size_t)TN, 3 * H, dp, act_Rh, cache2, partial, dgamma2, v)));
   }
   HASTE_HIP_PROPAGATE((column_sum<T, 0>(stream, (size_t)TN, 3 * H, dp, nullptr, nullptr, partial, dbx)));
   HASTE_HIP_PROPAGATE(ln_forward_rows<T>(stream, (size_t)TN, 3 * H, gamma1, nullptr, act_Wx, nullptr, stats1));
