@@ -744,9 +744,10 @@ int gru_forward_impl(hipStream_t stream, int training, int T, int N, int C, int 
                      tile.reg_groups == 0 && C <= 512 && C % 4 == 0 &&
                      (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
   if (fused) HASTE_HIP_PROPAGATE(input_projection_in_recurrence(stream, T, N, C, H, 3 * H, &fused));
-  // The recurrence on the bf16 matrix cores, where it is the faster one (split_forward.h).
+  // The recurrence on the bf16 matrix cores, where it is the faster one (split_forward.h).  Widened half
+  // tensors have a product of their own in tiles of up to 8 rows only.
   int split_rows = 0;
-  if (!half_product)
+  if (!half_product || tile.nb > 8)
     HASTE_HIP_PROPAGATE(split_forward_rule(stream, T, N, C, H, 3 * H, wx_ready, fused, &split_rows));
   if (split_rows > 0) fused = false;
   const int xsg = C <= 256 ? 1 : 2;
@@ -866,10 +867,11 @@ int gru_backward_impl(hipStream_t stream, int T, int N, int C, int H,
                               : tile.nb == 8 && paired_lds <= kMaxLdsBytes;
   const int sets = paired ? 2 : 1;
 
-  // Tiles of 8 and 16 rows: on the bf16 matrix cores (split_backward.h).
+  // Tiles of 8 and 16 rows: on the bf16 matrix cores (split_backward.h).  Widened half tensors have a
+  // product of their own in the scattered form only.
   int split_rows = 0;
   size_t split_sums = 0, split_floats = 0;
-  if (!half_product)
+  if (!half_product || !scatter)
     HASTE_HIP_PROPAGATE(split_backward_rule(stream, N, H, 6, &split_rows, &split_sums, &split_floats));
 
   Workspace ws;

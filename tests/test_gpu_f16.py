@@ -91,6 +91,12 @@ def test_f16_gru_inference_and_iterate():
     assert relerr(host(torch.stack(hs)), host(h)) < 4e-3
 
 
+# Batches whose tiles have 16 rows: the recurrences in sums of three bf16 (forward from H = 225, backward from H = 65 on).
+@pytest.mark.parametrize("T,N,C,H", [(6, 72, 24, 300), (5, 128, 16, 478), (5, 100, 8, 96), (4, 70, 16, 224)])
+def test_f16_gru_tiles_of_16_rows(T, N, C, H):
+    test_f16_gru_training_forward_backward(T, N, C, H, 0.3)
+
+
 @pytest.mark.parametrize("N,C,H", [(1, 512, 512), (3, 40, 100), (8, 24, 36), (5, 700, 16), (9, 33, 31), (40, 60, 1500),
                                    (128, 512, 512)])
 def test_f16_gru_single_step_of_a_small_batch(N, C, H):
