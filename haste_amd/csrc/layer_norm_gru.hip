@@ -665,7 +665,12 @@ int haste_hip_layer_norm_gru_forward_f32(int training, int steps, int batch_size
   hipStream_t stream = as_stream(stream_);
   const ForwardTile tile = pick_forward_tile(3, N, H, 2 * sizeof(float), kMaxLdsBytes, true,
                                              3);
-  if (!tile.ok)
+  // As in layer_norm_lstm.hip (us a step kept / streamed: H = 1280, N = 64 27.0 / 22.9, H = 1792 N = 40 41 / 29 and
+  // N = 24 25.7 / 23.8; but H = 1536, N = 32 19.5 / 20.9).
+  bool streamed = !tile.ok;
+  if (tile.ok && tile.reg_groups > 0 && ((tile.nb >= 64 && H > 1240) || (tile.nb >= 32 && H > 1700)))
+    HASTE_HIP_PROPAGATE(workspace_has_room(stream, workspace_scratch_bound(T, N, C, H), &streamed));
+  if (streamed)
     return layer_norm_gru_forward_streamed(stream, training, T, N, C, H, W, R, bx, br, x, h, v, act_Wx,
                                            gamma1, cache1, tmp_Wx_norm, act_Rh, gamma2, cache2,
                                            zoneout_prob, zoneout_mask);
@@ -735,7 +740,12 @@ int haste_hip_layer_norm_gru_backward_f32(int steps, int batch_size, int input_s
   hipStream_t stream = as_stream(stream_);
   // per row: 9 column-sum accumulators of 16 floats (or the partial tiles, whichever is more) + 4 sums
   const BackwardTile tile = pick_backward_tile(ln_gru_backward_k(H), N, H, 9 * 16, 4, true);
-  if (!tile.ok)
+  // As in layer_norm_lstm.hip (us a step kept / streamed: H = 896, N = 8 14.9 / 13.7, H = 1408 N = 8 19.8 / 17.3 and
+  // N = 48 33.9 / 31.8, H = 1280 N = 128 59 / 44; but H = 1024, N = 16 14.0 / 15.2 and N = 128 27 / 37).
+  bool streamed = !tile.ok;
+  if (tile.ok && tile.reg_groups > 0 && ((N <= 8 && H > 880) || (N > 32 && H > 1240)))
+    HASTE_HIP_PROPAGATE(workspace_has_room(stream, workspace_scratch_bound(T, N, C, H), &streamed));
+  if (streamed)
     return layer_norm_gru_backward_streamed(stream, T, N, C, H, W_t, R_t, x_t, h, v, dh_new, dx, dW, dR,
                                             dbx, dbr, dh, dp, dq, act_Wx, gamma1, dgamma1, act_Rh,
                                             gamma2, dgamma2, cache2, zoneout_mask);
