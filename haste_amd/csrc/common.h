@@ -319,9 +319,11 @@ size_t cut_scratch_bound(int N, int H, int cus);
 // One forward step as a single kernel (single_step.hip): what the Iterate entry points and one-step
 // Run calls use, for batches up to a size (single_step_rule: most_blocks blocks of 16 units, rows and
 // contraction indices) that depends on what the step would run on otherwise.
-constexpr long long kStepStreamed = 60 << 10, kStepResident = 128 << 10, kStepHalf = 1ll << 40;
+constexpr long long kStepStreamed = 60 << 10, kStepResident = 128 << 10, kStepHalf = 1ll << 40,
+                    kStepDouble = 16 << 10;
 // staged_bytes: staged_state_bytes() of the call, scratch for a state that is updated in place.
-int single_step_rule(hipStream_t stream, int N, int C, int H, long long most_blocks, size_t staged_bytes, bool* applies);
+int single_step_rule(hipStream_t stream, int N, int C, int H, size_t element, long long most_blocks, size_t staged_bytes,
+                     bool* applies);
 size_t staged_state_bytes(int N, int H, const void* h, const void* h_out, size_t element);
 int lstm_forward_single_step(hipStream_t stream, int training, int N, int C, int H, const float* W,
                              const float* R, const float* b, const float* x, const float* h,
@@ -332,6 +334,15 @@ int gru_forward_single_step(hipStream_t stream, int training, int N, int C, int 
                             const float* R, const float* bx, const float* br, const float* x,
                             const float* h, float* h_out, float* v, float zoneout_prob,
                             const float* zoneout_mask, const float* dc_mask, float dc_scale);
+int lstm_forward_single_step(hipStream_t stream, int training, int N, int C, int H, const double* W,
+                             const double* R, const double* b, const double* x, const double* h,
+                             const double* c, double* h_out, double* c_out, double* v,
+                             float zoneout_prob, const double* zoneout_mask, const double* dc_mask,
+                             float dc_scale);
+int gru_forward_single_step(hipStream_t stream, int training, int N, int C, int H, const double* W,
+                            const double* R, const double* bx, const double* br, const double* x,
+                            const double* h, double* h_out, double* v, float zoneout_prob,
+                            const double* zoneout_mask, const double* dc_mask, float dc_scale);
 // Half tensors (IEEE binary16), sums and pointwise step in float.
 int gru_forward_single_step_half(hipStream_t stream, int training, int N, int C, int H, const void* W,
                                  const void* R, const void* bx, const void* br, const void* x,

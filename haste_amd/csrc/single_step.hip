@@ -8,7 +8,8 @@
 // 32 batch rows and a run of the contraction, parks its partial sums, and the last workgroup of
 // an output tile to finish adds the runs in index order and does the pointwise step (gates, cell
 // update, zoneout) -- one launch, no float atomics, results independent of timing.  The GRU's
-// half entry points use the same kernel on half tensors (sums and pointwise step in float).
+// half entry points use the same kernel on half tensors (sums and pointwise step in float), and the
+// double ones in double.
 //
 // Arithmetic: reference lib/lstm_forward_gpu.cu.cc:55-86, lib/gru_forward_gpu.cu.cc:46-84.
 #include "recurrent.h"
@@ -24,8 +25,34 @@ constexpr int kStageStride = kStageGroups * kGroupRows + 4;  // floats a row: 16
 constexpr int kStepTiles = 4096;    // output tiles: the counters of the control block
 
 typedef _Float16 half_t;
+typedef double double4_t __attribute__((ext_vector_type(4)));
 
-// T: the caller's tensors (float, or half with the sums and the pointwise step in float).
+// What sums and the pointwise step are in, and the matrix instruction: A[row = lane % 16][k = lane / 16] times
+// B[k = lane / 16][column = lane % 16]; element i of a lane is row row(lane, i) and column lane % 16.
+template <typename T> struct Step {
+  typedef float Sum;
+  typedef float4_t Sum4;
+  static constexpr bool kQuads = true;  // a lane's elements are rows of one quad
+  static __device__ __forceinline__ Sum4 mfma(float a, float b, Sum4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int lane, int i) { return 4 * (lane >> 4) + i; }
+  static __device__ __forceinline__ float sigmoid(float x) { return sigmoid_f(x); }
+  static __device__ __forceinline__ float tanh_(float x) { return tanh_f(x); }
+};
+template <> struct Step<double> {
+  typedef double Sum;
+  typedef double4_t Sum4;
+  static constexpr bool kQuads = false;
+  static __device__ __forceinline__ Sum4 mfma(double a, double b, Sum4 c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int lane, int i) { return (lane >> 4) + 4 * i; }
+  static __device__ __forceinline__ double sigmoid(double x) { return 1.0 / (1.0 + exp(-x)); }
+  static __device__ __forceinline__ double tanh_(double x) { return tanh(x); }
+};
+
+// T: the caller's tensors (float, double, or half with the sums and the pointwise step in float).
 template <typename T>
 struct StepParams {
   int training, N, C, H;
@@ -43,62 +70,89 @@ struct StepParams {
   const T* zoneout_mask;      // [N, H] or null
   const T* dc_mask;           // DropConnect mask of R or null
   float dc_scale;
-  float* h_stage;        // [N, H] when h_out overlaps h (state updated in place), else null
-  float* partial;        // [runs][output tiles][4 sums][quads of rows][64]; unused with one run
+  typename Step<T>::Sum* h_stage;  // [N, H] when h_out overlaps h (state updated in place), else null
+  typename Step<T>::Sum* partial;  // [runs][output tiles][4 sums][quads of rows][64]; unused with one run
   ControlBlock* cb;
   int runs, row_blocks, unit_blocks, quads;  // quads: of rows, in an output tile
 };
 
+// Sums between workgroups of a launch (agent scope: store_agent, load_exchanged).
+__device__ __forceinline__ float load_sum(const float* p) { return load_exchanged(p); }
+__device__ __forceinline__ double load_sum(const double* p) {
+  return __longlong_as_double((long long)__hip_atomic_load(reinterpret_cast<const unsigned long long*>(p), __ATOMIC_RELAXED,
+                                                           __HIP_MEMORY_SCOPE_AGENT));
+}
+__device__ __forceinline__ void store_sum(float* p, float v) { store_agent(p, v); }
+__device__ __forceinline__ void store_sum(double* p, double v) {
+  __hip_atomic_store(reinterpret_cast<unsigned long long*>(p), (unsigned long long)__double_as_longlong(v),
+                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void store_sum4(float* p, float4_t v) {
+  unsigned long long* q = reinterpret_cast<unsigned long long*>(p);
+  const unsigned long long lo = (unsigned long long)__float_as_uint(v.y) << 32 | __float_as_uint(v.x);
+  const unsigned long long hi = (unsigned long long)__float_as_uint(v.w) << 32 | __float_as_uint(v.z);
+  __hip_atomic_store(q, lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(q + 1, hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void store_sum4(double* p, double4_t v) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) store_sum(p + i, v[i]);
+}
+
 // What the pointwise step of one unit of one row reads beside the sums.
+template <typename A>
 struct UnitInputs {
-  float h, c, b[4], mask;
+  A h, c, b[4], mask;
 };
 
 template <int GATES, typename T>
-__device__ __forceinline__ UnitInputs unit_inputs(const StepParams<T>& p, int n, int j) {
-  UnitInputs u = {};
+__device__ __forceinline__ UnitInputs<typename Step<T>::Sum> unit_inputs(const StepParams<T>& p, int n, int j) {
+  typedef typename Step<T>::Sum A;
+  UnitInputs<A> u = {};
   const int H = p.H;
   const size_t e = (size_t)n * H + j;
-  u.h = (float)p.h[e];
+  u.h = (A)p.h[e];
   if constexpr (GATES == 4) {
-    u.c = (float)p.c[e];
+    u.c = (A)p.c[e];
 #pragma unroll
-    for (int g = 0; g < 4; ++g) u.b[g] = (float)p.b[g * H + j];
+    for (int g = 0; g < 4; ++g) u.b[g] = (A)p.b[g * H + j];
   } else {
-    u.b[0] = (float)p.b[j] + (float)p.br[j];
-    u.b[1] = (float)p.b[H + j] + (float)p.br[H + j];
-    u.b[2] = (float)p.b[2 * H + j];
-    u.b[3] = (float)p.br[2 * H + j];
+    u.b[0] = (A)p.b[j] + (A)p.br[j];
+    u.b[1] = (A)p.b[H + j] + (A)p.br[H + j];
+    u.b[2] = (A)p.b[2 * H + j];
+    u.b[3] = (A)p.br[2 * H + j];
   }
-  if (p.training && p.zoneout_prob != 0.f && p.zoneout_mask != nullptr) u.mask = (float)p.zoneout_mask[e];
+  if (p.training && p.zoneout_prob != 0.f && p.zoneout_mask != nullptr) u.mask = (A)p.zoneout_mask[e];
   return u;
 }
 
 // Unit j of row n from its sums a: LSTM the four gates of [x | h] * [W; R]; GRU the update and the
 // reset gate, x * W and h * R of the candidate gate.
 template <int GATES, typename T>
-__device__ __forceinline__ void finish_unit(const StepParams<T>& p, int n, int j, const float (&a)[4],
-                                            const UnitInputs& in) {
+__device__ __forceinline__ void finish_unit(const StepParams<T>& p, int n, int j, const typename Step<T>::Sum (&a)[4],
+                                            const UnitInputs<typename Step<T>::Sum>& in) {
+  typedef typename Step<T>::Sum A;
+  typedef Step<T> S;
   const int H = p.H;
   const size_t e = (size_t)n * H + j;
   const bool zoneout = p.zoneout_prob != 0.f && p.zoneout_mask != nullptr;
-  float h_new;
+  A h_new;
   if constexpr (GATES == 4) {
-    const float gi = sigmoid_f(a[0] + in.b[0]), gg = tanh_f(a[1] + in.b[1]);
-    const float gf = sigmoid_f(a[2] + in.b[2]), go = sigmoid_f(a[3] + in.b[3]);
-    const float c_new = gf * in.c + gi * gg;
-    h_new = go * tanh_f(c_new);
+    const A gi = S::sigmoid(a[0] + in.b[0]), gg = S::tanh_(a[1] + in.b[1]);
+    const A gf = S::sigmoid(a[2] + in.b[2]), go = S::sigmoid(a[3] + in.b[3]);
+    const A c_new = gf * in.c + gi * gg;
+    h_new = go * S::tanh_(c_new);
     p.c_out[e] = (T)c_new;
     if (p.training) {
       T* vt = p.v + (size_t)n * 4 * H + j;
       vt[0] = (T)gi; vt[H] = (T)gg; vt[2 * H] = (T)gf; vt[3 * H] = (T)go;
     }
   } else {
-    const float z = sigmoid_f(a[0] + in.b[0]);
-    const float r = sigmoid_f(a[1] + in.b[1]);
-    const float qg = a[3] + in.b[3];
-    const float g = tanh_f(a[2] + r * qg + in.b[2]);
-    h_new = z * in.h + (1.0f - z) * g;
+    const A z = S::sigmoid(a[0] + in.b[0]);
+    const A r = S::sigmoid(a[1] + in.b[1]);
+    const A qg = a[3] + in.b[3];
+    const A g = S::tanh_(a[2] + r * qg + in.b[2]);
+    h_new = z * in.h + (A(1) - z) * g;
     if (p.training && p.v != nullptr) {
       T* vt = p.v + (size_t)n * 4 * H + j;
       vt[0] = (T)z; vt[H] = (T)r; vt[2 * H] = (T)g; vt[3 * H] = (T)qg;
@@ -106,10 +160,10 @@ __device__ __forceinline__ void finish_unit(const StepParams<T>& p, int n, int j
   }
   if (zoneout) {
     if (p.training) h_new = (h_new - in.h) * in.mask + in.h;
-    else h_new = p.zoneout_prob * in.h + (1.0f - p.zoneout_prob) * h_new;
+    else h_new = A(p.zoneout_prob) * in.h + (A(1) - A(p.zoneout_prob)) * h_new;
   }
   if (p.h_stage == nullptr) p.h_out[e] = (T)h_new;
-  else store_agent(&p.h_stage[e], h_new);
+  else store_sum(&p.h_stage[e], h_new);
 }
 
 // h_out overlaps h: other workgroups may still be reading h when a column block is finished,
@@ -130,15 +184,7 @@ __device__ __forceinline__ void copy_staged_state(const StepParams<T>& p, unsign
   __syncthreads();
   if (*flag == 0u) return;
   const int count = p.N * p.H;
-  for (int i = threadIdx.x; i < count; i += 256) p.h_out[i] = (T)load_exchanged(&p.h_stage[i]);
-}
-
-__device__ __forceinline__ void store_agent4(float* p, float4_t v) {
-  unsigned long long* q = reinterpret_cast<unsigned long long*>(p);
-  const unsigned long long lo = (unsigned long long)__float_as_uint(v.y) << 32 | __float_as_uint(v.x);
-  const unsigned long long hi = (unsigned long long)__float_as_uint(v.w) << 32 | __float_as_uint(v.z);
-  __hip_atomic_store(q, lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  __hip_atomic_store(q + 1, hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  for (int i = threadIdx.x; i < count; i += 256) p.h_out[i] = (T)load_sum(&p.h_stage[i]);
 }
 
 // GATES = 4: LSTM (i, g, f, o); GATES = 3: GRU (z, r, g).  RT: tiles of 16 batch rows a workgroup
@@ -152,7 +198,9 @@ __device__ __forceinline__ void store_agent4(float* p, float4_t v) {
 template <int GATES, int RT, bool DROPCONNECT, typename T>
 __global__ __launch_bounds__(256)
 void forward_step_kernel(StepParams<T> p) {
-  __shared__ __attribute__((aligned(16))) float s_in[RT * 16 * kStageStride];
+  typedef typename Step<T>::Sum A;
+  typedef typename Step<T>::Sum4 A4;
+  __shared__ __attribute__((aligned(16))) A s_in[RT * 16 * kStageStride];
   __shared__ unsigned int s_flag;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int N = p.N, H = p.H;
@@ -202,14 +250,14 @@ void forward_step_kernel(StepParams<T> p) {
     }
   };
 
-  const float4_t zero4 = {0.f, 0.f, 0.f, 0.f};
-  float4_t acc[RT];
+  const A4 zero4 = {A(0), A(0), A(0), A(0)};
+  A4 acc[RT];
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) acc[rt] = zero4;
   // Groups g .., staged from s0 on.  Every batch is summed by itself, in four sums side by side: short chains,
   // whose rounding errors stay those of many small runs.
   auto multiply = [&](int g, int s0, const T (&w)[kBatchGroups][4], const T (&m)[kBatchGroups][4]) {
-    float4_t part[RT][4];
+    A4 part[RT][4];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
@@ -220,19 +268,19 @@ void forward_step_kernel(StepParams<T> p) {
       if (gg < my_first || gg >= my_last) continue;  // the same for a whole wavefront
       const bool recurrent = gg >= groups_w;
       const int left = (recurrent ? len_r : len_w) - (recurrent ? gg - groups_w : gg) * kGroupRows;
-      float4_t a[RT];
+      A4 a[RT];
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt)
-        a[rt] = *reinterpret_cast<const float4_t*>(
+        a[rt] = *reinterpret_cast<const A4*>(
             &s_in[(rt * 16 + (lane & 15)) * kStageStride + (gg - s0) * kGroupRows + k_lane]);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        float weight = (float)w[q][i];
-        if constexpr (DROPCONNECT) weight = recurrent ? weight * (float)m[q][i] * p.dc_scale : weight;
-        weight = k_lane + i < left ? weight : 0.f;
+        A weight = (A)w[q][i];
+        if constexpr (DROPCONNECT) weight = recurrent ? weight * (A)m[q][i] * A(p.dc_scale) : weight;
+        weight = k_lane + i < left ? weight : A(0);
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt)
-          part[rt][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[rt][i], weight, part[rt][i], 0, 0, 0);
+          part[rt][i] = Step<T>::mfma(a[rt][i], weight, part[rt][i]);
       }
     }
 #pragma unroll
@@ -247,16 +295,16 @@ void forward_step_kernel(StepParams<T> p) {
       const bool recurrent = mine >= groups_w;
       const int len = recurrent ? len_r : len_w, k = (recurrent ? mine - groups_w : mine) * kGroupRows + (lane & 15);
       const T* in = (recurrent ? p.h : p.x) + (k < len ? k : len - 1);
-      float value[4 * RT];
+      A value[4 * RT];
 #pragma unroll
       for (int i = 0; i < 4 * RT; ++i) {
         const int n = n0 + wave + 4 * i;
-        value[i] = (float)in[(size_t)(n < N ? n : N - 1) * len];
+        value[i] = (A)in[(size_t)(n < N ? n : N - 1) * len];
       }
 #pragma unroll
       for (int i = 0; i < 4 * RT; ++i)
         s_in[(wave + 4 * i) * kStageStride + (g - s0) * kGroupRows + lane] =
-            k < len && n0 + wave + 4 * i < N ? value[i] : 0.f;
+            k < len && n0 + wave + 4 * i < N ? value[i] : A(0);
     }
     __syncthreads();
   };
@@ -279,27 +327,26 @@ void forward_step_kernel(StepParams<T> p) {
     g += kBatchGroups;
   }
 
-  // Lane l of wavefront w holds sum w of rows 4 (l / 16) .. + 3 of each tile and unit l % 16.
-  // Thread t finishes row 4 (t / 64) + t % 4 and unit (t / 4) % 16 of each: its sums lie side by
-  // side with its neighbours'.
-  const int row = 4 * (tid >> 6) + (tid & 3), j = j0 + ((tid >> 2) & 15);
-  const unsigned slot = 64 * p.quads, run_stride = tiles * 4 * slot;  // floats of one sum of a tile, of a run
+  // Lane l of wavefront w holds sum w of four rows of each tile and unit l % 16.  Thread t finishes element t % 4
+  // of lane t / 4: its sums lie side by side with its neighbours'.
+  const int row = Step<T>::row(tid >> 2, tid & 3), j = j0 + ((tid >> 2) & 15);
+  const unsigned slot = 64 * p.quads, run_stride = tiles * 4 * slot;  // one sum of a tile, all of a run
   if (p.runs == 1) {
     __syncthreads();
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
-      *reinterpret_cast<float4_t*>(&s_in[(wave * RT + rt) * 256 + 4 * lane]) = acc[rt];
+      *reinterpret_cast<A4*>(&s_in[(wave * RT + rt) * 256 + 4 * lane]) = acc[rt];
   } else {
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
-      if (4 * rt + (lane >> 4) < p.quads)
-        store_agent4(p.partial + run * run_stride + (4 * tile + wave) * slot + rt * 256 + 4 * lane, acc[rt]);
+      if (!Step<T>::kQuads || 4 * rt + (lane >> 4) < p.quads)
+        store_sum4(p.partial + run * run_stride + (4 * tile + wave) * slot + rt * 256 + 4 * lane, acc[rt]);
   }
   // What the pointwise step reads is on its way while the sums are handed over.
-  UnitInputs in[RT];
+  UnitInputs<A> in[RT];
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
-    in[rt] = UnitInputs{};
+    in[rt] = UnitInputs<A>{};
     const int n = n0 + 16 * rt + row;
     if (n < N && j < H) in[rt] = unit_inputs<GATES, T>(p, n, j);
   }
@@ -309,19 +356,19 @@ void forward_step_kernel(StepParams<T> p) {
   for (int rt = 0; rt < RT; ++rt) {
     const int n = n0 + 16 * rt + row;
     if (n >= N || j >= H) continue;
-    float a[4] = {0.f, 0.f, 0.f, 0.f};
+    A a[4] = {A(0), A(0), A(0), A(0)};
     if (p.runs == 1) {
 #pragma unroll
       for (int g = 0; g < 4; ++g) a[g] = s_in[(g * RT + rt) * 256 + tid];
     } else {
       const unsigned at = 4 * tile * slot + rt * 256 + tid;
       for (int r0 = 0; r0 < p.runs; r0 += 16) {  // 64 loads in flight
-        float run_sum[16][4];
+        A run_sum[16][4];
 #pragma unroll
         for (int i = 0; i < 16; ++i)
 #pragma unroll
           for (int g = 0; g < 4; ++g)
-            run_sum[i][g] = r0 + i < p.runs ? load_exchanged(p.partial + (at + (r0 + i) * run_stride + g * slot)) : 0.f;
+            run_sum[i][g] = r0 + i < p.runs ? load_sum(p.partial + (at + (r0 + i) * run_stride + g * slot)) : A(0);
 #pragma unroll
         for (int width = 8; width > 0; width /= 2)
 #pragma unroll
@@ -340,7 +387,7 @@ void forward_step_kernel(StepParams<T> p) {
 // How a step is cut up.
 struct StepCut {
   int rt, row_blocks, unit_blocks, runs, quads;
-  size_t partial_floats() const {
+  size_t sums() const {
     return runs > 1 ? (size_t)runs * row_blocks * unit_blocks * 4 * 64 * quads : 0;
   }
 };
@@ -357,13 +404,13 @@ long long step_blocks(int N, int C, int H) {
 // more than 32 groups, up to four workgroups per CU (GRU, N = 8, C = 64, H = 3776: 46.0 -> 44.5 us).
 // 32 rows a workgroup halve the reading of weights, once there are enough tiles for it (LSTM,
 // C = H = 512, us with 16 / 32 rows: N = 64, 128 tiles of 16, 12.2 / 14.2; N = 128, 256 tiles, 17.6 / 16.5).
-StepCut step_cut(int N, int C, int H) {
+StepCut step_cut(int N, int C, int H, size_t element) {
   StepCut s;
   const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
   s.unit_blocks = (H + kStepUnits - 1) / kStepUnits;
-  s.rt = N > 16 && (N + 15) / 16 * (long long)s.unit_blocks >= cus ? 2 : 1;
+  s.rt = element < 8 && N > 16 && (N + 15) / 16 * (long long)s.unit_blocks >= cus ? 2 : 1;
   s.row_blocks = (N + 16 * s.rt - 1) / (16 * s.rt);
-  s.quads = s.row_blocks > 1 ? 4 * s.rt : (N + 3) / 4;
+  s.quads = s.row_blocks > 1 || element == 8 ? 4 * s.rt : (N + 3) / 4;
   const int groups = (C + kGroupRows - 1) / kGroupRows + (H + kGroupRows - 1) / kGroupRows;
   const long long tiles = (long long)s.row_blocks * s.unit_blocks;
   long long runs = (2 * cus + tiles - 1) / tiles;
@@ -378,21 +425,22 @@ StepCut step_cut(int N, int C, int H) {
 
 template <int GATES, typename T>
 int launch_step(hipStream_t stream, StepParams<T>& p, const char* name) {
-  StepCut cut = step_cut(p.N, p.C, p.H);
+  typedef typename Step<T>::Sum A;
+  StepCut cut = step_cut(p.N, p.C, p.H, sizeof(T));
   const size_t state_bytes = staged_state_bytes(p.N, p.H, p.h, p.h_out, sizeof(T));
   for (bool room = false; !room && cut.runs > 1;) {
-    HASTE_HIP_PROPAGATE(workspace_has_room(stream, cut.partial_floats() * sizeof(float) + state_bytes + 256, &room));
+    HASTE_HIP_PROPAGATE(workspace_has_room(stream, cut.sums() * sizeof(A) + state_bytes + 256, &room));
     if (!room) cut.runs = (cut.runs + 1) / 2;
   }
-  const size_t partial_bytes = cut.partial_floats() * sizeof(float);
+  const size_t partial_bytes = cut.sums() * sizeof(A);
   Workspace ws;
   HASTE_HIP_PROPAGATE(get_workspace(stream, partial_bytes + state_bytes + 256, &ws));
   if (PlannedPass* pass = planned_pass()) {
     pass->kernel = kPlanSingleStep;
     return HASTE_HIP_OK;
   }
-  p.partial = ws.scratch;
-  p.h_stage = state_bytes > 0 ? ws.scratch + partial_bytes / sizeof(float) : nullptr;
+  p.partial = reinterpret_cast<A*>(ws.scratch);
+  p.h_stage = state_bytes > 0 ? p.partial + cut.sums() : nullptr;
   p.cb = ws.control;
   p.runs = cut.runs; p.row_blocks = cut.row_blocks; p.unit_blocks = cut.unit_blocks; p.quads = cut.quads;
   const dim3 grid((unsigned)cut.row_blocks * cut.unit_blocks * cut.runs);
@@ -402,7 +450,10 @@ int launch_step(hipStream_t stream, StepParams<T>& p, const char* name) {
     if (p.dc_mask != nullptr) forward_step_kernel<GATES, RT_, true, T><<<grid, dim3(256), 0, stream>>>(p);  \
     else forward_step_kernel<GATES, RT_, false, T><<<grid, dim3(256), 0, stream>>>(p);                      \
   }
-  HASTE_LAUNCH_STEP(1) HASTE_LAUNCH_STEP(2)
+  HASTE_LAUNCH_STEP(1)
+  if constexpr (Step<T>::kQuads) {
+    HASTE_LAUNCH_STEP(2)
+  }
 #undef HASTE_LAUNCH_STEP
   HASTE_HIP_TRY(hipGetLastError());
   return HASTE_HIP_OK;
@@ -410,26 +461,29 @@ int launch_step(hipStream_t stream, StepParams<T>& p, const char* name) {
 
 }  // namespace
 
-// Whether a step of N rows is this kernel's.  Up to 8 rows always, as long as its tiles have counters.  Beyond, the other way is the
-// all-steps kernels, which fetch their slice of R in a single row of loads (kStepResident: they keep R on
-// chip; LSTM, us there / here: N = 43, C = 32, H = 128 13.6 / 5.7, N = 64, C = 64, H = 2048 82 / 52), or a GEMM
-// per side, faster from some size on because it keeps more of both operands on chip (kStepStreamed; N = 16,
-// C = 64, H = 4096, 66 560 blocks, 53 / 63; N = 128, C = 512, H = 1536, 98 304 blocks, 51 / 60; N = 128, C = 256,
-// H = 1024, 40 960 blocks, 48 / 30).  The half GRU's other way converts its weights: here at every size (N = 64,
-// C = 64, H = 2048 125 / 48, N = 128, C = 512, H = 4096 420 / 290).
-int single_step_rule(hipStream_t stream, int N, int C, int H, long long most_blocks, size_t staged_bytes, bool* applies) {
-  const StepCut cut = step_cut(N, C, H);
+// Whether a step of N rows is this kernel's (most_blocks: kStep...).  In float up to 8 rows always, as long as its
+// tiles have counters.  Beyond, the other way is the all-steps kernels, which fetch their slice of R for one use
+// (kStepResident: they keep R on chip; LSTM, us there / here: N = 43, C = 32, H = 128 13.6 / 5.7, N = 64, C = 64,
+// H = 2048 82 / 52), or a GEMM per side, faster from some size on because it keeps more of both operands on chip
+// (kStepStreamed; N = 16, C = 64, H = 4096, 66 560 blocks, 53 / 63; N = 128, C = 512, H = 1536, 98 304 blocks,
+// 51 / 60; N = 128, C = 256, H = 1024, 40 960 blocks, 48 / 30).  The half GRU's other way converts its weights: here
+// at every size (N = 64, C = 64, H = 2048 125 / 42, N = 128, C = 512, H = 4096 420 / 261).  In double (kStepDouble) it is a
+// product per side and a pointwise launch: LSTM N = 1, C = H = 512 17.4 / 11.5, N = 43, C = 64, H = 192 14.1 / 9.7,
+// N = 128, C = H = 512, 16 384 blocks, 32.9 / 27.8; GRU N = 8, C = 64, H = 2048, 16 896 blocks, 29.9 / 31.3.
+int single_step_rule(hipStream_t stream, int N, int C, int H, size_t element, long long most_blocks, size_t staged_bytes,
+                     bool* applies) {
+  const StepCut cut = step_cut(N, C, H, element);
   *applies = (long long)cut.row_blocks * cut.unit_blocks <= kStepTiles;
-  if (!*applies || N <= 8) return HASTE_HIP_OK;
+  if (!*applies || (N <= 8 && element != 8)) return HASTE_HIP_OK;
   *applies = step_blocks(N, C, H) <= most_blocks;
   if (!*applies) return HASTE_HIP_OK;
-  return workspace_has_room(stream, cut.partial_floats() * sizeof(float) + staged_bytes + 256, applies);
+  return workspace_has_room(stream, cut.sums() * (element == 8 ? 8 : 4) + staged_bytes + 256, applies);
 }
 
 size_t staged_state_bytes(int N, int H, const void* h, const void* h_out, size_t element) {
   const uintptr_t from = reinterpret_cast<uintptr_t>(h), to = reinterpret_cast<uintptr_t>(h_out);
   const size_t floats = (size_t)N * H;
-  return to < from + floats * element && from < to + floats * element ? floats * sizeof(float) : 0;
+  return to < from + floats * element && from < to + floats * element ? floats * (element == 8 ? 8 : 4) : 0;
 }
 
 int lstm_forward_single_step(hipStream_t stream, int training, int N, int C, int H, const float* W,
@@ -457,6 +511,33 @@ int gru_forward_single_step(hipStream_t stream, int training, int N, int C, int 
   p.zoneout_prob = zoneout_prob; p.zoneout_mask = zoneout_mask;
   p.dc_mask = dc_mask; p.dc_scale = dc_scale;
   return launch_step<3>(stream, p, "gru_forward_step");
+}
+
+int lstm_forward_single_step(hipStream_t stream, int training, int N, int C, int H, const double* W,
+                             const double* R, const double* b, const double* x, const double* h,
+                             const double* c, double* h_out, double* c_out, double* v,
+                             float zoneout_prob, const double* zoneout_mask, const double* dc_mask,
+                             float dc_scale) {
+  StepParams<double> p = {};
+  p.training = training; p.N = N; p.C = C; p.H = H;
+  p.W = W; p.R = R; p.b = b; p.x = x; p.h = h; p.c = c;
+  p.h_out = h_out; p.c_out = c_out; p.v = v;
+  p.zoneout_prob = zoneout_prob; p.zoneout_mask = zoneout_mask;
+  p.dc_mask = dc_mask; p.dc_scale = dc_scale;
+  return launch_step<4>(stream, p, "lstm_forward_step_double");
+}
+
+int gru_forward_single_step(hipStream_t stream, int training, int N, int C, int H, const double* W,
+                            const double* R, const double* bx, const double* br, const double* x,
+                            const double* h, double* h_out, double* v, float zoneout_prob,
+                            const double* zoneout_mask, const double* dc_mask, float dc_scale) {
+  StepParams<double> p = {};
+  p.training = training; p.N = N; p.C = C; p.H = H;
+  p.W = W; p.R = R; p.b = bx; p.br = br; p.x = x; p.h = h;
+  p.h_out = h_out; p.v = v;
+  p.zoneout_prob = zoneout_prob; p.zoneout_mask = zoneout_mask;
+  p.dc_mask = dc_mask; p.dc_scale = dc_scale;
+  return launch_step<3>(stream, p, "gru_forward_step_double");
 }
 
 int gru_forward_single_step_half(hipStream_t stream, int training, int N, int C, int H, const void* W,

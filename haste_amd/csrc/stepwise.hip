@@ -1227,6 +1227,14 @@ int lstm_forward_steps(hipStream_t stream, int training, int steps, int N, int C
                        const T* W, const T* R, const T* b, const T* x, const T* h, const T* c,
                        T* h_out, T* c_out, T* v, float zoneout_prob, const T* zoneout_mask,
                        const T* dc_mask, float dc_scale) {
+  if constexpr (std::is_same<T, double>::value) {
+    bool single = false;
+    if (steps == 1)
+      HASTE_HIP_PROPAGATE(single_step_rule(stream, N, C, H, sizeof(T), kStepDouble, staged_state_bytes(N, H, h, h_out, sizeof(T)), &single));
+    if (single)
+      return lstm_forward_single_step(stream, training, N, C, H, W, R, b, x, h, c, h_out, c_out, v, zoneout_prob, zoneout_mask, dc_mask,
+                                      dc_scale);
+  }
   const size_t NH = (size_t)N * H, N4H = NH * 4, r_count = (size_t)H * 4 * H;
   size_t own = padded(N4H * sizeof(T)) + (dc_mask ? padded(r_count * sizeof(T)) : 0);
   const Room room = max2(gemm_room<T>(steps * N, 4 * H, C), gemm_room<T>(N, 4 * H, H));
@@ -1302,6 +1310,13 @@ int gru_forward_steps(hipStream_t stream, int training, int steps, int N, int C,
                       const T* R, const T* bx, const T* br, const T* x, const T* h, T* h_out, T* v,
                       T* tmp_Wx, float zoneout_prob, const T* zoneout_mask, const T* dc_mask,
                       float dc_scale) {
+  if constexpr (std::is_same<T, double>::value) {
+    bool single = false;
+    if (steps == 1)
+      HASTE_HIP_PROPAGATE(single_step_rule(stream, N, C, H, sizeof(T), kStepDouble, staged_state_bytes(N, H, h, h_out, sizeof(T)), &single));
+    if (single)
+      return gru_forward_single_step(stream, training, N, C, H, W, R, bx, br, x, h, h_out, v, zoneout_prob, zoneout_mask, dc_mask, dc_scale);
+  }
   const size_t NH = (size_t)N * H, N3H = NH * 3, N4H = NH * 4, r_count = (size_t)H * 3 * H;
   size_t own = padded(N3H * sizeof(T)) + (dc_mask ? padded(r_count * sizeof(T)) : 0);
   const Room room = max2(gemm_room<T>(steps * N, 3 * H, C), gemm_room<T>(N, 3 * H, H));
@@ -2093,7 +2108,7 @@ int haste_hip_gru_forward_f16(int training, int steps, int batch_size, int input
     return gru_forward_half(as_stream(stream), training, steps, batch_size, input_size, hidden_size, W, R,
                             bx, br, x, h, v, zoneout_prob, zoneout_mask, nullptr, 1.f);
   bool single = false;
-  HASTE_HIP_PROPAGATE(single_step_rule(as_stream(stream), batch_size, input_size, hidden_size, kStepHalf,
+  HASTE_HIP_PROPAGATE(single_step_rule(as_stream(stream), batch_size, input_size, hidden_size, sizeof(half_t), kStepHalf,
                                        staged_state_bytes(batch_size, hidden_size, h, hp(h) + NH, sizeof(half_t)), &single));
   if (single)
     return gru_forward_single_step_half(as_stream(stream), training, batch_size, input_size, hidden_size,
@@ -2119,7 +2134,7 @@ int haste_hip_gru_forward_dropconnect_f16(int training, int steps, int batch_siz
                             bx, br, x, h, v, zoneout_prob, zoneout_mask, dropconnect_mask,
                             dropconnect_scale);
   bool single = false;
-  HASTE_HIP_PROPAGATE(single_step_rule(as_stream(stream), batch_size, input_size, hidden_size, kStepHalf,
+  HASTE_HIP_PROPAGATE(single_step_rule(as_stream(stream), batch_size, input_size, hidden_size, sizeof(half_t), kStepHalf,
                                        staged_state_bytes(batch_size, hidden_size, h, hp(h) + NH, sizeof(half_t)), &single));
   if (single)
     return gru_forward_single_step_half(as_stream(stream), training, batch_size, input_size, hidden_size,
@@ -2160,7 +2175,7 @@ int haste_hip_gru_forward_iterate_f16(int training, int batch_size, int input_si
   HASTE_HIP_REQUIRE(batch_size > 0 && input_size > 0 && hidden_size > 0);
   HASTE_HIP_REQUIRE(W && R && bx && br && x && h && h_out && tmp_Wx && (v || !training));
   bool single = false;
-  HASTE_HIP_PROPAGATE(single_step_rule(as_stream(stream), batch_size, input_size, hidden_size, kStepHalf,
+  HASTE_HIP_PROPAGATE(single_step_rule(as_stream(stream), batch_size, input_size, hidden_size, sizeof(half_t), kStepHalf,
                                        staged_state_bytes(batch_size, hidden_size, h, h_out, sizeof(half_t)), &single));
   if (single)
     return gru_forward_single_step_half(as_stream(stream), training, batch_size, input_size, hidden_size,

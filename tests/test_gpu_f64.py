@@ -91,6 +91,18 @@ def test_f64_iterate(double_precision, T, N, C, H, zoneout):
     test_gpu_iterate.test_gru_iterate(T, N, C, H, zoneout)
 
 
+# One kernel for a step: a row, partly filled tiles of 16 rows and units, several runs, sides of any length.
+@pytest.mark.parametrize("training", [True, False])
+@pytest.mark.parametrize("N,C,H", [(1, 512, 512), (3, 100, 333), (16, 16, 512), (17, 5, 47), (40, 60, 1500), (128, 3, 1)])
+def test_f64_single_step_kernel(double_precision, N, C, H, training):
+    test_gpu_iterate.test_single_step_kernel(N, C, H, training, 0.25)
+
+
+@pytest.mark.parametrize("N,C,H", [(4, 48, 200), (33, 48, 200)])
+def test_f64_single_step_dropconnect(double_precision, N, C, H):
+    test_gpu_lstm.test_lstm_dropconnect_fused_equals_premasked_weights(1, N, C, H)
+
+
 @pytest.mark.parametrize("trans_a,M,N,K", [(False, 1, 1, 1), (False, 37, 53, 29), (False, 128, 192, 64),
                                            (True, 70, 130, 45), (True, 5, 20, 33), (False, 300, 100, 1000),
                                            # few tiles, long contractions: cut along K into pieces
