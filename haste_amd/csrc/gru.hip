@@ -164,7 +164,11 @@ void gru_forward_kernel(GruFwdParams p) {
 #pragma unroll
         for (int g = 0; g < 3; ++g) wx_next[pp][g] = wt[g * H];
       }
-      if (zoneout && p.training) mk_next[pp] = p.zoneout_mask[(size_t)tt * NH + row * H + unit];
+      if (zoneout && p.training) {
+        const size_t at = (size_t)tt * NH + row * H + unit;
+        if (HALF && p.half_io) mk_next[pp] = (float)reinterpret_cast<const _Float16*>(p.zoneout_mask)[at];
+        else mk_next[pp] = p.zoneout_mask[at];
+      }
     }
   };
   fetch(0);
@@ -250,12 +254,23 @@ void gru_forward_kernel(GruFwdParams p) {
 #pragma unroll
     for (int pp = 0; pp < PP; ++pp) {
       if (act[pp]) {
+        const size_t v_at = ((size_t)t * N + pn[pp]) * 4 * H + pj[pp];
+        const size_t h_at = (size_t)t * NH + (size_t)pn[pp] * H + pj[pp];
+        if (HALF && p.half_io) {
+          if (p.training) {
+            _Float16* vt = reinterpret_cast<_Float16*>(p.v) + v_at;
+#pragma unroll
+            for (int g = 0; g < 4; ++g) vt[g * H] = (_Float16)saved[pp][g];
+          }
+          reinterpret_cast<_Float16*>(p.h_out)[h_at] = (_Float16)h_prev[pp];
+          continue;
+        }
         if (p.training) {
-          float* vt = p.v + ((size_t)t * N + pn[pp]) * 4 * H + pj[pp];
+          float* vt = p.v + v_at;
 #pragma unroll
           for (int g = 0; g < 4; ++g) vt[g * H] = saved[pp][g];
         }
-        p.h_out[(size_t)t * NH + (size_t)pn[pp] * H + pj[pp]] = h_prev[pp];
+        p.h_out[h_at] = h_prev[pp];
       }
     }
   }
@@ -693,15 +708,35 @@ bool gru_backward_resident(int N, int H) {
   return pick_backward_tile(gru_backward_k(H), N, H, 6 * 16, 0, true).ok;
 }
 
+// Whether the recurrence of a pass on widened half tensors (half_product, T > 1) reads and writes the caller's half
+// tensors itself: forward h_out, v and zoneout_mask, backward (products == false) h, v, dh_next and zoneout_mask, and
+// dp and dq.  The kernels whose product is on the half matrix cores do, and nothing else is tried before them up to 512
+// units.
+static bool half_forward(const ForwardTile& tile, int H) {
+  if (H > 512 || !tile.ok || tile.reg_groups > 0) return false;
+  return tile.nb == 4 || (tile.nb == 8 && paired_lds_bytes((H + 63) / 64 * 64, tile.ct) <= kWorkgroupLdsBytes);
+}
+static bool scattered_backward(const BackwardTile& tile, int H) {
+  return tile.ok && tile.reg_groups == 0 && H <= 512 && (tile.nb == 8 || (tile.nb == 4 && H > 320));
+}
+bool gru_forward_half_io(int N, int H) {
+  return !(N == 1 && H <= 512 && xcd_local_fits((H + 15) / 16, 1)) &&
+         half_forward(pick_forward_tile(3, N, H, 0, kWorkgroupLdsBytes, false, 3), H);
+}
+bool gru_backward_half_io(int N, int H) {
+  return scattered_backward(pick_backward_tile(gru_backward_k(H), N, H, 6 * 16, 0, true), H);
+}
+
 // h: [N,H] state before the first step; h_out: [T,N,H] states after each step.
 // wx_ready (T > 1, gru_forward_resident): tmp_Wx already holds x*W, and W and x are not looked at.
 // half_product: the tensors are widened half tensors (gru_half.hip); with 4-row tiles the step's
 // product h * R goes to the half matrix cores (h rounded to half there, as such a cell stores it).
+// half_io (gru_forward_half_io): h_out, v and zoneout_mask are half tensors.
 int gru_forward_impl(hipStream_t stream, int training, int T, int N, int C, int H,
                      const float* W, const float* R, const float* bx, const float* br,
                      const float* x, const float* h, float* h_out, float* v, float* tmp_Wx,
                      float zoneout_prob, const float* zoneout_mask, const float* dc_mask,
-                     float dc_scale, bool wx_ready, bool half_product) {
+                     float dc_scale, bool wx_ready, bool half_product, bool half_io) {
   HASTE_HIP_REQUIRE(T > 0 && N > 0 && C > 0 && H > 0);
   HASTE_HIP_REQUIRE(R && bx && br && h && h_out && tmp_Wx && (wx_ready || (W && x)));
   HASTE_HIP_REQUIRE(!training || v != nullptr);
@@ -718,10 +753,11 @@ int gru_forward_impl(hipStream_t stream, int training, int T, int N, int C, int 
       return gru_forward_single_step(stream, training, N, C, H, W, R, bx, br, x, h, h_out, v,
                                      zoneout_prob, zoneout_mask, dc_mask, dc_scale);
   }
-  if (N == 1 && H <= 512 && xcd_local_fits((H + 15) / 16, 1))
+  if (N == 1 && H <= 512 && xcd_local_fits((H + 15) / 16, 1) && !half_io)
     return gru_forward_single_row(stream, training, T, C, H, W, R, bx, br, x, h, h_out, v, tmp_Wx,
                                   zoneout_prob, zoneout_mask, dc_mask, dc_scale, wx_ready);
   const ForwardTile tile = pick_forward_tile(3, N, H, 0, kWorkgroupLdsBytes, false, 3);
+  HASTE_HIP_REQUIRE(!half_io || (half_product && half_forward(tile, H)));
   bool taken = false;
   HASTE_HIP_PROPAGATE(gru_forward_cut(stream, training, T, N, C, H, W, R, bx, br, x, h, h_out, v, tmp_Wx, zoneout_prob,
                                       zoneout_mask, dc_mask, dc_scale, wx_ready, !tile.ok || tile.reg_groups > 0, &taken));
@@ -771,6 +807,7 @@ int gru_forward_impl(hipStream_t stream, int training, int T, int N, int C, int 
   p.zoneout_prob = zoneout_prob; p.zoneout_mask = zoneout_mask;
   p.dc_mask = dc_mask; p.dc_scale = dc_scale;
   p.xh = ws.scratch;
+  p.half_io = half_io;
   if (split_rows > 0)
     return launch_split_forward<GruForwardCell>("gru_forward_recurrence", stream, ws, split_rows, p);
   LaunchPlan plan;
@@ -828,11 +865,12 @@ int gru_forward_impl(hipStream_t stream, int training, int T, int N, int C, int 
 // caller computes dx, dW and dR from dp and dq itself, and W_t, x_t, dx, dW, dR are not looked at.
 // half_product: the tensors are widened half tensors (gru_half.hip); where the scattered form
 // runs, its product dh = (gate gradients) * R_t goes to the half matrix cores.
+// half_io (products == false, gru_backward_half_io): h, v, dh_next, zoneout_mask, dp and dq are half tensors.
 int gru_backward_impl(hipStream_t stream, int T, int N, int C, int H,
                       const float* W_t, const float* R_t, const float* x_t, const float* h,
                       const float* v, const float* dh_next, float* dx, float* dW, float* dR,
                       float* dbx, float* dbr, float* dh, float* dp, float* dq,
-                      const float* zoneout_mask, bool products, bool half_product) {
+                      const float* zoneout_mask, bool products, bool half_product, bool half_io) {
   HASTE_HIP_REQUIRE(T > 0 && N > 0 && C > 0 && H > 0);
   HASTE_HIP_REQUIRE(R_t && h && v && dh_next && (!products || (W_t && x_t)));
   HASTE_HIP_REQUIRE(dbx && dbr && dh && dp && dq && (!products || (dx && dW && dR)));
@@ -846,6 +884,7 @@ int gru_backward_impl(hipStream_t stream, int T, int N, int C, int H,
   };
   // per row: the partial tiles or the 6 bias-gradient columns of 16 floats
   const BackwardTile tile = pick_backward_tile(gru_backward_k(H), N, H, 6 * 16, 0, true);
+  HASTE_HIP_REQUIRE(!half_io || (half_product && !products && scattered_backward(tile, H)));
   bool taken = false;
   HASTE_HIP_PROPAGATE(gru_backward_cut(stream, T, N, H, R_t, h, v, dh_next, dbx, dbr, dh, dp, dq, zoneout_mask,
                                        !tile.ok || tile.reg_groups > 0, &taken));
@@ -861,8 +900,7 @@ int gru_backward_impl(hipStream_t stream, int T, int N, int C, int H,
   // (Measured against the other form over H = 64 ... 512, T = 100: with two sets per workgroup it is 5-15 % faster
   // at every H, with one set from H = 384 on; below, one set is 5-20 % faster the other way.  Two sets run where
   // split_backward_rule() below declines.)
-  const bool scatter = tile.reg_groups == 0 && H <= 512 &&
-                       (tile.nb == 8 || (tile.nb == 4 && H > 320));
+  const bool scatter = scattered_backward(tile, H);
   const bool paired = scatter ? tile.nb == 8
                               : tile.nb == 8 && paired_lds <= kMaxLdsBytes;
   const int sets = paired ? 2 : 1;
@@ -900,6 +938,8 @@ int gru_backward_impl(hipStream_t stream, int T, int N, int C, int H,
   int rc = HASTE_HIP_ERROR_UNSUPPORTED_SIZE;
   const char* name = "gru_backward_recurrence";
   if (split_rows > 0) rc = launch_split_backward<GruScatterCell>(name, stream, ws, split_rows, p);
+  else if (scatter && half_io)
+    rc = launch_scatter_backward<GruHalfScatterCell, true>(name, H, sets, plan, p, stream);
   else if (scatter && half_product) rc = launch_scatter_backward<GruScatterCell, true>(name, H, sets, plan, p, stream);
   else if (scatter) rc = launch_scatter_backward<GruScatterCell>(name, H, sets, plan, p, stream);
   else
@@ -938,7 +978,7 @@ int haste_hip_gru_forward_f32(int training, int steps, int batch_size, int input
   return haste_hip::gru_forward_impl(haste_hip::as_stream(stream), training, steps, batch_size,
                                      input_size, hidden_size, W, R, bx, br, x, h,
                                      h + (size_t)batch_size * hidden_size, v, tmp_Wx,
-                                     zoneout_prob, zoneout_mask, nullptr, 1.0f, false, false);
+                                     zoneout_prob, zoneout_mask, nullptr, 1.0f, false, false, false);
 }
 
 int haste_hip_gru_forward_dropconnect_f32(int training, int steps, int batch_size,
@@ -954,7 +994,7 @@ int haste_hip_gru_forward_dropconnect_f32(int training, int steps, int batch_siz
                                      input_size, hidden_size, W, R, bx, br, x, h,
                                      h + (size_t)batch_size * hidden_size, v, tmp_Wx,
                                      zoneout_prob, zoneout_mask, dropconnect_mask,
-                                     dropconnect_scale, false, false);
+                                     dropconnect_scale, false, false, false);
 }
 
 int haste_hip_gru_backward_f32(int steps, int batch_size, int input_size, int hidden_size,
@@ -969,7 +1009,7 @@ int haste_hip_gru_backward_f32(int steps, int batch_size, int input_size, int hi
   return haste_hip::gru_backward_impl(haste_hip::as_stream(stream), steps, batch_size, input_size,
                                       hidden_size, W_t, R_t, x_t, h, v,
                                       dh_new + (size_t)batch_size * hidden_size, dx, dW, dR, dbx,
-                                      dbr, dh, dp, dq, zoneout_mask, true, false);
+                                      dbr, dh, dp, dq, zoneout_mask, true, false, false);
 }
 
 int haste_hip_gru_forward_iterate_f32(int training, int batch_size, int input_size,
@@ -982,7 +1022,7 @@ int haste_hip_gru_forward_iterate_f32(int training, int batch_size, int input_si
   (void)tmp_Rh;
   return haste_hip::gru_forward_impl(haste_hip::as_stream(stream), training, 1, batch_size,
                                      input_size, hidden_size, W, R, bx, br, x, h, h_out, v, tmp_Wx,
-                                     zoneout_prob, zoneout_mask, nullptr, 1.0f, false, false);
+                                     zoneout_prob, zoneout_mask, nullptr, 1.0f, false, false, false);
 }
 
 int haste_hip_gru_backward_iterate_f32(int batch_size, int input_size, int hidden_size,
@@ -995,7 +1035,7 @@ int haste_hip_gru_backward_iterate_f32(int batch_size, int input_size, int hidde
   (void)br;
   return haste_hip::gru_backward_impl(haste_hip::as_stream(stream), 1, batch_size, input_size,
                                       hidden_size, W_t, R_t, x_t, h, v, dh_new, dx, dW, dR, dbx,
-                                      dbr, dh, dp, dq, zoneout_mask, true, false);
+                                      dbr, dh, dp, dq, zoneout_mask, true, false, false);
 }
 
 }  // extern "C"

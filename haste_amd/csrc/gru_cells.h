@@ -23,6 +23,7 @@ struct GruFwdParams {
   const float* dc_mask;  // DropConnect mask [H,3H] or null
   float dc_scale;
   float* xh;             // polled exchange tiles of h: [batch tiles][4][Kpad/4][NB][4]
+  int half_io;           // (kernels with a product on the half matrix cores) h_out, v and zoneout_mask are in half
   LaunchShape ls;
 };
 
@@ -201,6 +202,33 @@ struct GruScatterCell {
   static constexpr int kCutInputs = kInputs;
   __device__ __forceinline__ static int cut_input(int i) { return i; }
   __device__ __forceinline__ void carry_inputs(float (&)[kInputs]) {}
+};
+
+// The same on the caller's half tensors: h, v, dh_next and zoneout_mask are read, dp and dq written in half.
+struct GruHalfScatterCell : GruScatterCell {
+  typedef _Float16 half_t;
+  __device__ __forceinline__ static void request(const Params& p, float (&in)[kInputs], size_t e, size_t ve,
+                                                 bool zoneout) {
+    auto half = [](const float* q) { return reinterpret_cast<const half_t*>(q); };
+    const half_t* vt = half(p.v) + ve;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) in[i] = (float)vt[i * (size_t)p.H];
+    in[4] = (float)half(p.h)[e];
+    in[5] = (float)half(p.dh_next)[e];
+    if (zoneout) in[6] = (float)half(p.zoneout_mask)[e];
+  }
+  __device__ __forceinline__ static void store_copy(const Params& p, int t, size_t n, size_t j, const float4_t& a) {
+    const size_t H = p.H;
+    const size_t o3 = ((size_t)t * p.N + n) * 3 * H + j;
+    half_t *dp = reinterpret_cast<half_t*>(p.dp) + o3, *dq = reinterpret_cast<half_t*>(p.dq) + o3;
+    const half_t z = (half_t)a[0], r = (half_t)a[1];
+    dp[0] = z;
+    dp[H] = r;
+    dp[2 * H] = (half_t)a[3];
+    dq[0] = z;
+    dq[H] = r;
+    dq[2 * H] = (half_t)a[2];
+  }
 };
 
 }  // namespace

@@ -4,9 +4,10 @@
 //
 // The recurrence is bound by the latency of its per-step exchange and by instruction issue,
 // not by the rate of the matrix units or by HBM, so the persistent fp32 kernels are also the
-// fastest way to run it on half tensors: what it reads is widened into a staging area at the
-// front of the stream's scratch buffer (one launch), it runs on the staged copies, and what the
-// caller gets back is rounded to half (one launch).  Between the steps the state stays in fp32:
+// fastest way to run it on half tensors: R, the biases, the first state and the gradients that are added
+// to are widened into a staging area at the front of the stream's scratch buffer (one launch).  What a step
+// reads and writes the kernels read and write in half themselves (gru_forward_half_io, gru_backward_half_io), or it is staged
+// as well and what the caller gets back rounded to half (one launch).  Between the steps the state stays in fp32:
 // the results are those of exact half inputs, rounded once, where the reference rounds every
 // step.  The products around the recurrence (x*W; dx, dW, dR) are bound by the matrix units,
 // and those run on the half matrix cores (gemm_half_nt.hip: half operands, the gate gradients
@@ -23,14 +24,16 @@ int gru_forward_impl(hipStream_t stream, int training, int T, int N, int C, int 
                      const float* W, const float* R, const float* bx, const float* br,
                      const float* x, const float* h, float* h_out, float* v, float* tmp_Wx,
                      float zoneout_prob, const float* zoneout_mask, const float* dc_mask,
-                     float dc_scale, bool wx_ready, bool half_product);
+                     float dc_scale, bool wx_ready, bool half_product, bool half_io);
 int gru_backward_impl(hipStream_t stream, int T, int N, int C, int H,
                       const float* W_t, const float* R_t, const float* x_t, const float* h,
                       const float* v, const float* dh_next, float* dx, float* dW, float* dR,
                       float* dbx, float* dbr, float* dh, float* dp, float* dq,
-                      const float* zoneout_mask, bool products, bool half_product);
+                      const float* zoneout_mask, bool products, bool half_product, bool half_io);
 bool gru_forward_resident(int N, int H);
 bool gru_backward_resident(int N, int H);
+bool gru_forward_half_io(int N, int H);
+bool gru_backward_half_io(int N, int H);
 // gemm_half_nt.hip
 bool gemm_half_nt_applies(bool a_float, int M, int N, int K, const void* A, int lda, const void* Bt, int ldb);
 int gemm_half_nt(hipStream_t stream, bool a_float, int M, int N, int K, const void* A, int lda,
@@ -199,6 +202,12 @@ int gru_forward_half(hipStream_t stream, int training, int T, int N, int C, int 
   float* f = nullptr;
   HASTE_HIP_PROPAGATE(staged_workspace(stream, T, N, C, H, bytes, &f));
 
+  // What the recurrence writes and reads per step, in the caller's tensors or staged.
+  const bool io = gru_forward_half_io(N, H);
+  float* h_out = io ? reinterpret_cast<float*>(static_cast<half_t*>(h) + NH) : f + oh + NH;
+  float* v_out = !training ? nullptr : io ? static_cast<float*>(v) : f + ov;
+  const float* mask = zoneout_mask == nullptr ? nullptr : io ? static_cast<const float*>(zoneout_mask) : f + om;
+
   // x*W on the half matrix cores, the recurrence alone in fp32
   if (gru_forward_resident(N, H) && (long long)T * N < (1ll << 31) &&
       gemm_half_nt_applies(false, (int)TN, 3 * H, C, x, C, f + at.Wt_half, C)) {
@@ -207,7 +216,7 @@ int gru_forward_half(hipStream_t stream, int training, int T, int N, int C, int 
     in.add(bx, f + obx, 3 * (size_t)H);
     in.add(br, f + obr, 3 * (size_t)H);
     in.add(h, f + oh, NH);
-    if (zoneout_mask) in.add(zoneout_mask, f + om, TN * H);
+    if (zoneout_mask && !io) in.add(zoneout_mask, f + om, TN * H);
     if (dc_mask) in.add(dc_mask, f + od, (size_t)H * 3 * H);
     HASTE_HIP_PROPAGATE(convert<true>(stream, in));
     HASTE_HIP_PROPAGATE(transpose_to_half(stream, false, C, 3 * H, W, f + at.Wt_half));
@@ -216,10 +225,11 @@ int gru_forward_half(hipStream_t stream, int training, int T, int N, int C, int 
       HASTE_HIP_PROPAGATE(gemm_half_nt(stream, false, (int)TN, 3 * H, C, x, C, f + at.Wt_half, C, f + oWx, 3 * H,
                                        false, 0));
       HASTE_HIP_PROPAGATE(gru_forward_impl(stream, training, T, N, C, H, nullptr, f + oR, f + obx, f + obr, nullptr,
-                                           f + oh, f + oh + NH, training ? f + ov : nullptr, f + oWx, zoneout_prob,
-                                           zoneout_mask ? f + om : nullptr, dc_mask ? f + od : nullptr, dc_scale,
-                                           true, true));
+                                           f + oh, h_out, v_out, f + oWx, zoneout_prob, mask,
+                                           dc_mask ? f + od : nullptr, dc_scale,
+                                           true, true, io));
     }
+    if (io) return HASTE_HIP_OK;
     ConvertList out;
     out.add(f + oh + NH, static_cast<half_t*>(h) + NH, TN * H);
     if (training) out.add(f + ov, v, TN * 4 * H);
@@ -233,16 +243,16 @@ int gru_forward_half(hipStream_t stream, int training, int T, int N, int C, int 
   in.add(br, f + obr, 3 * (size_t)H);
   in.add(x, f + ox, TN * C);
   in.add(h, f + oh, NH);
-  if (zoneout_mask) in.add(zoneout_mask, f + om, TN * H);
+  if (zoneout_mask && !io) in.add(zoneout_mask, f + om, TN * H);
   if (dc_mask) in.add(dc_mask, f + od, (size_t)H * 3 * H);
   HASTE_HIP_PROPAGATE(convert<true>(stream, in));
   {
     ScratchPrefix keep(bytes);
     HASTE_HIP_PROPAGATE(gru_forward_impl(stream, training, T, N, C, H, f + oW, f + oR, f + obx, f + obr,
-                                         f + ox, f + oh, f + oh + NH, training ? f + ov : nullptr, f + oWx,
-                                         zoneout_prob, zoneout_mask ? f + om : nullptr,
-                                         dc_mask ? f + od : nullptr, dc_scale, false, true));
+                                         f + ox, f + oh, h_out, v_out, f + oWx, zoneout_prob, mask,
+                                         dc_mask ? f + od : nullptr, dc_scale, false, true, io));
   }
+  if (io) return HASTE_HIP_OK;
   ConvertList out;
   out.add(f + oh + NH, static_cast<half_t*>(h) + NH, TN * H);
   if (training) out.add(f + ov, v, TN * 4 * H);
@@ -269,17 +279,21 @@ int gru_backward_half(hipStream_t stream, int T, int N, int C, int H, const void
 
   // the recurrence alone in fp32; dx = dp * W_t, dW += x_t * dp, dR += h^T * dq on the half
   // matrix cores, every operand with the contraction index contiguous
+  // (where it runs on the caller's tensors, dp and dq are in half as well)
   const int iTN = (int)TN, iH3 = 3 * H;
+  const bool io = gru_backward_half_io(N, H);
   if (gru_backward_resident(N, H) && (long long)T * N < (1ll << 31) &&
-      gemm_half_nt_applies(true, iTN, C, iH3, f + odp, iH3, f + at.W_half, iH3) &&
+      gemm_half_nt_applies(!io, iTN, C, iH3, f + odp, iH3, f + at.W_half, iH3) &&
       gemm_half_nt_applies(false, C, iH3, iTN, x_t, iTN, f + at.dpT_half, iTN) &&
       gemm_half_nt_applies(false, H, iH3, iTN, f + at.hT_half, iTN, f + at.dqT_half, iTN)) {
     ConvertList in;
     in.add(R_t, f + oRt, H3 * H);
-    in.add(h, f + oh, (T + 1) * NH);
-    in.add(v, f + ov, TN * 4 * H);
-    in.add(dh_next, f + odn, TN * H);
-    if (zoneout_mask) in.add(zoneout_mask, f + om, TN * H);
+    if (!io) {
+      in.add(h, f + oh, (T + 1) * NH);
+      in.add(v, f + ov, TN * 4 * H);
+      in.add(dh_next, f + odn, TN * H);
+      if (zoneout_mask) in.add(zoneout_mask, f + om, TN * H);
+    }
     in.add(dW, f + odW, C * H3);
     in.add(dR, f + odR, H * H3);
     in.add(dbx, f + odbx, H3);
@@ -290,12 +304,13 @@ int gru_backward_half(hipStream_t stream, int T, int N, int C, int H, const void
     HASTE_HIP_PROPAGATE(transpose_to_half(stream, false, iTN, H, h, f + at.hT_half));
     {
       ScratchPrefix keep(bytes);
-      HASTE_HIP_PROPAGATE(gru_backward_impl(stream, T, N, C, H, nullptr, f + oRt, nullptr, f + oh, f + ov, f + odn,
-                                            nullptr, nullptr, nullptr, f + odbx, f + odbr, f + odh, f + odp, f + odq,
-                                            zoneout_mask ? f + om : nullptr, false, true));
-      HASTE_HIP_PROPAGATE(transpose_to_half(stream, true, iTN, iH3, f + odp, f + at.dpT_half));
-      HASTE_HIP_PROPAGATE(transpose_to_half(stream, true, iTN, iH3, f + odq, f + at.dqT_half));
-      HASTE_HIP_PROPAGATE(gemm_half_nt(stream, true, iTN, C, iH3, f + odp, iH3, f + at.W_half, iH3, f + odx, C, false, 0));
+      auto tensor = [&](const void* given, size_t staged) { return io ? static_cast<const float*>(given) : f + staged; };
+      HASTE_HIP_PROPAGATE(gru_backward_impl(stream, T, N, C, H, nullptr, f + oRt, nullptr, tensor(h, oh), tensor(v, ov),
+                                            tensor(dh_next, odn), nullptr, nullptr, nullptr, f + odbx, f + odbr, f + odh,
+                                            f + odp, f + odq, zoneout_mask ? tensor(zoneout_mask, om) : nullptr, false, true, io));
+      HASTE_HIP_PROPAGATE(transpose_to_half(stream, !io, iTN, iH3, f + odp, f + at.dpT_half));
+      HASTE_HIP_PROPAGATE(transpose_to_half(stream, !io, iTN, iH3, f + odq, f + at.dqT_half));
+      HASTE_HIP_PROPAGATE(gemm_half_nt(stream, !io, iTN, C, iH3, f + odp, iH3, f + at.W_half, iH3, f + odx, C, false, 0));
       HASTE_HIP_PROPAGATE(gemm_half_nt(stream, false, C, iH3, iTN, x_t, iTN, f + at.dpT_half, iTN, f + odW, iH3, true, 0));
       HASTE_HIP_PROPAGATE(gemm_half_nt(stream, false, H, iH3, iTN, f + at.hT_half, iTN, f + at.dqT_half, iTN, f + odR,
                                        iH3, true, 0));
@@ -328,7 +343,7 @@ int gru_backward_half(hipStream_t stream, int T, int N, int C, int H, const void
     ScratchPrefix keep(bytes);
     HASTE_HIP_PROPAGATE(gru_backward_impl(stream, T, N, C, H, f + oWt, f + oRt, f + oxt, f + oh, f + ov,
                                           f + odn, f + odx, f + odW, f + odR, f + odbx, f + odbr, f + odh,
-                                          f + odp, f + odq, zoneout_mask ? f + om : nullptr, true, true));
+                                          f + odp, f + odq, zoneout_mask ? f + om : nullptr, true, true, false));
   }
   ConvertList out;
   out.add(f + odx, dx, TN * C);

@@ -15,11 +15,11 @@ int lstm_backward_impl(hipStream_t stream, int T, int N, int C, int H, const flo
 int gru_forward_impl(hipStream_t stream, int training, int T, int N, int C, int H, const float* W, const float* R,
                      const float* bx, const float* br, const float* x, const float* h, float* h_out, float* v,
                      float* tmp_Wx, float zoneout_prob, const float* zoneout_mask, const float* dc_mask, float dc_scale,
-                     bool wx_ready, bool half_product);
+                     bool wx_ready, bool half_product, bool half_io);
 int gru_backward_impl(hipStream_t stream, int T, int N, int C, int H, const float* W_t, const float* R_t,
                       const float* x_t, const float* h, const float* v, const float* dh_next, float* dx, float* dW,
                       float* dR, float* dbx, float* dbr, float* dh, float* dp, float* dq, const float* zoneout_mask,
-                      bool products, bool half_product);
+                      bool products, bool half_product, bool half_io);
 size_t recurrence64_scratch_bytes(int in_gates, int out_gates, int steps, int N, int H);
 int lstm_forward_recurrence64(hipStream_t stream, int training, int T, int N, int H, const double* R, const double* b,
                               const double* h, const double* c, double* h_out, double* c_out, double* v,
@@ -68,9 +68,9 @@ int plan_recurrence(int gates, int element_bytes, bool backward, int T, int N, i
   float* a = reinterpret_cast<float*>(uintptr_t(256));
   if (backward)
     return lstm ? lstm_backward_impl(nullptr, T, N, C, H, a, a, a, a, a, a, a, a, a, a, a, a, a, a, a, nullptr)
-                : gru_backward_impl(nullptr, T, N, C, H, a, a, a, a, a, a, a, a, a, a, a, a, a, a, nullptr, true, false);
+                : gru_backward_impl(nullptr, T, N, C, H, a, a, a, a, a, a, a, a, a, a, a, a, a, a, nullptr, true, false, false);
   return lstm ? lstm_forward_impl(nullptr, 1, T, N, C, H, a, a, a, a, a, a, a, a, a, 0.f, nullptr, nullptr, 1.f)
-              : gru_forward_impl(nullptr, 1, T, N, C, H, a, a, a, a, a, a, a, a, a, 0.f, nullptr, nullptr, 1.f, false, false);
+              : gru_forward_impl(nullptr, 1, T, N, C, H, a, a, a, a, a, a, a, a, a, 0.f, nullptr, nullptr, 1.f, false, false, false);
 }
 
 }  // namespace haste_hip
