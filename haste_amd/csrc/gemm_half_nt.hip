@@ -8,8 +8,8 @@
 // contraction index contiguous -- what the instruction wants of a lane, eight consecutive k
 // of one row -- so a tile goes from global memory to LDS to the operand registers in 16-byte
 // pieces with no transposition anywhere; callers transpose the operand that is not laid out
-// that way once (transpose_to_half).  128 x 128 tile per 256-thread workgroup, each wavefront a
-// 64 x 64 quadrant as 2 x 2 MFMA tiles, 64 k per step through a double-buffered LDS stage.  A
+// that way once (transpose_to_half).  128 x 128 tile per workgroup of four or eight wavefronts, each
+// with a 64 x 64 or 64 x 32 block of it, 64 k per step through a double-buffered LDS stage.  A
 // row of an LDS tile is 8 chunks of 8 halves; chunk c of row r sits at position c ^ ((r >> 1) & 7),
 // which makes the 16 rows x one chunk that a quarter of a wavefront reads (and the 8 rows x 8
 // chunks it writes) cover all 64 banks.  Lane layout of the instruction: a = A[i = lane%32]
@@ -50,18 +50,24 @@ __device__ __forceinline__ uint4_t pack8(float4_t lo, float4_t hi) {
   return __builtin_bit_cast(uint4_t, h);
 }
 
-// One 128 x 128 tile over k in [k_begin, k_end); K % 8 == 0, rows 16-byte aligned.
-template <bool A_FLOAT>
-__global__ __launch_bounds__(256, 2)
+// One 128 x 128 tile over k in [k_begin, k_end); K % 8 == 0, rows 16-byte aligned.  WAVES = 4: 64 x 64 of it a
+// wavefront, the fewest reads of LDS; 8: 64 x 32, so that a SIMD has two wavefronts where a CU has one workgroup.
+template <bool A_FLOAT, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, 2)
 void gemm_half_nt_kernel(int M, int N, int K, const void* __restrict__ A, int lda,
                          const half_t* __restrict__ Bt, int ldb, float* __restrict__ C, int ldc,
                          int accumulate, int tiles_n, int tiles, int k_per_piece,
                          float* __restrict__ partial) {
   __shared__ __attribute__((aligned(16))) uint4_t lds[2][2][kTileChunks];  // [buffer][A, B][chunk]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int piece = blockIdx.x / tiles, tile = blockIdx.x % tiles;
+  // Workgroups go to the XCDs in turn.  Short pieces: each XCD is given a range of the work, tiles that share rows
+  // of A.  Long ones: as they come, which gives an XCD tiles of many rows and few columns (4096^3 188 -> 172 us).
+  const int xcd = blockIdx.x & 7, each = gridDim.x >> 3, rest = gridDim.x & 7;
+  const int work = WAVES == 8 ? xcd * each + (xcd < rest ? xcd : rest) + (blockIdx.x >> 3) : blockIdx.x;
+  const int piece = work / tiles, tile = work % tiles;
   const int m0 = (tile / tiles_n) * QM, n0 = (tile % tiles_n) * QN;
-  const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
+  constexpr int WCOLS = WAVES / 2, NJ = 4 / WCOLS;  // wavefronts side by side, 32-column blocks of one
+  const int wm = (wave / WCOLS) * 64, wn = (wave % WCOLS) * 32 * NJ;
   const int k_begin = piece * k_per_piece;
   const int k_end = k_begin + k_per_piece < K ? k_begin + k_per_piece : K;
 
@@ -71,13 +77,13 @@ void gemm_half_nt_kernel(int M, int N, int K, const void* __restrict__ A, int ld
       panel(static_cast<const char*>(A) + (size_t)m0 * lda * ASZ, ((long long)(rows_a - 1) * lda + K) * ASZ);
   const __amdgpu_buffer_rsrc_t pb = panel(Bt + (size_t)n0 * ldb, ((long long)(rows_b - 1) * ldb + K) * 2);
 
-  // A thread's four chunks of each tile: chunk c = tid % 8 of rows tid / 8 + 32 * i.  Two
+  // A thread's chunks of each tile: chunk c = tid % 8 of rows tid / 8 + 8 WAVES i.  Two
   // steps of operands are kept in flight in two register sets (a step's 512 cycles of MFMAs
   // are a fraction of a load's latency).  An fp32 A stays as loaded until it is parked:
   // converted at the request it would make the request wait for its own loads.
   const int c = tid & 7, r = tid >> 3;
-  constexpr int AR = A_FLOAT ? 8 : 4;
-  uint4_t ra[2][AR], rb[2][4];
+  constexpr int CH = 16 / WAVES, ROWS = 8 * WAVES, AR = A_FLOAT ? 2 * CH : CH;
+  uint4_t ra[2][AR], rb[2][CH];
   // A thread's offsets into the panels are fixed; the step enters as the loads' scalar offset
   // (which the range check ignores: chunks beyond the end of K, in the last step of a ragged K
   // only, get an offset beyond the panel instead).  The offsets pass through an empty asm
@@ -85,18 +91,18 @@ void gemm_half_nt_kernel(int M, int N, int K, const void* __restrict__ A, int ld
   // and a wait for all loads before it (8192^3: 565 -> 814 TFLOP/s without them).  Loads issued
   // straight from the fixed offsets, with nothing between them, are slower again (783): more
   // loads in flight are not what the step lacks.
-  unsigned int va[4], vb[4];
+  unsigned int va[CH], vb[CH];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    va[i] = (unsigned int)(((size_t)(r + 32 * i) * lda + 8 * c) * ASZ);
-    vb[i] = (unsigned int)(((size_t)(r + 32 * i) * ldb + 8 * c) * 2);
+  for (int i = 0; i < CH; ++i) {
+    va[i] = (unsigned int)(((size_t)(r + ROWS * i) * lda + 8 * c) * ASZ);
+    vb[i] = (unsigned int)(((size_t)(r + ROWS * i) * ldb + 8 * c) * 2);
   }
   auto request = [&](auto set_c, int k0) {
     constexpr int SET = decltype(set_c)::value;
     const int sa = k0 * ASZ, sb = k0 * 2;
     const bool gone = k0 + 8 * c >= k_end;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < CH; ++i) {
       unsigned int oa = gone ? kNowhere : va[i], ob = gone ? kNowhere : vb[i];
       asm volatile("" : "+v"(oa), "+v"(ob));
       if constexpr (A_FLOAT) {
@@ -111,21 +117,21 @@ void gemm_half_nt_kernel(int M, int N, int K, const void* __restrict__ A, int ld
   auto park = [&](auto set_c) {
     constexpr int SET = decltype(set_c)::value;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < CH; ++i) {
       if constexpr (A_FLOAT)
-        lds[SET][0][lds_chunk(r + 32 * i, c)] = pack8(__builtin_bit_cast(float4_t, ra[SET][2 * i]),
+        lds[SET][0][lds_chunk(r + ROWS * i, c)] = pack8(__builtin_bit_cast(float4_t, ra[SET][2 * i]),
                                                       __builtin_bit_cast(float4_t, ra[SET][2 * i + 1]));
       else
-        lds[SET][0][lds_chunk(r + 32 * i, c)] = ra[SET][i];
-      lds[SET][1][lds_chunk(r + 32 * i, c)] = rb[SET][i];
+        lds[SET][0][lds_chunk(r + ROWS * i, c)] = ra[SET][i];
+      lds[SET][1][lds_chunk(r + ROWS * i, c)] = rb[SET][i];
     }
   };
 
-  float16_t acc[2][2];
+  float16_t acc[2][NJ];
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < NJ; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
 
@@ -133,16 +139,15 @@ void gemm_half_nt_kernel(int M, int N, int K, const void* __restrict__ A, int ld
 #pragma unroll
     for (int ks = 0; ks < QK / 16; ++ks) {
       const int cc = 2 * ks + (lane >> 5), o = lane & 31;
-      half8_t a[2], b[2];
+      half8_t a[2], b[NJ];
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        a[i] = __builtin_bit_cast(half8_t, lds[buf][0][lds_chunk(wm + 32 * i + o, cc)]);
-        b[i] = __builtin_bit_cast(half8_t, lds[buf][1][lds_chunk(wn + 32 * i + o, cc)]);
-      }
+      for (int i = 0; i < 2; ++i) a[i] = __builtin_bit_cast(half8_t, lds[buf][0][lds_chunk(wm + 32 * i + o, cc)]);
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) b[j] = __builtin_bit_cast(half8_t, lds[buf][1][lds_chunk(wn + 32 * j + o, cc)]);
 #pragma unroll
       for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < NJ; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i], b[j], acc[i][j], 0, 0, 0);
     }
   };
@@ -178,7 +183,7 @@ void gemm_half_nt_kernel(int M, int N, int K, const void* __restrict__ A, int ld
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < NJ; ++j) {
       const int col = n0 + wn + 32 * j + (lane & 31);
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
@@ -311,12 +316,18 @@ int gemm_half_nt(hipStream_t stream, bool a_float, int M, int N, int K, const vo
   const dim3 grid((unsigned)(tiles * pieces));
   const half_t* b = static_cast<const half_t*>(Bt);
   ScopedKernelTimer timer("gemm_half_nt", stream);
-  if (a_float)
-    gemm_half_nt_kernel<true><<<grid, dim3(256), 0, stream>>>(M, N, K, A, lda, b, ldb, C, ldc, accumulate ? 1 : 0,
-                                                              tiles_n, tiles, per, part);
-  else
-    gemm_half_nt_kernel<false><<<grid, dim3(256), 0, stream>>>(M, N, K, A, lda, b, ldb, C, ldc, accumulate ? 1 : 0,
-                                                               tiles_n, tiles, per, part);
+  // A short piece is bound by the latency of its steps, which two wavefronts a SIMD share; a long one by reads of LDS
+  // (us with 4 / 8 wavefronts: 6400 x 1536 x 512 26.4 / 23.6, 6400 x 512 x 1536 26.2 / 23.3, 512 x 1536 x 6400 in pieces
+  // of 1600 31.4 / 28.2, 12800 x 1536 x 512 43.6 / 35.5; 1024 x 3072 x 3200 43.5 / 44.8, 4096^3 172 / 186).
+  const bool eight = per <= 2048;
+#define HASTE_LAUNCH_NT(A_FLOAT_, WAVES_)                                                                       \
+  gemm_half_nt_kernel<A_FLOAT_, WAVES_><<<grid, dim3(64 * WAVES_), 0, stream>>>(                                \
+      M, N, K, A, lda, b, ldb, C, ldc, accumulate ? 1 : 0, tiles_n, tiles, per, part)
+  if (a_float && eight) HASTE_LAUNCH_NT(true, 8);
+  else if (a_float) HASTE_LAUNCH_NT(true, 4);
+  else if (eight) HASTE_LAUNCH_NT(false, 8);
+  else HASTE_LAUNCH_NT(false, 4);
+#undef HASTE_LAUNCH_NT
   HASTE_HIP_TRY(hipGetLastError());
   if (pieces > 1) {
     const size_t n = (size_t)M * N;

@@ -23,8 +23,8 @@ struct GruFwdParams {
   const float* dc_mask;  // DropConnect mask [H,3H] or null
   float dc_scale;
   float* xh;             // polled exchange tiles of h: [batch tiles][4][Kpad/4][NB][4]
-  int half_io;           // (kernels with a product on the half matrix cores) h_out, v and zoneout_mask are in half
   LaunchShape ls;
+  int half_io;           // (kernels with a product on the half matrix cores) h_out, v and zoneout_mask are in half
 };
 
 struct GruBwdParams {
