@@ -46,7 +46,7 @@ constexpr int kMaxWorkgroups = 2048;  // workgroups a persistent kernel may have
 constexpr int kCounterStride = 32;    // uint32 slots between counters (128 B apart)
 struct ControlBlock {
   unsigned int step_flags[kMaxWorkgroups];                 // per-workgroup arrival counts
-  unsigned int grid_exit_counter[kCounterStride];          // unused (kept for the layout)
+  unsigned int grid_exit_counter[kCounterStride];          // finished tiles of a single step in place
   unsigned int tile_counter[4096];                         // arrivals per column block at the end of a launch
   unsigned int xcd_ticket[16 * kCounterStride];            // per-XCD role tickets (only ever grow)
   unsigned int abort_flag[kCounterStride];                 // set when a barrier wait gives up
@@ -265,6 +265,7 @@ int gru_backward_streamed(hipStream_t stream, int T, int N, int C, int H,
                           const float* v, const float* dh_next, float* dx, float* dW, float* dR,
                           float* dbx, float* dbr, float* dh, float* dp, float* dq,
                           const float* zoneout_mask);
+size_t layer_norm_streamed_bytes(int gates, bool backward, int T, int N, int C, int H);
 int layer_norm_lstm_forward_streamed(hipStream_t stream, int training, int T, int N, int C, int H,
                                      const float* W, const float* R, const float* b, const float* x,
                                      float* h, float* c, float* act_Wx, const float* gamma1,

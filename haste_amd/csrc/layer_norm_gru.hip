@@ -669,7 +669,7 @@ int haste_hip_layer_norm_gru_forward_f32(int training, int steps, int batch_size
   // N = 24 25.7 / 23.8; but H = 1536, N = 32 19.5 / 20.9).
   bool streamed = !tile.ok;
   if (tile.ok && tile.reg_groups > 0 && ((tile.nb >= 64 && H > 1240) || (tile.nb >= 32 && H > 1700)))
-    HASTE_HIP_PROPAGATE(workspace_has_room(stream, workspace_scratch_bound(T, N, C, H), &streamed));
+    HASTE_HIP_PROPAGATE(workspace_has_room(stream, layer_norm_streamed_bytes(3, false, T, N, C, H), &streamed));
   if (streamed)
     return layer_norm_gru_forward_streamed(stream, training, T, N, C, H, W, R, bx, br, x, h, v, act_Wx,
                                            gamma1, cache1, tmp_Wx_norm, act_Rh, gamma2, cache2,
@@ -744,7 +744,7 @@ int haste_hip_layer_norm_gru_backward_f32(int steps, int batch_size, int input_s
   // N = 48 33.9 / 31.8, H = 1280 N = 128 59 / 44; but H = 1024, N = 16 14.0 / 15.2 and N = 128 27 / 37).
   bool streamed = !tile.ok;
   if (tile.ok && tile.reg_groups > 0 && ((N <= 8 && H > 880) || (N > 32 && H > 1240)))
-    HASTE_HIP_PROPAGATE(workspace_has_room(stream, workspace_scratch_bound(T, N, C, H), &streamed));
+    HASTE_HIP_PROPAGATE(workspace_has_room(stream, layer_norm_streamed_bytes(3, true, T, N, C, H), &streamed));
   if (streamed)
     return layer_norm_gru_backward_streamed(stream, T, N, C, H, W_t, R_t, x_t, h, v, dh_new, dx, dW, dR,
                                             dbx, dbr, dh, dp, dq, act_Wx, gamma1, dgamma1, act_Rh,

@@ -854,7 +854,7 @@ int haste_hip_layer_norm_lstm_forward_f32(int training, int steps, int batch_siz
   // N = 40 34 / 24, H = 1792 N = 8 26.9 / 23.8 and N = 48 65 / 31; but H = 1056, N = 12 15.3 / 16.2.)
   bool streamed = !tile.ok;
   if (tile.ok && tile.reg_groups > 0 && (H > 1600 || (tile.nb >= 32 && H > 1024)))
-    HASTE_HIP_PROPAGATE(workspace_has_room(stream, workspace_scratch_bound(T, N, C, H), &streamed));
+    HASTE_HIP_PROPAGATE(workspace_has_room(stream, layer_norm_streamed_bytes(4, false, T, N, C, H), &streamed));
   if (streamed)
     return layer_norm_lstm_forward_streamed(stream, training, T, N, C, H, W, R, b, x, h, c, act_Wx,
                                             gamma1, cache1, act_Wx_norm, act_Rh, gamma2, cache2,
@@ -953,7 +953,7 @@ int haste_hip_layer_norm_lstm_backward_f32(int steps, int batch_size, int input_
   // 19.3 / 18.4, N = 32 21.1 / 23.5; H = 1056, N = 12 22.8 / 20.7; H = 896, N = 8 15.2 / 17.0).
   bool streamed = !tile.ok;
   if (tile.ok && tile.reg_groups > 0 && N <= 16 && H > 960)
-    HASTE_HIP_PROPAGATE(workspace_has_room(stream, workspace_scratch_bound(T, N, C, H), &streamed));
+    HASTE_HIP_PROPAGATE(workspace_has_room(stream, layer_norm_streamed_bytes(4, true, T, N, C, H), &streamed));
   if (streamed)
     return layer_norm_lstm_backward_streamed(stream, T, N, C, H, W_t, R_t, x_t, h, c, dh_new, dc_new,
                                              dx, dW, dR, db, dh, dc, act_Wx, gamma1, dgamma1,

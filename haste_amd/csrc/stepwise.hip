@@ -1,6 +1,7 @@
 // Every cell in step-wise form, for `float` and `double`: the recurrent product of each step
-// is a GEMM that streams R from HBM, followed by row-wise layer-norm kernels (layer-norm
-// cells) and one or two pointwise kernels -- the structure of the reference
+// is a GEMM that streams R from HBM, followed by one or two pointwise kernels, or for the
+// layer-norm cells one kernel with a workgroup per row (rows beyond 4096 units: row-wise norms and
+// pointwise kernels) -- the structure of the reference
 // (lib/lstm_forward_gpu.cu.cc:210-310, lib/lstm_backward_gpu.cu.cc:246-317,
 // lib/gru_forward_gpu.cu.cc:214-312, lib/gru_backward_gpu.cu.cc:252-319,
 // lib/layer_norm_lstm_forward_gpu.cu.cc:276-340, lib/layer_norm_lstm_backward_gpu.cu.cc:255-352,
@@ -1387,6 +1388,25 @@ int gru_backward_steps(hipStream_t stream, int steps, int N, int C, int H, const
   return HASTE_HIP_OK;
 }
 
+// Scratch of a layer-norm cell's pass: buffers of its own, and the products'.
+template <typename T>
+size_t ln_own_bytes(int gates, bool backward, int steps, int N, int H) {
+  if (!backward) return padded((size_t)N * gates * H * sizeof(T));
+  const size_t TN = (size_t)steps * N;
+  return column_sum_bytes<T>(TN, (size_t)N, gates * H) + padded(TN * 2 * sizeof(T));
+}
+template <typename T>
+Room ln_product_room(int gates, bool backward, int steps, int N, int C, int H) {
+  const int TN = steps * N, GH = gates * H;
+  if (!backward) return max2(gemm_room<T>(TN, GH, C), gemm_room<T>(N, GH, H));
+  return max2(max2(gemm_room<T>(N, H, GH), gemm_room<T>(C, GH, TN)), max2(gemm_room<T>(H, GH, TN), gemm_room<T>(TN, C, GH)));
+}
+// What the reverse pass of the LSTM keeps beside them when a row is held by a workgroup: each row's share of dgamma2.
+template <typename T>
+size_t ln_lstm_sums_bytes(int N, int H) {
+  return rows_held(H) ? padded((size_t)N * 4 * H * sizeof(T)) : 0;
+}
+
 template <typename T>
 int ln_lstm_forward_steps(hipStream_t stream, int training, int steps, int N, int C, int H,
                           const T* W, const T* R, const T* b, const T* x, T* h, T* c, T* act_Wx,
@@ -1396,7 +1416,8 @@ int ln_lstm_forward_steps(hipStream_t stream, int training, int steps, int N, in
   const size_t NH = (size_t)N * H, N4H = NH * 4;
   const int TN = steps * N;
   Scratch sc;
-  HASTE_HIP_PROPAGATE(open_scratch(stream, padded(N4H * sizeof(T)), max2(gemm_room<T>(TN, 4 * H, C), gemm_room<T>(N, 4 * H, H)), &sc));
+  HASTE_HIP_PROPAGATE(open_scratch(stream, ln_own_bytes<T>(4, false, steps, N, H),
+                                   ln_product_room<T>(4, false, steps, N, C, H), &sc));
   T* rhn = sc.take<T>(N4H);
   HASTE_HIP_PROPAGATE(gemm(stream, false, TN, 4 * H, C, x, C, W, 4 * H, act_Wx, 4 * H, false, sc.gemm_offset()));
   HASTE_HIP_PROPAGATE(ln_forward_rows<T>(stream, (size_t)TN, 4 * H, gamma1, nullptr, act_Wx, act_Wx_norm, cache1));
@@ -1446,11 +1467,10 @@ int ln_lstm_backward_steps(hipStream_t stream, int steps, int N, int C, int H, c
   const size_t NH = (size_t)N * H, N4H = NH * 4;
   const int TN = steps * N;
   const size_t part_bytes = column_sum_bytes<T>((size_t)TN, (size_t)N, 4 * H);
-  size_t own = part_bytes + padded((size_t)TN * 2 * sizeof(T));
-  Room room = max2(gemm_room<T>(N, H, 4 * H), gemm_room<T>(C, 4 * H, TN));
-  room = max2(room, max2(gemm_room<T>(H, 4 * H, TN), gemm_room<T>(TN, C, 4 * H)));
+  size_t own = ln_own_bytes<T>(4, true, steps, N, H);
+  const Room room = ln_product_room<T>(4, true, steps, N, C, H);
   // Rows held by a workgroup each, where there is room for their sums of dgamma2.
-  const size_t sums_bytes = padded(N4H * sizeof(T));
+  const size_t sums_bytes = ln_lstm_sums_bytes<T>(N, H);
   bool held = rows_held(H);
   if (held) HASTE_HIP_PROPAGATE(workspace_has_room(stream, own + sums_bytes + room.need + 256, &held));
   if (held) own += sums_bytes;
@@ -1521,7 +1541,8 @@ int ln_gru_forward_steps(hipStream_t stream, int training, int steps, int N, int
   const size_t NH = (size_t)N * H, N3H = NH * 3, N4H = NH * 4;
   const int TN = steps * N;
   Scratch sc;
-  HASTE_HIP_PROPAGATE(open_scratch(stream, padded(N3H * sizeof(T)), max2(gemm_room<T>(TN, 3 * H, C), gemm_room<T>(N, 3 * H, H)), &sc));
+  HASTE_HIP_PROPAGATE(open_scratch(stream, ln_own_bytes<T>(3, false, steps, N, H),
+                                   ln_product_room<T>(3, false, steps, N, C, H), &sc));
   T* rhn = sc.take<T>(N3H);
   HASTE_HIP_PROPAGATE(gemm(stream, false, TN, 3 * H, C, x, C, W, 3 * H, act_Wx, 3 * H, false, sc.gemm_offset()));
   HASTE_HIP_PROPAGATE(ln_forward_rows<T>(stream, (size_t)TN, 3 * H, gamma1, nullptr, act_Wx, tmp_Wx_norm, cache1));
@@ -1565,11 +1586,9 @@ int ln_gru_backward_steps(hipStream_t stream, int steps, int N, int C, int H, co
   const size_t NH = (size_t)N * H, N3H = NH * 3, N4H = NH * 4;
   const int TN = steps * N;
   const size_t part_bytes = column_sum_bytes<T>((size_t)TN, (size_t)N, 3 * H);
-  const size_t own = part_bytes + padded((size_t)TN * 2 * sizeof(T));
-  Room room = max2(gemm_room<T>(N, H, 3 * H), gemm_room<T>(C, 3 * H, TN));
-  room = max2(room, max2(gemm_room<T>(H, 3 * H, TN), gemm_room<T>(TN, C, 3 * H)));
   Scratch sc;
-  HASTE_HIP_PROPAGATE(open_scratch(stream, own, room, &sc));
+  HASTE_HIP_PROPAGATE(open_scratch(stream, ln_own_bytes<T>(3, true, steps, N, H),
+                                   ln_product_room<T>(3, true, steps, N, C, H), &sc));
   void* partial = sc.take<char>(part_bytes);
   T* stats1 = sc.take<T>((size_t)TN * 2);
   {
@@ -1721,6 +1740,12 @@ int layer_norm_backward_wide(hipStream_t stream, int rows, int dim, const float*
   float* stats = sc.take<float>((size_t)rows * 2);
   HASTE_HIP_PROPAGATE(ln_forward_rows<float>(stream, (size_t)rows, dim, gamma, nullptr, x, nullptr, stats));
   return ln_backward_rows<float>(stream, (size_t)rows, dim, gamma, x, dy, dx, dgamma, dbeta, stats, partial);
+}
+
+// Bytes of scratch that a layer-norm cell's pass asks for when it streams R, in float.
+size_t layer_norm_streamed_bytes(int gates, bool backward, int T, int N, int C, int H) {
+  return ln_own_bytes<float>(gates, backward, T, N, H) + (gates == 4 && backward ? ln_lstm_sums_bytes<float>(N, H) : 0) +
+         ln_product_room<float>(gates, backward, T, N, C, H).wish + 256;
 }
 
 int layer_norm_lstm_forward_streamed(hipStream_t stream, int training, int T, int N, int C, int H,

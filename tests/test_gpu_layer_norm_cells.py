@@ -140,3 +140,53 @@ def test_layer_norm_lstm_backward_with_badly_scaled_sums(T, N, C, H):
     names = ("dx", "dh0", "dc0", "dW", "dR", "db", "dgamma", "dgamma_h", "dbeta_h")
     for name, ours in zip(names, grads):
         assert relerr(host(ours), g[name]) < TOL, name
+
+
+@pytest.mark.parametrize("cell,T,N,C,H", [("lstm", 3, 5, 8, 1700), ("gru", 3, 50, 8, 1300)])
+def test_streamed_wide_slices_under_capture_and_in_little_memory(cell, T, N, C, H):
+    """Slices that would stay on chip with a part in registers and stream R because that is faster: replays of a graph give the
+    eager bits, and whatever lent memory is not refused gives the same results (the smallest keeps the slice on chip)."""
+    from haste_amd import lib, ops
+    import torch
+    p = problem(17, T, N, C, H, 4 if cell == "lstm" else 3, 0.0)
+
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        x, W, R = dev(p["x"]), dev(p["W"]), dev(p["R"])
+        rest = [dev(p[k]) for k in (("h0", "c0") if cell == "lstm" else ("h0",))]
+        weights = [dev(p[k]) for k in (("b", "gamma", "gamma_h", "beta_h") if cell == "lstm" else ("b", "b2", "gamma"))]
+        forward = ops.layer_norm_lstm_forward if cell == "lstm" else ops.layer_norm_gru_forward
+        none = dev(None)
+
+        def step():
+            return forward(True, 0.0, x, *rest, W, R, *weights, none)[0]
+
+        eager = step().clone()
+        s.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=s):
+            out = step()
+        for _ in range(3):
+            out.fill_(float("nan"))
+            graph.replay()
+            s.synchronize()
+            assert torch.equal(out, eager)
+        del graph
+        taken = 0
+        try:
+            for kib in (256, 512, 1024, 2048, 4096, 8192, 16384, 32768):
+                lent = torch.empty(kib << 10, dtype=torch.uint8, device="cuda")
+                ops.set_workspace(lent)
+                try:
+                    h = step()
+                except lib.HasteHipError as e:
+                    assert e.code == 2 and taken == 0, (kib, e.code)
+                    continue
+                s.synchronize()
+                ops.stream_status()
+                taken += 1
+                assert relerr(host(h), host(eager)) < TOL, kib
+        finally:
+            s.synchronize()
+            ops.set_workspace(None)
+        assert taken >= 2
