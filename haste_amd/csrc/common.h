@@ -325,7 +325,7 @@ constexpr long long kStepStreamed = 60 << 10, kStepResident = 128 << 10, kStepHa
 // staged_bytes: staged_state_bytes() of the call, scratch for a state that is updated in place.
 int single_step_rule(hipStream_t stream, int N, int C, int H, size_t element, long long most_blocks, size_t staged_bytes,
                      bool* applies);
-size_t staged_state_bytes(int N, int H, const void* h, const void* h_out, size_t element);
+size_t staged_state_bytes(int N, int C, int H, const void* x, const void* h, const void* h_out, size_t element);
 int lstm_forward_single_step(hipStream_t stream, int training, int N, int C, int H, const float* W,
                              const float* R, const float* b, const float* x, const float* h,
                              const float* c, float* h_out, float* c_out, float* v,

@@ -712,7 +712,7 @@ int lstm_forward_impl(hipStream_t stream, int training, int T, int N, int C, int
   // A single step (Iterate): one kernel, nothing kept on chip.
   if (T == 1) {
     bool single = false;
-    const size_t staged = staged_state_bytes(N, H, h, h_out, sizeof(float));
+    const size_t staged = staged_state_bytes(N, C, H, x, h, h_out, sizeof(float));
     HASTE_HIP_PROPAGATE(single_step_rule(stream, N, C, H, sizeof(float), kStepStreamed, staged, &single));
     if (!single && pick_forward_tile(4, N, H, 0, kWorkgroupLdsBytes, false, 2).ok)
       HASTE_HIP_PROPAGATE(single_step_rule(stream, N, C, H, sizeof(float), kStepResident, staged, &single));

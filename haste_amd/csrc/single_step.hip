@@ -70,7 +70,7 @@ struct StepParams {
   const T* zoneout_mask;      // [N, H] or null
   const T* dc_mask;           // DropConnect mask of R or null
   float dc_scale;
-  typename Step<T>::Sum* h_stage;  // [N, H] when h_out overlaps h (state updated in place), else null
+  typename Step<T>::Sum* h_stage;  // [N, H] when h_out overlaps h (state updated in place) or x, else null
   typename Step<T>::Sum* partial;  // [runs][output tiles][4 sums][quads of rows][64]; unused with one run
   ControlBlock* cb;
   int runs, row_blocks, unit_blocks, quads;  // quads: of rows, in an output tile
@@ -166,8 +166,8 @@ __device__ __forceinline__ void finish_unit(const StepParams<T>& p, int n, int j
   else store_sum(&p.h_stage[e], h_new);
 }
 
-// h_out overlaps h: other workgroups may still be reading h when a column block is finished,
-// so the new state is parked and copied out by the last column block to finish, when every
+// h_out overlaps h or x: other workgroups may still be reading them when a column block is
+// finished, so the new state is parked and copied out by the last column block to finish, when every
 // run of every block has been read.  Called by the finishing workgroups, all threads.
 template <typename T>
 __device__ __forceinline__ void copy_staged_state(const StepParams<T>& p, unsigned int* flag) {
@@ -427,7 +427,7 @@ template <int GATES, typename T>
 int launch_step(hipStream_t stream, StepParams<T>& p, const char* name) {
   typedef typename Step<T>::Sum A;
   StepCut cut = step_cut(p.N, p.C, p.H, sizeof(T));
-  const size_t state_bytes = staged_state_bytes(p.N, p.H, p.h, p.h_out, sizeof(T));
+  const size_t state_bytes = staged_state_bytes(p.N, p.C, p.H, p.x, p.h, p.h_out, sizeof(T));
   for (bool room = false; !room && cut.runs > 1;) {
     HASTE_HIP_PROPAGATE(workspace_has_room(stream, cut.sums() * sizeof(A) + state_bytes + 256, &room));
     if (!room) cut.runs = (cut.runs + 1) / 2;
@@ -480,10 +480,14 @@ int single_step_rule(hipStream_t stream, int N, int C, int H, size_t element, lo
   return workspace_has_room(stream, cut.sums() * (element == 8 ? 8 : 4) + staged_bytes + 256, applies);
 }
 
-size_t staged_state_bytes(int N, int H, const void* h, const void* h_out, size_t element) {
-  const uintptr_t from = reinterpret_cast<uintptr_t>(h), to = reinterpret_cast<uintptr_t>(h_out);
+size_t staged_state_bytes(int N, int C, int H, const void* x, const void* h, const void* h_out, size_t element) {
+  const uintptr_t to = reinterpret_cast<uintptr_t>(h_out);
   const size_t floats = (size_t)N * H;
-  return to < from + floats * element && from < to + floats * element ? floats * (element == 8 ? 8 : 4) : 0;
+  auto overlaps = [&](const void* in, size_t count) {
+    const uintptr_t from = reinterpret_cast<uintptr_t>(in);
+    return to < from + count * element && from < to + floats * element;
+  };
+  return overlaps(h, floats) || overlaps(x, (size_t)N * C) ? floats * (element == 8 ? 8 : 4) : 0;
 }
 
 int lstm_forward_single_step(hipStream_t stream, int training, int N, int C, int H, const float* W,

@@ -142,6 +142,27 @@ def test_single_step_kernel_of_larger_batches(N, C, H, training, zoneout):
     test_single_step_kernel(N, C, H, training, zoneout)
 
 
+@pytest.mark.parametrize("N,H", [(3, 512), (40, 512), (128, 300)])
+def test_single_step_whose_output_replaces_its_input(N, H):
+    """The new state in the memory of x (a layer fed with its own output): the bits of a call with memory of its own."""
+    from haste_amd import ops
+    import torch
+    p = problem(41 + N, 1, N, H, H, 4)
+    x, h0, c0 = dev(p["x"][0]), dev(p["h0"]), dev(p["c0"])
+    W, R, b, b2 = dev(p["W"]), dev(p["R"]), dev(p["b"]), dev(p["b2"])
+    W3, R3, bx, br = (t[..., :3 * H].contiguous() for t in (W, R, b, b2))
+    for state in (h0, x):  # also: x and the state are the same memory
+        want, _, _ = ops.lstm_forward_iterate(False, 0.0, x, state, c0, W, R, b)
+        want3, _ = ops.gru_forward_iterate(False, 0.0, x, state, W3, R3, bx, br)
+        for _ in range(3):
+            xi = x.clone()
+            got, _, _ = ops.lstm_forward_iterate(False, 0.0, xi, xi if state is x else state, c0, W, R, b, h_out=xi)
+            xg = x.clone()
+            got3, _ = ops.gru_forward_iterate(False, 0.0, xg, xg if state is x else state, W3, R3, bx, br, h_out=xg)
+            torch.cuda.synchronize()
+            assert torch.equal(got, want) and torch.equal(got3, want3)
+
+
 @pytest.mark.parametrize("N,C,H", [(4, 48, 200), (8, 512, 512), (33, 48, 200), (70, 100, 1030)])
 def test_single_step_dropconnect_equals_premasked_weights(N, C, H):
     from haste_amd import ops
