@@ -322,10 +322,12 @@ size_t cut_scratch_bound(int N, int H, int cus);
 // contraction indices) that depends on what the step would run on otherwise.
 constexpr long long kStepStreamed = 60 << 10, kStepResident = 128 << 10, kStepHalf = 1ll << 40,
                     kStepDouble = 16 << 10;
-// staged_bytes: staged_state_bytes() of the call, scratch for a state that is updated in place.
-int single_step_rule(hipStream_t stream, int N, int C, int H, size_t element, long long most_blocks, size_t staged_bytes,
-                     bool* applies);
-size_t staged_state_bytes(int N, int C, int H, const void* x, const void* h, const void* h_out, size_t element);
+struct StepTensors {
+  const void *x, *h, *c, *mask;   // what it reads (GRU: no c; no mask: null)
+  const void *h_out, *c_out, *v;  // what it writes (GRU: no c_out; v: in training)
+};
+int single_step_rule(hipStream_t stream, int N, int C, int H, size_t element, long long most_blocks,
+                     const StepTensors& tensors, bool* applies);
 int lstm_forward_single_step(hipStream_t stream, int training, int N, int C, int H, const float* W,
                              const float* R, const float* b, const float* x, const float* h,
                              const float* c, float* h_out, float* c_out, float* v,

@@ -745,10 +745,10 @@ int gru_forward_impl(hipStream_t stream, int training, int T, int N, int C, int 
   // scratch of the other paths and is left alone).
   if (T == 1) {
     bool single = false;
-    const size_t staged = staged_state_bytes(N, C, H, x, h, h_out, sizeof(float));
-    HASTE_HIP_PROPAGATE(single_step_rule(stream, N, C, H, sizeof(float), kStepStreamed, staged, &single));
+    const StepTensors tensors = {x, h, nullptr, zoneout_mask, h_out, nullptr, training ? v : nullptr};
+    HASTE_HIP_PROPAGATE(single_step_rule(stream, N, C, H, sizeof(float), kStepStreamed, tensors, &single));
     if (!single && pick_forward_tile(3, N, H, 0, kWorkgroupLdsBytes, false, 3).ok)
-      HASTE_HIP_PROPAGATE(single_step_rule(stream, N, C, H, sizeof(float), kStepResident, staged, &single));
+      HASTE_HIP_PROPAGATE(single_step_rule(stream, N, C, H, sizeof(float), kStepResident, tensors, &single));
     if (single)
       return gru_forward_single_step(stream, training, N, C, H, W, R, bx, br, x, h, h_out, v,
                                      zoneout_prob, zoneout_mask, dc_mask, dc_scale);

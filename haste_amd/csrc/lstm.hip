@@ -712,10 +712,10 @@ int lstm_forward_impl(hipStream_t stream, int training, int T, int N, int C, int
   // A single step (Iterate): one kernel, nothing kept on chip.
   if (T == 1) {
     bool single = false;
-    const size_t staged = staged_state_bytes(N, C, H, x, h, h_out, sizeof(float));
-    HASTE_HIP_PROPAGATE(single_step_rule(stream, N, C, H, sizeof(float), kStepStreamed, staged, &single));
+    const StepTensors tensors = {x, h, c, zoneout_mask, h_out, c_out, training ? v : nullptr};
+    HASTE_HIP_PROPAGATE(single_step_rule(stream, N, C, H, sizeof(float), kStepStreamed, tensors, &single));
     if (!single && pick_forward_tile(4, N, H, 0, kWorkgroupLdsBytes, false, 2).ok)
-      HASTE_HIP_PROPAGATE(single_step_rule(stream, N, C, H, sizeof(float), kStepResident, staged, &single));
+      HASTE_HIP_PROPAGATE(single_step_rule(stream, N, C, H, sizeof(float), kStepResident, tensors, &single));
     if (single)
       return lstm_forward_single_step(stream, training, N, C, H, W, R, b, x, h, c, h_out, c_out, v,
                                       zoneout_prob, zoneout_mask, dc_mask, dc_scale);

@@ -70,7 +70,8 @@ struct StepParams {
   const T* zoneout_mask;      // [N, H] or null
   const T* dc_mask;           // DropConnect mask of R or null
   float dc_scale;
-  typename Step<T>::Sum* h_stage;  // [N, H] when h_out overlaps h (state updated in place) or x, else null
+  typename Step<T>::Sum* h_stage;  // [N, H] where h_out is memory that others still read (StepStaging), else null
+  typename Step<T>::Sum* c_stage;  // LSTM: the same for c_out
   typename Step<T>::Sum* partial;  // [runs][output tiles][4 sums][quads of rows][64]; unused with one run
   ControlBlock* cb;
   int runs, row_blocks, unit_blocks, quads;  // quads: of rows, in an output tile
@@ -142,7 +143,8 @@ __device__ __forceinline__ void finish_unit(const StepParams<T>& p, int n, int j
     const A gf = S::sigmoid(a[2] + in.b[2]), go = S::sigmoid(a[3] + in.b[3]);
     const A c_new = gf * in.c + gi * gg;
     h_new = go * S::tanh_(c_new);
-    p.c_out[e] = (T)c_new;
+    if (p.c_stage == nullptr) p.c_out[e] = (T)c_new;
+    else store_sum(&p.c_stage[e], c_new);
     if (p.training) {
       T* vt = p.v + (size_t)n * 4 * H + j;
       vt[0] = (T)gi; vt[H] = (T)gg; vt[2 * H] = (T)gf; vt[3 * H] = (T)go;
@@ -166,11 +168,11 @@ __device__ __forceinline__ void finish_unit(const StepParams<T>& p, int n, int j
   else store_sum(&p.h_stage[e], h_new);
 }
 
-// h_out overlaps h or x: other workgroups may still be reading them when a column block is
+// h_out or c_out overlaps h or x: other workgroups may still be reading them when a column block is
 // finished, so the new state is parked and copied out by the last column block to finish, when every
 // run of every block has been read.  Called by the finishing workgroups, all threads.
 template <typename T>
-__device__ __forceinline__ void copy_staged_state(const StepParams<T>& p, unsigned int* flag) {
+__device__ __forceinline__ void copy_staged_states(const StepParams<T>& p, unsigned int* flag) {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -184,7 +186,10 @@ __device__ __forceinline__ void copy_staged_state(const StepParams<T>& p, unsign
   __syncthreads();
   if (*flag == 0u) return;
   const int count = p.N * p.H;
-  for (int i = threadIdx.x; i < count; i += 256) p.h_out[i] = (T)load_sum(&p.h_stage[i]);
+  if (p.h_stage != nullptr)
+    for (int i = threadIdx.x; i < count; i += 256) p.h_out[i] = (T)load_sum(&p.h_stage[i]);
+  if (p.c_stage != nullptr)
+    for (int i = threadIdx.x; i < count; i += 256) p.c_out[i] = (T)load_sum(&p.c_stage[i]);
 }
 
 // GATES = 4: LSTM (i, g, f, o); GATES = 3: GRU (z, r, g).  RT: tiles of 16 batch rows a workgroup
@@ -381,7 +386,7 @@ void forward_step_kernel(StepParams<T> p) {
     }
     finish_unit<GATES, T>(p, n, j, a, in[rt]);
   }
-  if (p.h_stage != nullptr) copy_staged_state(p, &s_flag);
+  if (p.h_stage != nullptr || p.c_stage != nullptr) copy_staged_states(p, &s_flag);
 }
 
 // How a step is cut up.
@@ -423,11 +428,40 @@ StepCut step_cut(int N, int C, int H, size_t element) {
   return s;
 }
 
+// Which results of a step are parked until all of its workgroups have read their inputs.  Every workgroup of a row block
+// reads x and h; an element of c and of the mask only the thread that writes the results of that element.
+struct StepStaging {
+  bool h = false, c = false;
+  bool possible = true;  // v is not parked
+  size_t bytes = 0;
+};
+
+StepStaging step_staging(int N, int C, int H, size_t element, const StepTensors& t) {
+  const size_t state = (size_t)N * H;
+  auto overlaps = [&](const void* out, size_t out_count, const void* in, size_t in_count) {
+    const uintptr_t to = reinterpret_cast<uintptr_t>(out), from = reinterpret_cast<uintptr_t>(in);
+    return out != nullptr && in != nullptr && to < from + in_count * element && from < to + out_count * element;
+  };
+  auto read_by_others = [&](const void* out, size_t count) {
+    return overlaps(out, count, t.x, (size_t)N * C) || overlaps(out, count, t.h, state) ||
+           (overlaps(out, count, t.c, state) && out != t.c) || (overlaps(out, count, t.mask, state) && out != t.mask);
+  };
+  StepStaging s;
+  if (planned_pass() != nullptr) return s;  // (whose tensors are all at one address)
+  s.h = read_by_others(t.h_out, state);
+  s.c = read_by_others(t.c_out, state);
+  s.possible = !read_by_others(t.v, 4 * state) && (t.v == nullptr || (t.v != t.c && t.v != t.mask));
+  s.bytes = ((s.h ? 1 : 0) + (s.c ? 1 : 0)) * state * (element == 8 ? 8 : 4);
+  return s;
+}
+
 template <int GATES, typename T>
 int launch_step(hipStream_t stream, StepParams<T>& p, const char* name) {
   typedef typename Step<T>::Sum A;
   StepCut cut = step_cut(p.N, p.C, p.H, sizeof(T));
-  const size_t state_bytes = staged_state_bytes(p.N, p.C, p.H, p.x, p.h, p.h_out, sizeof(T));
+  const StepStaging staging = step_staging(p.N, p.C, p.H, sizeof(T), {p.x, p.h, p.c, p.zoneout_mask, p.h_out, p.c_out,
+                                                                      p.training ? p.v : nullptr});
+  const size_t state_bytes = staging.bytes;
   for (bool room = false; !room && cut.runs > 1;) {
     HASTE_HIP_PROPAGATE(workspace_has_room(stream, cut.sums() * sizeof(A) + state_bytes + 256, &room));
     if (!room) cut.runs = (cut.runs + 1) / 2;
@@ -440,7 +474,9 @@ int launch_step(hipStream_t stream, StepParams<T>& p, const char* name) {
     return HASTE_HIP_OK;
   }
   p.partial = reinterpret_cast<A*>(ws.scratch);
-  p.h_stage = state_bytes > 0 ? p.partial + cut.sums() : nullptr;
+  A* stage = p.partial + cut.sums();
+  p.h_stage = staging.h ? stage : nullptr;
+  p.c_stage = staging.c ? stage + (staging.h ? (size_t)p.N * p.H : 0) : nullptr;
   p.cb = ws.control;
   p.runs = cut.runs; p.row_blocks = cut.row_blocks; p.unit_blocks = cut.unit_blocks; p.quads = cut.quads;
   const dim3 grid((unsigned)cut.row_blocks * cut.unit_blocks * cut.runs);
@@ -470,24 +506,15 @@ int launch_step(hipStream_t stream, StepParams<T>& p, const char* name) {
 // at every size (N = 64, C = 64, H = 2048 125 / 42, N = 128, C = 512, H = 4096 420 / 261).  In double (kStepDouble) it is a
 // product per side and a pointwise launch: LSTM N = 1, C = H = 512 17.4 / 11.5, N = 43, C = 64, H = 192 14.1 / 9.7,
 // N = 128, C = H = 512, 16 384 blocks, 32.9 / 27.8; GRU N = 8, C = 64, H = 2048, 16 896 blocks, 29.9 / 31.3.
-int single_step_rule(hipStream_t stream, int N, int C, int H, size_t element, long long most_blocks, size_t staged_bytes,
-                     bool* applies) {
+int single_step_rule(hipStream_t stream, int N, int C, int H, size_t element, long long most_blocks,
+                     const StepTensors& tensors, bool* applies) {
   const StepCut cut = step_cut(N, C, H, element);
-  *applies = (long long)cut.row_blocks * cut.unit_blocks <= kStepTiles;
+  const StepStaging staging = step_staging(N, C, H, element, tensors);
+  *applies = (long long)cut.row_blocks * cut.unit_blocks <= kStepTiles && staging.possible;
   if (!*applies || (N <= 8 && element != 8)) return HASTE_HIP_OK;
   *applies = step_blocks(N, C, H) <= most_blocks;
   if (!*applies) return HASTE_HIP_OK;
-  return workspace_has_room(stream, cut.sums() * (element == 8 ? 8 : 4) + staged_bytes + 256, applies);
-}
-
-size_t staged_state_bytes(int N, int C, int H, const void* x, const void* h, const void* h_out, size_t element) {
-  const uintptr_t to = reinterpret_cast<uintptr_t>(h_out);
-  const size_t floats = (size_t)N * H;
-  auto overlaps = [&](const void* in, size_t count) {
-    const uintptr_t from = reinterpret_cast<uintptr_t>(in);
-    return to < from + count * element && from < to + floats * element;
-  };
-  return overlaps(h, floats) || overlaps(x, (size_t)N * C) ? floats * (element == 8 ? 8 : 4) : 0;
+  return workspace_has_room(stream, cut.sums() * (element == 8 ? 8 : 4) + staging.bytes + 256, applies);
 }
 
 int lstm_forward_single_step(hipStream_t stream, int training, int N, int C, int H, const float* W,

@@ -1231,7 +1231,8 @@ int lstm_forward_steps(hipStream_t stream, int training, int steps, int N, int C
   if constexpr (std::is_same<T, double>::value) {
     bool single = false;
     if (steps == 1)
-      HASTE_HIP_PROPAGATE(single_step_rule(stream, N, C, H, sizeof(T), kStepDouble, staged_state_bytes(N, C, H, x, h, h_out, sizeof(T)), &single));
+      HASTE_HIP_PROPAGATE(single_step_rule(stream, N, C, H, sizeof(T), kStepDouble,
+                                           {x, h, c, zoneout_mask, h_out, c_out, training ? v : nullptr}, &single));
     if (single)
       return lstm_forward_single_step(stream, training, N, C, H, W, R, b, x, h, c, h_out, c_out, v, zoneout_prob, zoneout_mask, dc_mask,
                                       dc_scale);
@@ -1314,7 +1315,8 @@ int gru_forward_steps(hipStream_t stream, int training, int steps, int N, int C,
   if constexpr (std::is_same<T, double>::value) {
     bool single = false;
     if (steps == 1)
-      HASTE_HIP_PROPAGATE(single_step_rule(stream, N, C, H, sizeof(T), kStepDouble, staged_state_bytes(N, C, H, x, h, h_out, sizeof(T)), &single));
+      HASTE_HIP_PROPAGATE(single_step_rule(stream, N, C, H, sizeof(T), kStepDouble,
+                                           {x, h, nullptr, zoneout_mask, h_out, nullptr, training ? v : nullptr}, &single));
     if (single)
       return gru_forward_single_step(stream, training, N, C, H, W, R, bx, br, x, h, h_out, v, zoneout_prob, zoneout_mask, dc_mask, dc_scale);
   }
@@ -2134,7 +2136,7 @@ int haste_hip_gru_forward_f16(int training, int steps, int batch_size, int input
                             bx, br, x, h, v, zoneout_prob, zoneout_mask, nullptr, 1.f);
   bool single = false;
   HASTE_HIP_PROPAGATE(single_step_rule(as_stream(stream), batch_size, input_size, hidden_size, sizeof(half_t), kStepHalf,
-                                       staged_state_bytes(batch_size, input_size, hidden_size, x, h, hp(h) + NH, sizeof(half_t)), &single));
+                                       {x, h, nullptr, zoneout_mask, hp(h) + NH, nullptr, training ? v : nullptr}, &single));
   if (single)
     return gru_forward_single_step_half(as_stream(stream), training, batch_size, input_size, hidden_size,
                                         W, R, bx, br, x, h, hp(h) + NH, v, zoneout_prob, zoneout_mask,
@@ -2160,7 +2162,7 @@ int haste_hip_gru_forward_dropconnect_f16(int training, int steps, int batch_siz
                             dropconnect_scale);
   bool single = false;
   HASTE_HIP_PROPAGATE(single_step_rule(as_stream(stream), batch_size, input_size, hidden_size, sizeof(half_t), kStepHalf,
-                                       staged_state_bytes(batch_size, input_size, hidden_size, x, h, hp(h) + NH, sizeof(half_t)), &single));
+                                       {x, h, nullptr, zoneout_mask, hp(h) + NH, nullptr, training ? v : nullptr}, &single));
   if (single)
     return gru_forward_single_step_half(as_stream(stream), training, batch_size, input_size, hidden_size,
                                         W, R, bx, br, x, h, hp(h) + NH, v, zoneout_prob, zoneout_mask,
@@ -2201,7 +2203,7 @@ int haste_hip_gru_forward_iterate_f16(int training, int batch_size, int input_si
   HASTE_HIP_REQUIRE(W && R && bx && br && x && h && h_out && tmp_Wx && (v || !training));
   bool single = false;
   HASTE_HIP_PROPAGATE(single_step_rule(as_stream(stream), batch_size, input_size, hidden_size, sizeof(half_t), kStepHalf,
-                                       staged_state_bytes(batch_size, input_size, hidden_size, x, h, h_out, sizeof(half_t)), &single));
+                                       {x, h, nullptr, zoneout_mask, h_out, nullptr, training ? v : nullptr}, &single));
   if (single)
     return gru_forward_single_step_half(as_stream(stream), training, batch_size, input_size, hidden_size,
                                         W, R, bx, br, x, h, h_out, v, zoneout_prob, zoneout_mask, nullptr,

@@ -163,6 +163,38 @@ def test_single_step_whose_output_replaces_its_input(N, H):
             assert torch.equal(got, want) and torch.equal(got3, want3)
 
 
+@pytest.mark.parametrize("dtype,N,H", [("float32", 3, 512), ("float32", 40, 512), ("float32", 128, 300), ("float32", 40, 1000),
+                                       ("float64", 3, 512), ("float64", 40, 300)])
+@pytest.mark.parametrize("training", [False, True])
+def test_single_lstm_step_whose_cell_state_replaces_its_inputs(dtype, N, H, training):
+    """c_out in the memory of x or h, both states exchanged, or moved by some rows: the bits of a call with memory of its
+    own."""
+    from haste_amd import ops
+    import torch
+    p = problem(43 + N, 1, N, H, H, 4, 0.1)
+    x, h0, c0, W, R, b, mask = (dev(a).to(getattr(torch, dtype)) for a in
+                                (p["x"][0], p["h0"], p["c0"], p["W"], p["R"], p["b"], p["mask"][0]))
+    step = lambda x, h, c, **out: ops.lstm_forward_iterate(training, 0.1, x, h, c, W, R, b, mask, **out)
+    want_h, want_c, want_v = step(x, h0, c0)
+    for _ in range(3):
+        for form in ("x", "h", "both", "exchanged", "moved"):
+            xi, hi, ci = x.clone(), h0.clone(), c0.clone()
+            rows = torch.cat([c0[:1], c0])
+            if form == "x":
+                got = step(xi, hi, ci, c_out=xi)
+            elif form == "h":
+                got = step(xi, hi, ci, c_out=hi)
+            elif form == "both":
+                got = step(xi, hi, ci, h_out=xi, c_out=hi)
+            elif form == "exchanged":
+                got = step(xi, hi, ci, h_out=ci, c_out=hi)
+            else:
+                got = step(xi, hi, rows[1:], h_out=hi, c_out=rows[:-1])
+            torch.cuda.synchronize()
+            assert torch.equal(got[0], want_h) and torch.equal(got[1], want_c), form
+            assert not training or torch.equal(got[2], want_v), form
+
+
 @pytest.mark.parametrize("N,C,H", [(4, 48, 200), (8, 512, 512), (33, 48, 200), (70, 100, 1030)])
 def test_single_step_dropconnect_equals_premasked_weights(N, C, H):
     from haste_amd import ops
