@@ -72,6 +72,7 @@ struct StepParams {
   float dc_scale;
   typename Step<T>::Sum* h_stage;  // [N, H] where h_out is memory that others still read (StepStaging), else null
   typename Step<T>::Sum* c_stage;  // LSTM: the same for c_out
+  int copies;                      // whether the kernel also copies them where they belong
   typename Step<T>::Sum* partial;  // [runs][output tiles][4 sums][quads of rows][64]; unused with one run
   ControlBlock* cb;
   int runs, row_blocks, unit_blocks, quads;  // quads: of rows, in an output tile
@@ -168,9 +169,23 @@ __device__ __forceinline__ void finish_unit(const StepParams<T>& p, int n, int j
   else store_sum(&p.h_stage[e], h_new);
 }
 
+// Elements first, first + stride .. of a parked state go where they belong, COPY of them on their way at a time.
+template <int COPY, typename T>
+__device__ __forceinline__ void copy_state(typename Step<T>::Sum* stage, T* out, int first, int stride, int count) {
+  typedef typename Step<T>::Sum A;
+  for (int i = first; i < count; i += COPY * stride) {
+    A v[COPY];
+#pragma unroll
+    for (int k = 0; k < COPY; ++k) v[k] = i + k * stride < count ? load_sum(&stage[i + k * stride]) : A(0);
+#pragma unroll
+    for (int k = 0; k < COPY; ++k)
+      if (i + k * stride < count) out[i + k * stride] = (T)v[k];
+  }
+}
+
 // h_out or c_out overlaps h or x: other workgroups may still be reading them when a column block is
-// finished, so the new state is parked and copied out by the last column block to finish, when every
-// run of every block has been read.  Called by the finishing workgroups, all threads.
+// finished, so the new state is parked.  Few elements (StepParams::copies) are copied out by the last column block to
+// finish, when every run of every block has been read.  Called by the finishing workgroups, all threads.
 template <typename T>
 __device__ __forceinline__ void copy_staged_states(const StepParams<T>& p, unsigned int* flag) {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -186,10 +201,17 @@ __device__ __forceinline__ void copy_staged_states(const StepParams<T>& p, unsig
   __syncthreads();
   if (*flag == 0u) return;
   const int count = p.N * p.H;
-  if (p.h_stage != nullptr)
-    for (int i = threadIdx.x; i < count; i += 256) p.h_out[i] = (T)load_sum(&p.h_stage[i]);
-  if (p.c_stage != nullptr)
-    for (int i = threadIdx.x; i < count; i += 256) p.c_out[i] = (T)load_sum(&p.c_stage[i]);
+  if (p.h_stage != nullptr) copy_state<4, T>(p.h_stage, p.h_out, threadIdx.x, 256, count);
+  if (p.c_stage != nullptr) copy_state<4, T>(p.c_stage, p.c_out, threadIdx.x, 256, count);
+}
+
+// More of them: a launch of its own.
+template <typename T>
+__global__ __launch_bounds__(256)
+void copy_staged_kernel(typename Step<T>::Sum* h_stage, T* h_out, typename Step<T>::Sum* c_stage, T* c_out, int count) {
+  const int first = blockIdx.x * 256 + threadIdx.x, stride = gridDim.x * 256;
+  if (h_stage != nullptr) copy_state<4, T>(h_stage, h_out, first, stride, count);
+  if (c_stage != nullptr) copy_state<4, T>(c_stage, c_out, first, stride, count);
 }
 
 // GATES = 4: LSTM (i, g, f, o); GATES = 3: GRU (z, r, g).  RT: tiles of 16 batch rows a workgroup
@@ -386,7 +408,7 @@ void forward_step_kernel(StepParams<T> p) {
     }
     finish_unit<GATES, T>(p, n, j, a, in[rt]);
   }
-  if (p.h_stage != nullptr || p.c_stage != nullptr) copy_staged_states(p, &s_flag);
+  if (p.copies) copy_staged_states(p, &s_flag);
 }
 
 // How a step is cut up.
@@ -455,6 +477,12 @@ StepStaging step_staging(int N, int C, int H, size_t element, const StepTensors&
   return s;
 }
 
+// Elements of parked states up to which the step's last workgroup copies them, a memory round trip for every 1024; a launch
+// of its own costs 2 - 3 us at any size.  (A step in place of N x H, C = 64, us in the step / with the launch: LSTM 4 x 64
+// 6.3 / 8.1, 2 x 1024 12.3 / 13.1, 8 x 512 11.5 / 11.6, 16 x 512 13.2 / 11.8; half GRU 1 x 512 10.6 / 11.2, 4 x 512 12.1 / 11.6, 8 x 512
+// 13.5 / 11.4; double LSTM 8 x 64 8.6 / 10.2, 8 x 256 13.1 / 13.6, 8 x 1024 21.2 / 19.2.)
+constexpr size_t kCopiedInStep = 2048;
+
 template <int GATES, typename T>
 int launch_step(hipStream_t stream, StepParams<T>& p, const char* name) {
   typedef typename Step<T>::Sum A;
@@ -477,6 +505,8 @@ int launch_step(hipStream_t stream, StepParams<T>& p, const char* name) {
   A* stage = p.partial + cut.sums();
   p.h_stage = staging.h ? stage : nullptr;
   p.c_stage = staging.c ? stage + (staging.h ? (size_t)p.N * p.H : 0) : nullptr;
+  const size_t parked = state_bytes / sizeof(A);
+  p.copies = parked > 0 && parked <= kCopiedInStep;
   p.cb = ws.control;
   p.runs = cut.runs; p.row_blocks = cut.row_blocks; p.unit_blocks = cut.unit_blocks; p.quads = cut.quads;
   const dim3 grid((unsigned)cut.row_blocks * cut.unit_blocks * cut.runs);
@@ -492,6 +522,11 @@ int launch_step(hipStream_t stream, StepParams<T>& p, const char* name) {
   }
 #undef HASTE_LAUNCH_STEP
   HASTE_HIP_TRY(hipGetLastError());
+  if (parked > kCopiedInStep) {
+    const unsigned count = (unsigned)p.N * p.H;
+    copy_staged_kernel<T><<<dim3((count + 1023) / 1024), dim3(256), 0, stream>>>(p.h_stage, p.h_out, p.c_stage, p.c_out, (int)count);
+    HASTE_HIP_TRY(hipGetLastError());
+  }
   return HASTE_HIP_OK;
 }
 

@@ -163,6 +163,29 @@ def test_single_step_whose_output_replaces_its_input(N, H):
             assert torch.equal(got, want) and torch.equal(got3, want3)
 
 
+# Parked states are copied by the step itself up to 2048 elements, beyond that by a launch of their own.
+@pytest.mark.parametrize("dtype", ["float16", "float32", "float64"])
+@pytest.mark.parametrize("N,C,H", [(1, 5, 1), (3, 20, 341), (2, 64, 1024), (1, 64, 2049), (33, 40, 100), (128, 70, 300)])
+def test_single_step_in_place(dtype, N, C, H):
+    """Both states updated where they are: the bits of a call with memory of its own, call after call."""
+    from haste_amd import ops
+    import torch
+    p = problem(47 + N, 1, N, C, H, 4)
+    x, h0, c0, W, R, b, b2 = (dev(a).to(getattr(torch, dtype)) for a in
+                              (p["x"][0], p["h0"], p["c0"], p["W"], p["R"], p["b"], p["b2"]))
+    W3, R3, bx, br = (t[..., :3 * H].contiguous() for t in (W, R, b, b2))
+    h, c, g = h0, c0, h0
+    hi, ci, gi = h0.clone(), c0.clone(), h0.clone()
+    for _ in range(4):
+        if dtype != "float16":  # (the LSTM has no half form)
+            h, c, _ = ops.lstm_forward_iterate(False, 0.0, x, h, c, W, R, b)
+            ops.lstm_forward_iterate(False, 0.0, x, hi, ci, W, R, b, h_out=hi, c_out=ci)
+        g, _ = ops.gru_forward_iterate(False, 0.0, x, g, W3, R3, bx, br)
+        ops.gru_forward_iterate(False, 0.0, x, gi, W3, R3, bx, br, h_out=gi)
+        torch.cuda.synchronize()
+        assert torch.equal(hi, h) and torch.equal(ci, c) and torch.equal(gi, g)
+
+
 @pytest.mark.parametrize("dtype,N,H", [("float32", 3, 512), ("float32", 40, 512), ("float32", 128, 300), ("float32", 40, 1000),
                                        ("float64", 3, 512), ("float64", 40, 300)])
 @pytest.mark.parametrize("training", [False, True])
