@@ -318,16 +318,14 @@ int gru_backward_cut(hipStream_t stream, int T, int N, int H, const float* R_t, 
 size_t cut_scratch_bound(int N, int H, int cus);
 
 // One forward step as a single kernel (single_step.hip): what the Iterate entry points and one-step
-// Run calls use, for batches up to a size (single_step_rule: most_blocks blocks of 16 units, rows and
-// contraction indices) that depends on what the step would run on otherwise.
-constexpr long long kStepStreamed = 60 << 10, kStepResident = 128 << 10, kStepHalf = 1ll << 40,
-                    kStepDouble = 16 << 10;
+// Run calls use, for batches up to a size (single_step_rule) that depends on what the step would run on otherwise.
+enum StepOther { kStepStreamed, kStepResident, kStepHalf, kStepDouble };
 struct StepTensors {
   const void *x, *h, *c, *mask;   // what it reads (GRU: no c; no mask: null)
   const void *h_out, *c_out, *v;  // what it writes (GRU: no c_out; v: in training)
 };
-int single_step_rule(hipStream_t stream, int N, int C, int H, size_t element, long long most_blocks,
-                     const StepTensors& tensors, bool* applies);
+int single_step_rule(hipStream_t stream, int N, int C, int H, size_t element, StepOther other, const StepTensors& tensors,
+                     bool* applies);
 int lstm_forward_single_step(hipStream_t stream, int training, int N, int C, int H, const float* W,
                              const float* R, const float* b, const float* x, const float* h,
                              const float* c, float* h_out, float* c_out, float* v,

@@ -706,7 +706,7 @@ size_t haste_hip_workspace_bytes(int time_steps, int batch_size, int input_size,
   b += 2 * cus * 64 * 64 * 8;
   b += 2 * cus * 2 * widest * sizeof(float);
   // Single forward steps: partial sums of every run of the contraction (four of 4 to 32 rows and 16 units a
-  // workgroup, at most four workgroups per CU and one per tile beyond: larger batches also use the room
+  // workgroup, at most about five workgroups per CU: larger batches also use the room
   // of the GEMM and the exchange tiles, which such a step does not touch), and the staged states.
   b += 64 * 2 * 8 * (H / 16 + 1) * 64 * sizeof(float) + 2 * 8 * H * sizeof(float) + 256;
   return kControlBytes + 4096 + (b + 255) / 256 * 256;

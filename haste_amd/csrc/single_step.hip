@@ -12,6 +12,8 @@
 // double ones in double.
 //
 // Arithmetic: reference lib/lstm_forward_gpu.cu.cc:55-86, lib/gru_forward_gpu.cu.cc:46-84.
+#include <algorithm>
+
 #include "recurrent.h"
 
 namespace haste_hip {
@@ -425,10 +427,21 @@ long long step_blocks(int N, int C, int H) {
   return (long long)((N + 15) / 16) * ((H + kStepUnits - 1) / kStepUnits) * groups;
 }
 
-// A step of few rows is bound by the latency of its chain (loads, sums out, a counter, sums in): two
-// workgroups per CU, but runs of at least 8 groups, since every run's sums meet in memory (N = 1,
-// C = H = 512: 8 runs 8.3 us, 16 runs of half the length 9.0, 32 runs 13.7).  Where that leaves runs of
-// more than 32 groups, up to four workgroups per CU (GRU, N = 8, C = 64, H = 3776: 46.0 -> 44.5 us).
+// A step is bound by the latency of its chain (loads, sums out, a counter, sums in).
+// Up to 16 rows a run is as few batches of weights (kBatchGroups groups, which are on their way together: a run of a batch
+// and a group takes two) as leave no more workgroups than a CU holds well at a time (three, with runs of more than 16
+// batches four, in double two) and not many more runs than batches: every run's sums meet in memory.  Measured, N = 1,
+// us by batches a run:
+//   float   C =  64, H =  256  1: 6.4   2: 7.3   3: 8.1   5 (one run): 8.5
+//           C =  64, H =  512  1: 7.6   2: 7.9   3: 8.5   5: 10.6
+//           C = 512, H =  512  1: 9.4   2: 8.7   4: 9.3
+//           C = 256, H = 1024  1: 12.8  2: 10.9  3: 11.6  4: 12.3
+//           C =  64, H = 2048  1: 25.4  3: 20.1  4: 20.5  6: 20.8  9: 21.2
+//   double  C =  64, H =  512  1: 11.7  2: 11.1  3: 12.1
+//           C = 512, H = 1536  2: 45.6  4: 32.6  8: 33.6
+// With more rows, runs of at least 8 groups, whose sums are then read by fewer: two workgroups per CU (double at most two:
+// N = 24, C = 64, H = 1280, 480 / 560 workgroups 25 / 38; float three: N = 320, C = 64, H = 768, 480 / 960 32 / 43), in float and
+// half, where that leaves runs of more than 32 groups, up to four.
 // 32 rows a workgroup halve the reading of weights, once there are enough tiles for it (LSTM,
 // C = H = 512, us with 16 / 32 rows: N = 64, 128 tiles of 16, 12.2 / 14.2; N = 128, 256 tiles, 17.6 / 16.5).
 StepCut step_cut(int N, int C, int H, size_t element) {
@@ -440,11 +453,23 @@ StepCut step_cut(int N, int C, int H, size_t element) {
   s.quads = s.row_blocks > 1 || element == 8 ? 4 * s.rt : (N + 3) / 4;
   const int groups = (C + kGroupRows - 1) / kGroupRows + (H + kGroupRows - 1) / kGroupRows;
   const long long tiles = (long long)s.row_blocks * s.unit_blocks;
-  long long runs = (2 * cus + tiles - 1) / tiles;
-  if (runs > groups / 8) runs = groups / 8;
-  if (runs < groups / 32) {
-    runs = (4 * cus + tiles - 1) / tiles;
-    if (runs > groups / 32) runs = groups / 32;
+  long long runs;
+  if (s.rt == 1 && s.row_blocks == 1) {
+    auto of = [&](int batches) { return (groups + batches * kBatchGroups - 1) / (batches * kBatchGroups); };
+    auto fewest = [&](int per_cu) {
+      int batches = groups <= 2 * kBatchGroups ? 2 : 1;
+      while (of(batches) > 1 && (tiles * of(batches) > (long long)per_cu * cus || of(batches) > 10 * batches)) ++batches;
+      return batches;
+    };
+    int batches = fewest(element == 8 ? 2 : 3);
+    if (batches > 16 && element < 8) batches = fewest(4);
+    runs = of(batches);
+  } else if (element == 8) {
+    runs = std::min<long long>(2 * cus / tiles, groups / 8);
+  } else {
+    runs = std::min<long long>((2 * cus + tiles - 1) / tiles, groups / 8);
+    if (element == 4 && tiles * runs > 3 * cus) runs = 3 * cus / tiles;
+    if (runs < groups / 32) runs = std::min<long long>((4 * cus + tiles - 1) / tiles, groups / 32);
   }
   s.runs = runs < 1 ? 1 : (int)runs;
   return s;
@@ -532,22 +557,42 @@ int launch_step(hipStream_t stream, StepParams<T>& p, const char* name) {
 
 }  // namespace
 
-// Whether a step of N rows is this kernel's (most_blocks: kStep...).  In float up to 8 rows always, as long as its
-// tiles have counters.  Beyond, the other way is the all-steps kernels, which fetch their slice of R for one use
-// (kStepResident: they keep R on chip; LSTM, us there / here: N = 43, C = 32, H = 128 13.6 / 5.7, N = 64, C = 64,
-// H = 2048 82 / 52), or a GEMM per side, faster from some size on because it keeps more of both operands on chip
-// (kStepStreamed; N = 16, C = 64, H = 4096, 66 560 blocks, 53 / 63; N = 128, C = 512, H = 1536, 98 304 blocks,
-// 51 / 60; N = 128, C = 256, H = 1024, 40 960 blocks, 48 / 30).  The half GRU's other way converts its weights: here
-// at every size (N = 64, C = 64, H = 2048 125 / 42, N = 128, C = 512, H = 4096 420 / 261).  In double (kStepDouble) it is a
-// product per side and a pointwise launch: LSTM N = 1, C = H = 512 17.4 / 11.5, N = 43, C = 64, H = 192 14.1 / 9.7,
-// N = 128, C = H = 512, 16 384 blocks, 32.9 / 27.8; GRU N = 8, C = 64, H = 2048, 16 896 blocks, 29.9 / 31.3.
-int single_step_rule(hipStream_t stream, int N, int C, int H, size_t element, long long most_blocks,
-                     const StepTensors& tensors, bool* applies) {
+// Whether a step of N rows is this kernel's rather than what it would run on otherwise.  In float and half up to 8 rows
+// always, as long as its tiles have counters.  Beyond (blocks: of 16 units, rows and contraction indices; tiles: of 16 or 32
+// rows, which up to one per CU do not wait for one another; us there / here):
+//  - float, all-steps kernels, which fetch their slice of R for one use: N = 43, C = 32, H = 128 13.6 / 5.7; N = 64, C = 64,
+//    H = 2048 82 / 55; N = 256, C = 512, H = 1024 (98 304 blocks) 66 / 51.
+//  - float, a GEMM per side, which keeps more of both operands on chip.  Up to H = 1024 slower as long as there are few
+//    blocks: N = 160, C = 64, H = 768 33 / 22, N = 160, C = 512, H = 1024 (61 440, 320 tiles) 48 / 42, N = 512, C = 512, H = 448
+//    (53 760, 448 tiles) 47 / 37; but with many tiles of a long contraction N = 208, C = 64, H = 1024 (56 576, 448 tiles) 40 / 51,
+//    and N = 320, C = 64, H = 896 (67 200) 38 / 47.  Beyond, with tiles for every CU at most: N = 96, C = 64, H = 1280 (240 tiles) 34 / 29, GRU 31 / 29; but
+//    N = 112, H = 1152 (288) 33 / 37 and N = 80, H = 1536 (288) 39 / 45.  From where no batch has a resident slice, the GEMM's
+//    small form: N = 16, C = 64, H = 2560 27 / 31, GRU 24 / 27; N = 16, H = 4096 52 / 60.
+//  - half, where the other way converts its weights: N = 64, C = 64, H = 2048 127 / 42, N = 128, C = 512, H = 4096 420 / 238.
+//  - double, a product per side and a pointwise launch: LSTM N = 1, C = H = 512 17.4 / 11.1, GRU N = 8, C = 512, H = 1536
+//    (12 288) 31 / 25, N = 128, C = H = 512 (16 384, 256 tiles) 33 / 28; more tiles than CUs N = 320, C = 64, H = 256 (6 400)
+//    22 / 17, but N = 128, C = 64, H = 576 (11 520, 288 tiles) 25 / 28.
+static bool step_pays(StepOther other, long long blocks, long long tiles, int H) {
+  const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
+  switch (other) {
+    case kStepResident: return blocks <= 128 << 10;
+    case kStepStreamed:
+      if (H > 1024) return blocks <= 60 << 10 && H <= 2048 && tiles <= cus;
+      return blocks <= (2 * tiles <= 3 * cus || H <= 512 ? 60 << 10 : 48 << 10);
+    case kStepHalf: return true;
+    case kStepDouble: return blocks <= (tiles <= cus ? 16 << 10 : 8 << 10);
+  }
+  return false;
+}
+
+int single_step_rule(hipStream_t stream, int N, int C, int H, size_t element, StepOther other, const StepTensors& tensors,
+                     bool* applies) {
   const StepCut cut = step_cut(N, C, H, element);
   const StepStaging staging = step_staging(N, C, H, element, tensors);
-  *applies = (long long)cut.row_blocks * cut.unit_blocks <= kStepTiles && staging.possible;
+  const long long tiles = (long long)cut.row_blocks * cut.unit_blocks;
+  *applies = tiles <= kStepTiles && staging.possible;
   if (!*applies || (N <= 8 && element != 8)) return HASTE_HIP_OK;
-  *applies = step_blocks(N, C, H) <= most_blocks;
+  *applies = step_pays(other, step_blocks(N, C, H), tiles, H);
   if (!*applies) return HASTE_HIP_OK;
   return workspace_has_room(stream, cut.sums() * (element == 8 ? 8 : 4) + staging.bytes + 256, applies);
 }

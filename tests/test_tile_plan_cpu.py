@@ -106,7 +106,10 @@ def test_single_steps(gates):
     is; a workspace too small for its sums leaves larger batches what they ran on before."""
     lib = hlib.load()
     for N, C, H, single in [(1, 512, 512, 1), (8, 64, 4096, 1), (9, 512, 512, 1), (128, 512, 512, 1), (64, 64, 2048, 1),
-                            (16, 512, 4096, 0), (128, 64, 3000, 0), (1024, 512, 512, 0)]:
+                            (16, 512, 4096, 0), (128, 64, 3000, 0), (1024, 512, 512, 0),
+                            # beyond what stays on chip: as long as there is no more than a tile per CU, and few blocks
+                            (16, 64, 2560, 0), (96, 64, 1280, 1), (112, 64, 1152, 0), (80, 64, 1536, 0),
+                            (160, 512, 1024, 1)]:
         rc, plan = _plan_pass(lib, 256, 8, gates, 4, 0, 1, N, C, H)
         assert rc == 0 and (plan[0] == 1) == bool(single), (N, C, H, rc, plan)
     # the sums of a step of 64 rows take 2 MiB; its all-steps kernel asks for less
