@@ -132,7 +132,7 @@ __device__ __forceinline__ UnitInputs<typename Step<T>::Sum> unit_inputs(const S
 
 // Unit j of row n from its sums a: LSTM the four gates of [x | h] * [W; R]; GRU the update and the
 // reset gate, x * W and h * R of the candidate gate.
-template <int GATES, typename T>
+template <int GATES, bool STAGED, typename T>
 __device__ __forceinline__ void finish_unit(const StepParams<T>& p, int n, int j, const typename Step<T>::Sum (&a)[4],
                                             const UnitInputs<typename Step<T>::Sum>& in) {
   typedef typename Step<T>::Sum A;
@@ -146,7 +146,7 @@ __device__ __forceinline__ void finish_unit(const StepParams<T>& p, int n, int j
     const A gf = S::sigmoid(a[2] + in.b[2]), go = S::sigmoid(a[3] + in.b[3]);
     const A c_new = gf * in.c + gi * gg;
     h_new = go * S::tanh_(c_new);
-    if (p.c_stage == nullptr) p.c_out[e] = (T)c_new;
+    if (!STAGED || p.c_stage == nullptr) p.c_out[e] = (T)c_new;
     else store_sum(&p.c_stage[e], c_new);
     if (p.training) {
       T* vt = p.v + (size_t)n * 4 * H + j;
@@ -167,7 +167,7 @@ __device__ __forceinline__ void finish_unit(const StepParams<T>& p, int n, int j
     if (p.training) h_new = (h_new - in.h) * in.mask + in.h;
     else h_new = A(p.zoneout_prob) * in.h + (A(1) - A(p.zoneout_prob)) * h_new;
   }
-  if (p.h_stage == nullptr) p.h_out[e] = (T)h_new;
+  if (!STAGED || p.h_stage == nullptr) p.h_out[e] = (T)h_new;
   else store_sum(&p.h_stage[e], h_new);
 }
 
@@ -223,8 +223,8 @@ void copy_staged_kernel(typename Step<T>::Sum* h_stage, T* h_out, typename Step<
 // Every weight goes from memory to the register of the one lane that feeds it to the matrix unit
 // (fp32 instruction: 16 rows of a batch against 16 units cost a quarter of what the loads take);
 // the inputs are staged in LDS.  Lane (column l % 16, l / 16) of a group's i-th instruction holds
-// contraction index 4 (l / 16) + i, so that its inputs are one 16-byte read.
-template <int GATES, int RT, bool DROPCONNECT, typename T>
+// contraction index 4 (l / 16) + i, so that its inputs are one 16-byte read.  STAGED: some of the new state is parked.
+template <int GATES, int RT, bool DROPCONNECT, bool STAGED, typename T>
 __global__ __launch_bounds__(256)
 void forward_step_kernel(StepParams<T> p) {
   typedef typename Step<T>::Sum A;
@@ -408,9 +408,9 @@ void forward_step_kernel(StepParams<T> p) {
         for (int g = 0; g < 4; ++g) a[g] += run_sum[0][g];
       }
     }
-    finish_unit<GATES, T>(p, n, j, a, in[rt]);
+    finish_unit<GATES, STAGED, T>(p, n, j, a, in[rt]);
   }
-  if (p.copies) copy_staged_states(p, &s_flag);
+  if (STAGED && p.copies) copy_staged_states(p, &s_flag);
 }
 
 // How a step is cut up.
@@ -536,10 +536,12 @@ int launch_step(hipStream_t stream, StepParams<T>& p, const char* name) {
   p.runs = cut.runs; p.row_blocks = cut.row_blocks; p.unit_blocks = cut.unit_blocks; p.quads = cut.quads;
   const dim3 grid((unsigned)cut.row_blocks * cut.unit_blocks * cut.runs);
   ScopedKernelTimer timer(name, stream);
-#define HASTE_LAUNCH_STEP(RT_)                                                                              \
-  if (cut.rt == RT_) {                                                                                      \
-    if (p.dc_mask != nullptr) forward_step_kernel<GATES, RT_, true, T><<<grid, dim3(256), 0, stream>>>(p);  \
-    else forward_step_kernel<GATES, RT_, false, T><<<grid, dim3(256), 0, stream>>>(p);                      \
+#define HASTE_LAUNCH_STEP(RT_)                                                                                     \
+  if (cut.rt == RT_) {                                                                                             \
+    if (p.dc_mask != nullptr && parked) forward_step_kernel<GATES, RT_, true, true, T><<<grid, 256, 0, stream>>>(p); \
+    else if (p.dc_mask != nullptr) forward_step_kernel<GATES, RT_, true, false, T><<<grid, 256, 0, stream>>>(p);     \
+    else if (parked) forward_step_kernel<GATES, RT_, false, true, T><<<grid, 256, 0, stream>>>(p);                   \
+    else forward_step_kernel<GATES, RT_, false, false, T><<<grid, 256, 0, stream>>>(p);                              \
   }
   HASTE_LAUNCH_STEP(1)
   if constexpr (Step<T>::kQuads) {
