@@ -298,21 +298,31 @@ int layer_norm_gru_backward_streamed(hipStream_t stream, int T, int N, int C, in
                                      float* dgamma2, const float* cache2,
                                      const float* zoneout_mask);
 
+// What a pass runs on otherwise: tiles of `rows` batch rows (0: a product a step), `beyond_lds`: whose slices of the weights
+// exceed LDS.
+struct CutOther {
+  int rows;
+  bool beyond_lds;
+};
+
+// Steps and rows for which that is looked at.
+constexpr int kCutMinSteps = 4, kCutMaxRows = 160;
+
 // The recurrence cut along the contraction and the columns (cut_recurrence.h), where it is the faster one: *taken.  Forward
-// with the product x * W (GRU: unless it is there), backward without the products around it.  beyond_lds: see cut_pays.
+// with the product x * W (GRU: unless it is there), backward without the products around it.
 int lstm_forward_cut(hipStream_t stream, int training, int T, int N, int C, int H, const float* W, const float* R,
                      const float* b, const float* x, const float* h, const float* c, float* h_out, float* c_out, float* v,
-                     float zoneout_prob, const float* zoneout_mask, const float* dc_mask, float dc_scale, bool beyond_lds, bool* taken);
+                     float zoneout_prob, const float* zoneout_mask, const float* dc_mask, float dc_scale, const CutOther& other, bool* taken);
 int lstm_backward_cut(hipStream_t stream, int T, int N, int H, const float* R_t, const float* c, const float* c_next,
                       const float* dh_next, const float* dc_next, float* db, float* dh, float* dc, float* v,
-                      const float* zoneout_mask, bool beyond_lds, bool* taken);
+                      const float* zoneout_mask, const CutOther& other, bool* taken);
 int gru_forward_cut(hipStream_t stream, int training, int T, int N, int C, int H, const float* W, const float* R,
                     const float* bx, const float* br, const float* x, const float* h, float* h_out, float* v,
                     float* tmp_Wx, float zoneout_prob, const float* zoneout_mask, const float* dc_mask, float dc_scale,
-                    bool wx_ready, bool beyond_lds, bool* taken);
+                    bool wx_ready, const CutOther& other, bool* taken);
 int gru_backward_cut(hipStream_t stream, int T, int N, int H, const float* R_t, const float* h, const float* v,
                      const float* dh_next, float* dbx, float* dbr, float* dh, float* dp, float* dq,
-                     const float* zoneout_mask, bool beyond_lds, bool* taken);
+                     const float* zoneout_mask, const CutOther& other, bool* taken);
 
 // Bytes of scratch they may ask for on a device of `cus` compute units, whatever its XCDs.
 size_t cut_scratch_bound(int N, int H, int cus);

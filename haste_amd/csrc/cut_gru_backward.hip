@@ -6,9 +6,9 @@ namespace haste_hip {
 
 int gru_backward_cut(hipStream_t stream, int T, int N, int H, const float* R_t, const float* h, const float* v,
                      const float* dh_next, float* dbx, float* dbr, float* dh, float* dp, float* dq,
-                     const float* zoneout_mask, bool beyond_lds, bool* taken) {
+                     const float* zoneout_mask, const CutOther& other, bool* taken) {
   CutPlan cut;
-  HASTE_HIP_PROPAGATE((cut_rule<GruScatterCell, true>(stream, T, N, H, beyond_lds, false, &cut)));
+  HASTE_HIP_PROPAGATE((cut_rule<GruScatterCell, true>(stream, T, N, H, other, false, &cut)));
   *taken = cut.ok;
   if (!cut.ok) return HASTE_HIP_OK;
   GruBwdParams p{};

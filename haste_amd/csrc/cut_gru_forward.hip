@@ -7,9 +7,9 @@ namespace haste_hip {
 int gru_forward_cut(hipStream_t stream, int training, int T, int N, int C, int H, const float* W, const float* R,
                     const float* bx, const float* br, const float* x, const float* h, float* h_out, float* v,
                     float* tmp_Wx, float zoneout_prob, const float* zoneout_mask, const float* dc_mask, float dc_scale,
-                    bool wx_ready, bool beyond_lds, bool* taken) {
+                    bool wx_ready, const CutOther& other, bool* taken) {
   CutPlan cut;
-  HASTE_HIP_PROPAGATE((cut_rule<GruForwardCell, false>(stream, T, N, H, beyond_lds, dc_mask != nullptr, &cut)));
+  HASTE_HIP_PROPAGATE((cut_rule<GruForwardCell, false>(stream, T, N, H, other, dc_mask != nullptr, &cut)));
   *taken = cut.ok;
   if (!cut.ok) return HASTE_HIP_OK;
   if (!wx_ready) HASTE_HIP_PROPAGATE(gemm_f32(stream, false, T * N, 3 * H, C, x, C, W, 3 * H, tmp_Wx, 3 * H, false));

@@ -6,9 +6,9 @@ namespace haste_hip {
 
 int lstm_backward_cut(hipStream_t stream, int T, int N, int H, const float* R_t, const float* c, const float* c_next,
                       const float* dh_next, const float* dc_next, float* db, float* dh, float* dc, float* v,
-                      const float* zoneout_mask, bool beyond_lds, bool* taken) {
+                      const float* zoneout_mask, const CutOther& other, bool* taken) {
   CutPlan cut;
-  HASTE_HIP_PROPAGATE((cut_rule<LstmScatterCell, true>(stream, T, N, H, beyond_lds, false, &cut)));
+  HASTE_HIP_PROPAGATE((cut_rule<LstmScatterCell, true>(stream, T, N, H, other, false, &cut)));
   *taken = cut.ok;
   if (!cut.ok) return HASTE_HIP_OK;
   LstmBwdParams p{};

@@ -6,9 +6,9 @@ namespace haste_hip {
 
 int lstm_forward_cut(hipStream_t stream, int training, int T, int N, int C, int H, const float* W, const float* R,
                      const float* b, const float* x, const float* h, const float* c, float* h_out, float* c_out, float* v,
-                     float zoneout_prob, const float* zoneout_mask, const float* dc_mask, float dc_scale, bool beyond_lds, bool* taken) {
+                     float zoneout_prob, const float* zoneout_mask, const float* dc_mask, float dc_scale, const CutOther& other, bool* taken) {
   CutPlan cut;
-  HASTE_HIP_PROPAGATE((cut_rule<LstmForwardCell, false>(stream, T, N, H, beyond_lds, dc_mask != nullptr, &cut)));
+  HASTE_HIP_PROPAGATE((cut_rule<LstmForwardCell, false>(stream, T, N, H, other, dc_mask != nullptr, &cut)));
   *taken = cut.ok;
   if (!cut.ok) return HASTE_HIP_OK;
   HASTE_HIP_PROPAGATE(gemm_f32(stream, false, T * N, 4 * H, C, x, C, W, 4 * H, v, 4 * H, false));

@@ -1124,48 +1124,66 @@ CutPlan cut_plan(int N, int H, int cus, int xcds) {
   return plan;
 }
 
-// Whether it pays.  `beyond_lds`: the other kernels' slices of the weights exceed LDS (they keep a part in registers and read
-// it at the rate of the fp32 instruction, or stream the weights step by step): always, up to 160 rows.  Otherwise their
-// steps are cheap while a tile of theirs has few rows; here 16 rows cost a whole tile (with the row tiles over 4, 2 or 1 groups).
-// Measured, C = 64, T = 60, the others -> this one, us:
-//   LSTM forward   H = 544  N = 64 276 -> 266   N = 96 291 -> 434   N = 128 534 -> 443
-//                  H = 672  N = 40 277 -> 260   N = 52 380 -> 266   N = 96 408 -> 451   N = 128 648 -> 474
-//                  H = 736  N = 12 212 -> 252   N = 20 297 -> 260   N = 40 412 -> 259   N = 96 647 -> 468
-//                  H = 1056 N = 12 292 -> 337   N = 20 434 -> 337   N = 52 767 -> 531   N = 128 1495 -> 1016
-//       beyond LDS H = 1536 N = 1 347 -> 283    N = 16 364 -> 324   N = 32 596 -> 520   N = 64 1082 -> 702
-//                  H = 2048 N = 1 419 -> 327    N = 16 437 -> 356   N = 32 757 -> 617   N = 64 1380 -> 879
-//   LSTM backward  H = 544  N = 28 307 -> 364   N = 40 375 -> 376   N = 52 415 -> 388   N = 96 503 -> 560   N = 128 754 -> 587
-//       beyond LDS H = 672  N = 6 435 -> 358    N = 28 467 -> 388   N = 64 (H = 640) 487 -> 415   N = 128 899 -> 653
-//                  H = 1024 N = 1 551 -> 410    N = 64 744 -> 555   H = 2048 N = 1 1045 -> 446   N = 16 1275 -> 565   N = 64 2131 -> 1530
-//   GRU forward    H = 672  N = 40 225 -> 256   N = 52 302 -> 256   N = 96 318 -> 447   H = 736 N = 40 234 -> 256   N = 52 333 -> 257
-//                  H = 800  N = 20 171 -> 299   N = 28 319 -> 302   H = 864 N = 12 224 -> 296   N = 20 344 -> 299   N = 96 711 -> 525
-//                  H = 1056 N = 28 435 -> 327   N = 40 362 -> 515   N = 52 589 -> 535   N = 96 629 -> 727   N = 128 1046 -> 911
-//       beyond LDS H = 2048 N = 1 405 -> 310    N = 16 425 -> 337   N = 64 1322 -> 851
-//   GRU backward   H = 544  N = 28 358 -> 364   N = 40 437 -> 374   H = 672 N = 20 371 -> 367  N = 28 424 -> 377   N = 96 543 -> 611
-//                  H = 736  N = 12 359 -> 366   N = 20 405 -> 379   N = 96 812 -> 637
-//       beyond LDS H = 864  N = 6 503 -> 416    N = 52 567 -> 483   H = 2048 N = 1 887 -> 437   N = 64 2195 -> 1514
+// Whether it pays.  Here a step takes a turn per batch tile of a group (the plan's row_tiles: 4, 2 or 1 groups share them,
+// H <= 1024, 1280 and beyond); the others' step grows with the rows of their tiles, which all go at once.  So it does where
+// theirs have many rows for every turn here, and where they stream the weights, always.  Measured, C = 64, T = 60, N rows in
+// tiles of theirs / turns here, the others -> this one, us:
+//   LSTM forward   H =  544  N = 40 8/1 241 -> 262   N = 64 16/1 282 -> 269 (not taken)  N = 96 16/2 293 -> 437  N = 128 64/2 537 -> 447
+//                  H =  640  N = 32 16/1 277 -> 262 (not taken)  N = 52 32/1 345 -> 263  N = 72 32/2 361 -> 436  N = 144 64/3 620 -> 623
+//                  H =  736  N = 12 8/1 220 -> 262   N = 20 16/1 305 -> 265  N = 40 32/1 417 -> 266  N = 96 64/2 645 -> 475
+//                  H = 1024  N = 28 16/1 297 -> 318  N = 48 32/1 447 -> 326  N = 128 64/2 900 -> 604
+//                  H = 1056  N = 16 16/1 305 -> 345  N = 28 32/1 457 -> 343  N = 52 64/2 765 -> 533
+//       beyond LDS H = 1280  N = 12 16/1 381 -> 348
+//                  H = 1536  N = 1 362 -> 284   N = 64 1092 -> 732   N = 128 2048 -> 1407  N = 160 2573 -> 1728
+//                  H = 2048  N = 1 430 -> 337   N = 64 1432 -> 940   N = 128 2458 -> 1790  N = 160 3649 -> 2216
+//   LSTM backward  H =  544  N = 28 4/1 320 -> 372   N = 40 8/1 388 -> 387   N = 52 8/1 428 -> 397   N = 96 16/2 528 -> 570
+//                  H =  608  N = 32 8/1 405 -> 387   N = 64 16/1 587 -> 421  N = 72 16/2 604 -> 558  N = 160 32/3 970 -> 838
+//                  H =  800  N = 72 16/2 691 -> 708  N = 96 32/2 1005 -> 771 N = 160 32/5 1188 -> 1277
+//                  H =  848  N = 160 64/5 1789 -> 1294
+//       beyond LDS H =  640  N = 1 16/1 400 -> 348   N = 72 16/2 524 -> 563  N = 160 32/3 925 -> 854
+//                  H = 1536  N = 1 792 -> 383   N = 64 1840 -> 1167  N = 128 2846 -> 2295  N = 160 3736 -> 2824
+//                  H = 2048  N = 1 1049 -> 455  N = 64 2368 -> 1699  N = 128 3986 -> 3350  N = 160 5343 -> 4130
+//   GRU forward    H =  544  N = 64 16/1 244 -> 267  N = 128 32/2 396 -> 435 H = 672  N = 64 16/1 310 -> 264  N = 96 16/2 323 -> 452
+//                  H =  736  N = 28 8/1 236 -> 266   N = 48 16/1 340 -> 264  N = 72 16/2 351 -> 449  N = 96 64/2 625 -> 455
+//                  H =  832  N = 20 16/1 326 -> 302  N = 40 32/1 433 -> 305  H = 1024 N = 28 16/1 290 -> 302
+//                  H = 1056  N = 28 32/1 441 -> 334
+//       beyond LDS H =  736  N = 144 32/3 566 -> 618
+//                  H = 1056  N = 40 16/2 368 -> 503  N = 52 32/2 594 -> 528  N = 96 32/3 626 -> 737  N = 128 64/4 1048 -> 914
+//                  H = 2048  N = 1 422 -> 323   N = 64 1369 -> 894   N = 160 2938 -> 2059
+//   GRU backward   H =  544  N = 28 4/1 373 -> 375   N = 40 8/1 449 -> 383   N = 96 16/2 619 -> 581  N = 144 32/3 736 -> 775
+//                  H =  672  N = 28 8/1 434 -> 385   N = 80 16/2 510 -> 604  N = 160 32/3 881 -> 892
+//                  H =  736  N = 72 16/2 616 -> 602  N = 160 32/3 988 -> 932
+//       beyond LDS H =  864  N = 8 16/1 527 -> 429   H = 1056 N = 48 16/2 651 -> 710  H = 1152 N = 48 16/2 754 -> 712
+//                  H = 1312  N = 40 16/3 899 -> 753  N = 80 32/5 1340 -> 1270
+//                  H = 2048  N = 1 891 -> 437   N = 64 2223 -> 1553  N = 160 4572 -> 3622
 // Whole passes of three steps are level with the others, of eight 0.65 - 1 of theirs.
-inline bool cut_pays(bool backward, int gates, int T, int N, int H, bool beyond_lds) {
-  if (T < 4 || H <= 512 || N > 160) return false;
-  if (beyond_lds) return true;
-  const bool one_tile_each = N > 48 && N <= 64, many = N > 96;  // on four groups
-  if (backward) {
-    if (gates == 4) return one_tile_each || many || (H > 576 && N > 32);
-    return H <= 576 ? N > 32 : (N > 24 && (H <= 640 || H > 704 || N <= 64 || many));
+inline bool cut_pays(bool backward, int gates, int N, int H, const CutPlan& plan, const CutOther& other) {
+  const int turns = plan.row_tiles;
+  if (other.rows == 0) return true;
+  if (!backward) {
+    if (other.rows > 16 * turns) return gates == 3 || turns <= 2 || H > 608;
+    // as many rows as a turn has: level with them, by how well either fits the size
+    return other.rows == 16 * turns && (other.beyond_lds || (turns == 1 && H > 640 && H <= 960));
   }
-  if (gates == 4) return H > 704 ? N > 16 : (H > 576 && (one_tile_each || many));
-  if (H > 1024) return (N > 16 && N <= 32) || one_tile_each || many;  // (two groups)
-  if (H > 832) return N > 16;
-  return H > 704 ? N > 48 : (H > 640 && one_tile_each);
+  // Their backward steps take longer, these hardly do, least where a group is the whole chip.
+  if (other.rows >= 16 * turns) return true;
+  if (other.rows < (plan.s.span == plan.s.xcds ? 5 : 8) * turns) return false;
+  if (gates == 4) {
+    if (turns == 1) return H > 576 || N > 48;
+    return other.rows > 16 || (H > 576 && (H <= 632 || H > 656));
+  }
+  if (turns == 1) return true;
+  if (other.rows > 16) return H > 576;
+  return H <= 656 || (H > 720 && H <= 1024) || H > 1100;
 }
 
 // `masked`: the weights are multiplied with a DropConnect mask first, which takes room for them.
 template <class Cell, bool BACK>
-int cut_rule(hipStream_t stream, int T, int N, int H, bool beyond_lds, bool masked, CutPlan* plan) {
+int cut_rule(hipStream_t stream, int T, int N, int H, const CutOther& other, bool masked, CutPlan* plan) {
   *plan = CutPlan();
-  if (!cut_pays(BACK, Cell::kGates, T, N, H, beyond_lds)) return HASTE_HIP_OK;
+  if (T < kCutMinSteps || H <= 512 || N > kCutMaxRows) return HASTE_HIP_OK;
   CutPlan found = cut_plan<Cell, BACK>(N, H, device_cu_count(), device_xcd_count());
-  if (!found.ok) return HASTE_HIP_OK;
+  if (!found.ok || !cut_pays(BACK, Cell::kGates, N, H, found, other)) return HASTE_HIP_OK;
   if (masked) found.weight_floats = ((size_t)Cell::kGates * H * H + 63) / 64 * 64;
   bool room = false;
   HASTE_HIP_PROPAGATE(workspace_has_room(stream, found.bytes(), &room));

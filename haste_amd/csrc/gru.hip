@@ -760,7 +760,7 @@ int gru_forward_impl(hipStream_t stream, int training, int T, int N, int C, int 
   HASTE_HIP_REQUIRE(!half_io || (half_product && half_forward(tile, H)));
   bool taken = false;
   HASTE_HIP_PROPAGATE(gru_forward_cut(stream, training, T, N, C, H, W, R, bx, br, x, h, h_out, v, tmp_Wx, zoneout_prob,
-                                      zoneout_mask, dc_mask, dc_scale, wx_ready, !tile.ok || tile.reg_groups > 0, &taken));
+                                      zoneout_mask, dc_mask, dc_scale, wx_ready, {tile.ok ? tile.nb : 0, tile.reg_groups > 0}, &taken));
   if (taken) return HASTE_HIP_OK;
   // No slice of R fits a CU: stream R from HBM every step instead.
   if (!tile.ok)
@@ -887,7 +887,7 @@ int gru_backward_impl(hipStream_t stream, int T, int N, int C, int H,
   HASTE_HIP_REQUIRE(!half_io || (half_product && !products && scattered_backward(tile, H)));
   bool taken = false;
   HASTE_HIP_PROPAGATE(gru_backward_cut(stream, T, N, H, R_t, h, v, dh_next, dbx, dbr, dh, dp, dq, zoneout_mask,
-                                       !tile.ok || tile.reg_groups > 0, &taken));
+                                       {tile.ok ? tile.nb : 0, tile.reg_groups > 0}, &taken));
   if (taken) return finish();
   if (!tile.ok)
     return planned_pass() != nullptr ? HASTE_HIP_OK : gru_backward_streamed(stream, T, N, C, H, W_t, R_t, x_t, h, v, dh_next, dx, dW, dR, dbx,

@@ -726,7 +726,7 @@ int lstm_forward_impl(hipStream_t stream, int training, int T, int N, int C, int
   const ForwardTile tile = pick_forward_tile(4, N, H, 0, kWorkgroupLdsBytes, false, 2);
   bool taken = false;
   HASTE_HIP_PROPAGATE(lstm_forward_cut(stream, training, T, N, C, H, W, R, b, x, h, c, h_out, c_out, v, zoneout_prob,
-                                       zoneout_mask, dc_mask, dc_scale, !tile.ok || tile.reg_groups > 0, &taken));
+                                       zoneout_mask, dc_mask, dc_scale, {tile.ok ? tile.nb : 0, tile.reg_groups > 0}, &taken));
   if (taken) return HASTE_HIP_OK;
   // No slice of R fits a CU: stream R from HBM every step instead.
   if (!tile.ok)
@@ -834,7 +834,7 @@ int lstm_backward_impl(hipStream_t stream, int T, int N, int C, int H,
   const BackwardTile tile = pick_backward_tile(4 * H, N, H, 4 * 16, 0, true);
   bool taken = false;
   HASTE_HIP_PROPAGATE(lstm_backward_cut(stream, T, N, H, R_t, c, c_next, dh_next, dc_next, db, dh, dc, v, zoneout_mask,
-                                        !tile.ok || tile.reg_groups > 0, &taken));
+                                        {tile.ok ? tile.nb : 0, tile.reg_groups > 0}, &taken));
   if (taken) return products();
   if (!tile.ok)
     return planned_pass() != nullptr ? HASTE_HIP_OK : lstm_backward_streamed(stream, T, N, C, H, W_t, R_t, x_t, h, c, c_next, dh_next, dc_next,

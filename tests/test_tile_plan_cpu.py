@@ -203,3 +203,14 @@ def test_the_tests_of_the_cut_recurrences_reach_them():
                 assert rc == 0 and few[0] != 3, (gates, backward, N, H)
     assert {(b, xcds) for b, xcds, _ in seen} == {(b, xcds) for b in (0, 1) for xcds in (2, 4, 8)}
     assert {(b, tiles) for b, _, tiles in seen} == {(b, tiles) for b in (0, 1) for tiles in (1, 2, 3)}
+
+
+@pytest.mark.parametrize("gates,backward,N,H,cut", [
+    (4, 0, 128, 544, 1), (4, 0, 64, 544, 0), (4, 0, 40, 672, 1), (4, 0, 28, 1024, 0), (4, 0, 160, 2048, 1),
+    (3, 0, 28, 800, 1), (3, 0, 72, 736, 0), (3, 0, 144, 800, 0), (3, 0, 40, 1056, 0), (3, 0, 52, 1056, 1), (3, 0, 160, 1536, 1),
+    (4, 1, 96, 544, 0), (4, 1, 72, 640, 0), (4, 1, 72, 624, 1), (4, 1, 160, 848, 1), (4, 1, 160, 2048, 1),
+    (3, 1, 144, 528, 0), (3, 1, 80, 672, 0), (3, 1, 48, 1056, 0), (3, 1, 40, 1312, 1)])
+def test_where_the_cut_recurrences_are_taken(gates, backward, N, H, cut):
+    """Where the batch tiles of the other kernels have many rows for every batch tile a group goes through, as measured."""
+    rc, plan = _plan_pass(hlib.load(), 256, 8, gates, 4, backward, 60, N, 64, H)
+    assert rc == 0 and (plan[0] == 3 and plan[3] > 32) == bool(cut), plan
