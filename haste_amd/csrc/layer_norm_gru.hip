@@ -741,9 +741,10 @@ int haste_hip_layer_norm_gru_backward_f32(int steps, int batch_size, int input_s
   // per row: 9 column-sum accumulators of 16 floats (or the partial tiles, whichever is more) + 4 sums
   const BackwardTile tile = pick_backward_tile(ln_gru_backward_k(H), N, H, 9 * 16, 4, true);
   // As in layer_norm_lstm.hip (us a step kept / streamed: H = 896, N = 8 14.9 / 13.7, H = 1408 N = 8 19.8 / 17.3 and
-  // N = 48 33.9 / 31.8, H = 1280 N = 128 59 / 44; but H = 1024, N = 16 14.0 / 15.2 and N = 128 27 / 37).
+  // N = 48 33.9 / 31.8, two batch tiles H = 1280 N = 128 58 / 44 and N = 64 34 / 31; but H = 1024, N = 16 14.0 / 15.2 and
+  // N = 128 27 / 37, three H = 1280 N = 48 23.5 / 28.8 and N = 96 36.8 / 39.3).
   bool streamed = !tile.ok;
-  if (tile.ok && tile.reg_groups > 0 && ((N <= 8 && H > 880) || (N > 32 && H > 1240)))
+  if (tile.ok && tile.reg_groups > 0 && ((N <= 8 && H > 880) || (N > 32 && H > (tile.gy <= 2 ? 1240 : 1376))))
     HASTE_HIP_PROPAGATE(workspace_has_room(stream, layer_norm_streamed_bytes(3, true, T, N, C, H), &streamed));
   if (streamed)
     return layer_norm_gru_backward_streamed(stream, T, N, C, H, W_t, R_t, x_t, h, v, dh_new, dx, dW, dR,

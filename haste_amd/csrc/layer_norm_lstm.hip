@@ -950,9 +950,9 @@ int haste_hip_layer_norm_lstm_backward_f32(int steps, int batch_size, int input_
   // per row: 10 column-sum accumulators of 16 floats (or the partial tiles, whichever is more) + 10 sums
   const BackwardTile tile = pick_backward_tile(4 * H, N, H, 10 * 16, 10, true);
   // A large slice with few rows: streaming R is faster (us a step kept / streamed: H = 1024, N = 8 19.4 / 17.1, N = 16
-  // 19.3 / 18.4, N = 32 21.1 / 23.5; H = 1056, N = 12 22.8 / 20.7; H = 896, N = 8 15.2 / 17.0).
+  // 19.3 / 18.4, N = 32 21.1 / 23.5; H = 1056, N = 12 22.8 / 20.7; but H = 896, N = 8 15.2 / 17.0, H = 976 N = 8 19.3 / 20.9).
   bool streamed = !tile.ok;
-  if (tile.ok && tile.reg_groups > 0 && N <= 16 && H > 960)
+  if (tile.ok && tile.reg_groups > 0 && N <= 16 && H > 1000)
     HASTE_HIP_PROPAGATE(workspace_has_room(stream, layer_norm_streamed_bytes(4, true, T, N, C, H), &streamed));
   if (streamed)
     return layer_norm_lstm_backward_streamed(stream, T, N, C, H, W_t, R_t, x_t, h, c, dh_new, dc_new,

@@ -229,6 +229,22 @@ int step_product<float>(hipStream_t s, int M, int N, int K, const float* A, cons
   return HASTE_HIP_OK;
 }
 
+// The same for a kernel that has a workgroup per row (a layer-norm cell's forward step).  In double the chunks of 33 to 64 rows
+// come from a kernel that walks the rows' operands in each of 16 columns' workgroups, slower than whole tiles and one more
+// launch from some width on; and with fewer rows and many units their sum is bound by one CU a row.  (LSTM forward, us a step
+// with chunks / whole: N = 40, H = 512 22 / 24, H = 640 30 / 27, H = 2048 122 / 71, H = 4096 350 / 197; N = 32, H = 1024
+// 34 / 34; GRU N = 20, H = 3072 93 / 104, H = 3500 146 / 121.)
+template <typename T>
+int row_product(hipStream_t s, int M, int N, int K, const T* A, const T* B, T* out, size_t scratch_offset, StepProduct<T>* p) {
+  if (!std::is_same<T, double>::value || (M > 32 ? K < 640 : M <= 16 || K <= 3072))
+    return step_product<T>(s, M, N, K, A, B, out, scratch_offset, p);
+  HASTE_HIP_PROPAGATE(gemm(s, false, M, N, K, A, K, B, N, out, N, false, scratch_offset));
+  p->base = out;
+  p->chunks = 1;
+  p->stride = 0;
+  return HASTE_HIP_OK;
+}
+
 // dh += (pending chunks): the recurrent contribution a reverse step leaves for the next
 // step's pointwise kernel, added for real after the last step.
 template <typename T>
@@ -1429,7 +1445,7 @@ int ln_lstm_forward_steps(hipStream_t stream, int training, int steps, int N, in
     T* rh_t = act_Rh + (size_t)t * N4H;
     if (rows_held(H)) {
       StepProduct<T> prod;
-      HASTE_HIP_PROPAGATE(step_product<T>(stream, N, 4 * H, H, h_t, R, rh_t, sc.gemm_offset(), &prod));
+      HASTE_HIP_PROPAGATE(row_product<T>(stream, N, 4 * H, H, h_t, R, rh_t, sc.gemm_offset(), &prod));
       LnLstmForwardRow<T> row;
       row.training = training; row.H = H;
       row.rh = rh_t; row.gamma2 = gamma2; row.cache2 = cache2 ? cache2 + (size_t)t * N * 2 : nullptr;
@@ -1554,7 +1570,7 @@ int ln_gru_forward_steps(hipStream_t stream, int training, int steps, int N, int
     T* rh_t = act_Rh + (size_t)t * N3H;
     if (rows_held(H)) {
       StepProduct<T> prod;
-      HASTE_HIP_PROPAGATE(step_product<T>(stream, N, 3 * H, H, h_t, R, rh_t, sc.gemm_offset(), &prod));
+      HASTE_HIP_PROPAGATE(row_product<T>(stream, N, 3 * H, H, h_t, R, rh_t, sc.gemm_offset(), &prod));
       LnGruForwardRow<T> row;
       row.training = training; row.H = H;
       row.rh = rh_t; row.gamma2 = gamma2; row.cache2 = cache2 ? cache2 + (size_t)t * N * 2 : nullptr;

@@ -52,9 +52,10 @@ def test_f64_layer_norm_cells(double_precision, T, N, C, H, zoneout):
     test_gpu_layer_norm_cells.test_layer_norm_gru_training_forward_backward(T, N, C, H, zoneout)
 
 
-# A workgroup a row: one wavefront and a unit more, 1, 2 and 4 units a thread at their ends, and a row that is not held.
+# A workgroup a row: one wavefront and a unit more, 1, 2 and 4 units a thread at their ends, and a row that is not held;
+# the product in chunks and, with more than 32 and 16 rows of many units, whole.
 @pytest.mark.parametrize("T,N,C,H", [(2, 3, 4, 64), (2, 3, 4, 65), (3, 2, 4, 1024), (2, 2, 4, 1025), (2, 2, 4, 2050),
-                                     (2, 2, 4, 4096), (2, 2, 4, 4100)])
+                                     (2, 2, 4, 4096), (2, 2, 4, 4100), (2, 33, 4, 639), (2, 33, 4, 640), (2, 17, 4, 3073)])
 def test_f64_layer_norm_cells_row_by_row(double_precision, T, N, C, H):
     test_f64_layer_norm_cells(None, T, N, C, H, 0.3)
 
