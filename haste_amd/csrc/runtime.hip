@@ -696,8 +696,6 @@ size_t haste_hip_workspace_bytes(int time_steps, int batch_size, int input_size,
   // Backward recurrences of 4-row tiles in scattered form (H <= 512): two tiles of pieces per
   // tile of 4 rows, [owners][up to 32 producers][64].
   if (H <= 512) b += (N / 4 + 2) * 2 * (H / 16 + 1) * 32 * 64 * sizeof(float);
-  // Recurrences cut along the contraction and the columns.
-  if (H > 512 && H <= 8192 && N <= 4096) b += cut_scratch_bound(batch_size, hidden_size, (int)cus);
   // Step-wise regime (any scalar type up to 8 bytes): the step's product [N, 4H], a scaled
   // copy of R, column sums in at most 128 chunks, row statistics of all steps, two [N, H]
   // buffers; the stand-alone layer norm's column sums (two workgroups per CU, two rows each).
@@ -709,6 +707,11 @@ size_t haste_hip_workspace_bytes(int time_steps, int batch_size, int input_size,
   // workgroup, at most about five workgroups per CU: larger batches also use the room
   // of the GEMM and the exchange tiles, which such a step does not touch), and the staged states.
   b += 64 * 2 * 8 * (H / 16 + 1) * 64 * sizeof(float) + 2 * 8 * H * sizeof(float) + 256;
+  // Recurrences cut along the contraction and the columns have the scratch to themselves.
+  if (time_steps >= kCutMinSteps && batch_size <= kCutMaxRows && H > 512 && H <= 8192) {
+    const size_t cut = cut_scratch_bound(batch_size, hidden_size, (int)cus);
+    if (cut > b) b = cut;
+  }
   return kControlBytes + 4096 + (b + 255) / 256 * 256;
 }
 

@@ -214,3 +214,18 @@ def test_where_the_cut_recurrences_are_taken(gates, backward, N, H, cut):
     """Where the batch tiles of the other kernels have many rows for every batch tile a group goes through, as measured."""
     rc, plan = _plan_pass(hlib.load(), 256, 8, gates, 4, backward, 60, N, 64, H)
     assert rc == 0 and (plan[0] == 3 and plan[3] > 32) == bool(cut), plan
+
+
+def test_workspace_bytes_of_the_cut_recurrences():
+    """Nothing else is in use beside them, and calls of more rows never take them: they do not add to the bound, and a buffer
+    of its size is enough for them."""
+    lib = hlib.load()
+    lib.haste_hip_workspace_bytes.restype = ctypes.c_size_t
+    assert lib.haste_hip_workspace_bytes(50, 64, 512, 2048) < 380 << 20
+    assert lib.haste_hip_workspace_bytes(4, 200, 64, 2048) < 440 << 20
+    for gates in (3, 4):
+        for backward in (0, 1):
+            for N, H in [(1, 1024), (64, 2048), (160, 1408), (160, 2048), (20, 736)]:
+                rc, plan = _plan_pass(lib, 256, 8, gates, 4, backward, 60, N, 64, H)
+                lent = lib.haste_hip_workspace_bytes(60, N, 64, H)
+                assert rc == 0 and _plan_pass(lib, 256, 8, gates, 4, backward, 60, N, 64, H, lent)[1][:6] == plan[:6]
