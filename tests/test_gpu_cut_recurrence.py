@@ -109,21 +109,52 @@ def test_states_that_are_no_numbers():
 
 
 @pytest.mark.parametrize("N,H", [(50, 700), (20, 1300)])
-def test_dropconnect_and_run_to_run(N, H):
-    """The masked weights give what R masked beforehand gives, and a pass what it gave before, bit for bit."""
+@pytest.mark.parametrize("cell,training", [("lstm", False), ("lstm", True), ("gru", False), ("gru", True)])
+def test_dropconnect_and_run_to_run(cell, training, N, H):
+    """The masked weights give what R masked beforehand gives, and a pass what it gave before, bit for bit, also where the
+    lent memory is what is stated for the sizes."""
     import torch
     from haste_amd import ops
     T, C = 5, 15
-    p = problem(77 + N, T, N, C, H, 4, 0.0)
+    zoneout = 0.2 if training else 0.0
+    p = problem(77 + N, T, N, C, H, 4 if cell == "lstm" else 3, zoneout)
     keep = (np.random.default_rng(N).uniform(size=p["R"].shape) >= 0.3).astype(np.float64)
     scale = 2.0
-    none = torch.empty(0, device="cuda")
-    first = (dev(p["x"]), dev(p["h0"]), dev(p["c0"]), dev(p["W"]))
-    a = ops.lstm_forward(False, 0.0, *first, dev(p["R"]), dev(p["b"]), none, dev(keep), scale)
-    b = ops.lstm_forward(False, 0.0, *first, dev(p["R"] * keep * scale), dev(p["b"]), none)
-    again = ops.lstm_forward(False, 0.0, *first, dev(p["R"]), dev(p["b"]), none, dev(keep), scale)
-    assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
-    assert torch.equal(a[0], again[0]) and torch.equal(a[1], again[1])
+    mask = dev(p["mask"]) if zoneout else torch.empty(0, device="cuda")
+    x, h0, c0, W, b, b2 = (dev(p[k]) for k in ("x", "h0", "c0", "W", "b", "b2"))
+
+    def run(R, *dropconnect):
+        if cell == "lstm":
+            return ops.lstm_forward(training, zoneout, x, h0, c0, W, R, b, mask, *dropconnect)
+        out = ops.gru_forward(training, zoneout, x, h0, W, R, b, b2, mask, *dropconnect)
+        return out if training else out[:1]  # (the second one is written in training only)
+
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        masked = (dev(p["R"]), dev(keep), scale)
+        want = run(dev(p["R"] * keep * scale))
+        first, again = run(*masked), run(*masked)
+        lent = torch.empty(ops.workspace_bytes(T, N, C, H), dtype=torch.uint8, device="cuda")
+        try:
+            ops.set_workspace(lent)
+            in_lent = run(*masked)
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=stream):
+                captured = run(*masked)
+            replays = []
+            for _ in range(3):
+                for t in captured:
+                    t.zero_()
+                graph.replay()
+                replays.append([t.clone() for t in captured])
+            stream.synchronize()
+            ops.stream_status()
+        finally:
+            ops.set_workspace(None)
+    states = 2 if cell == "lstm" else 1  # (the LSTM's third one is scratch where it does not train)
+    for got in [first, again, in_lent] + replays:
+        assert all(torch.equal(a, b) for a, b in zip(got[:None if training else states], want))
 
 
 def test_graph_replay():
