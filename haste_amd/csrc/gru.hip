@@ -20,12 +20,13 @@ namespace {
 // which a single tile of 2*NB rows cannot do.
 // REG > 0 (tiles of 16 rows and more): the slice exceeds LDS; every wavefront keeps the first REG
 // k-groups of its share of the contraction in registers (tall_tile_product).
-// HALF (4-row tiles): the step's product on the half matrix cores, for widened half tensors.
+// HALF (4-row tiles): the step's product on the half matrix cores, for widened half tensors.  HALF_IO: h_out, v and
+// zoneout_mask are half tensors (told apart at run time every step is 2 - 6 % longer: N = 16, H = 256 0.87 -> 0.91 us).
 // XSG > 0 (4-row tiles, 16 units per workgroup): the kernel also computes the input projection
 // x[t] * W beside its waits (see InputProjection): the z and r columns into the accumulators of
 // the recurrent product, the candidate gate's -- which needs x*W and h*R apart -- into a tile of
 // its own, which rides behind the slice's three in the partial tiles (rows of 64 columns).
-template <int NB, int CT, int HS, int SETS, int REG = 0, bool HALF = false, int XSG = 0>
+template <int NB, int CT, int HS, int SETS, int REG = 0, bool HALF = false, int XSG = 0, bool HALF_IO = false>
 __global__ __launch_bounds__(256 * SETS, 1)
 void gru_forward_kernel(GruFwdParams p) {
   static_assert(!HALF || (NB == 4 && REG == 0), "half product: 4-row tiles");
@@ -166,7 +167,7 @@ void gru_forward_kernel(GruFwdParams p) {
       }
       if (zoneout && p.training) {
         const size_t at = (size_t)tt * NH + row * H + unit;
-        if (HALF && p.half_io) mk_next[pp] = (float)reinterpret_cast<const _Float16*>(p.zoneout_mask)[at];
+        if constexpr (HALF_IO) mk_next[pp] = (float)reinterpret_cast<const _Float16*>(p.zoneout_mask)[at];
         else mk_next[pp] = p.zoneout_mask[at];
       }
     }
@@ -256,13 +257,17 @@ void gru_forward_kernel(GruFwdParams p) {
       if (act[pp]) {
         const size_t v_at = ((size_t)t * N + pn[pp]) * 4 * H + pj[pp];
         const size_t h_at = (size_t)t * NH + (size_t)pn[pp] * H + pj[pp];
-        if (HALF && p.half_io) {
-          if (p.training) {
-            _Float16* vt = reinterpret_cast<_Float16*>(p.v) + v_at;
+        if constexpr (HALF_IO) {
+          // (Two sets: behind a condition that always holds, so that the compiler keeps this in a block of its own; as part of
+          // the step's code N = 64, H = 512 takes 1.5 % longer, N = 16, H = 256 with one set 3 % less.)
+          if (SETS == 1 || p.h_out != nullptr) {
+            if (p.training) {
+              _Float16* vt = reinterpret_cast<_Float16*>(p.v) + v_at;
 #pragma unroll
-            for (int g = 0; g < 4; ++g) vt[g * H] = (_Float16)saved[pp][g];
+              for (int g = 0; g < 4; ++g) vt[g * H] = (_Float16)saved[pp][g];
+            }
+            reinterpret_cast<_Float16*>(p.h_out)[h_at] = (_Float16)h_prev[pp];
           }
-          reinterpret_cast<_Float16*>(p.h_out)[h_at] = (_Float16)h_prev[pp];
           continue;
         }
         if (p.training) {
@@ -807,7 +812,6 @@ int gru_forward_impl(hipStream_t stream, int training, int T, int N, int C, int 
   p.zoneout_prob = zoneout_prob; p.zoneout_mask = zoneout_mask;
   p.dc_mask = dc_mask; p.dc_scale = dc_scale;
   p.xh = ws.scratch;
-  p.half_io = half_io;
   if (split_rows > 0)
     return launch_split_forward<GruForwardCell>("gru_forward_recurrence", stream, ws, split_rows, p);
   LaunchPlan plan;
@@ -834,6 +838,9 @@ int gru_forward_impl(hipStream_t stream, int training, int T, int N, int C, int 
 #undef HASTE_LAUNCH_FWD_RESIDENT
   if (tile.reg_groups > 0) return HASTE_HIP_ERROR_UNSUPPORTED_SIZE;
 #define HASTE_LAUNCH_FWD_PAIRED(CT_, HS_)                                                     \
+  if (paired && tile.hs == HS_ && half_io)                                                    \
+    return launch_persistent("gru_forward_recurrence", gru_forward_kernel<4, CT_, HS_, 2, 0, true, 0, true>, \
+                             plan, p, stream);                                                \
   if (paired && tile.hs == HS_ && half_product)                                               \
     return launch_persistent("gru_forward_recurrence", gru_forward_kernel<4, CT_, HS_, 2, 0, true>, \
                              plan, p, stream);                                                \
@@ -847,6 +854,9 @@ int gru_forward_impl(hipStream_t stream, int training, int T, int N, int C, int 
     return launch_persistent("gru_forward_recurrence", gru_forward_kernel<NB_, CT_, HS_, 1>,  \
                              plan, p, stream);
 #define HASTE_LAUNCH_FWD_HALF(CT_, HS_)                                                             \
+  if (half_io && tile.nb == 4 && tile.hs == HS_)                                                    \
+    return launch_persistent("gru_forward_recurrence", gru_forward_kernel<4, CT_, HS_, 1, 0, true, 0, true>, \
+                             plan, p, stream);                                                      \
   if (half_product && tile.nb == 4 && tile.hs == HS_)                                               \
     return launch_persistent("gru_forward_recurrence", gru_forward_kernel<4, CT_, HS_, 1, 0, true>, \
                              plan, p, stream);

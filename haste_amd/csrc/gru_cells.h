@@ -24,7 +24,6 @@ struct GruFwdParams {
   float dc_scale;
   float* xh;             // polled exchange tiles of h: [batch tiles][4][Kpad/4][NB][4]
   LaunchShape ls;
-  int half_io;           // (kernels with a product on the half matrix cores) h_out, v and zoneout_mask are in half
 };
 
 struct GruBwdParams {
