@@ -52,7 +52,7 @@ __device__ __forceinline__ uint4_t pack8(float4_t lo, float4_t hi) {
 
 // One 128 x 128 tile over k in [k_begin, k_end); K % 8 == 0, rows 16-byte aligned.  WAVES = 4: 64 x 64 of it a
 // wavefront, the fewest reads of LDS; 8: 64 x 32, so that a SIMD has two wavefronts where a CU has one workgroup.
-template <bool A_FLOAT, int WAVES>
+template <bool A_FLOAT, int WAVES, bool RANGES>
 __global__ __launch_bounds__(64 * WAVES, 2)
 void gemm_half_nt_kernel(int M, int N, int K, const void* __restrict__ A, int lda,
                          const half_t* __restrict__ Bt, int ldb, float* __restrict__ C, int ldc,
@@ -60,10 +60,10 @@ void gemm_half_nt_kernel(int M, int N, int K, const void* __restrict__ A, int ld
                          float* __restrict__ partial) {
   __shared__ __attribute__((aligned(16))) uint4_t lds[2][2][kTileChunks];  // [buffer][A, B][chunk]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  // Workgroups go to the XCDs in turn.  Short pieces: each XCD is given a range of the work, tiles that share rows
-  // of A.  Long ones: as they come, which gives an XCD tiles of many rows and few columns (4096^3 188 -> 172 us).
+  // Workgroups go to the XCDs in turn.  RANGES: each XCD is given a range of the work, tiles that share rows
+  // of A.  Otherwise as they come, which gives an XCD tiles of many rows and few columns.
   const int xcd = blockIdx.x & 7, each = gridDim.x >> 3, rest = gridDim.x & 7;
-  const int work = WAVES == 8 ? xcd * each + (xcd < rest ? xcd : rest) + (blockIdx.x >> 3) : blockIdx.x;
+  const int work = RANGES ? xcd * each + (xcd < rest ? xcd : rest) + (blockIdx.x >> 3) : blockIdx.x;
   const int piece = work / tiles, tile = work % tiles;
   const int m0 = (tile / tiles_n) * QM, n0 = (tile % tiles_n) * QN;
   constexpr int WCOLS = WAVES / 2, NJ = 4 / WCOLS;  // wavefronts side by side, 32-column blocks of one
@@ -320,13 +320,20 @@ int gemm_half_nt(hipStream_t stream, bool a_float, int M, int N, int K, const vo
   // (us with 4 / 8 wavefronts: 6400 x 1536 x 512 26.4 / 23.6, 6400 x 512 x 1536 26.2 / 23.3, 512 x 1536 x 6400 in pieces
   // of 1600 31.4 / 28.2, 12800 x 1536 x 512 43.6 / 35.5; 1024 x 3072 x 3200 43.5 / 44.8, 4096^3 172 / 186).
   const bool eight = per <= 2048;
-#define HASTE_LAUNCH_NT(A_FLOAT_, WAVES_)                                                                       \
-  gemm_half_nt_kernel<A_FLOAT_, WAVES_><<<grid, dim3(64 * WAVES_), 0, stream>>>(                                \
+  // Ranges where a row of tiles is short: all of B stays in an XCD's L2, and A is read once.  With more columns B goes
+  // through it for every few rows; and short pieces of very many tiles are bound by writing C.  (us, ranges / as they come:
+  // 25600 x 768 x 512 32 / 42, fp32 A 38 / 60, 12800 x 1536 x 512 33 / 36; 8192 x 4096 x 1024 113 / 90, 25600 x 3072 x 512
+  // 154 / 127; 51200 x 1536 x 64 70 / 55. Four wavefronts: 4096^3 172 as they come, 188 in ranges.)
+  const bool ranges = eight && (per <= 64 || tiles_n <= 20) && (per > 256 || tiles <= 2400);
+#define HASTE_LAUNCH_NT(A_FLOAT_, WAVES_, RANGES_)                                                              \
+  gemm_half_nt_kernel<A_FLOAT_, WAVES_, RANGES_><<<grid, dim3(64 * WAVES_), 0, stream>>>(                       \
       M, N, K, A, lda, b, ldb, C, ldc, accumulate ? 1 : 0, tiles_n, tiles, per, part)
-  if (a_float && eight) HASTE_LAUNCH_NT(true, 8);
-  else if (a_float) HASTE_LAUNCH_NT(true, 4);
-  else if (eight) HASTE_LAUNCH_NT(false, 8);
-  else HASTE_LAUNCH_NT(false, 4);
+  if (a_float && ranges) HASTE_LAUNCH_NT(true, 8, true);
+  else if (a_float && eight) HASTE_LAUNCH_NT(true, 8, false);
+  else if (a_float) HASTE_LAUNCH_NT(true, 4, false);
+  else if (ranges) HASTE_LAUNCH_NT(false, 8, true);
+  else if (eight) HASTE_LAUNCH_NT(false, 8, false);
+  else HASTE_LAUNCH_NT(false, 4, false);
 #undef HASTE_LAUNCH_NT
   HASTE_HIP_TRY(hipGetLastError());
   if (pieces > 1) {
