@@ -208,11 +208,16 @@ def test_f16_gru_with_a_lent_workspace():
 @pytest.mark.parametrize("a_float", [False, True])
 @pytest.mark.parametrize("accumulate", [False, True])
 @pytest.mark.parametrize("M,N,K", [(1, 1, 8), (37, 53, 24), (128, 128, 64), (130, 257, 200), (300, 100, 1000),
-                                   (64, 1536, 512), (512, 200, 6400), (1000, 512, 1536)])
+                                   (64, 1536, 512), (512, 200, 6400), (1000, 512, 1536),
+                                   # rows of more than 20 tiles, in short and longer pieces and cut; more than 2400
+                                   # tiles; one piece beyond 2048 k
+                                   (130, 2700, 64), (130, 2700, 136), (130, 2700, 800), (38500, 1000, 72),
+                                   (1500, 2050, 2056)])
 def test_f16_gemm_nt(M, N, K, accumulate, a_float):
     """The half GRU's product kernel, C (+)= A * Bt^T in fp32 from half operands (A also from
     fp32, rounded as it is read), against numpy on the same half values: whole and ragged tiles,
-    tails of K, products cut along K."""
+    tails of K, products cut along K, tiles given to the XCDs in ranges and as they come, either
+    number of wavefronts."""
     from haste_amd import lib as hlib
     import torch
     r = np.random.default_rng(M + 3 * N + 7 * K)
